@@ -5,8 +5,8 @@
 // the traversal stack, stays bounded.  The collapse pulls grandchildren up
 // by largest surface area until a node has four children (Wald et al.,
 // "Getting rid of packets", 2008), so a node fetch is one 128-byte line that
-// tests four boxes.  Child boxes are widened by two ulps outward so the
-// kernel's conservative slab test never drops a triangle the watertight
+// tests four boxes.  Child boxes are widened outward by OMV_BOX_PAD_ULPS so
+// the kernel's conservative slab test never drops a triangle the watertight
 // test would hit.
 #include "bvh.h"
 
@@ -35,8 +35,8 @@ inline float halfArea(const float lo[3], const float hi[3]) {
     float d0 = std::max(0.0f, hi[0] - lo[0]), d1 = std::max(0.0f, hi[1] - lo[1]), d2 = std::max(0.0f, hi[2] - lo[2]);
     return d0 * d1 + d1 * d2 + d2 * d0;
 }
-inline float padDown(float v) { return std::nextafter(std::nextafter(v, -INFINITY), -INFINITY); }
-inline float padUp(float v) { return std::nextafter(std::nextafter(v, INFINITY), INFINITY); }
+inline float padDown(float v) { for (int k = 0; k < OMV_BOX_PAD_ULPS; ++k) v = std::nextafter(v, -INFINITY); return v; }
+inline float padUp(float v) { for (int k = 0; k < OMV_BOX_PAD_ULPS; ++k) v = std::nextafter(v, INFINITY); return v; }
 
 struct Builder {
     const std::vector<BuildBox>& boxes;

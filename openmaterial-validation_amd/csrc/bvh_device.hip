@@ -17,7 +17,7 @@
 //      level per launch: a node takes its binary node's two children and
 //      keeps replacing the largest-area one by its children until it has
 //      four; subtrees of <= leafMax triangles become leaves (their triangles
-//      are contiguous in sorted order); child boxes widened two ulps outward,
+//      are contiguous in sorted order); child boxes widened outward,
 //      as the host builder does;
 //   6. triangle records (v0 + id, v1, v2) in sorted order.
 //
@@ -38,8 +38,8 @@ constexpr int kChunk = 256;          // keys per sort lane
 constexpr int kBlock = 256;
 constexpr uint32_t kLeafBit = 0x80000000u;
 
-__device__ inline float padDown(float v) { return nextafterf(nextafterf(v, -INFINITY), -INFINITY); }
-__device__ inline float padUp(float v) { return nextafterf(nextafterf(v, INFINITY), INFINITY); }
+__device__ inline float padDown(float v) { for (int k = 0; k < OMV_BOX_PAD_ULPS; ++k) v = nextafterf(v, -INFINITY); return v; }
+__device__ inline float padUp(float v) { for (int k = 0; k < OMV_BOX_PAD_ULPS; ++k) v = nextafterf(v, INFINITY); return v; }
 
 // 1. triangle boxes and centroids; block partials of the centroid bounds
 __global__ void lbBoxes(const float* __restrict__ vtx, uint32_t vtxOff, uint32_t stride, const uint32_t* __restrict__ faces,

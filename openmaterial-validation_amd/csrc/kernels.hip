@@ -164,8 +164,8 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_fc_kernel(OmvSceneView S, omv_c
     const uint32_t gthreads = gridDim.x * blockDim.x;
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     Stack st;
-    st.init(gstack, gtid, gthreads);
-    Counters cnt; cnt.nodes = 0; cnt.tris = 0; cnt.overflow = 0;
+    st.init(gstack, gthreads);
+    Counters cnt; cnt.zero();
     uint32_t rays = 0, camRays = 0;
     const uint64_t npix = (uint64_t)cam.width * cam.height;
     const bool fcDensity = S.fc_subject == OMV_FC_MD || S.fc_subject == OMV_FC_SG;

@@ -20,6 +20,7 @@
 #define OMV_BVH_LEAF_MAX 2   // triangles per BVH4 leaf: 2 traced fastest of 1-4 (100k- and 2M-triangle scenes)
 #define OMV_STACK_LDS 28      // per-lane traversal stack entries kept in LDS
 #define OMV_STACK_TOTAL 128   // LDS + global overflow; the builder proves the bound
+#define OMV_BOX_PAD_ULPS 4    // child boxes are built this many ulps larger on every side (the slab test's error bound)
 #define OMV_EMPTY_CHILD ((int32_t)0x80000000)
 #define OMV_MAX_NODES ((size_t)1 << 25)   // node byte offsets (node * 128) stay below 2^32
 
@@ -39,6 +40,7 @@ enum { OMV_BG_NONE = 0, OMV_BG_CONSTANT = 1, OMV_BG_HDR = 2 };
 #define OMV_ENT(kind, payload) (((uint32_t)(kind) << OMV_ENT_SHIFT) | (uint32_t)(payload))
 #define OMV_ENT_END 0xFFFFFFFFu    // end of an instance's BLAS (stack only)
 #define OMV_ENT_NONE 0xFFFFFFFEu   // empty child slot (never pushed)
+#define OMV_ENT_DONE 0xFFFFFFFDu   // bottom of the stack: the traversal is over
 static_assert(OMV_BVH_LEAF_MAX >= 1 && OMV_BVH_LEAF_MAX <= 8, "leaf size must fit the entry's 3-bit count");
 
 struct alignas(64) OmvNode4 {

@@ -796,53 +796,69 @@ DEV void matGetRayAndBrdf(const OmvSceneView& S, const Ext& X, const SP& sp, con
 }
 
 // ------------------------------------------------------------ traversal
-struct Counters { uint32_t nodes, tris, overflow; };
+// Node visits and triangle tests of a lane; a stack overflow (the builder
+// proves there is none) sets the top bit of `tris` rather than hold a
+// register of its own through the traversal loop.
+struct Counters {
+    uint32_t nodes, tris;
+    DEV void zero() { nodes = tris = 0u; }
+    DEV void lose() { tris |= 0x80000000u; }
+    DEV uint32_t overflow() const { return tris >> 31; }
+};
 
 // Per-lane traversal stack: entries 0 .. OMV_STACK_LDS-1 in the kernel's
 // dynamic LDS (omv_lds_stack, [entry][lane]), the rest in a global spill
-// area.  The two parts are addressed through their own address spaces, so
-// the LDS entries compile to ds_read / ds_write (LDS counter only) rather
-// than to flat accesses, which would also wait on the vector memory counter
-// behind every node and triangle fetch in flight.
-typedef __attribute__((address_space(1))) uint32_t GlobalU32;
+// area [entry - OMV_STACK_LDS][lane of the grid].  The two parts are
+// addressed through their own address spaces, so the LDS entries compile to
+// ds_read / ds_write (LDS counter only) rather than to flat accesses, which
+// would also wait on the vector memory counter behind every node and
+// triangle fetch in flight.  The one per-lane register is `top`, the LDS
+// byte offset of the slot above the top (kLane * lane of the block + kRow *
+// entry); the spill area's base and stride are wave-uniform.
 // Every kernel that traverses runs OMV_BLOCK-lane workgroups with
-// OMV_STACK_LDS * OMV_BLOCK words of dynamic LDS, so the LDS stride is a
-// constant (a shift, not a multiply, per push and pop).
+// OMV_STACK_LDS * OMV_BLOCK words of dynamic LDS.
+typedef __attribute__((address_space(1))) uint32_t GlobalU32;
+typedef __attribute__((address_space(3))) uint32_t LdsU32;
 struct Stack {
-    uint32_t col;        // this lane's LDS column: omv_lds_stack[col + entry * OMV_BLOCK]
-    GlobalU32* glb;      // this lane's spill area, stride = glbStride
+    static constexpr uint32_t kLane = 4u, kRow = 4u * OMV_BLOCK;
+    static constexpr uint32_t kLds = kRow * OMV_STACK_LDS, kTotal = kRow * OMV_STACK_TOTAL;
+    uint32_t top;
+    GlobalU32* glb;
     uint32_t glbStride;
-    int sp;
-    // lane `tid` of `threads` (spill stacks interleaved by lane in gstack)
-    DEV void init(uint32_t* gstack, uint32_t tid, uint32_t threads) {
-        col = threadIdx.x;
-        glb = (GlobalU32*)(gstack + tid); glbStride = threads;
-        sp = 0;
+    // `threads` lanes in the grid, their spill stacks interleaved by lane in gstack
+    DEV void init(uint32_t* gstack, uint32_t threads) {
+        glb = (GlobalU32*)gstack; glbStride = threads;
+        clear();
+    }
+    DEV void clear() { top = kLane * threadIdx.x; }
+    DEV LdsU32& lds(uint32_t at) const { return *(LdsU32*)((__attribute__((address_space(3))) char*)(LdsU32*)omv_lds_stack + at); }
+    DEV GlobalU32& spill(uint32_t at) const {
+        return glb[(at / kRow - OMV_STACK_LDS) * glbStride + blockIdx.x * OMV_BLOCK + (at % kRow) / kLane];
     }
     DEV void push(uint32_t e, Counters& c) {
-        if (sp < OMV_STACK_LDS) omv_lds_stack[col + (uint32_t)sp * OMV_BLOCK] = e;
-        else if (sp < OMV_STACK_TOTAL) glb[(uint32_t)(sp - OMV_STACK_LDS) * glbStride] = e;
-        else { ++c.overflow; return; }
-        ++sp;
+        if (top < kLds) lds(top) = e;
+        else if (top < kTotal) spill(top) = e;
+        else { c.lose(); return; }
+        top += kRow;
     }
     // push e if `valid`, without a branch on it: the slot above the top is
     // written either way (free space) and the top moves only for a valid entry
     DEV void pushIf(uint32_t e, bool valid, Counters& c) {
-        if (sp < OMV_STACK_LDS) omv_lds_stack[col + (uint32_t)sp * OMV_BLOCK] = e;
-        else if (sp < OMV_STACK_TOTAL) glb[(uint32_t)(sp - OMV_STACK_LDS) * glbStride] = e;
-        const bool room = sp < OMV_STACK_TOTAL;
-        c.overflow += (valid && !room) ? 1u : 0u;
-        sp += (valid && room) ? 1 : 0;
+        if (top < kLds) lds(top) = e;
+        else if (top < kTotal) spill(top) = e;
+        const bool room = top < kTotal;
+        if (valid && !room) c.lose();
+        top += (valid && room) ? kRow : 0u;
     }
     // pushIf of three entries; when no active lane of the wave could reach
     // the spill area (a wave-uniform test) the entries go to LDS without the
     // per-entry LDS / spill / overflow branches
     DEV void push3If(const uint32_t e[3], const bool v[3], Counters& c) {
-        if (__ballot(sp > OMV_STACK_LDS - 3) == 0ull) {
+        if (__ballot(top >= kLds - 2u * kRow) == 0ull) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                omv_lds_stack[col + (uint32_t)sp * OMV_BLOCK] = e[k];
-                sp += v[k] ? 1 : 0;
+                lds(top) = e[k];
+                top += v[k] ? kRow : 0u;
             }
         } else {
 #pragma unroll
@@ -850,68 +866,77 @@ struct Stack {
         }
     }
     DEV uint32_t pop() {
-        --sp;
-        if (__ballot(sp >= OMV_STACK_LDS) == 0ull) return omv_lds_stack[col + (uint32_t)sp * OMV_BLOCK];   // wave-uniform: LDS only
-        return sp < OMV_STACK_LDS ? omv_lds_stack[col + (uint32_t)sp * OMV_BLOCK] : glb[(uint32_t)(sp - OMV_STACK_LDS) * glbStride];
+        top -= kRow;
+        if (__ballot(top >= kLds) == 0ull) return lds(top);   // wave-uniform: LDS only
+        return top < kLds ? lds(top) : spill(top);
     }
 };
 
 enum : uint32_t {
     E_KIND_SHIFT = OMV_ENT_SHIFT,
     E_BLAS_NODE = OMV_ENT_BLAS_NODE, E_BLAS_LEAF = OMV_ENT_BLAS_LEAF, E_TLAS_NODE = OMV_ENT_TLAS_NODE, E_INST = OMV_ENT_INST,
-    E_END = OMV_ENT_END, E_NONE = OMV_ENT_NONE,
+    E_END = OMV_ENT_END, E_NONE = OMV_ENT_NONE, E_DONE = OMV_ENT_DONE,
 };
 
-// Component selection for the ray's axis permutation by bit masks: k in
-// {0, 1, 2} gives m1 = all ones iff k == 1 and m2 = all ones iff k == 2,
-// and pick() takes y over x by m1, then z by m2 (two v_bfi_b32).  The masks
-// pass through an empty asm so the optimiser does not turn the selects back
-// into a compare chain (lowered as branches) or a dynamic vector index
+// The triangle test's view of a ray (Woop, Benthin & Wald 2013): its origin,
+// the shear of the axes (kx, ky, kz) = (kz + 1, kz + 2, kz) mod 3 with kz the
+// direction's largest axis, and the axis permutation as bit masks (m0: all
+// ones iff kz == 0, m1: iff kz == 1), so that a component is picked with two
+// v_bfi_b32.  The published test swaps kx and ky for a negative d[kz]; that
+// only negates U, V, W and det exactly, which leaves t, u, v and every
+// comparison as they are, so it is left out and the masks depend on kz alone.
+// The masks pass through an empty asm so the optimiser does not turn the
+// picks into a compare chain (lowered as branches) or a dynamic vector index
 // (lowered through scratch memory).
-struct PermMask { uint32_t m1, m2; };
-DEV PermMask permMask(int k) {
-    PermMask r;
-    r.m1 = 0u - (uint32_t)(k & 1);
-    r.m2 = 0u - (uint32_t)((k >> 1) & 1);
-    asm("" : "+v"(r.m1), "+v"(r.m2));
-    return r;
-}
-DEV float pick(const f3& v, const PermMask& m) {
-    const uint32_t a = (__float_as_uint(v.x) & ~m.m1) | (__float_as_uint(v.y) & m.m1);
-    return __uint_as_float((a & ~m.m2) | (__float_as_uint(v.z) & m.m2));
+struct TriRay { f3 o; float Sx, Sy, Sz; uint32_t m0, m1; };
+DEV float bfi(uint32_t m, float a, float b) { return __uint_as_float((__float_as_uint(a) & m) | (__float_as_uint(b) & ~m)); }
+DEV f3 permute(const f3& v, uint32_t m0, uint32_t m1) {
+    return mk3(bfi(m0, v.y, bfi(m1, v.z, v.x)), bfi(m0, v.z, bfi(m1, v.x, v.y)), bfi(m0, v.x, bfi(m1, v.y, v.z)));
 }
 
-struct Pre { int kx, ky, kz; float Sx, Sy, Sz; f3 o, d, idir; };
-
-DEV bool rayPrep(const f3& o, const f3& d, Pre& p) {
-    float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
+DEV bool rayPrep(const f3& o, const f3& d, TriRay& p) {
+    const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
     if (!(ax > 0.0f || ay > 0.0f || az > 0.0f)) return false;   // zero / NaN direction: no hit
-    int kz = 0; float m = ax;
-    if (ay > m) { kz = 1; m = ay; }
-    if (az > m) { kz = 2; }
-    int kx = kz + 1; if (kx == 3) kx = 0;
-    int ky = kx + 1; if (ky == 3) ky = 0;
-    float dkz = pick(d, permMask(kz));
-    if (dkz < 0.0f) { int t = kx; kx = ky; ky = t; }
-    p.kx = kx; p.ky = ky; p.kz = kz;
-    p.Sx = pick(d, permMask(kx)) / dkz;
-    p.Sy = pick(d, permMask(ky)) / dkz;
-    p.Sz = 1.0f / dkz;
-    p.o = o; p.d = d;
-    p.idir = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+    const bool y = ay > ax;
+    const bool z = az > (y ? ay : ax);
+    p.m0 = (y || z) ? 0u : 0xFFFFFFFFu;
+    p.m1 = (y && !z) ? 0xFFFFFFFFu : 0u;
+    asm("" : "+v"(p.m0), "+v"(p.m1));
+    const f3 k = permute(d, p.m0, p.m1);
+    p.o = o;
+    // Sx = k.x / k.z, Sy = k.y / k.z, Sz = 1 / k.z, correctly rounded.  With all
+    // three magnitudes well inside the float range (a wave-uniform test) one
+    // reciprocal, refined once, serves the three quotients, each with two
+    // residual corrections (Markstein 1990): the operations of the compiler's
+    // own division without its scaling, which does nothing in that range.
+    const float lo = fminf(fabsf(k.x), fabsf(k.y)), hi = fabsf(k.z);
+    if (__ballot(!(lo >= 1e-18f && hi <= 1e18f)) == 0ull) {
+        float r = __builtin_amdgcn_rcpf(k.z);
+        r = __builtin_fmaf(__builtin_fmaf(-k.z, r, 1.0f), r, r);
+        auto quot = [&](float a) {
+            float q = a * r;
+            q = __builtin_fmaf(__builtin_fmaf(-k.z, q, a), r, q);
+            return __builtin_fmaf(__builtin_fmaf(-k.z, q, a), r, q);
+        };
+        p.Sx = quot(k.x);
+        p.Sy = quot(k.y);
+        p.Sz = quot(1.0f);
+    } else {
+        p.Sx = k.x / k.z;
+        p.Sy = k.y / k.z;
+        p.Sz = 1.0f / k.z;
+    }
     return true;
 }
 
 // Woop, Benthin & Wald 2013; t in (tnear, tfar]
-DEV bool triIntersect(const Pre& p, const float4 r0, const float4 r1, const float4 r2, float tnear, float tfar, float& t, float& u, float& v) {
-    f3 A = mk3(r0.x - p.o.x, r0.y - p.o.y, r0.z - p.o.z);
-    f3 B = mk3(r1.x - p.o.x, r1.y - p.o.y, r1.z - p.o.z);
-    f3 C = mk3(r2.x - p.o.x, r2.y - p.o.y, r2.z - p.o.z);
-    const PermMask mx = permMask(p.kx), my = permMask(p.ky), mz = permMask(p.kz);
-    const float Akz = pick(A, mz), Bkz = pick(B, mz), Ckz = pick(C, mz);
-    float Ax = pick(A, mx) - p.Sx * Akz, Ay = pick(A, my) - p.Sy * Akz;
-    float Bx = pick(B, mx) - p.Sx * Bkz, By = pick(B, my) - p.Sy * Bkz;
-    float Cx = pick(C, mx) - p.Sx * Ckz, Cy = pick(C, my) - p.Sy * Ckz;
+DEV bool triIntersect(const TriRay& p, const float4 r0, const float4 r1, const float4 r2, float tnear, float tfar, float& t, float& u, float& v) {
+    const f3 A = permute(mk3(r0.x - p.o.x, r0.y - p.o.y, r0.z - p.o.z), p.m0, p.m1);
+    const f3 B = permute(mk3(r1.x - p.o.x, r1.y - p.o.y, r1.z - p.o.z), p.m0, p.m1);
+    const f3 C = permute(mk3(r2.x - p.o.x, r2.y - p.o.y, r2.z - p.o.z), p.m0, p.m1);
+    float Ax = A.x - p.Sx * A.z, Ay = A.y - p.Sy * A.z;
+    float Bx = B.x - p.Sx * B.z, By = B.y - p.Sy * B.z;
+    float Cx = C.x - p.Sx * C.z, Cy = C.y - p.Sy * C.z;
     float U = Cx * By - Cy * Bx, V = Ax * Cy - Ay * Cx, W = Bx * Ay - By * Ax;
     const bool zero = U == 0.0f || V == 0.0f || W == 0.0f;
     // the FP64 recomputation is rare: a wave-uniform branch around it keeps
@@ -927,7 +952,7 @@ DEV bool triIntersect(const Pre& p, const float4 r0, const float4 r1, const floa
     if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return false;
     float det = U + V + W;
     if (det == 0.0f) return false;
-    float Az = p.Sz * Akz, Bz = p.Sz * Bkz, Cz = p.Sz * Ckz;
+    float Az = p.Sz * A.z, Bz = p.Sz * B.z, Cz = p.Sz * C.z;
     float T = U * Az + V * Bz + W * Cz;
     float rcp = 1.0f / det;
     float tt = T * rcp;
@@ -936,12 +961,15 @@ DEV bool triIntersect(const Pre& p, const float4 r0, const float4 r1, const floa
     return true;
 }
 
-DEV void offer(Hit& h, bool& found, float t, float u, float v, int inst, int prim) {
-    if (!found || t < h.t) { h.t = t; h.u = u; h.v = v; h.inst = inst; h.prim = prim; h.tie = false; found = true; return; }
+// Keeps the (t, instance, primitive) minimum; h.inst < 0: nothing found yet.
+// Returns true when h.t changed.
+DEV bool offer(Hit& h, float t, float u, float v, int inst, int prim) {
+    if (h.inst < 0 || t < h.t) { h.t = t; h.u = u; h.v = v; h.inst = inst; h.prim = prim; h.tie = false; return true; }
     if (t == h.t) {
         if (inst != h.inst || prim != h.prim) h.tie = true;
         if (inst < h.inst || (inst == h.inst && prim < h.prim)) { h.u = u; h.v = v; h.inst = inst; h.prim = prim; }
     }
+    return false;
 }
 
 // 4-wide slab test, conservative (Ize 2013: tmax scaled by 1 + 2*gamma(3)).
@@ -1003,140 +1031,198 @@ DEV void boxTest4Rows(const OmvNode4* nodes, uint32_t idx, uint32_t rows, const 
     ent[0] = en.x; ent[1] = en.y; ent[2] = en.z; ent[3] = en.w;
 }
 
-// push the hit children farthest first; the nearest is not pushed but
-// returned in nxt (hasNext), so the next step needs no stack round trip.
-// Branch-free: a missed child becomes (key +inf, entry E_NONE), the
-// 5-comparator network sorts descending by key with selects, so the misses
-// come first and the nearest hit (if any) last; entries are pushed unless
-// E_NONE.  Hits at equal keys may come out in either order -- the closest
-// hit does not depend on the visiting order.
-DEV void pushSorted(Stack& st, Counters& c, uint32_t e[4], float t[4], const bool h[4], uint32_t& nxt, bool& hasNext) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        t[i] = h[i] ? t[i] : INFINITY;
-        e[i] = h[i] ? e[i] : (uint32_t)E_NONE;
-    }
-#define OMV_CSWAP(a, b)                                             \
-    {                                                               \
-        const bool sw = t[b] > t[a];                                \
-        const float ta = t[a], tb = t[b];                           \
-        const uint32_t ea = e[a], eb = e[b];                        \
-        t[a] = sw ? tb : ta; t[b] = sw ? ta : tb;                   \
-        e[a] = sw ? eb : ea; e[b] = sw ? ea : eb;                   \
-    }
-    OMV_CSWAP(0, 1) OMV_CSWAP(2, 3) OMV_CSWAP(0, 2) OMV_CSWAP(1, 3) OMV_CSWAP(1, 2)
-#undef OMV_CSWAP
-    const bool v[3] = {e[0] != (uint32_t)E_NONE, e[1] != (uint32_t)E_NONE, e[2] != (uint32_t)E_NONE};
-    st.push3If(e, v, c);
-    nxt = e[3];
-    hasNext = e[3] != (uint32_t)E_NONE;
+// A ray as the node visits test it.  On each axis the distance of plane p is
+// p * idir - o * idir, one multiply-add against a bias computed once per ray
+// and instance: nb for a near plane (error bound taken off) and fb for a far
+// one (added).  Conservative: with r = v_rcp_f32(d) (1 ulp) the computed
+// distance is off the exact (p - o) / d by at most 3 roundings of |p r| (r,
+// the multiply-add) and 5 of |o r| (r, o * r, the bias, the multiply-add),
+// 2^-24 each.  The builders widen every child plane by 4 ulps (>= 4 * 2^-24
+// |p|) and the bias carries 6 * 2^-24 |o r|, so a box the exact ray meets is
+// never missed; the widening also covers the rounding of a hit's t, as
+// kBoxUp does on the far side.  A component below 1e-30 (0, NaN) does not
+// cull on its axis: idir 0, nb -inf, fb +inf.
+struct BoxRay { f3 idir, nb, fb; uint32_t rows; };
+DEV void boxAxis(float o, float d, float& idir, float& nb, float& fb) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    const float od = o * r;
+    const bool ok = fabsf(d) >= 1e-30f;
+    idir = ok ? r : 0.0f;
+    nb = ok ? __builtin_fmaf(fabsf(od), -3.57627869e-7f, -od) : -INFINITY;   // 6 * 2^-24
+    fb = ok ? __builtin_fmaf(fabsf(od), 3.57627869e-7f, -od) : INFINITY;
 }
+DEV void boxRay(const f3& o, const f3& d, BoxRay& b) {
+    boxAxis(o.x, d.x, b.idir.x, b.nb.x, b.fb.x);
+    boxAxis(o.y, d.y, b.idir.y, b.nb.y, b.fb.y);
+    boxAxis(o.z, d.z, b.idir.z, b.nb.z, b.fb.z);
+    b.rows = nearRows(b.idir);
+    // computed where it is asked for: hoisted out of the mask loop it would be
+    // kept in scratch memory across the traversal
+    asm volatile("" : "+v"(b.idir.x), "+v"(b.idir.y), "+v"(b.idir.z));
+}
+constexpr float kBoxUp = 1.0000004f;
+
+// A child's sort key: distance (high word) and entry (low word), compared as
+// one double -- for distances >= 0 the order of their bits.  Minimum and
+// maximum as instructions: fmin / fmax would first quiet both operands,
+// which are no NaNs here.
+typedef uint32_t Key __attribute__((ext_vector_type(2)));   // x entry, y distance bits
+DEV Key keyMin(Key a, Key b) { Key r; asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+DEV Key keyMax(Key a, Key b) { Key r; asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b)); return r; }
+DEV bool keyHit(Key a) { return __uint_as_float(a.y) < INFINITY; }
 
 // Closest hit of a world-space ray over the two-level BVH, as a resumable
-// traversal: start() sets the TLAS root as the next entry, every step()
-// consumes one entry (TLAS/BLAS node, leaf, instance entry or instance end):
-// the nearest hit child of the last node when there is one (kept in a
-// register), else the top of the stack; more() says whether entries remain.  The result
+// traversal: start() sets the TLAS root as the current entry `cur`; node(),
+// leaf() and inst() consume it and leave the next one (the nearest hit child
+// of a node, kept in a register, else the top of the stack); E_DONE ends.
+// TLAS and BLAS nodes are one case: `box` holds the ray of the level the
+// traversal is at, set when an instance is entered and left.  The result
 // does not depend on the visiting order: boxes are tested conservatively
 // against the current closest t, triangles accept t in (tnear, t_closest],
 // and offer() keeps the (t, instance, primitive) minimum.
 struct Trav {
-    f3 wo, wd, widir;   // world ray (TLAS boxes, instance transforms)
-    Pre op;             // object ray of the current instance (BLAS boxes, triangles)
-    uint32_t wrows, orows;   // nearRows of the world and object rays
-    Hit h;
-    float tnear, tfar;
+    f3 wo, wd;       // world ray
+    BoxRay box;      // the ray in the space of cur's node
+    TriRay tri;      // object ray of the current instance (triangles)
+    Hit h;           // closest hit so far; h.t = the far end while h.inst < 0
+    float tnear;
+    float tcull;     // boxes entered after it are skipped: h.t * kBoxUp, finite
     float tstop;     // occlusion early-out: the traversal ends at the first hit with t <= tstop (< 0: closest hit only)
     int curInst;
-    bool found;
-    uint32_t nxt;    // next entry when hasNext
-    bool hasNext;
-    DEV bool more(const Stack& st) const { return hasNext || st.sp > 0; }
+    uint32_t cur;
+    DEV bool more() const { return cur != (uint32_t)E_DONE; }
+    DEV bool found() const { return h.inst >= 0; }
+    DEV bool isNode() const { return (cur & (1u << E_KIND_SHIFT)) == 0u; }            // BLAS or TLAS node
+    DEV bool isLeaf() const { return (cur >> E_KIND_SHIFT) == (uint32_t)E_BLAS_LEAF; }
     DEV bool start(const OmvSceneView& S, const f3& o, const f3& d, float tn, float tf, Stack& st, Counters& c) {
-        found = false;
-        hasNext = false;
         h.tie = false; h.t = tf; h.u = 0.0f; h.v = 0.0f; h.inst = -1; h.prim = 0;
-        tnear = tn; tfar = tf;
+        tnear = tn;
+        tcull = fminf(tf * kBoxUp, FLT_MAX);
         tstop = -1.0f;
-        st.sp = 0;
+        st.clear();
+        cur = E_DONE;
         const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
         if (!(ax > 0.0f || ay > 0.0f || az > 0.0f)) return false;   // zero / NaN direction: no hit (as rayPrep)
         wo = o; wd = d;
-        widir = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-        wrows = nearRows(widir);
-        orows = wrows;
+        boxRay(o, d, box);
         curInst = -1;
-        nxt = (E_TLAS_NODE << E_KIND_SHIFT) | (uint32_t)S.tlas_root;
-        hasNext = true;
+        st.push(E_DONE, c);
+        cur = (E_TLAS_NODE << E_KIND_SHIFT) | (uint32_t)S.tlas_root;
         return true;
     }
-    DEV uint32_t take(Stack& st) {
-        if (hasNext) { hasNext = false; return nxt; }
-        return st.pop();
-    }
-    DEV static bool isLeaf(uint32_t e) { return e != E_END && (e >> E_KIND_SHIFT) == E_BLAS_LEAF; }
     // triangles of a BLAS leaf entry (object ray of the current instance)
-    DEV void leaf(const OmvSceneView& S, uint32_t e, Stack& st, Counters& c) {
-        const uint32_t idx = e & 0x3FFFFFFFu;
+    DEV void leaf(const OmvSceneView& S, Stack& st, Counters& c) {
+        const uint32_t idx = cur & 0x3FFFFFFFu;
         const uint32_t first = idx >> 3, cnt = (idx & 7u) + 1u;
+        cur = st.pop();
         for (uint32_t k = 0; k < cnt; ++k) {
             const float4* rec = reinterpret_cast<const float4*>(S.tris) + 3u * (first + k);
             float4 r0 = rec[0], r1 = rec[1], r2 = rec[2];
             ++c.tris;
             float t, u, v;
-            if (triIntersect(op, r0, r1, r2, tnear, found ? h.t : tfar, t, u, v)) offer(h, found, t, u, v, curInst, __float_as_int(r0.w));
+            if (triIntersect(tri, r0, r1, r2, tnear, h.t, t, u, v) && offer(h, t, u, v, curInst, __float_as_int(r0.w)))
+                tcull = fminf(t * kBoxUp, FLT_MAX);
         }
         // a hit at or before tstop decides an occlusion query: the closest hit
         // is at least as near, so the traversal ends here
-        if (found && h.t <= tstop) { st.sp = 0; hasNext = false; }
+        if (h.inst >= 0 && h.t <= tstop) cur = E_DONE;
     }
-    // any other entry: instance end, instance entry, TLAS or BLAS node
-    DEV void visit(const OmvSceneView& S, uint32_t e, Stack& st, Counters& c) {
-        if (e == E_END) { curInst = -1; return; }
-        const uint32_t kind = e >> E_KIND_SHIFT;
-        const uint32_t idx = e & 0x3FFFFFFFu;
-        const float tb = found ? h.t : tfar;
-        if (kind == E_INST) {
-            const int inst = (int)(idx & 0x1FFFFFFFu);
-            const OmvInstance& in = S.insts[inst];
-            const float* I = in.inv;
-            const f3 o = wo, d = wd;
-            f3 oo = mk3(I[0] * o.x + I[1] * o.y + I[2] * o.z + I[3], I[4] * o.x + I[5] * o.y + I[6] * o.z + I[7],
-                        I[8] * o.x + I[9] * o.y + I[10] * o.z + I[11]);
-            f3 od = mk3(I[0] * d.x + I[1] * d.y + I[2] * d.z, I[4] * d.x + I[5] * d.y + I[6] * d.z, I[8] * d.x + I[9] * d.y + I[10] * d.z);
-            if (!rayPrep(oo, od, op)) return;
-            orows = nearRows(op.idir);
-            curInst = inst;
-            st.push(E_END, c);
-            nxt = (E_BLAS_NODE << E_KIND_SHIFT) | (uint32_t)in.blas_root;
-            hasNext = true;
+    // entry into an instance, or the end of one
+    DEV void inst(const OmvSceneView& S, Stack& st, Counters& c) {
+        if (cur == (uint32_t)E_END) {
+            curInst = -1;
+            boxRay(wo, wd, box);
+            cur = st.pop();
             return;
         }
-        // internal node (TLAS uses the world ray, BLAS the object ray)
-        const bool tl = kind == E_TLAS_NODE;
+        const int i = (int)(cur & 0x1FFFFFFFu);
+        const OmvInstance& in = S.insts[i];
+        const float* I = in.inv;
+        const f3 o = wo, d = wd;
+        f3 oo = mk3(I[0] * o.x + I[1] * o.y + I[2] * o.z + I[3], I[4] * o.x + I[5] * o.y + I[6] * o.z + I[7],
+                    I[8] * o.x + I[9] * o.y + I[10] * o.z + I[11]);
+        f3 od = mk3(I[0] * d.x + I[1] * d.y + I[2] * d.z, I[4] * d.x + I[5] * d.y + I[6] * d.z, I[8] * d.x + I[9] * d.y + I[10] * d.z);
+        if (!rayPrep(oo, od, tri)) { cur = st.pop(); return; }
+        boxRay(oo, od, box);
+        curInst = i;
+        st.push(E_END, c);
+        cur = (E_BLAS_NODE << E_KIND_SHIFT) | (uint32_t)in.blas_root;
+    }
+    // Internal node: its four boxes against the ray, the hit children pushed
+    // farthest first except the nearest, which becomes cur.  The planes are
+    // fetched by the direction's signs (nearRows).  A child that is missed
+    // gets the key +inf; the 5-comparator network sorts (distance, entry)
+    // pairs as doubles, two instructions a comparator.  An empty slot (planes
+    // at +inf) is always missed, since tcull is finite.
+    DEV void node(const OmvSceneView& S, Stack& st, Counters& c) {
         ++c.nodes;
-        float tent[4]; bool hit[4]; uint32_t ent[4];
-        boxTest4Rows(S.nodes, idx, tl ? wrows : orows, tl ? wo : op.o, tl ? widir : op.idir, tnear, tb, tent, hit, ent);
-        pushSorted(st, c, ent, tent, hit, nxt, hasNext);
+        const char* base = reinterpret_cast<const char*>(S.nodes);
+        const uint32_t nb = cur << 7;   // byte offset: the kind bits leave at the top (OMV_MAX_NODES)
+        const uint32_t ax = nb | (box.rows & 0xFFu), ay = nb | ((box.rows >> 8) & 0xFFu), az = nb | (box.rows >> 16);
+        const float4 nx = ldRow(base, ax), fx = ldRow(base, ax ^ 16u);
+        const float4 ny = ldRow(base, ay), fy = ldRow(base, ay ^ 16u);
+        const float4 nz = ldRow(base, az), fz = ldRow(base, az ^ 16u);
+        const uint4 en = *reinterpret_cast<const uint4*>(base + (nb | 112u));
+        const float NX[4] = {nx.x, nx.y, nx.z, nx.w}, FX[4] = {fx.x, fx.y, fx.z, fx.w};
+        const float NY[4] = {ny.x, ny.y, ny.z, ny.w}, FY[4] = {fy.x, fy.y, fy.z, fy.w};
+        const float NZ[4] = {nz.x, nz.y, nz.z, nz.w}, FZ[4] = {fz.x, fz.y, fz.z, fz.w};
+        const uint32_t E[4] = {en.x, en.y, en.z, en.w};
+        Key k[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float tmin = fmaxf(fmaxf(__builtin_fmaf(NX[i], box.idir.x, box.nb.x), __builtin_fmaf(NY[i], box.idir.y, box.nb.y)),
+                                     fmaxf(__builtin_fmaf(NZ[i], box.idir.z, box.nb.z), tnear));
+            const float tmax = fminf(fminf(__builtin_fmaf(FX[i], box.idir.x, box.fb.x), __builtin_fmaf(FY[i], box.idir.y, box.fb.y)),
+                                     fminf(__builtin_fmaf(FZ[i], box.idir.z, box.fb.z), tcull));
+            k[i].x = E[i];
+            k[i].y = __float_as_uint(tmin <= tmax ? tmin : INFINITY);
+        }
+        const Key a0 = keyMax(k[0], k[1]), b0 = keyMin(k[0], k[1]), a1 = keyMax(k[2], k[3]), b1 = keyMin(k[2], k[3]);
+        const Key last = keyMax(a0, a1), first = keyMin(b0, b1), m0 = keyMin(a0, a1), m1 = keyMax(b0, b1);
+        const Key third = keyMax(m0, m1), second = keyMin(m0, m1);
+        const uint32_t push[3] = {last.x, third.x, second.x};
+        const bool valid[3] = {keyHit(last), keyHit(third), keyHit(second)};
+        st.push3If(push, valid, c);
+        cur = first.x;
+        if (!keyHit(first)) cur = st.pop();
     }
     // one entry, whatever its kind (the persistent traversal's unit of work)
     DEV void step(const OmvSceneView& S, Stack& st, Counters& c) {
-        const uint32_t e = take(st);
-        if (isLeaf(e)) leaf(S, e, st, c);
-        else visit(S, e, st, c);
+        if (isNode()) node(S, st, c);
+        else if (isLeaf()) leaf(S, st, c);
+        else inst(S, st, c);
     }
 };
 
+// Traversal launches are bound by VALU issue (0.8 - 0.99 of the issue cycles
+// on MI355X, a quarter of the lanes active on secondary rays), so what counts
+// is instructions per entry and how many entry kinds an iteration mixes.  The
+// blocks of the loop are taken by the lanes whose entry is of that kind, and
+// a wave pays each block that any of its lanes needs; a ray visits four to
+// six nodes for each leaf and instance entry, so an iteration holds
+// kNodeSteps node visits for one leaf and one instance block.  1 / 2 / 3:
+// instanced 1080p x 16 10.25 / 9.99 / 10.05 ms, torus knot 512^2 x 64 5.72 /
+// 5.60 / 5.63.  With the one multiply-add per plane, the double-keyed sort (a
+// node visit: 136 -> 85 instructions), the shared reciprocal at instance
+// entry (155 -> 95) and the mask loop compiled out: traversal launches 7.91
+// -> 6.28 ms and 4.23 -> 3.55 ms.
+constexpr int kNodeSteps = 2;
 DEV bool traceClosest(const OmvSceneView& S, const f3& o, const f3& d, float tnear, float tfar, Hit& h, Stack& st, Counters& c,
                       float tstop = -1.0f) {
     Trav T;
     const bool ok = T.start(S, o, d, tnear, tfar, st, c);
     T.tstop = tstop;
     if (ok) {
-        while (T.more(st)) T.step(S, st, c);
+        do {
+#pragma unroll
+            for (int k = 0; k < kNodeSteps; ++k)
+                if (T.isNode()) T.node(S, st, c);
+            if (T.isLeaf()) T.leaf(S, st, c);
+            if (!T.isNode() && !T.isLeaf() && T.more()) T.inst(S, st, c);
+        } while (T.more());
     }
     h = T.h;
-    return ok && T.found;
+    return ok && T.found();
 }
 
 // --------------------------------------------------------- path helpers
@@ -1170,8 +1256,15 @@ DEV int maskStep(const OmvSceneView& S, const f3& org, const f3& dir, const Hit&
     return tfar <= tnear ? 2 : 1;
 }
 
+// kMask = false: the caller knows that no material of the scene is masked, and
+// one trace decides (the loop would keep the ray's set-up across the trace).
+template <bool kMask = true>
 DEV bool sceneIntersect(const OmvSceneView& S, const f3& org, const f3& dir, float& tnear, float tfar, Hit& h, Stack& st, Counters& c, uint32_t& rays,
                         float tstop = -1.0f) {
+    if (!kMask) {
+        ++rays;
+        return traceClosest(S, org, dir, tnear, tfar, h, st, c, S.closest_only ? -1.0f : tstop);
+    }
     const float t1 = tfar;
     if (S.any_masked || S.closest_only) tstop = -1.0f;
     for (int itr = 10; itr > 0; --itr) {
@@ -1461,7 +1554,7 @@ DEV uint64_t waveSum(uint64_t v) {
 }
 
 DEV void flushCounters(unsigned long long* g, uint32_t rays, uint32_t cam, uint32_t light, uint32_t shadow, const Counters& c) {
-    uint64_t v[7] = {rays, cam, light, shadow, c.nodes, c.tris, c.overflow};
+    uint64_t v[7] = {rays, cam, light, shadow, c.nodes, c.tris & 0x7FFFFFFFu, c.overflow()};
 #pragma unroll
     for (int i = 0; i < 7; ++i) {
         uint64_t s = waveSum(v[i]);
@@ -1499,8 +1592,8 @@ struct Lane {
 };
 
 DEV void laneInit(Lane& L, uint32_t* gstack, float* lv, uint32_t gtid, uint32_t gthreads) {
-    L.st.init(gstack, gtid, gthreads);
-    L.cnt.nodes = 0; L.cnt.tris = 0; L.cnt.overflow = 0;
+    L.st.init(gstack, gthreads);
+    L.cnt.zero();
     L.rays = L.camRays = L.lightRays = L.shadowRays = 0;
     L.splat = nullptr;
     L.lv = lv ? lv + gtid : nullptr; L.lvStride = gthreads;

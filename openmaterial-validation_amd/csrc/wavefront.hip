@@ -24,12 +24,11 @@
 
 #include "path_device.h"
 
-// Traversal kernels are compiled for 5 waves per SIMD (<= 96 VGPRs; a few
-// bytes of spill in the camera and fused kernels) with a 28-entry LDS stack,
-// so 10 workgroups fit a CU's 160 KB of LDS.  Measured on MI355X against 4
-// waves (<= 128 VGPRs, 32-entry LDS stack): 2M-triangle instanced scene
-// 15.85 -> 15.23 ms, torus knot 8.93 -> 8.53 ms per render; 3 waves
-// (6 workgroups per CU) was 16 % slower than 4.
+// Traversal kernels are compiled for 5 waves per SIMD (<= 96 VGPRs; without
+// masked materials 12 bytes of spill in the camera kernel, none in the
+// others) with a 28-entry LDS stack, so 10 workgroups fit a CU's 160 KB of
+// LDS.  Measured on MI355X against 4 waves (<= 128 VGPRs): 2M-triangle
+// instanced scene 10.01 -> 9.60 ms, torus knot 5.69 -> 5.41 ms per render.
 #define OMV_TRACE_WAVES 5
 // Resident waves per SIMD the camera-shading kernel is compiled for (the
 // register budget it gets: 3 -> 168 VGPRs, 4 -> 128).  Measured on MI355X:
@@ -109,8 +108,6 @@ DEV uint32_t waveAppend(uint32_t* counter, bool want) {
     base = __shfl(base, leader, 64);
     return base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
 }
-
-DEV void stackInit(Stack& st, uint32_t* gstack, uint32_t gtid, uint32_t gthreads) { st.init(gstack, gtid, gthreads); }
 
 // The traversal launches add their ray and visit counts into one of
 // OMV_STAT_SLOTS slots (128 bytes apart) by workgroup, for the same reason
@@ -393,28 +390,25 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_gen(OmvSceneView S, omv_came
         }
     }
     if (kLights) {
-        Counters c; c.nodes = culled; c.tris = 0; c.overflow = 0;
+        Counters c; c.nodes = culled; c.tris = 0;
         flushCounters(statSlot(counters), culled, 0u, culled, 0u, c);
     }
 }
 
 // ---------------------------------------------------------------- trace
 // sceneIntersect (BDPTRenderer.cpp:75-102) over a queue.  kKind 0: camera
-// rays, 1: light rays (closest hit + the re-trace tnear), 2: connection
-// rays (the visibility decision of isConnected, BDPTRenderer.cpp:221-234),
-// 3: environment rays of OMV_EXT_HDRI_NEE (visible iff nothing is hit),
-// 4: pinhole rays of OMV_EXT_LIGHT_SPLAT (visible iff nothing is hit; the
-//    visible contributions are added to the splat film).
-template <int kKind>
+// rays, 1: light rays (closest hit + the re-trace tnear), 4: pinhole rays of
+// OMV_EXT_LIGHT_SPLAT (visible iff nothing is hit; the visible contributions
+// are added to the splat film).  kMask: some material is alpha-masked.
+template <int kKind, bool kMask>
 __global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace(OmvSceneView S, WfQueue q, WfShadowQ sq, WfSeg count,
-                                                          WfHits H, uint8_t* __restrict__ vis, uint32_t nslots, int lc,
-                                                          uint32_t* __restrict__ gstack, unsigned long long* __restrict__ counters,
-                                                          float* __restrict__ splat, uint32_t xcds, WfGen G) {
+                                                          WfHits H, uint32_t* __restrict__ gstack,
+                                                          unsigned long long* __restrict__ counters, float* __restrict__ splat,
+                                                          uint32_t xcds, WfGen G) {
     const uint32_t gthreads = gridDim.x * blockDim.x;
-    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     Stack st;
-    stackInit(st, gstack, gtid, gthreads);
-    Counters cnt; cnt.nodes = 0; cnt.tris = 0; cnt.overflow = 0;
+    st.init(gstack, gthreads);
+    Counters cnt; cnt.zero();
     uint32_t rays = 0;
     XcdWalk w;
     __shared__ SegTable cur;
@@ -423,30 +417,10 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace(OmvSc
         const uint32_t e = w.e;                                       // logical entry (hit records)
         const uint32_t p = kKind == 0 && G.gen ? e : cur.phys(e);   // its queue slot
         Hit h;
-        if (kKind == 2) {
+        if (kKind == 4) {
             const float4 a = sq.o[p], dd = sq.d[p], b = sq.b[p];
             float tnear = a.w;
-            bool visible;
-            if (!sceneIntersect(S, xyz(a), xyz(dd), tnear, dd.w, h, st, cnt, rays, connectStop(xyz(a), xyz(b)))) {
-                visible = true;
-            } else {
-                f3 df = sub3(hitPosition(S, h), xyz(b));
-                float sd = dot3(df, df);
-                float safeD = 10.0f * FLT_EPSILON * maxAbs(xyz(b));
-                visible = sd <= safeD * safeD;
-            }
-            const uint32_t id = __float_as_uint(b.w);
-            const uint32_t slot = id / (uint32_t)lc, l = id - slot * (uint32_t)lc;
-            vis[(uint64_t)l * nslots + slot] = visible ? 2 : 0;
-        } else if (kKind == 3) {
-            const float4 o = q.o[p], d = q.d[p];
-            float tnear = o.w;
-            const bool hit = sceneIntersect(S, xyz(o), xyz(d), tnear, FLT_MAX, h, st, cnt, rays, FLT_MAX);
-            vis[__float_as_uint(d.w)] = hit ? 0 : 2;
-        } else if (kKind == 4) {
-            const float4 a = sq.o[p], dd = sq.d[p], b = sq.b[p];
-            float tnear = a.w;
-            const bool hit = sceneIntersect(S, xyz(a), xyz(dd), tnear, dd.w, h, st, cnt, rays, FLT_MAX);
+            const bool hit = sceneIntersect<kMask>(S, xyz(a), xyz(dd), tnear, dd.w, h, st, cnt, rays, FLT_MAX);
             splatAdd(splat, !hit, __float_as_uint(b.w), xyz(b));
         } else {
             f3 org, dir;
@@ -457,7 +431,7 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace(OmvSc
                 const float4 o = q.o[p], d = q.d[p];
                 org = xyz(o); dir = xyz(d); tnear = o.w;
             }
-            const bool hit = sceneIntersect(S, org, dir, tnear, FLT_MAX, h, st, cnt, rays);
+            const bool hit = sceneIntersect<kMask>(S, org, dir, tnear, FLT_MAX, h, st, cnt, rays);
             float4 r; r.x = h.t; r.y = h.u; r.z = h.v; r.w = tnear;
             int2 id; id.x = hit ? h.inst : -1; id.y = h.prim | (h.tie ? (int)0x80000000 : 0);
             if (hit) H.h[e] = r;   // read by the shading kernels for hits only
@@ -477,15 +451,15 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace(OmvSc
 // exactly the per-ray arithmetic of its own kind, so the outputs are those
 // of three separate launches; one launch pays one latency tail instead of
 // up to three.  A null count is an empty queue.
+template <bool kMask>
 __global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace_fused(
     OmvSceneView S, WfQueue q, WfSeg qCount, WfShadowQ sq, WfSeg sqCount, WfQueue eq, WfSeg eqCount, WfHits H, uint8_t* __restrict__ vis,
     uint8_t* __restrict__ nvis, uint32_t nslots, int lc, uint32_t* __restrict__ gstack, unsigned long long* __restrict__ counters,
     uint32_t xcds) {
     const uint32_t gthreads = gridDim.x * blockDim.x;
-    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     Stack st;
-    stackInit(st, gstack, gtid, gthreads);
-    Counters cnt; cnt.nodes = 0; cnt.tris = 0; cnt.overflow = 0;
+    st.init(gstack, gthreads);
+    Counters cnt; cnt.zero();
     uint32_t rays = 0;
     __shared__ SegTable cA, cB, cC;
     segLoad(cA, qCount); segLoad(cB, sqCount); segLoad(cC, eqCount);
@@ -513,7 +487,7 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace_fused
         }
         Hit h;
         float tnear = o.w;
-        const bool hit = sceneIntersect(S, xyz(o), xyz(d), tnear, tfar, h, st, cnt, rays, tstop);
+        const bool hit = sceneIntersect<kMask>(S, xyz(o), xyz(d), tnear, tfar, h, st, cnt, rays, tstop);
         if (kind == 0) {
             float4 r; r.x = h.t; r.y = h.u; r.z = h.v; r.w = tnear;
             int2 id; id.x = hit ? h.inst : -1; id.y = h.prim | (h.tie ? (int)0x80000000 : 0);
@@ -568,10 +542,11 @@ DEV uint64_t wuni64(uint64_t v) { return ((uint64_t)wuni((uint32_t)(v >> 32)) <<
 
 struct PacketRay {   // one lane's ray and closest hit
     f3 wo, wd, widir;   // world ray
-    Pre op;             // object ray of the packet's current instance
+    TriRay op;          // object ray of the packet's current instance
+    f3 oidir;
     Hit h;
     float tnear, tfar;
-    bool found;
+    DEV bool found() const { return h.inst >= 0; }
 };
 
 // One traceClosest of every lane in M0 (closest hit, no occlusion early-out).
@@ -601,8 +576,7 @@ DEV void packetTrace(const OmvSceneView& S, PacketRay& R, uint64_t M0, uint32_t*
                 if (act) {
                     ++c.tris;
                     float t, u, v;
-                    if (triIntersect(R.op, r0, r1, r2, R.tnear, R.found ? R.h.t : R.tfar, t, u, v))
-                        offer(R.h, R.found, t, u, v, curInst, __float_as_int(r0.w));
+                    if (triIntersect(R.op, r0, r1, r2, R.tnear, R.h.t, t, u, v)) offer(R.h, t, u, v, curInst, __float_as_int(r0.w));
                 }
             }
             continue;
@@ -620,6 +594,7 @@ DEV void packetTrace(const OmvSceneView& S, PacketRay& R, uint64_t M0, uint32_t*
                             I[8] * o.x + I[9] * o.y + I[10] * o.z + I[11]);
                 f3 od = mk3(I[0] * d.x + I[1] * d.y + I[2] * d.z, I[4] * d.x + I[5] * d.y + I[6] * d.z, I[8] * d.x + I[9] * d.y + I[10] * d.z);
                 ok = rayPrep(oo, od, R.op);
+                R.oidir = mk3(1.0f / od.x, 1.0f / od.y, 1.0f / od.z);
             }
             const uint64_t M2 = __ballot(ok);
             if (M2 == 0ull) continue;
@@ -636,10 +611,10 @@ DEV void packetTrace(const OmvSceneView& S, PacketRay& R, uint64_t M0, uint32_t*
 #pragma unroll
             for (int i = 0; i < 8; ++i) dst[i] = ldUniform(S.nodes + idx, (uint32_t)i);
         }
-        const float tb = R.found ? R.h.t : R.tfar;
+        const float tb = R.h.t;
         float tent[4]; bool hit[4];
         if (kind == E_TLAS_NODE) boxTest4(nd, R.wo, R.widir, R.tnear, tb, tent, hit);
-        else boxTest4(nd, R.op.o, R.op.idir, R.tnear, tb, tent, hit);
+        else boxTest4(nd, R.op.o, R.oidir, R.tnear, tb, tent, hit);
         if (act) ++c.nodes;
         uint64_t m[4];
 #pragma unroll
@@ -672,7 +647,7 @@ DEV void packetTrace(const OmvSceneView& S, PacketRay& R, uint64_t M0, uint32_t*
                 stM[sp] = m[k];
                 ++sp;
             } else if ((m[k] >> lane) & 1ull) {
-                ++c.overflow;
+                c.lose();
             }
         }
         e = ent[3];
@@ -694,7 +669,7 @@ __global__ __launch_bounds__(OMV_BLOCK, 6) void omv_wf_trace_cam1(OmvSceneView S
     __shared__ SegTable cur;
     segLoad(cur, count);
     const uint32_t wave = threadIdx.x >> 6;
-    Counters cnt; cnt.nodes = 0; cnt.tris = 0; cnt.overflow = 0;
+    Counters cnt; cnt.zero();
     uint32_t rays = 0, nCam = 0;
     XcdWalk w;
     // the wave stays together: lanes past the end of the queue go on with
@@ -714,7 +689,6 @@ __global__ __launch_bounds__(OMV_BLOCK, 6) void omv_wf_trace_cam1(OmvSceneView S
         R.widir = mk3(1.0f / dir.x, 1.0f / dir.y, 1.0f / dir.z);
         R.tnear = 0.0f;
         R.tfar = FLT_MAX;
-        R.found = false;
         R.h.t = R.tfar; R.h.u = 0.0f; R.h.v = 0.0f; R.h.inst = -1; R.h.prim = 0; R.h.tie = false;
         bool need = has, hit = false;
         int itr = 10;
@@ -722,13 +696,12 @@ __global__ __launch_bounds__(OMV_BLOCK, 6) void omv_wf_trace_cam1(OmvSceneView S
             const uint64_t M = __ballot(need && dirOk);
             if (need) {
                 ++rays;
-                R.found = false;
                 R.h.t = R.tfar; R.h.u = 0.0f; R.h.v = 0.0f; R.h.inst = -1; R.h.prim = 0; R.h.tie = false;
             }
             if (M != 0ull) packetTrace(S, R, M, stE[wave], stM[wave], cnt);
             if (need) {
                 --itr;
-                if (!R.found) {
+                if (!R.found()) {
                     hit = false; need = false;
                 } else {
                     const int ms = maskStep(S, org, dir, R.h, R.tnear, R.tfar, FLT_MAX);
@@ -774,10 +747,9 @@ struct WfTraceArgs {
 template <int kKind>
 __global__ __launch_bounds__(OMV_BLOCK, 4) void omv_wf_trace_pt(OmvSceneView S, WfTraceArgs A) {
     const uint32_t gthreads = gridDim.x * blockDim.x;
-    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     Stack st;
-    stackInit(st, A.gstack, gtid, gthreads);
-    Counters cnt; cnt.nodes = 0; cnt.tris = 0; cnt.overflow = 0;
+    st.init(A.gstack, gthreads);
+    Counters cnt; cnt.zero();
     uint32_t rays = 0, nCam = 0, nLight = 0, nShadow = 0;
     // entries [0, nA) camera / light rays of q, [nA, nA + nB) rays of sq,
     // [nA + nB, total) environment rays of eq (by kKind)
@@ -831,10 +803,10 @@ __global__ __launch_bounds__(OMV_BLOCK, 4) void omv_wf_trace_pt(OmvSceneView S, 
         // step until fewer than keep lanes of the wave are busy
         for (;;) {
             if (busy) {
-                if (T.more(st)) T.step(S, st, cnt);
-                if (!T.more(st)) {
+                if (T.more()) T.step(S, st, cnt);
+                if (!T.more()) {
                     // one traceClosest call finished: sceneIntersect's masked re-trace loop
-                    bool done = true, hit = T.found;
+                    bool done = true, hit = T.found();
                     if (hit && S.any_masked) {
                         const int mesh = S.insts[T.h.inst].mesh_id;
                         const OmvMaterial& M = S.mats[S.meshes[mesh].mat_id];
@@ -1390,14 +1362,13 @@ int wavefrontCounterCount(int B, int lvCap) { return OMV_QSEG * (2 * (lvCap + 2)
 
 void wavefrontBlocksPerCU(int out[9]) {
     const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
-    int t = occ(omv_wf_trace<0>, lds);
-    for (int k : {occ(omv_wf_trace<1>, lds), occ(omv_wf_trace<2>, lds), occ(omv_wf_trace<3>, lds), occ(omv_wf_trace<4>, lds),
-                  occ(omv_wf_trace_fused, lds)})
+    int t = occ(omv_wf_trace<0, true>, lds);
+    for (int k : {occ(omv_wf_trace<0, false>, lds), occ(omv_wf_trace<1, true>, lds), occ(omv_wf_trace<1, false>, lds),
+                  occ(omv_wf_trace<4, true>, lds), occ(omv_wf_trace<4, false>, lds), occ(omv_wf_trace_fused<true>, lds),
+                  occ(omv_wf_trace_fused<false>, lds)})
         t = std::min(t, k);
     int tp = occ(omv_wf_trace_pt<0>, lds);
-    for (int k : {occ(omv_wf_trace_pt<1>, lds), occ(omv_wf_trace_pt<2>, lds), occ(omv_wf_trace_pt<3>, lds), occ(omv_wf_trace_pt<4>, lds),
-                  occ(omv_wf_trace_pt<5>, lds)})
-        tp = std::min(tp, k);
+    for (int k : {occ(omv_wf_trace_pt<1>, lds), occ(omv_wf_trace_pt<4>, lds), occ(omv_wf_trace_pt<5>, lds)}) tp = std::min(tp, k);
     out[0] = t;
     out[4] = tp;
     out[1] = occ(omv_wf_shade_cam<true, true>, 0);
@@ -1507,6 +1478,13 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
     auto mark = [&]() {
         if (L.traceEv && L.traceEvUsed && *L.traceEvUsed < L.traceEvCap) (void)hipEventRecord(L.traceEv[(*L.traceEvUsed)++], stream);
     };
+    enum { kTraceCamera, kTraceLight, kTraceSplat };
+    auto launchTrace = [&](int what, const WfQueue& q, const WfSeg& count, const WfGen& gen) {
+        auto k = what == kTraceCamera ? (S.any_masked ? omv_wf_trace<0, true> : omv_wf_trace<0, false>)
+                 : what == kTraceLight ? (S.any_masked ? omv_wf_trace<1, true> : omv_wf_trace<1, false>)
+                                       : (S.any_masked ? omv_wf_trace<4, true> : omv_wf_trace<4, false>);
+        hipLaunchKernelGGL(k, dim3(L.blocksTrace), blk, lds, stream, S, q, sq, count, H, L.gstack, stats, L.splat, xcds, gen);
+    };
     hipLaunchKernelGGL(omv_wf_fill_u32, dim3((ncnt + 63) / 64), dim3(64), 0, stream, L.qcount, ncnt);
     hipLaunchKernelGGL(omv_wf_fill_u32, dim3(OMV_STAT_SLOTS * 32 / 64), dim3(64), 0, stream, reinterpret_cast<uint32_t*>(stats),
                        OMV_STAT_SLOTS * 32);
@@ -1540,8 +1518,7 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
                 hipLaunchKernelGGL(omv_wf_trace_pt<1>, dim3(L.blocksTrace), blk, lds, stream, S,
                                    ptArgs(in, lightCnt(i), none, eq, none));
             else
-                hipLaunchKernelGGL(omv_wf_trace<1>, dim3(L.blocksTrace), blk, lds, stream, S, in, sq, lightCnt(i), H, W.vis, n, L.lc, L.gstack,
-                                   stats, L.splat, xcds, Gen0);
+                launchTrace(kTraceLight, in, lightCnt(i), Gen0);
             mark();
             if (splat) {
                 hipLaunchKernelGGL(omv_wf_shade_light<true>, dim3(L.blocksShade), blk, 0, stream, S, L.cam, P, L.sample0, i, W, in, lightCnt(i),
@@ -1551,8 +1528,7 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
                     hipLaunchKernelGGL(omv_wf_trace_pt<4>, dim3(L.blocksTrace), blk, lds, stream, S,
                                        ptArgs(in, none, splCnt(i), eq, none));
                 else
-                    hipLaunchKernelGGL(omv_wf_trace<4>, dim3(L.blocksTrace), blk, lds, stream, S, in, sq, splCnt(i), H, W.vis, n, L.lc, L.gstack,
-                                       stats, L.splat, xcds, Gen0);
+                    launchTrace(kTraceSplat, in, splCnt(i), Gen0);
                 mark();
             } else {
                 hipLaunchKernelGGL(omv_wf_shade_light<false>, dim3(L.blocksShade), blk, 0, stream, S, L.cam, P, L.sample0, i, W, in, lightCnt(i),
@@ -1562,7 +1538,7 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
         }
     }
     WfQueue in = qa, out = qb, spare = qc;   // qc is free once the light rounds are done
-    // With connection or environment rays (and the one-pass traversal), the
+    // With connection or environment rays, the
     // traversal of bounce i's visibility rays is fused with that of bounce
     // i + 1's camera rays: shade(i) -> fused trace -> connect(i) -> shade(i + 1).
     // connect(i) still runs before shade(i + 1) (which reads the connection
@@ -1603,8 +1579,7 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
             else if (i == 1 && Gen1.gen && L.blocksPacket > 0)
                 hipLaunchKernelGGL(omv_wf_trace_cam1, dim3(L.blocksPacket), blk, 0, stream, S, camCnt(1), H, stats, xcds, Gen1);
             else
-                hipLaunchKernelGGL(omv_wf_trace<0>, dim3(L.blocksTrace), blk, lds, stream, S, in, sq, camCnt(i), H, W.vis, n, L.lc,
-                                   L.gstack, stats, L.splat, xcds, i == 1 ? Gen1 : Gen0);
+                launchTrace(kTraceCamera, in, camCnt(i), i == 1 ? Gen1 : Gen0);
             mark();
         }
         traced = false;
@@ -1642,32 +1617,11 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
                                    ptArgs(next, nextInWavefront ? camCnt(i + 1) : none, lights ? shCnt(i) : none, eq,
                                           nee ? envCnt(i) : none));
             else
-                hipLaunchKernelGGL(omv_wf_trace_fused, dim3(L.blocksTrace), blk, lds, stream, S, next, nextInWavefront ? camCnt(i + 1) : none,
+                hipLaunchKernelGGL(S.any_masked ? omv_wf_trace_fused<true> : omv_wf_trace_fused<false>, dim3(L.blocksTrace), blk, lds, stream, S, next, nextInWavefront ? camCnt(i + 1) : none,
                                    sq, lights ? shCnt(i) : none, eq, nee ? envCnt(i) : none, H, W.vis, W.nvis, n, L.lc, L.gstack,
                                    stats, xcds);
             mark();
             traced = nextInWavefront;
-        } else {
-            if (lights) {
-                mark();
-                if (L.traceKeep > 0)
-                    hipLaunchKernelGGL(omv_wf_trace_pt<2>, dim3(L.blocksTrace), blk, lds, stream, S,
-                                       ptArgs(in, none, shCnt(i), eq, none));
-                else
-                    hipLaunchKernelGGL(omv_wf_trace<2>, dim3(L.blocksTrace), blk, lds, stream, S, in, sq, shCnt(i), H, W.vis, n, L.lc,
-                                       L.gstack, stats, L.splat, xcds, Gen0);
-                mark();
-            }
-            if (nee) {
-                mark();
-                if (L.traceKeep > 0)
-                    hipLaunchKernelGGL(omv_wf_trace_pt<3>, dim3(L.blocksTrace), blk, lds, stream, S,
-                                       ptArgs(in, none, none, eq, envCnt(i)));
-                else
-                    hipLaunchKernelGGL(omv_wf_trace<3>, dim3(L.blocksTrace), blk, lds, stream, S, eq, sq, envCnt(i), H, W.nvis, n, L.lc,
-                                       L.gstack, stats, L.splat, xcds, Gen0);
-                mark();
-            }
         }
         if (lights || nee)
             hipLaunchKernelGGL(omv_wf_connect, dim3(L.blocksShade), blk, 0, stream, W, in, camCnt(i), L.rad, lights ? 1 : 0, nee ? 1 : 0, i,
