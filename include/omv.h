@@ -343,9 +343,10 @@ int omv_renderer_get_schedule(const omv_renderer* r, int* schedule);
 /* Launch tuning of the wavefront schedule (no reference counterpart; the
  * film does not depend on it). */
 typedef struct omv_render_tuning {
-    int trace_keep;           /* 1..64: persistent traversal, a wave refills its
-                                 idle lanes once fewer than trace_keep are busy;
-                                 0: one pass over the queue, one ray per lane   */
+    int trace_keep;           /* 1..64: a traversal wave gives its idle lanes new
+                                 rays once fewer than trace_keep are busy (1:
+                                 when all are done); 0 = default: 1 for the
+                                 first bounce's camera rays, 32 for all others */
     int trace_blocks_per_cu;  /* resident traversal workgroups per CU
                                  (0 = occupancy limit)                          */
     int chunk_samples;        /* samples per wavefront chunk, rounded down to

@@ -52,7 +52,7 @@ struct WfLaunch {
     uint32_t* gstack;          // spill stacks of blocksTrace * OMV_BLOCK lanes
     unsigned long long* counters;
     int blocksGen, blocksTrace, blocksShade;
-    int traceKeep;             // > 0: persistent traversal, refill below this many busy lanes
+    int traceKeep;             // > 0: idle lanes refilled below this many busy ones; 0: the default of each launch
     hipEvent_t* traceEv;       // optional: an event pair around every traversal launch
     int traceEvCap;            // events available from traceEv
     int* traceEvUsed;          // events recorded so far (in/out)

@@ -1186,12 +1186,8 @@ struct Trav {
         cur = first.x;
         if (!keyHit(first)) cur = st.pop();
     }
-    // one entry, whatever its kind (the persistent traversal's unit of work)
-    DEV void step(const OmvSceneView& S, Stack& st, Counters& c) {
-        if (isNode()) node(S, st, c);
-        else if (isLeaf()) leaf(S, st, c);
-        else inst(S, st, c);
-    }
+    // Up to kNodeSteps nodes, a leaf and an instance entry, each if it is next.
+    DEV void iterate(const OmvSceneView& S, Stack& st, Counters& c);
 };
 
 // Traversal launches are bound by VALU issue (0.8 - 0.99 of the issue cycles
@@ -1205,21 +1201,25 @@ struct Trav {
 // 5.60 / 5.63.  With the one multiply-add per plane, the double-keyed sort (a
 // node visit: 136 -> 85 instructions), the shared reciprocal at instance
 // entry (155 -> 95) and the mask loop compiled out: traversal launches 7.91
-// -> 6.28 ms and 4.23 -> 3.55 ms.
+// -> 6.28 ms and 4.23 -> 3.55 ms.  Making lanes wait with a leaf until 12, 16
+// or 24 lanes hold one is slower (knot 4.85 -> 5.02 / 5.08 / 5.23 ms): rays
+// then take more iterations, and each is also a chain of dependent fetches.
 constexpr int kNodeSteps = 2;
+DEV void Trav::iterate(const OmvSceneView& S, Stack& st, Counters& c) {
+#pragma unroll
+    for (int k = 0; k < kNodeSteps; ++k)
+        if (isNode()) node(S, st, c);
+    if (isLeaf()) leaf(S, st, c);
+    if (!isNode() && !isLeaf() && more()) inst(S, st, c);
+}
 DEV bool traceClosest(const OmvSceneView& S, const f3& o, const f3& d, float tnear, float tfar, Hit& h, Stack& st, Counters& c,
                       float tstop = -1.0f) {
     Trav T;
     const bool ok = T.start(S, o, d, tnear, tfar, st, c);
     T.tstop = tstop;
     if (ok) {
-        do {
-#pragma unroll
-            for (int k = 0; k < kNodeSteps; ++k)
-                if (T.isNode()) T.node(S, st, c);
-            if (T.isLeaf()) T.leaf(S, st, c);
-            if (!T.isNode() && !T.isLeaf() && T.more()) T.inst(S, st, c);
-        } while (T.more());
+        do T.iterate(S, st, c);
+        while (T.more());
     }
     h = T.h;
     return ok && T.found();

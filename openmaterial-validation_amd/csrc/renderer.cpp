@@ -391,9 +391,8 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
     const uint64_t slots = std::min(npix, chunkPix) * (uint64_t)spp;
     if (slots * (uint64_t)lc >= (1ull << 32)) { setError("render: too many samples per pixel for one chunk"); return OMV_E_RANGE; }
     if (!wfPerCu_[0]) wavefrontBlocksPerCU(wfPerCu_);
-    // resident traversal workgroups per CU: the occupancy limit of the traversal
-    // kernel in use (the persistent form holds more registers)
-    const int traceOcc = tuning_.trace_keep > 0 ? wfPerCu_[4] : wfPerCu_[0];
+    // resident traversal workgroups per CU: the occupancy limit of the traversal kernels
+    const int traceOcc = wfPerCu_[0];
     const int blocksTrace = cus_ * (tuning_.trace_blocks_per_cu > 0 ? std::min(tuning_.trace_blocks_per_cu, traceOcc) : traceOcc);
     hipError_t e;
     if ((e = dStack_.reserve((uint64_t)blocksTrace * OMV_BLOCK * (OMV_STACK_TOTAL - OMV_STACK_LDS) * sizeof(uint32_t))) != hipSuccess)

@@ -139,7 +139,7 @@ inline WfSeg segOf(uint32_t* cnt, uint32_t K, uint32_t cap) { WfSeg g; g.cnt = c
 struct SegTable {
     uint32_t pre[OMV_QSEG + 1];
     uint32_t K, cap;
-    DEV uint32_t total() const { return pre[K]; }
+    DEV uint32_t total() const { return (uint32_t)__builtin_amdgcn_readfirstlane((int)pre[K]); }
     DEV uint32_t phys(uint32_t L) const {
         uint32_t r = 0;
 #pragma unroll
@@ -274,36 +274,36 @@ struct WfLightVerts {
     }
 };
 
-// XCD-banded walk over a queue of `total` entries.  Workgroups are dispatched
-// to the X XCDs round-robin (workgroup b on XCD b mod X), and each XCD has an
-// L2 of its own.  The queue is cut into chunks of C entries (a power of two,
-// 128 .. 32768, about total / 16X), dealt to the XCDs round-robin, and the
-// workgroups of one XCD stride over that XCD's chunks as over one array, so
-// the rays an XCD traces at a time come from a few contiguous stretches of
-// the queue (for camera rays: of the image) and share their node and
-// triangle lines in that XCD's L2.  Every entry below `total` is visited by
-// exactly one thread: chunk g belongs to XCD g mod X as its chunk g div X,
-// and within an XCD the offsets v = local thread + k * (threads of the XCD)
-// cover 0, 1, 2, ... once each.  With X = 1, or a grid that is not a
-// multiple of X, it is the plain grid stride.  Entries must stay below 2^31.
-struct XcdWalk {
-    uint32_t x, X, logC, v, stride, total, e;
+// A wave's list of the entries of a queue of `total`, 64 at a time, banded
+// over the XCDs.  Workgroups are dispatched to the X XCDs round-robin
+// (workgroup b on XCD b mod X), and each XCD has an L2 of its own.  The queue
+// is cut into chunks of C entries (a power of two, 128 .. 32768, about total
+// / 16X), dealt to the XCDs round-robin, and the waves of one XCD stride over
+// that XCD's chunks as over one array, so the rays an XCD traces at a time
+// come from a few contiguous stretches of the queue (for camera rays: of the
+// image) and share their node and triangle lines in that XCD's L2.  Every
+// entry below `total` is in exactly one list: chunk g belongs to XCD g mod X
+// as its chunk g div X, and within an XCD item c of wave i is offset
+// ((c div 64) * waves + i) * 64 + c mod 64, which covers 0, 1, 2, ... once
+// each.  A list's entries grow with the item, so it is over at the first one
+// past the end.  With X = 1, or a grid that is not a multiple of X, it is the
+// plain stride.  Entries must stay below 2^31.
+struct XcdList {
+    uint32_t x, X, logC, wave, waves, total;
     DEV void start(uint32_t tot, uint32_t nX) {
         total = tot;
         X = nX > 1u && gridDim.x % nX == 0u ? nX : 1u;
         x = blockIdx.x % X;
-        v = (blockIdx.x / X) * blockDim.x + threadIdx.x;
-        stride = (gridDim.x / X) * blockDim.x;
+        wave = (blockIdx.x / X) * (OMV_BLOCK / 64u) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        waves = (gridDim.x / X) * (OMV_BLOCK / 64u);
         const uint32_t want = tot / (16u * X);
         logC = 7u;
         while (logC < 15u && (2u << logC) <= want) ++logC;
-        e = at(v);
     }
-    DEV uint32_t at(uint32_t vv) const {
-        return ((((vv >> logC) * X) + x) << logC) | (vv & ((1u << logC) - 1u));
+    DEV uint32_t entry(uint32_t c) const {
+        const uint32_t v = (((c >> 6) * waves + wave) << 6) | (c & 63u);
+        return ((((v >> logC) * X) + x) << logC) | (v & ((1u << logC) - 1u));
     }
-    DEV bool more() const { return e < total; }
-    DEV void next() { v += stride; e = at(v); }
 };
 
 }  // namespace
@@ -311,8 +311,8 @@ struct XcdWalk {
 // ------------------------------------------------------------------ gen
 // Camera ray of every slot (PinholeCamera::getRay, 2 draws) and, with
 // lights, the light-subpath start (tryComputeLightPath, BDPTRenderer.cpp:194-206).
-// With writeQueues = 0 the round-1 camera rays are not stored: the round-1
-// camera kernels compute them (WfGen).  Light rays are stored (their
+// The round-1 camera rays are not stored: the round-1 camera kernels compute
+// them (WfGen).  Light rays are stored (their
 // direction comes from a rejection loop, cheaper to keep than to redo) by
 // appending to the segmented round-1 light queue (lightSeg, whose regions
 // are sized for this launch's grid) -- except a ray that
@@ -325,8 +325,8 @@ struct XcdWalk {
 // (lightBelowRoot); their directions are not drawn.
 template <bool kLights>
 __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_gen(OmvSceneView S, omv_camera_desc cam, RP P, int spp, uint64_t sample0,
-                                                        WfState W, WfQueue camQ, WfQueue lightQ, uint32_t* __restrict__ camCount,
-                                                        WfSeg lightSeg, float* __restrict__ rad, int writeQueues,
+                                                        WfState W, WfQueue lightQ, uint32_t* __restrict__ camCount,
+                                                        WfSeg lightSeg, float* __restrict__ rad,
                                                         unsigned long long* __restrict__ counters, unsigned long long* __restrict__ lost) {
     const uint32_t gthreads = gridDim.x * blockDim.x;
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -340,14 +340,7 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_gen(OmvSceneView S, omv_came
         // after 1 vertex, connection sum 0, 2 draws consumed) is not stored:
         // camera round 1 and its connect kernel start from it
         W.flags[slot] = 0u;
-        if (camRays) {
-            if (writeQueues) {
-                f3 org, D;
-                genCameraRay(cam, P.seed, spp, s, org, D);
-                camQ.o[slot] = f4of(org, 0.0f);
-                camQ.d[slot] = f4of(D, __uint_as_float(slot));
-            }
-        } else {
+        if (!camRays) {
             // no camera vertex: conn * 1 + radiance with both zero
             rad[(uint64_t)slot * 3 + 0] = 0.0f;
             rad[(uint64_t)slot * 3 + 1] = 0.0f;
@@ -396,122 +389,159 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_gen(OmvSceneView S, omv_came
 }
 
 // ---------------------------------------------------------------- trace
-// sceneIntersect (BDPTRenderer.cpp:75-102) over a queue.  kKind 0: camera
-// rays, 1: light rays (closest hit + the re-trace tnear), 4: pinhole rays of
-// OMV_EXT_LIGHT_SPLAT (visible iff nothing is hit; the visible contributions
-// are added to the splat film).  kMask: some material is alpha-masked.
-template <int kKind, bool kMask>
-__global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace(OmvSceneView S, WfQueue q, WfShadowQ sq, WfSeg count,
-                                                          WfHits H, uint32_t* __restrict__ gstack,
-                                                          unsigned long long* __restrict__ counters, float* __restrict__ splat,
-                                                          uint32_t xcds, WfGen G) {
-    const uint32_t gthreads = gridDim.x * blockDim.x;
-    Stack st;
-    st.init(gstack, gthreads);
-    Counters cnt; cnt.zero();
-    uint32_t rays = 0;
-    XcdWalk w;
-    __shared__ SegTable cur;
-    segLoad(cur, count);
-    for (w.start(cur.total(), xcds); w.more(); w.next()) {
-        const uint32_t e = w.e;                                       // logical entry (hit records)
-        const uint32_t p = kKind == 0 && G.gen ? e : cur.phys(e);   // its queue slot
-        Hit h;
-        if (kKind == 4) {
-            const float4 a = sq.o[p], dd = sq.d[p], b = sq.b[p];
-            float tnear = a.w;
-            const bool hit = sceneIntersect<kMask>(S, xyz(a), xyz(dd), tnear, dd.w, h, st, cnt, rays, FLT_MAX);
-            splatAdd(splat, !hit, __float_as_uint(b.w), xyz(b));
-        } else {
-            f3 org, dir;
-            float tnear = 0.0f;
-            if (kKind == 0 && G.gen) {   // round 1: the camera ray of slot e
-                genCameraRay(G.cam, G.seed, G.spp, G.sample0 + e, org, dir);
-            } else {
-                const float4 o = q.o[p], d = q.d[p];
-                org = xyz(o); dir = xyz(d); tnear = o.w;
-            }
-            const bool hit = sceneIntersect<kMask>(S, org, dir, tnear, FLT_MAX, h, st, cnt, rays);
-            float4 r; r.x = h.t; r.y = h.u; r.z = h.v; r.w = tnear;
-            int2 id; id.x = hit ? h.inst : -1; id.y = h.prim | (h.tie ? (int)0x80000000 : 0);
-            if (hit) H.h[e] = r;   // read by the shading kernels for hits only
-            H.id[e] = id;
-        }
-    }
-    // every entry below the total is traced once, so the ray kinds are
-    // counted once per launch rather than per lane
-    const uint32_t all = blockIdx.x == 0 && threadIdx.x == 0 ? cur.total() : 0u;
-    flushCounters(statSlot(counters), rays, kKind == 0 ? all : 0u, kKind == 1 ? all : 0u, kKind >= 2 ? all : 0u, cnt);
-}
+// The queues of one traversal launch: camera (kKind 0) or light (1) rays in
+// q, pinhole rays (4) in sq, or (5) the rays of one camera round boundary,
+// back to back: the camera rays of bounce i + 1 in q, then the connection
+// rays in sq and the environment rays in eq of bounce i.  A null count is an
+// empty queue.
+struct WfTraceArgs {
+    WfQueue q; WfSeg qCount;
+    WfShadowQ sq; WfSeg sqCount;
+    WfQueue eq; WfSeg eqCount;
+    WfHits H;
+    uint8_t* vis; uint8_t* nvis;
+    uint32_t nslots; int lc;
+    uint32_t* gstack; unsigned long long* counters; float* splat;
+    uint32_t xcds;
+    int keep;
+    WfGen G;
+};
 
-// Fused traversal of one camera round boundary: the camera extension rays of
-// bounce i + 1 (kind 0), then the connection rays (kind 2) and environment
-// rays (kind 3) of bounce i, one grid over the three queues back to back.
-// The three are independent given bounce i's shading, and each entry gets
-// exactly the per-ray arithmetic of its own kind, so the outputs are those
-// of three separate launches; one launch pays one latency tail instead of
-// up to three.  A null count is an empty queue.
-template <bool kMask>
-__global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace_fused(
-    OmvSceneView S, WfQueue q, WfSeg qCount, WfShadowQ sq, WfSeg sqCount, WfQueue eq, WfSeg eqCount, WfHits H, uint8_t* __restrict__ vis,
-    uint8_t* __restrict__ nvis, uint32_t nslots, int lc, uint32_t* __restrict__ gstack, unsigned long long* __restrict__ counters,
-    uint32_t xcds) {
-    const uint32_t gthreads = gridDim.x * blockDim.x;
+// sceneIntersect (BDPTRenderer.cpp:75-102) over the queues of a launch.
+//   camera, light rays: closest hit + the re-trace tnear into H
+//   connection rays: the visibility decision of isConnected
+//     (BDPTRenderer.cpp:221-234)
+//   environment rays of OMV_EXT_HDRI_NEE: visible iff nothing is hit
+//   pinhole rays of OMV_EXT_LIGHT_SPLAT: likewise; the visible
+//     contributions are added to the splat film
+// Each entry gets the arithmetic of its own kind, so one launch over three
+// queues gives what three would and pays one latency tail.  kMask: some
+// material is alpha-masked (the re-trace loop).
+//
+// Each lane holds one ray.  The lanes of a wave need very different numbers
+// of steps (secondary rays: a quarter of the lanes active when a wave waits
+// for its longest ray), so finished lanes stand idle only until fewer than
+// `keep` are busy; then all of them write their results and take the wave's
+// next entries together, which keeps the code outside the traversal loop at
+// one pass per 64 - keep rays.  keep = 1: the wave waits for its last ray.
+// MI355X, traversal ms per render, keep 1 -> 32 on the secondary launches:
+// torus knot 512^2 x 64 3.46 -> 3.00 (lanes active 0.30 -> 0.40), with NEE
+// 333 x 511 x 32 2.80 -> 2.37, instanced 1080p x 16 6.16 -> 5.85, masked
+// scene with lights 3.17 -> 2.93; 20 and 44 are within 1 % of 32.  Round-1
+// camera rays are coherent (lanes 0.7 - 0.8) and lose by it: knot 3.00 ->
+// 3.30, instanced 5.85 -> 6.25.
+constexpr int kKeepPrimary = 1, kKeepSecondary = 32;
+template <int kKind, bool kMask>
+__global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace(OmvSceneView S, WfTraceArgs A) {
     Stack st;
-    st.init(gstack, gthreads);
+    st.init(A.gstack, gridDim.x * OMV_BLOCK);
     Counters cnt; cnt.zero();
-    uint32_t rays = 0;
+    uint32_t retraced = 0;
+    // entries [0, nA) of q, [nA, nA + nB) of sq, [nA + nB, total) of eq
     __shared__ SegTable cA, cB, cC;
-    segLoad(cA, qCount); segLoad(cB, sqCount); segLoad(cC, eqCount);
-    const uint32_t nA = cA.total(), nB = cB.total(), nC = cC.total();
-    XcdWalk w;
-    for (w.start(nA + nB + nC, xcds); w.more(); w.next()) {
-        const uint32_t e = w.e;
-        // the entry's ray: one traversal call site for the three kinds (the
-        // arguments each kind's own launch would pass), then its epilogue
-        const int kind = e < nA ? 0 : (e < nA + nB ? 2 : 3);
-        float4 o, d;
-        float tfar = FLT_MAX, tstop = -1.0f;
-        if (kind == 0) {
-            const uint32_t p = cA.phys(e);
-            o = q.o[p]; d = q.d[p];
-        } else if (kind == 2) {
-            const uint32_t k = cB.phys(e - nA);
-            o = sq.o[k]; d = sq.d[k];
-            tfar = d.w;
-            tstop = connectStop(xyz(o), xyz(sq.b[k]));   // the target is read again after the traversal
-        } else {
-            const uint32_t k = cC.phys(e - nA - nB);
-            o = eq.o[k]; d = eq.d[k];
-            tstop = FLT_MAX;
-        }
-        Hit h;
-        float tnear = o.w;
-        const bool hit = sceneIntersect<kMask>(S, xyz(o), xyz(d), tnear, tfar, h, st, cnt, rays, tstop);
-        if (kind == 0) {
-            float4 r; r.x = h.t; r.y = h.u; r.z = h.v; r.w = tnear;
-            int2 id; id.x = hit ? h.inst : -1; id.y = h.prim | (h.tie ? (int)0x80000000 : 0);
-            if (hit) H.h[e] = r;   // read by the shading kernels for hits only
-            H.id[e] = id;
-        } else if (kind == 2) {
-            const float4 b = sq.b[cB.phys(e - nA)];   // not held in registers across the traversal
-            bool visible = true;
-            if (hit) {
-                f3 df = sub3(hitPosition(S, h), xyz(b));
-                float sd = dot3(df, df);
-                float safeD = 10.0f * FLT_EPSILON * maxAbs(xyz(b));
-                visible = sd <= safeD * safeD;
+    if (kKind != 4) segLoad(cA, A.qCount);
+    if (kKind >= 4) segLoad(cB, A.sqCount);
+    if (kKind == 5) segLoad(cC, A.eqCount);
+    const uint32_t nA = kKind != 4 ? cA.total() : 0u, nB = kKind >= 4 ? cB.total() : 0u, nC = kKind == 5 ? cC.total() : 0u;
+    const uint64_t before = (1ull << (threadIdx.x & 63u)) - 1ull;
+    XcdList list;
+    list.start(nA + nB + nC, A.xcds);
+    uint32_t item = 0;                          // the wave's next item
+    bool left = list.entry(0) < list.total;     // it has one
+    Trav T;
+    T.cur = E_DONE;
+    bool has = false;
+    uint32_t e = 0;                             // the lane's entry
+    int itr = 0;
+    for (;;) {
+        if (has && !T.more()) {
+            bool hit = T.found();
+            has = false;
+            if (kMask && hit) {
+                const bool query = kKind == 4 || (kKind == 5 && e >= nA && e < nA + nB);
+                const float t1 = query ? A.sq.d[cB.phys(e - nA)].w : FLT_MAX;
+                float tfar;
+                const int m = maskStep(S, T.wo, T.wd, T.h, T.tnear, tfar, t1);
+                hit = m == 0;
+                if (m == 1 && --itr > 0) {
+                    ++retraced;
+                    const float ts = T.tstop, tn = T.tnear;
+                    T.start(S, T.wo, T.wd, tn, tfar, st, cnt);
+                    T.tstop = ts;
+                    has = true;
+                }
             }
-            const uint32_t id = __float_as_uint(b.w);
-            const uint32_t slot = id / (uint32_t)lc, l = id - slot * (uint32_t)lc;
-            vis[(uint64_t)l * nslots + slot] = visible ? 2 : 0;
-        } else {
-            nvis[__float_as_uint(eq.d[cC.phys(e - nA - nB)].w)] = hit ? 0 : 2;   // the slot, read again
+            if (has) {
+            } else if (kKind < 4 || (kKind == 5 && e < nA)) {
+                float4 r; r.x = T.h.t; r.y = T.h.u; r.z = T.h.v; r.w = T.tnear;
+                int2 id; id.x = hit ? T.h.inst : -1; id.y = T.h.prim | (T.h.tie ? (int)0x80000000 : 0);
+                if (hit) A.H.h[e] = r;   // read by the shading kernels for hits only
+                A.H.id[e] = id;
+            } else if (kKind == 4 || e < nA + nB) {
+                const float4 b = A.sq.b[cB.phys(e - nA)];   // not held in registers across the traversal
+                if (kKind == 4) {
+                    splatAdd(A.splat, !hit, __float_as_uint(b.w), xyz(b));
+                } else {
+                    bool visible = true;
+                    if (hit) {
+                        f3 df = sub3(hitPosition(S, T.h), xyz(b));
+                        float sd = dot3(df, df);
+                        float safeD = 10.0f * FLT_EPSILON * maxAbs(xyz(b));
+                        visible = sd <= safeD * safeD;
+                    }
+                    const uint32_t id = __float_as_uint(b.w);
+                    const uint32_t slot = id / (uint32_t)A.lc, l = id - slot * (uint32_t)A.lc;
+                    A.vis[(uint64_t)l * A.nslots + slot] = visible ? 2 : 0;
+                }
+            } else {
+                A.nvis[__float_as_uint(A.eq.d[cC.phys(e - nA - nB)].w)] = hit ? 0 : 2;
+            }
         }
+        if (left) {
+            const uint64_t idle = __ballot(!has);
+            if (!has) {
+                e = list.entry(item + (uint32_t)__popcll(idle & before));
+                if (e < list.total) {
+                    f3 org, dir;
+                    float tnear = 0.0f, tfar = FLT_MAX, tstop = -1.0f;
+                    if (kKind == 0 && A.G.gen) {   // round 1: the camera ray of slot e
+                        genCameraRay(A.G.cam, A.G.seed, A.G.spp, A.G.sample0 + e, org, dir);
+                    } else {
+                        float4 o, d;
+                        if (kKind < 4 || (kKind == 5 && e < nA)) {
+                            const uint32_t p = cA.phys(e);
+                            o = A.q.o[p]; d = A.q.d[p];
+                        } else if (kKind == 4 || e < nA + nB) {
+                            const uint32_t p = cB.phys(e - nA);
+                            o = A.sq.o[p]; d = A.sq.d[p];
+                            tfar = d.w;
+                            tstop = kKind == 4 ? FLT_MAX : connectStop(xyz(o), xyz(A.sq.b[p]));
+                        } else {
+                            const uint32_t p = cC.phys(e - nA - nB);
+                            o = A.eq.o[p]; d = A.eq.d[p];
+                            tstop = FLT_MAX;
+                        }
+                        org = xyz(o); dir = xyz(d); tnear = o.w;
+                    }
+                    T.start(S, org, dir, tnear, tfar, st, cnt);
+                    T.tstop = kMask || S.closest_only ? -1.0f : tstop;   // kMask: a cut-out hit must be the closest
+                    itr = 10;
+                    has = true;
+                }
+            }
+            item += (uint32_t)__popcll(idle);
+            left = list.entry(item) < list.total;
+        }
+        if (__ballot(has) == 0ull) break;
+        const int keep = left ? A.keep : 1;
+        do {
+            T.iterate(S, st, cnt);
+        } while (__popcll(__ballot(T.more())) >= keep);
     }
     // every entry is traced once: the kinds are counted once per launch
     const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-    flushCounters(statSlot(counters), rays, first ? nA : 0u, 0u, first ? nB + nC : 0u, cnt);
+    const uint32_t all = first ? nA : 0u, vis = first ? nB + nC : 0u;
+    flushCounters(statSlot(A.counters), all + vis + retraced, kKind != 1 ? all : 0u, kKind == 1 ? all : 0u, vis, cnt);
 }
 
 // ------------------------------------------------ packet traversal (round 1)
@@ -671,13 +701,14 @@ __global__ __launch_bounds__(OMV_BLOCK, 6) void omv_wf_trace_cam1(OmvSceneView S
     const uint32_t wave = threadIdx.x >> 6;
     Counters cnt; cnt.zero();
     uint32_t rays = 0, nCam = 0;
-    XcdWalk w;
+    XcdList list;
+    list.start(cur.total(), xcds);
     // the wave stays together: lanes past the end of the queue go on with
     // the loop (inactive in every packet) until no lane has an entry
-    for (w.start(cur.total(), xcds);; w.next()) {
-        const bool has = w.more();
+    for (uint32_t item = threadIdx.x & 63u;; item += 64u) {
+        const uint32_t e = list.entry(item);
+        const bool has = e < list.total;
         if (__ballot(has) == 0ull) break;
-        const uint32_t e = w.e;
         f3 org = mk3(0.0f, 0.0f, 0.0f), dir = mk3(0.0f, 0.0f, 0.0f);
         if (has) {
             genCameraRay(G.cam, G.seed, G.spp, G.sample0 + e, org, dir);
@@ -719,143 +750,6 @@ __global__ __launch_bounds__(OMV_BLOCK, 6) void omv_wf_trace_cam1(OmvSceneView S
         }
     }
     flushCounters(statSlot(counters), rays, nCam, 0u, 0u, cnt);
-}
-
-// Arguments of the refilling traversal: the queues of one launch (kKind
-// 0..4 as omv_wf_trace: q or sq with its count; kKind 5: the fused launch's
-// camera, connection and environment queues back to back).
-struct WfTraceArgs {
-    WfQueue q; WfSeg qCount;
-    WfShadowQ sq; WfSeg sqCount;
-    WfQueue eq; WfSeg eqCount;
-    WfHits H;
-    uint8_t* vis; uint8_t* nvis;
-    uint32_t nslots; int lc;
-    uint32_t* gstack; unsigned long long* counters; float* splat;
-    uint32_t xcds;
-    int keep;
-};
-
-// Refilling form of the traversal (tuning trace_keep > 0): each lane holds
-// one ray and steps its traversal entry by entry; once fewer than `keep`
-// lanes of the wave are busy, every idle lane takes the next ray of its own
-// list (the XCD-banded walk over the launch's entries, the same hand-out as
-// omv_wf_trace: no atomics, each entry once), so lanes do not idle behind
-// the longest traversal of their wave.  Same per-ray arithmetic (Trav + the
-// masked re-trace loop of sceneIntersect, the occlusion early-out) and the
-// same outputs as omv_wf_trace / omv_wf_trace_fused.
-template <int kKind>
-__global__ __launch_bounds__(OMV_BLOCK, 4) void omv_wf_trace_pt(OmvSceneView S, WfTraceArgs A) {
-    const uint32_t gthreads = gridDim.x * blockDim.x;
-    Stack st;
-    st.init(A.gstack, gthreads);
-    Counters cnt; cnt.zero();
-    uint32_t rays = 0, nCam = 0, nLight = 0, nShadow = 0;
-    // entries [0, nA) camera / light rays of q, [nA, nA + nB) rays of sq,
-    // [nA + nB, total) environment rays of eq (by kKind)
-    __shared__ SegTable cA, cB, cC;
-    segLoad(cA, A.qCount); segLoad(cB, A.sqCount); segLoad(cC, A.eqCount);
-    const uint32_t nA = cA.total(), nB = cB.total(), nC = cC.total();
-    XcdWalk w;
-    w.start(nA + nB + nC, A.xcds);
-    Trav T;
-    bool busy = false;
-    int kind = 0, itr = 0;   // kind of the held ray: 0 q (camera / light), 2 connection / pinhole, 3 environment
-    uint32_t k = 0;          // its index in its own queue
-    f3 org = mk3(0.0f, 0.0f, 0.0f), dir = org, B = org;
-    float t1 = 0.0f;
-    for (;;) {
-        // idle lanes take the next entry of their list
-        if (!busy && w.more()) {
-            const uint32_t e = w.e;
-            w.next();
-            float tn, ts;
-            if (e < nA) {
-                k = e;                       // logical: the hit record's index
-                kind = 0;
-                const uint32_t p = cA.phys(e);
-                const float4 o = A.q.o[p], d = A.q.d[p];
-                org = xyz(o); dir = xyz(d); tn = o.w; t1 = FLT_MAX; ts = -1.0f;
-                if (kKind == 1) ++nLight; else ++nCam;
-            } else if (e < nA + nB) {
-                k = cB.phys(e - nA);         // physical: re-read at the end
-                kind = 2;
-                const float4 a = A.sq.o[k], dd = A.sq.d[k], b = A.sq.b[k];
-                org = xyz(a); dir = xyz(dd); B = xyz(b); tn = a.w; t1 = dd.w;
-                ts = kKind == 4 ? FLT_MAX : connectStop(org, B);
-                ++nShadow;
-            } else {
-                k = cC.phys(e - nA - nB);
-                kind = 3;
-                const float4 o = A.eq.o[k], d = A.eq.d[k];
-                org = xyz(o); dir = xyz(d); tn = o.w; t1 = FLT_MAX; ts = FLT_MAX;
-                ++nShadow;
-            }
-            itr = 10;
-            ++rays;
-            // a zero or NaN direction leaves nothing to traverse: its
-            // result (no hit) is written at the next step
-            T.start(S, org, dir, tn, t1, st, cnt);
-            T.tstop = (S.any_masked || S.closest_only) ? -1.0f : ts;
-            busy = true;
-        }
-        if (__ballot(busy) == 0ull) break;
-        // step until fewer than keep lanes of the wave are busy
-        for (;;) {
-            if (busy) {
-                if (T.more()) T.step(S, st, cnt);
-                if (!T.more()) {
-                    // one traceClosest call finished: sceneIntersect's masked re-trace loop
-                    bool done = true, hit = T.found();
-                    if (hit && S.any_masked) {
-                        const int mesh = S.insts[T.h.inst].mesh_id;
-                        const OmvMaterial& M = S.mats[S.meshes[mesh].mat_id];
-                        if (M.type == OMV_MAT_PBR && M.alpha_mode == OMV_ALPHA_MASK &&
-                            isMaskedHit(S, mesh, T.h.prim, mk3(1.0f - T.h.u - T.h.v, T.h.u, T.h.v))) {
-                            f3 o2 = mk3(org.x + T.h.t * dir.x, org.y + T.h.t * dir.y, org.z + T.h.t * dir.z);
-                            float v = maxAbs(o2);
-                            v = v > T.h.t ? v : T.h.t;
-                            float delta = 3.0f * FLT_EPSILON * v;
-                            const float tn = T.h.t + delta;
-                            hit = false;
-                            T.tnear = tn;
-                            if (!(t1 <= tn) && --itr > 0) {
-                                ++rays;
-                                T.start(S, org, dir, tn, t1, st, cnt);
-                                done = false;
-                            }
-                        }
-                    }
-                    if (done) {
-                        if (kind == 2 && kKind != 4) {
-                            bool visible = true;
-                            if (hit) {
-                                f3 df = sub3(hitPosition(S, T.h), B);
-                                float sd = dot3(df, df);
-                                float safeD = 10.0f * FLT_EPSILON * maxAbs(B);
-                                visible = sd <= safeD * safeD;
-                            }
-                            const uint32_t id = __float_as_uint(A.sq.b[k].w);
-                            const uint32_t slot = id / (uint32_t)A.lc, l = id - slot * (uint32_t)A.lc;
-                            A.vis[(uint64_t)l * A.nslots + slot] = visible ? 2 : 0;
-                        } else if (kind == 2) {
-                            splatAdd(A.splat, !hit, __float_as_uint(A.sq.b[k].w), B);
-                        } else if (kind == 3) {
-                            A.nvis[__float_as_uint(A.eq.d[k].w)] = hit ? 0 : 2;
-                        } else {
-                            float4 r; r.x = T.h.t; r.y = T.h.u; r.z = T.h.v; r.w = T.tnear;
-                            int2 id; id.x = hit ? T.h.inst : -1; id.y = T.h.prim | (T.h.tie ? (int)0x80000000 : 0);
-                            if (hit) A.H.h[k] = r;   // read by the shading kernels for hits only
-                            A.H.id[k] = id;
-                        }
-                        busy = false;
-                    }
-                }
-            }
-            if (__popcll(__ballot(busy)) < A.keep) break;
-        }
-    }
-    flushCounters(statSlot(A.counters), rays, nCam, nLight, nShadow, cnt);
 }
 
 // ---------------------------------------------------------- shade light
@@ -1364,13 +1258,11 @@ void wavefrontBlocksPerCU(int out[9]) {
     const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
     int t = occ(omv_wf_trace<0, true>, lds);
     for (int k : {occ(omv_wf_trace<0, false>, lds), occ(omv_wf_trace<1, true>, lds), occ(omv_wf_trace<1, false>, lds),
-                  occ(omv_wf_trace<4, true>, lds), occ(omv_wf_trace<4, false>, lds), occ(omv_wf_trace_fused<true>, lds),
-                  occ(omv_wf_trace_fused<false>, lds)})
+                  occ(omv_wf_trace<4, true>, lds), occ(omv_wf_trace<4, false>, lds), occ(omv_wf_trace<5, true>, lds),
+                  occ(omv_wf_trace<5, false>, lds)})
         t = std::min(t, k);
-    int tp = occ(omv_wf_trace_pt<0>, lds);
-    for (int k : {occ(omv_wf_trace_pt<1>, lds), occ(omv_wf_trace_pt<4>, lds), occ(omv_wf_trace_pt<5>, lds)}) tp = std::min(tp, k);
     out[0] = t;
-    out[4] = tp;
+    out[4] = t;
     out[1] = occ(omv_wf_shade_cam<true, true>, 0);
     out[5] = occ(omv_wf_shade_cam<true, false>, 0);
     out[6] = occ(omv_wf_shade_cam<false, true>, 0);
@@ -1467,45 +1359,37 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
     const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
     const dim3 blk(OMV_BLOCK);
     const uint32_t xcds = L.xcdBands > 1 ? (uint32_t)L.xcdBands : 1u;
-    // refilling traversal (trace_keep > 0): one argument block per launch
-    auto ptArgs = [&](const WfQueue& q, const WfSeg& qc, const WfSeg& sqc, const WfQueue& e, const WfSeg& ec) {
-        WfTraceArgs a;
-        a.q = q; a.qCount = qc; a.sq = sq; a.sqCount = sqc; a.eq = e; a.eqCount = ec; a.H = H;
-        a.vis = W.vis; a.nvis = W.nvis; a.nslots = n; a.lc = L.lc;
-        a.gstack = L.gstack; a.counters = stats; a.splat = L.splat; a.xcds = xcds; a.keep = L.traceKeep;
-        return a;
-    };
     auto mark = [&]() {
         if (L.traceEv && L.traceEvUsed && *L.traceEvUsed < L.traceEvCap) (void)hipEventRecord(L.traceEv[(*L.traceEvUsed)++], stream);
     };
-    enum { kTraceCamera, kTraceLight, kTraceSplat };
-    auto launchTrace = [&](int what, const WfQueue& q, const WfSeg& count, const WfGen& gen) {
-        auto k = what == kTraceCamera ? (S.any_masked ? omv_wf_trace<0, true> : omv_wf_trace<0, false>)
-                 : what == kTraceLight ? (S.any_masked ? omv_wf_trace<1, true> : omv_wf_trace<1, false>)
-                                       : (S.any_masked ? omv_wf_trace<4, true> : omv_wf_trace<4, false>);
-        hipLaunchKernelGGL(k, dim3(L.blocksTrace), blk, lds, stream, S, q, sq, count, H, L.gstack, stats, L.splat, xcds, gen);
+    auto launchTrace = [&](void (*kernel)(OmvSceneView, WfTraceArgs), const WfQueue& q, const WfSeg& qc, const WfSeg& sqc, const WfSeg& ec,
+                           const WfGen& gen, int keep) {
+        WfTraceArgs a;
+        a.q = q; a.qCount = qc; a.sq = sq; a.sqCount = sqc; a.eq = eq; a.eqCount = ec; a.H = H;
+        a.vis = W.vis; a.nvis = W.nvis; a.nslots = n; a.lc = L.lc;
+        a.gstack = L.gstack; a.counters = stats; a.splat = L.splat; a.xcds = xcds;
+        a.keep = L.traceKeep > 0 ? L.traceKeep : keep; a.G = gen;
+        hipLaunchKernelGGL(kernel, dim3(L.blocksTrace), blk, lds, stream, S, a);
     };
     hipLaunchKernelGGL(omv_wf_fill_u32, dim3((ncnt + 63) / 64), dim3(64), 0, stream, L.qcount, ncnt);
     hipLaunchKernelGGL(omv_wf_fill_u32, dim3(OMV_STAT_SLOTS * 32 / 64), dim3(64), 0, stream, reinterpret_cast<uint32_t*>(stats),
                        OMV_STAT_SLOTS * 32);
-    // Round-1 camera rays: computed by the round-1 camera kernels from the
-    // slot (Gen1), or with the refilling traversal stored by gen in qa;
-    // round-1 light rays are stored in qb
+    // Round-1 camera rays are computed by the round-1 camera kernels from the
+    // slot (Gen1); round-1 light rays are stored in qb
     WfGen Gen1;
     std::memset(&Gen1, 0, sizeof(Gen1));
-    Gen1.gen = L.traceKeep > 0 ? 0 : 1;
+    Gen1.gen = 1;
     Gen1.cam = L.cam; Gen1.seed = P.seed; Gen1.spp = L.p.samples_per_pixel; Gen1.sample0 = L.sample0;
     WfGen Gen0 = Gen1;
     Gen0.gen = 0;
-    const int writeQueues = Gen1.gen ? 0 : 1;
     // with lights, gen appends the round-1 light rays (the queue regions are
     // sized for its grid too: wavefrontSegCap)
     if (lights)
-        hipLaunchKernelGGL(omv_wf_gen<true>, dim3(L.blocksGen), blk, 0, stream, S, L.cam, P, L.p.samples_per_pixel, L.sample0, W, qa, qb,
-                           camCnt(1).cnt, lightCnt(1), L.rad, writeQueues, stats, lost);
+        hipLaunchKernelGGL(omv_wf_gen<true>, dim3(L.blocksGen), blk, 0, stream, S, L.cam, P, L.p.samples_per_pixel, L.sample0, W, qb,
+                           camCnt(1).cnt, lightCnt(1), L.rad, stats, lost);
     else
-        hipLaunchKernelGGL(omv_wf_gen<false>, dim3(L.blocksGen), blk, 0, stream, S, L.cam, P, L.p.samples_per_pixel, L.sample0, W, qa, qb,
-                           camCnt(1).cnt, lightCnt(1), L.rad, writeQueues, stats, lost);
+        hipLaunchKernelGGL(omv_wf_gen<false>, dim3(L.blocksGen), blk, 0, stream, S, L.cam, P, L.p.samples_per_pixel, L.sample0, W, qb,
+                           camCnt(1).cnt, lightCnt(1), L.rad, stats, lost);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // with S.lights_leave generation queues no light ray, and the light
@@ -1514,21 +1398,13 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
         WfQueue in = qb, out = qc;
         for (int i = 1; i < L.lvCap; ++i) {
             mark();
-            if (L.traceKeep > 0)
-                hipLaunchKernelGGL(omv_wf_trace_pt<1>, dim3(L.blocksTrace), blk, lds, stream, S,
-                                   ptArgs(in, lightCnt(i), none, eq, none));
-            else
-                launchTrace(kTraceLight, in, lightCnt(i), Gen0);
+            launchTrace(S.any_masked ? omv_wf_trace<1, true> : omv_wf_trace<1, false>, in, lightCnt(i), none, none, Gen0, kKeepSecondary);
             mark();
             if (splat) {
                 hipLaunchKernelGGL(omv_wf_shade_light<true>, dim3(L.blocksShade), blk, 0, stream, S, L.cam, P, L.sample0, i, W, in, lightCnt(i),
                                    H, out, lightCnt(i + 1), sq, splCnt(i), lost);
                 mark();
-                if (L.traceKeep > 0)
-                    hipLaunchKernelGGL(omv_wf_trace_pt<4>, dim3(L.blocksTrace), blk, lds, stream, S,
-                                       ptArgs(in, none, splCnt(i), eq, none));
-                else
-                    launchTrace(kTraceSplat, in, splCnt(i), Gen0);
+                launchTrace(S.any_masked ? omv_wf_trace<4, true> : omv_wf_trace<4, false>, in, none, splCnt(i), none, Gen0, kKeepSecondary);
                 mark();
             } else {
                 hipLaunchKernelGGL(omv_wf_shade_light<false>, dim3(L.blocksShade), blk, 0, stream, S, L.cam, P, L.sample0, i, W, in, lightCnt(i),
@@ -1573,13 +1449,11 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
         }
         if (!traced) {
             mark();
-            if (L.traceKeep > 0)
-                hipLaunchKernelGGL(omv_wf_trace_pt<0>, dim3(L.blocksTrace), blk, lds, stream, S,
-                                   ptArgs(in, camCnt(i), none, eq, none));
-            else if (i == 1 && Gen1.gen && L.blocksPacket > 0)
+            if (i == 1 && L.blocksPacket > 0)
                 hipLaunchKernelGGL(omv_wf_trace_cam1, dim3(L.blocksPacket), blk, 0, stream, S, camCnt(1), H, stats, xcds, Gen1);
             else
-                launchTrace(kTraceCamera, in, camCnt(i), i == 1 ? Gen1 : Gen0);
+                launchTrace(S.any_masked ? omv_wf_trace<0, true> : omv_wf_trace<0, false>, in, camCnt(i), none, none, i == 1 ? Gen1 : Gen0,
+                            i == 1 ? kKeepPrimary : kKeepSecondary);
             mark();
         }
         traced = false;
@@ -1612,14 +1486,8 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
         // the next round's hits go to H, which this round's connect does not read
         if (fuse) {
             mark();
-            if (L.traceKeep > 0)
-                hipLaunchKernelGGL(omv_wf_trace_pt<5>, dim3(L.blocksTrace), blk, lds, stream, S,
-                                   ptArgs(next, nextInWavefront ? camCnt(i + 1) : none, lights ? shCnt(i) : none, eq,
-                                          nee ? envCnt(i) : none));
-            else
-                hipLaunchKernelGGL(S.any_masked ? omv_wf_trace_fused<true> : omv_wf_trace_fused<false>, dim3(L.blocksTrace), blk, lds, stream, S, next, nextInWavefront ? camCnt(i + 1) : none,
-                                   sq, lights ? shCnt(i) : none, eq, nee ? envCnt(i) : none, H, W.vis, W.nvis, n, L.lc, L.gstack,
-                                   stats, xcds);
+            launchTrace(S.any_masked ? omv_wf_trace<5, true> : omv_wf_trace<5, false>, next, nextInWavefront ? camCnt(i + 1) : none,
+                        lights ? shCnt(i) : none, nee ? envCnt(i) : none, Gen0, kKeepSecondary);
             mark();
             traced = nextInWavefront;
         }

@@ -101,3 +101,28 @@ def test_schedules_agree(pkg, wl, frame, place):
         films.append(r.render(cam))
         assert r.stats()["stack_overflows"] == 0
     assert np.array_equal(films[0], films[1])
+
+
+@pytest.mark.parametrize("keep", [0, 1, 33, 64])
+@pytest.mark.parametrize("size", [(1, 1), (63, 1), (64, 1), (65, 1), (129, 3)])
+def test_refill_at_the_edges_of_a_list(pkg, wl, keep, size):
+    """The refilling traversal at queue lengths around a wave's 64 entries, and
+    at several lists per wave (few workgroups), banded and not: every entry is
+    traced once, so films and ray counts equal the per-sample schedule's."""
+    desc, view = wl.mixed_test_scene(hdr=True, lights=True)
+    view.width, view.height = size
+    s = pkg.Scene()
+    desc.apply(s, pkg.pbr_desc)
+    cam = pkg.Camera(view.width, view.height, view.position, view.forward, view.up, view.yfov)
+    params = dict(samples_per_pixel=1, camera_bounces=5, light_bounces=3, max_path_length=6, seed=21, extensions=pkg.EXT_HDRI_NEE)
+    ref = pkg.Renderer(pkg.default_params(**params))
+    ref.set_scene(s)
+    ref.set_schedule(pkg.SCHEDULE_PER_SAMPLE)
+    want, st = ref.render(cam), ref.stats()
+    for tuning in (dict(), dict(trace_blocks_per_cu=1, xcd_bands=1), dict(xcd_bands=16)):
+        r = pkg.Renderer(pkg.default_params(**params))
+        r.set_scene(s)
+        r.set_tuning(trace_keep=keep, **tuning)
+        assert np.array_equal(r.render(cam), want)
+        for k in ("rays", "camera_rays", "light_rays", "shadow_rays"):
+            assert r.stats()[k] == st[k], k
