@@ -426,7 +426,7 @@ int omv_encode_image(const char* ext, const float* rgba, int width, int height, 
  * Renders the renderer's committed scene with its parameters from camera c
  * into film_dev (device pointer, W*H*4 floats: the normalised film
  * omv_renderer_render gives, bit for bit) on `stream` (a hipStream_t; NULL =
- * the null stream), as one persistent per-pixel kernel.  It calls no
+ * the null stream), as one persistent kernel.  It calls no
  * hipMalloc / hipFree: its only device memory besides the scene and film_dev
  * is a fixed array of OMV_NOALLOC_SCRATCH_BYTES per GPU (counters, traversal
  * spill stacks, light vertices of the resident lanes), which each GPU the
@@ -494,8 +494,8 @@ typedef struct omv_batch omv_batch;
 typedef struct omv_batch_tuning {
     int blocks_per_cu;   /* per-pixel kernel: resident workgroups per CU
                             (0 = occupancy limit)                          */
-    int tile_waves;      /* per-pixel kernel: pixels per work item =
-                            64 * tile_waves (>= 1)                         */
+    int tile_waves;      /* per-pixel kernel: samples per work item, about
+                            256 * tile_waves (>= 1), in whole pixels       */
     int use_graph;       /* 1: replay a captured hipGraph, 0: plain launch */
     int streams;         /* 0: one persistent per-pixel kernel over all
                             jobs; N >= 1: each job's wavefront launch

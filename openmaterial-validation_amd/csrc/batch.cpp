@@ -111,10 +111,10 @@ int BatchRunner::prepare() {
         dirty_ = false;
         return OMV_OK;
     }
-    const uint64_t tilePix = 64ull * (uint64_t)tuning_.tile_waves;
     std::vector<uint64_t> tileEnd(jobs_.size());
     uint64_t t = 0;
     for (size_t i = 0; i < order.size(); ++i) {
+        const uint64_t tilePix = tilePixels(256ull * (uint64_t)tuning_.tile_waves, jobs_[order[i]].p.samples_per_pixel);
         t += (jobs_[order[i]].npix + tilePix - 1) / tilePix;
         tileEnd[i] = t;
     }

@@ -45,11 +45,10 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_bdpt_kernel(OmvSceneView S, omv
 }
 
 // Batched validation jobs in one persistent launch.  Work unit: a tile of
-// 64 x tileWaves consecutive pixels of one job, claimed by a whole wave
-// through one atomic on the work counter; each lane renders all spp samples
-// of its pixel in sample order (the reference's PinholeCamera::hit order)
-// and writes the normalised pixel, so no per-sample buffer is needed and the
-// film equals the plain render's bit for bit.
+// about 256 x tileWaves samples (whole consecutive pixels of one job), claimed
+// by a whole wave through one atomic on the work counter and rendered by
+// renderTile, so no per-sample buffer is needed and the film equals the plain
+// render's bit for bit.
 struct OmvJobDev {
     OmvSceneView S;
     omv_camera_desc cam;
@@ -69,6 +68,7 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_batch_kernel(const OmvJobDev* _
     const uint32_t gthreads = gridDim.x * blockDim.x;
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
+    __shared__ TileStage stage[OMV_BLOCK / 64];
     Lane L;
     laneInit(L, gstack, lv, gtid, gthreads);
     for (;;) {
@@ -82,12 +82,10 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_batch_kernel(const OmvJobDev* _
         const int job = __builtin_amdgcn_readfirstlane(lo);
         const OmvJobDev& J = jobs[job];
         const uint64_t first = (job ? tileEnd[job - 1] : 0ull);
-        const uint64_t pix0 = (t - first) * 64ull * (uint64_t)tileWaves;
-        for (int w = 0; w < tileWaves; ++w) {
-            const uint64_t p = pix0 + (uint64_t)w * 64ull + (uint64_t)lane;
-            if (p >= J.npix) continue;
-            reinterpret_cast<float4*>(J.film)[p] = renderPixel<true, kNee>(J.S, J.cam, J.P, J.spp, p, L);
-        }
+        const uint64_t tilePix = omv::tilePixels(256ull * (uint64_t)tileWaves, J.spp);
+        const uint64_t pix0 = (t - first) * tilePix;
+        renderTile<true, kNee>(J.S, J.cam, J.P, J.spp, pix0, (uint32_t)min(tilePix, J.npix - pix0), J.film,
+                               stage[threadIdx.x >> 6], L);
     }
     flushCounters(counters, L.rays, L.camRays, L.lightRays, L.shadowRays, L.cnt);
 }

@@ -2,7 +2,7 @@
 //
 // Some callers cannot allocate device memory at render time (code under HIP
 // graph capture, tight serving loops, harnesses that forbid hipMalloc).  For
-// them the render runs as one persistent per-pixel kernel whose only device
+// them the render runs as one persistent kernel whose only device
 // memory beyond the committed scene (input) and the caller's film (output)
 // is the file-scope array `scratch` below: the counters, the traversal spill
 // stacks and the light-vertex scratch of every resident lane.  Each GPU the
@@ -28,7 +28,6 @@ namespace {
 // then, 256-aligned, the light vertices, lanes * lvCap * 6 * 4.
 constexpr size_t kCounterBytes = 256;
 constexpr size_t kSpillPerLane = (size_t)(OMV_STACK_TOTAL - OMV_STACK_LDS) * sizeof(uint32_t);
-constexpr int kTileWaves = 2;                // pixels per work item = 64 * kTileWaves
 
 static_assert(OMV_NOALLOC_SCRATCH_BYTES % 256 == 0, "scratch size must be a multiple of 256");
 // the documented light-vertex limit is exactly what the scratch holds for
@@ -41,31 +40,26 @@ static_assert(kCounterBytes + 2 * 256 + (size_t)OMV_NOALLOC_MIN_BLOCKS * OMV_BLO
               "OMV_NOALLOC_MAX_LIGHT_VERTICES is below what the scratch holds");
 static __device__ __align__(256) unsigned char scratch[OMV_NOALLOC_SCRATCH_BYTES];
 
-// One pass over the film: a wave claims kTileWaves * 64 consecutive pixels
-// with one atomic on the work counter; each lane renders its pixel's spp
-// samples in sample order and writes the normalised pixel.  Every wave leaves
-// the loop once the counter has passed the last tile.
+// One pass over the film: a wave claims a tile of tilePix (<= 64) consecutive
+// pixels with one atomic on the work counter and renders it (renderTile).
+// Every wave leaves the loop once the counter has passed the last tile.
 template <bool kLights, bool kNee>
-__global__ __launch_bounds__(OMV_BLOCK) void omv_pixel_kernel(OmvSceneView S, omv_camera_desc cam, RP P, int spp, uint64_t npix,
-                                                              uint64_t tiles, unsigned long long* __restrict__ counters,
-                                                              uint32_t* __restrict__ gstack, float* __restrict__ lv,
-                                                              float* __restrict__ film) {
+__global__ __launch_bounds__(OMV_BLOCK) void omv_noalloc_kernel(OmvSceneView S, omv_camera_desc cam, RP P, int spp, uint64_t npix,
+                                                                uint64_t tiles, uint32_t tilePix, unsigned long long* __restrict__ counters,
+                                                                uint32_t* __restrict__ gstack, float* __restrict__ lv,
+                                                                float* __restrict__ film) {
+    __shared__ TileStage stage[OMV_BLOCK / 64];
     const uint32_t gthreads = gridDim.x * blockDim.x;
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
     Lane L;
     laneInit(L, gstack, lv, gtid, gthreads);
     for (;;) {
         unsigned long long t = 0;
-        if (lane == 0) t = atomicAdd(counters + 8, 1ull);
+        if ((threadIdx.x & 63u) == 0u) t = atomicAdd(counters + 8, 1ull);
         t = __shfl(t, 0, 64);
         if (t >= tiles) break;
-        const uint64_t pix0 = t * 64ull * (uint64_t)kTileWaves;
-        for (int w = 0; w < kTileWaves; ++w) {
-            const uint64_t p = pix0 + (uint64_t)w * 64ull + (uint64_t)lane;
-            if (p >= npix) continue;
-            reinterpret_cast<float4*>(film)[p] = renderPixel<kLights, kNee>(S, cam, P, spp, p, L);
-        }
+        const uint64_t pix0 = t * tilePix;
+        renderTile<kLights, kNee>(S, cam, P, spp, pix0, (uint32_t)min((uint64_t)tilePix, npix - pix0), film, stage[threadIdx.x >> 6], L);
     }
     flushCounters(counters, L.rays, L.camRays, L.lightRays, L.shadowRays, L.cnt);
 }
@@ -94,10 +88,10 @@ void setUp(DeviceSetup& d, int dev) {
     if ((e = hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) { d.err = e; return; }
     const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
     hipError_t o[4];
-    o[0] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[0], omv_pixel_kernel<false, false>, OMV_BLOCK, lds);
-    o[1] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[1], omv_pixel_kernel<false, true>, OMV_BLOCK, lds);
-    o[2] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[2], omv_pixel_kernel<true, false>, OMV_BLOCK, lds);
-    o[3] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[3], omv_pixel_kernel<true, true>, OMV_BLOCK, lds);
+    o[0] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[0], omv_noalloc_kernel<false, false>, OMV_BLOCK, lds);
+    o[1] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[1], omv_noalloc_kernel<false, true>, OMV_BLOCK, lds);
+    o[2] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[2], omv_noalloc_kernel<true, false>, OMV_BLOCK, lds);
+    o[3] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[3], omv_noalloc_kernel<true, true>, OMV_BLOCK, lds);
     for (int i = 0; i < 4; ++i) {
         if (o[i] != hipSuccess) { d.err = o[i]; return; }
         if (d.occ[i] < 1) d.occ[i] = 1;
@@ -138,15 +132,19 @@ int renderNoalloc(const OmvSceneView& S, const omv_camera_desc& cam, const omv_r
         return OMV_E_RANGE;
     }
     const uint64_t npix = (uint64_t)cam.width * (uint64_t)cam.height;
-    const uint64_t tiles = (npix + 64ull * kTileWaves - 1) / (64ull * kTileWaves);
     // resident blocks: the occupancy limit, as many as the scratch holds, and
-    // no more than there are work items for (two waves per block)
+    // no more than there are batches of 64 samples for (two waves per block)
+    const int spp = p.samples_per_pixel;
+    const uint64_t samples = npix * (uint64_t)std::max(spp, 1);
     const int occ = d.occ[(lights ? 2 : 0) + (P.x.nee ? 1 : 0)];
     uint64_t blocks = (uint64_t)d.cus * (uint64_t)occ;
     const uint64_t fit = ((size_t)OMV_NOALLOC_SCRATCH_BYTES - kCounterBytes - 2 * 256) / (perLane * OMV_BLOCK);
     blocks = std::min(blocks, fit);
-    blocks = std::min<uint64_t>(blocks, std::max<uint64_t>(1, (tiles + 1) / 2));
+    blocks = std::min<uint64_t>(blocks, (samples + OMV_BLOCK - 1) / OMV_BLOCK);
     blocks = std::max<uint64_t>(blocks, 1);
+    // about four tiles for every resident wave
+    const uint32_t tilePix = (uint32_t)tilePixels(samples / (blocks * (OMV_BLOCK / 64) * 4), spp);
+    const uint64_t tiles = (npix + tilePix - 1) / tilePix;
     const uint64_t lanes = blocks * OMV_BLOCK;
     unsigned long long* counters = reinterpret_cast<unsigned long long*>(d.ptr);
     uint32_t* gstack = reinterpret_cast<uint32_t*>(d.ptr + kCounterBytes);
@@ -159,15 +157,14 @@ int renderNoalloc(const OmvSceneView& S, const omv_camera_desc& cam, const omv_r
     if ((err = hipGetLastError()) != hipSuccess) { what = "render_noalloc: clear launch"; return OMV_E_DEVICE; }
     const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
     const dim3 g((unsigned)blocks), b(OMV_BLOCK);
-    const int spp = p.samples_per_pixel;
     if (lights && P.x.nee)
-        hipLaunchKernelGGL((omv_pixel_kernel<true, true>), g, b, lds, stream, S, cam, P, spp, npix, tiles, counters, gstack, lv, film);
+        hipLaunchKernelGGL((omv_noalloc_kernel<true, true>), g, b, lds, stream, S, cam, P, spp, npix, tiles, tilePix, counters, gstack, lv, film);
     else if (lights)
-        hipLaunchKernelGGL((omv_pixel_kernel<true, false>), g, b, lds, stream, S, cam, P, spp, npix, tiles, counters, gstack, lv, film);
+        hipLaunchKernelGGL((omv_noalloc_kernel<true, false>), g, b, lds, stream, S, cam, P, spp, npix, tiles, tilePix, counters, gstack, lv, film);
     else if (P.x.nee)
-        hipLaunchKernelGGL((omv_pixel_kernel<false, true>), g, b, lds, stream, S, cam, P, spp, npix, tiles, counters, gstack, lv, film);
+        hipLaunchKernelGGL((omv_noalloc_kernel<false, true>), g, b, lds, stream, S, cam, P, spp, npix, tiles, tilePix, counters, gstack, lv, film);
     else
-        hipLaunchKernelGGL((omv_pixel_kernel<false, false>), g, b, lds, stream, S, cam, P, spp, npix, tiles, counters, gstack, lv, film);
+        hipLaunchKernelGGL((omv_noalloc_kernel<false, false>), g, b, lds, stream, S, cam, P, spp, npix, tiles, tilePix, counters, gstack, lv, film);
     if ((err = hipGetLastError()) != hipSuccess) { what = "render_noalloc: kernel launch"; return OMV_E_DEVICE; }
     if (statsOut) {
         if ((err = hipMemcpyAsync(statsOut, counters, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, stream)) != hipSuccess) {

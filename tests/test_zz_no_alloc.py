@@ -103,3 +103,24 @@ def test_noalloc_refusals(pkg, wl):
     want, _ = _plain(pkg, scene, p3, cam)
     got, _ = _noalloc(pkg, r3, cam)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("spp", [0, 1, 5, 63, 64, 65, 200])
+@pytest.mark.parametrize("size", [(1, 1), (63, 1), (13, 5)])
+def test_noalloc_tiles(pkg, wl, spp, size):
+    """A wave renders a tile of whole pixels 64 samples at a time: sample counts
+    below, at and above a batch, with tiles and films that do not fill one.
+    The batch form of the same film (its default tuning) agrees too."""
+    scene, view, params = _setup(pkg, wl, samples_per_pixel=spp, camera_bounces=3, light_bounces=2, max_path_length=3)
+    cam = _cam(pkg, view, *size)
+    want, _ = _plain(pkg, scene, params, cam)
+    r = pkg.Renderer(pkg.default_params(**params))
+    r.set_scene(scene)
+    got, _ = _noalloc(pkg, r, cam)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    b = pkg.Batch()
+    for _ in range(2):
+        b.add_job(scene, cam, pkg.default_params(**params))
+    b.set_tuning(tile_waves=3, use_graph=False)
+    b.run()
+    assert np.array_equal(b.film(1).view(np.uint32), want.view(np.uint32))
