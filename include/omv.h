@@ -335,6 +335,9 @@ int omv_renderer_get_stats(const omv_renderer* r, omv_render_stats* out);
  *   OMV_SCHEDULE_WAVEFRONT   (default) ray queues: gen, then per bounce a
  *                            traversal kernel and a shading kernel
  *                            (+ connection visibility and sum with lights);
+ *                            with the default tuning a render of at most
+ *                            2^18 samples is one launch over film tiles
+ *                            (counted as one traversal launch);
  *   OMV_SCHEDULE_PER_SAMPLE  one persistent kernel, one lane per sample. */
 #define OMV_SCHEDULE_WAVEFRONT   0
 #define OMV_SCHEDULE_PER_SAMPLE  1

@@ -44,10 +44,10 @@ static __device__ __align__(256) unsigned char scratch[OMV_NOALLOC_SCRATCH_BYTES
 // pixels with one atomic on the work counter and renders it (renderTile).
 // Every wave leaves the loop once the counter has passed the last tile.
 template <bool kLights, bool kNee>
-__global__ __launch_bounds__(OMV_BLOCK) void omv_noalloc_kernel(OmvSceneView S, omv_camera_desc cam, RP P, int spp, uint64_t npix,
-                                                                uint64_t tiles, uint32_t tilePix, unsigned long long* __restrict__ counters,
-                                                                uint32_t* __restrict__ gstack, float* __restrict__ lv,
-                                                                float* __restrict__ film) {
+__global__ __launch_bounds__(OMV_BLOCK) void omv_tile_kernel(OmvSceneView S, omv_camera_desc cam, RP P, int spp, uint64_t npix,
+                                                             uint64_t tiles, uint32_t tilePix, unsigned long long* __restrict__ counters,
+                                                             unsigned long long* __restrict__ work, uint32_t* __restrict__ gstack,
+                                                             float* __restrict__ lv, float* __restrict__ film) {
     __shared__ TileStage stage[OMV_BLOCK / 64];
     const uint32_t gthreads = gridDim.x * blockDim.x;
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_noalloc_kernel(OmvSceneView S, 
     laneInit(L, gstack, lv, gtid, gthreads);
     for (;;) {
         unsigned long long t = 0;
-        if ((threadIdx.x & 63u) == 0u) t = atomicAdd(counters + 8, 1ull);
+        if ((threadIdx.x & 63u) == 0u) t = atomicAdd(work, 1ull);
         t = __shfl(t, 0, 64);
         if (t >= tiles) break;
         const uint64_t pix0 = t * tilePix;
@@ -88,10 +88,10 @@ void setUp(DeviceSetup& d, int dev) {
     if ((e = hipDeviceGetAttribute(&d.cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) { d.err = e; return; }
     const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
     hipError_t o[4];
-    o[0] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[0], omv_noalloc_kernel<false, false>, OMV_BLOCK, lds);
-    o[1] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[1], omv_noalloc_kernel<false, true>, OMV_BLOCK, lds);
-    o[2] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[2], omv_noalloc_kernel<true, false>, OMV_BLOCK, lds);
-    o[3] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[3], omv_noalloc_kernel<true, true>, OMV_BLOCK, lds);
+    o[0] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[0], omv_tile_kernel<false, false>, OMV_BLOCK, lds);
+    o[1] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[1], omv_tile_kernel<false, true>, OMV_BLOCK, lds);
+    o[2] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[2], omv_tile_kernel<true, false>, OMV_BLOCK, lds);
+    o[3] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&d.occ[3], omv_tile_kernel<true, true>, OMV_BLOCK, lds);
     for (int i = 0; i < 4; ++i) {
         if (o[i] != hipSuccess) { d.err = o[i]; return; }
         if (d.occ[i] < 1) d.occ[i] = 1;
@@ -103,6 +103,31 @@ size_t alignUp(size_t x) { return (x + 255) & ~(size_t)255; }
 }  // namespace
 
 namespace omv {
+
+int tileBlocksPerCU(bool lights, bool nee) {
+    int n = 0;
+    const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
+    auto k = lights ? (nee ? omv_tile_kernel<true, true> : omv_tile_kernel<true, false>)
+                    : (nee ? omv_tile_kernel<false, true> : omv_tile_kernel<false, false>);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, OMV_BLOCK, lds) != hipSuccess || n < 1) n = 1;
+    return n;
+}
+
+hipError_t launchTiles(const OmvSceneView& S, const omv_camera_desc& cam, const omv_renderer_params& p, float* film,
+                       unsigned long long* counters, unsigned long long* work, uint32_t* gstack, float* lv, int blocks, hipStream_t stream) {
+    RP P = toRP(p);
+    if (!S.env_tex_pdf) P.x.nee = false;   // no HDR environment: nothing to sample
+    P.x.splat = false;
+    const uint64_t npix = (uint64_t)cam.width * (uint64_t)cam.height, samples = npix * (uint64_t)std::max(p.samples_per_pixel, 1);
+    // about four tiles for every resident wave
+    const uint32_t tilePix = (uint32_t)tilePixels(samples / ((uint64_t)blocks * (OMV_BLOCK / 64) * 4), p.samples_per_pixel);
+    const uint64_t tiles = (npix + tilePix - 1) / tilePix;
+    auto k = S.num_lights > 0 ? (P.x.nee ? omv_tile_kernel<true, true> : omv_tile_kernel<true, false>)
+                              : (P.x.nee ? omv_tile_kernel<false, true> : omv_tile_kernel<false, false>);
+    hipLaunchKernelGGL(k, dim3((unsigned)blocks), dim3(OMV_BLOCK), (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t), stream, S, cam, P,
+                       p.samples_per_pixel, npix, tiles, tilePix, counters, work, gstack, lv, film);
+    return hipGetLastError();
+}
 
 size_t noallocLaneBytes(int lvCap, bool lights) {
     return kSpillPerLane + (lights ? (size_t)lvCap * 6 * sizeof(float) : 0);
@@ -134,17 +159,13 @@ int renderNoalloc(const OmvSceneView& S, const omv_camera_desc& cam, const omv_r
     const uint64_t npix = (uint64_t)cam.width * (uint64_t)cam.height;
     // resident blocks: the occupancy limit, as many as the scratch holds, and
     // no more than there are batches of 64 samples for (two waves per block)
-    const int spp = p.samples_per_pixel;
-    const uint64_t samples = npix * (uint64_t)std::max(spp, 1);
+    const uint64_t samples = npix * (uint64_t)std::max(p.samples_per_pixel, 1);
     const int occ = d.occ[(lights ? 2 : 0) + (P.x.nee ? 1 : 0)];
     uint64_t blocks = (uint64_t)d.cus * (uint64_t)occ;
     const uint64_t fit = ((size_t)OMV_NOALLOC_SCRATCH_BYTES - kCounterBytes - 2 * 256) / (perLane * OMV_BLOCK);
     blocks = std::min(blocks, fit);
     blocks = std::min<uint64_t>(blocks, (samples + OMV_BLOCK - 1) / OMV_BLOCK);
     blocks = std::max<uint64_t>(blocks, 1);
-    // about four tiles for every resident wave
-    const uint32_t tilePix = (uint32_t)tilePixels(samples / (blocks * (OMV_BLOCK / 64) * 4), spp);
-    const uint64_t tiles = (npix + tilePix - 1) / tilePix;
     const uint64_t lanes = blocks * OMV_BLOCK;
     unsigned long long* counters = reinterpret_cast<unsigned long long*>(d.ptr);
     uint32_t* gstack = reinterpret_cast<uint32_t*>(d.ptr + kCounterBytes);
@@ -155,17 +176,10 @@ int renderNoalloc(const OmvSceneView& S, const omv_camera_desc& cam, const omv_r
 
     hipLaunchKernelGGL(omv_noalloc_clear, dim3(1), dim3(64), 0, stream, counters);
     if ((err = hipGetLastError()) != hipSuccess) { what = "render_noalloc: clear launch"; return OMV_E_DEVICE; }
-    const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
-    const dim3 g((unsigned)blocks), b(OMV_BLOCK);
-    if (lights && P.x.nee)
-        hipLaunchKernelGGL((omv_noalloc_kernel<true, true>), g, b, lds, stream, S, cam, P, spp, npix, tiles, tilePix, counters, gstack, lv, film);
-    else if (lights)
-        hipLaunchKernelGGL((omv_noalloc_kernel<true, false>), g, b, lds, stream, S, cam, P, spp, npix, tiles, tilePix, counters, gstack, lv, film);
-    else if (P.x.nee)
-        hipLaunchKernelGGL((omv_noalloc_kernel<false, true>), g, b, lds, stream, S, cam, P, spp, npix, tiles, tilePix, counters, gstack, lv, film);
-    else
-        hipLaunchKernelGGL((omv_noalloc_kernel<false, false>), g, b, lds, stream, S, cam, P, spp, npix, tiles, tilePix, counters, gstack, lv, film);
-    if ((err = hipGetLastError()) != hipSuccess) { what = "render_noalloc: kernel launch"; return OMV_E_DEVICE; }
+    if ((err = launchTiles(S, cam, p, film, counters, counters + 8, gstack, lv, (int)blocks, stream)) != hipSuccess) {
+        what = "render_noalloc: kernel launch";
+        return OMV_E_DEVICE;
+    }
     if (statsOut) {
         if ((err = hipMemcpyAsync(statsOut, counters, 8 * sizeof(unsigned long long), hipMemcpyDeviceToHost, stream)) != hipSuccess) {
             what = "render_noalloc: counter read-back";

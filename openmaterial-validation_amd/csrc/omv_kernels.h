@@ -72,6 +72,11 @@ __host__ __device__ inline uint64_t tilePixels(uint64_t samples, int spp) {
     const uint64_t pix = want / n;
     return pix < 1 ? 1 : (pix > 64 ? 64 : pix);
 }
+// A whole film as one persistent launch over such tiles (noalloc.hip): work is
+// a zeroed work counter, gstack and lv hold blocks * OMV_BLOCK lanes.
+int tileBlocksPerCU(bool lights, bool nee);
+hipError_t launchTiles(const OmvSceneView& S, const omv_camera_desc& cam, const omv_renderer_params& p, float* film,
+                       unsigned long long* counters, unsigned long long* work, uint32_t* gstack, float* lv, int blocks, hipStream_t stream);
 // Ray queues are appended to through OMV_QSEG counters each (one per group of
 // producing workgroups); wavefrontSegCap is the entries of one group's region
 // for a producing launch of gridShade workgroups (blocksShade).

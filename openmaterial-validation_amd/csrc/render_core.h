@@ -170,6 +170,7 @@ private:
     int initStream();
     int renderSamples(PinholeCamera& cam, double& kernelMs);
     int renderWavefront(PinholeCamera& cam, double& kernelMs);
+    int renderTiles(PinholeCamera& cam, int lvCap);
     void collectWavefrontTiming(double& kernelMs);
     int wfEvUsed_ = 0;
     bool wfTimingPending_ = false;
@@ -178,6 +179,7 @@ private:
     omv_render_tuning tuning_{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     OmvSceneView viewForLaunch() const;   // the scene view with the tuning's traversal order
     int wfPerCu_[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    int tilePerCu_[4] = {0, 0, 0, 0};   // [lights][nee]
     RenderScene* scene_ = nullptr;
     omv_render_stats stats_{};
     hipStream_t stream_ = nullptr;

@@ -371,6 +371,20 @@ hipError_t launchBatch(const void* jobs, int njobs, const uint64_t* tileEnd, uin
     });
     return hipSuccess;
 }
+int tileBlocksPerCU(bool, bool) { return 4; }
+hipError_t launchTiles(const OmvSceneView& S, const omv_camera_desc& cam, const omv_renderer_params& p, float* film,
+                       unsigned long long* counters, unsigned long long* work, uint32_t* gstack, float* lv, int blocks, hipStream_t stream) {
+    op(stream, "tiles", [=]() {
+        inRange(film, (size_t)cam.width * cam.height * 16, "tiles film");
+        inRange(counters, 56, "tiles counters");
+        inRange(work, 8, "tiles work counter");
+        inRange(gstack, (size_t)blocks * OMV_BLOCK * (OMV_STACK_TOTAL - OMV_STACK_LDS) * 4, "tiles gstack");
+        if (S.num_lights > 0)
+            inRange(lv, (size_t)blocks * OMV_BLOCK * std::max(std::min(p.light_bounces + 1, std::max(p.max_path_length, 1)), 1) * 24, "tiles lv");
+        sceneCheck(S, "tiles");
+    });
+    return hipSuccess;
+}
 hipError_t launchBdpt(const OmvSceneView& S, const omv_camera_desc&, const omv_renderer_params&, uint64_t, uint64_t nsamples, float* rad, float*,
                       uint32_t*, unsigned long long* counters, int, float*, hipStream_t stream) {
     op(stream, "bdpt", [=]() { inRange(rad, nsamples * 12, "bdpt rad"); inRange(counters, 64, "bdpt counters"); sceneCheck(S, "bdpt"); });

@@ -65,3 +65,27 @@ def test_small_film_ids(pkg, wl, ref, w, h):
     desc.apply(rs, ref.pbr_desc)
     rfilm, rids, rtie = rs.render_fc(ref.default_params(seed=7), cam.desc())
     assert np.array_equal(ids, rids) and np.array_equal(tie, rtie) and np.array_equal(film, rfilm)
+
+
+@pytest.mark.parametrize("ext", [0, 1, 2])
+@pytest.mark.parametrize("lights", [False, True])
+def test_default_schedule_at_the_tile_limit(pkg, wl, lights, ext):
+    """With the default tuning a render of at most 2^18 samples is one launch
+    over film tiles, a larger one ray-queue rounds: on both sides of the limit
+    film and ray counts equal those of the rounds (any tuning set) bit for bit,
+    also when one renderer goes from one to the other and back."""
+    desc, view = wl.mixed_test_scene(hdr=True, lights=lights, masked=True)
+    s = pkg.Scene()
+    desc.apply(s, pkg.pbr_desc)
+    params = dict(samples_per_pixel=4, camera_bounces=3, light_bounces=2, max_path_length=4, seed=5, extensions=ext)
+    r, q = pkg.Renderer(pkg.default_params(**params)), pkg.Renderer(pkg.default_params(**params))
+    q.set_tuning(tail_round=1)
+    for x in (r, q):
+        x.set_scene(s)
+    for w, h in ((256, 256), (257, 256), (37, 5)):
+        cam = pkg.Camera(w, h, view.position, view.forward, view.up, view.yfov)
+        assert np.array_equal(r.render(cam), q.render(cam))
+        a, b = r.stats(), q.stats()
+        for k in ("samples", "rays", "camera_rays", "light_rays", "shadow_rays", "stack_overflows"):
+            assert a[k] == b[k], k
+        assert (a["trace_launches"] == 1) == (w * h * 4 <= 1 << 18)
