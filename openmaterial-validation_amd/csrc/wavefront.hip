@@ -49,14 +49,21 @@
 namespace {
 
 // ----------------------------------------------------------- state layout
-struct WfQueue {       // one ray queue
+// One ray queue.  What a path carries from round to round travels in its
+// queue entry, so shading reads it in order with the ray; indexed by the
+// path's slot it cost 76 scattered bytes a vertex, and a vertex count, a
+// radiance that is still zero and flags besides (MI355X: instanced 1080p x 16
+// 9.13 -> 8.90 ms, torus knot 512^2 x 64 4.85 -> 4.76, batch 30.8 -> 30.0).
+struct WfQueue {
     float4* o;         // origin xyz, tnear
     float4* d;         // direction xyz, as_float(slot)
+    float4* t;         // camera rays of round 2 on: throughput xyz, as_float(camera stream draws consumed)
+    float* w;          // likewise, OMV_EXT_HDRI_NEE: MIS weight of an escape
 };
 struct WfShadowQ {     // connection visibility rays (isConnected, BDPTRenderer.cpp:208-235)
     float4* o;         // A xyz (light vertex), tnear = safeD
     float4* d;         // unit direction xyz, tfar
-    float4* b;         // B xyz (camera vertex), as_float(slot * lc + l)
+    float4* b;         // B xyz (camera vertex), as_float(entry * lc + l)
 };
 struct WfHits {
     float4* h;         // t, u, v, tnear after the masked re-trace loop (written for hits only)
@@ -64,19 +71,17 @@ struct WfHits {
 };
 struct WfState {
     uint32_t n;        // slots
-    float4* thr;       // camera throughput xyz, MIS weight of an escape (OMV_EXT_HDRI_NEE)
-    float4* radc;      // camera radiance xyz, as_float(vertex count)
+    float4* rad;       // camera radiance so far xyz (written and read with emission or OMV_EXT_HDRI_NEE only)
     float4* conn;      // connection sum xyz
-    uint32_t* csn;     // camera stream draws consumed
-    uint32_t* flags;   // 0 running, 1 ends after this round's connections, 2 written
-    uint32_t* nconn;   // connections staged this round
+    uint32_t* info;    // [entry of the round] connections staged << 2 | 0 running, 1 ends after this round's
+                       // connections, 2 written (lights or OMV_EXT_HDRI_NEE only)
     float4* lthr;      // light throughput xyz, first-hit attenuation rD
     uint32_t* lsn;     // light stream draws consumed
     int* lidx;         // sampled light
     int* lplen;        // light subpath vertex count
     float* lv;         // light vertices [vertex][6][slot]
-    float* cc;         // staged connection contributions [l][3][slot]
-    uint8_t* vis;      // [l][slot] 0 none/blocked, 1 pending, 2 visible
+    float* cc;         // staged connection contributions [l][3][entry]
+    uint8_t* vis;      // [l][entry] 0 none/blocked, 1 pending, 2 visible
     float4* lbeta;     // light-tracer particle weight for the next vertex (OMV_EXT_LIGHT_SPLAT)
     float4* neeC;      // staged next-event contribution xyz (OMV_EXT_HDRI_NEE)
     uint8_t* nvis;     // [slot] its visibility: 0 none/blocked, 1 pending, 2 visible
@@ -339,13 +344,11 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_gen(OmvSceneView S, omv_came
         // the initial camera state (throughput 1, escape weight 1, radiance 0
         // after 1 vertex, connection sum 0, 2 draws consumed) is not stored:
         // camera round 1 and its connect kernel start from it
-        W.flags[slot] = 0u;
         if (!camRays) {
             // no camera vertex: conn * 1 + radiance with both zero
             rad[(uint64_t)slot * 3 + 0] = 0.0f;
             rad[(uint64_t)slot * 3 + 1] = 0.0f;
             rad[(uint64_t)slot * 3 + 2] = 0.0f;
-            W.flags[slot] = 2u;
         }
         if (kLights) {
             // light vertex 0 is the sampled light itself (read from the light
@@ -490,8 +493,8 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TRACE_WAVES) void omv_wf_trace(OmvSc
                         visible = sd <= safeD * safeD;
                     }
                     const uint32_t id = __float_as_uint(b.w);
-                    const uint32_t slot = id / (uint32_t)A.lc, l = id - slot * (uint32_t)A.lc;
-                    A.vis[(uint64_t)l * A.nslots + slot] = visible ? 2 : 0;
+                    const uint32_t entry = id / (uint32_t)A.lc, l = id - entry * (uint32_t)A.lc;
+                    A.vis[(uint64_t)l * A.nslots + entry] = visible ? 2 : 0;
                 }
             } else {
                 A.nvis[__float_as_uint(A.eq.d[cC.phys(e - nA - nB)].w)] = hit ? 0 : 2;
@@ -855,36 +858,44 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
     const uint64_t N = W.n;
     const int q = P.q;
     const bool gen = G.gen && i == 1;
+    const bool glow = kNee || S.any_emissive;   // radiance is collected before the path's end
     for (uint32_t e = gtid; e < total; e += gthreads) {
         uint32_t slot;
         f3 pDir;
+        f3 of = mk3(1.0f, 1.0f, 1.0f), radiance = mk3(0.0f, 0.0f, 0.0f);
+        float escIn = 1.0f;
+        uint32_t draws = 2u;   // the camera jitter's
+        const int2 id = H.id[e];
+        const bool first = i == 1;
         if (gen) {   // round 1: the camera ray of slot e
             f3 org;
             slot = e;
             genCameraRay(G.cam, G.seed, G.spp, G.sample0 + e, org, pDir);
         } else {
-            const float4 dd = in.d[cur.phys(e)];
+            const uint32_t p = cur.phys(e);
+            const float4 dd = in.d[p];
             slot = __float_as_uint(dd.w);
             pDir = xyz(dd);
+            if (!first) {
+                const float4 th = in.t[p];
+                of = xyz(th);
+                draws = __float_as_uint(th.w);
+                if (kNee) escIn = in.w[p];
+                if (glow) radiance = xyz(W.rad[slot]);
+            }
         }
-        const int2 id = H.id[e];
-        const bool first = i == 1;
-        const float4 rc = first ? f4of(mk3(0.0f, 0.0f, 0.0f), __int_as_float(1)) : W.radc[slot];
-        f3 radiance = xyz(rc);
-        int n = __float_as_int(rc.w);
-        const float4 th = first ? f4of(mk3(1.0f, 1.0f, 1.0f), 1.0f) : W.thr[slot];
-        f3 of = xyz(th);
+        int n = i;   // vertices so far: every round before this one added one
         bool emit = false, envRay = false;
         f3 eOrg = mk3(0.0f, 0.0f, 0.0f), eDir = eOrg;
         f3 nPos = mk3(0.0f, 0.0f, 0.0f), nDir = nPos;
-        float nTnear = 0.0f;
+        float nTnear = 0.0f, escW = 1.0f;
         if (id.x < 0) {
             // escape (BDPTRenderer.cpp:251-258); no connections this round
             // (the path is written here, so the connect kernel reads nothing else of it)
             if (S.bg_type != OMV_BG_NONE && n <= q) {
                 f3 bg = background(S, pDir);
                 bg = mk3(bg.x * of.x, bg.y * of.y, bg.z * of.z);
-                if (kNee) bg = mk3(bg.x * th.w, bg.y * th.w, bg.z * th.w);
+                if (kNee) bg = mk3(bg.x * escIn, bg.y * escIn, bg.z * escIn);
                 radiance = mk3(bg.x * 1.0f + radiance.x, bg.y * 1.0f + radiance.y, bg.z * 1.0f + radiance.z);
             }
             // the connection sum exists with point lights only (0 before round 1's connect)
@@ -892,8 +903,9 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
             rad[(uint64_t)slot * 3 + 0] = conn.x * 1.0f + radiance.x;
             rad[(uint64_t)slot * 3 + 1] = conn.y * 1.0f + radiance.y;
             rad[(uint64_t)slot * 3 + 2] = conn.z * 1.0f + radiance.z;
-            W.flags[slot] = 2u;
+            if (kLights || kNee) W.info[e] = 2u;
         } else {
+            uint32_t staged = 0u;
             const float4 hr = H.h[e];
             Hit h; h.t = hr.x; h.u = hr.y; h.v = hr.z; h.inst = id.x; h.prim = id.y & 0x7FFFFFFF; h.tie = id.y < 0;
             SP sp;
@@ -907,7 +919,7 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
                 const f3 lightInt = ld3(Lt.intensity);
                 const int lEnd = min(S.lights_leave ? 1 : W.lplen[slot], q - i + 1);
                 const f3 outV = neg3(pDir);
-                W.nconn[slot] = (uint32_t)max(lEnd, 0);
+                staged = (uint32_t)max(lEnd, 0);
                 for (int l = 0; l < lEnd; ++l) {
                     f3 lPos = l == 0 ? ld3(Lt.pos)
                                      : mk3(W.lv[((uint64_t)l * 6 + 0) * N + slot], W.lv[((uint64_t)l * 6 + 1) * N + slot],
@@ -947,9 +959,9 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
                                 v = 1;
                                 ray = true;
                             }
-                            W.cc[((uint64_t)l * 3 + 0) * N + slot] = lc.x;
-                            W.cc[((uint64_t)l * 3 + 1) * N + slot] = lc.y;
-                            W.cc[((uint64_t)l * 3 + 2) * N + slot] = lc.z;
+                            W.cc[((uint64_t)l * 3 + 0) * N + e] = lc.x;
+                            W.cc[((uint64_t)l * 3 + 1) * N + e] = lc.y;
+                            W.cc[((uint64_t)l * 3 + 2) * N + e] = lc.z;
                         }
                     }
                     // connections to the light itself grouped by light (key = light index),
@@ -958,16 +970,16 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
                     const uint32_t key = nk > 1u ? (l == 0 ? (uint32_t)li : (uint32_t)S.num_lights) : 0u;
                     const uint32_t k = segAppendKeyed(sqCount, ray, key, nk, lost);
                     if (ray && k == OMV_SEG_NONE) v = 0;   // a full region (cannot happen with the host's sizing)
-                    W.vis[(uint64_t)l * N + slot] = v;
+                    W.vis[(uint64_t)l * N + e] = v;
                     if (k != OMV_SEG_NONE) {
                         sq.o[k] = f4of(A, tnear);
                         sq.d[k] = f4of(dir, tfar);
-                        sq.b[k] = f4of(B, __uint_as_float(slot * (uint32_t)W.lc + (uint32_t)l));
+                        sq.b[k] = f4of(B, __uint_as_float(e * (uint32_t)W.lc + (uint32_t)l));
                     }
                 }
             }
             Rng cs;
-            rngRestore(cs, P.seed, STREAM_CAMERA, sample0 + slot, first ? 2u : W.csn[slot]);   // 2: the camera jitter's draws
+            rngRestore(cs, P.seed, STREAM_CAMERA, sample0 + slot, draws);
             f3 outRay, brdf, erad;
             BounceInfo bi;
             matGetRayAndBrdf(S, P.x, sp, pDir, outRay, brdf, erad, true, cs, kNee ? &bi : nullptr, kLights ? &mi : nullptr);
@@ -975,7 +987,6 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
             const f3 ofPrev = of;
             of = mk3(of.x * brdf.x * ct, of.y * brdf.y * ct, of.z * brdf.z * ct);
             radiance = mk3(radiance.x + of.x * erad.x, radiance.y + of.y * erad.y, radiance.z + of.z * erad.z);
-            float escW = 1.0f;
             if (kNee) {
                 f3 c;
                 envRay = neePrepare(S, P, sp, bi, ofPrev, outRay, i, sample0 + slot, escW, c, eOrg, eDir);
@@ -983,9 +994,8 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
                 W.nvis[slot] = envRay ? 1 : 0;
             }
             ++n;
-            W.csn[slot] = rngConsumed(cs);
-            W.thr[slot] = f4of(of, escW);
-            W.radc[slot] = f4of(radiance, __int_as_float(n));
+            draws = rngConsumed(cs);
+            if (glow) W.rad[slot] = f4of(radiance, 0.0f);
             // continue unless the loop ends (i == B) or an exact shortcut stops it
             const bool zero = of.x == 0.0f && of.y == 0.0f && of.z == 0.0f;
             const bool cont = i < P.camera_bounces && !zero && (S.any_emissive || n <= q);
@@ -995,20 +1005,20 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
                 nPos = mk3(sp.pos.x + delta * outRay.x, sp.pos.y + delta * outRay.y, sp.pos.z + delta * outRay.z);
                 nDir = outRay;
                 nTnear = hr.w;
-            } else if (kLights || kNee) {
-                W.flags[slot] = 1u;   // written by the connect kernel of this round
-            } else {
+            } else if (!(kLights || kNee)) {   // else written by the connect kernel of this round
                 const f3 conn = mk3(0.0f, 0.0f, 0.0f);   // no point lights: no connections
                 rad[(uint64_t)slot * 3 + 0] = conn.x * 1.0f + radiance.x;
                 rad[(uint64_t)slot * 3 + 1] = conn.y * 1.0f + radiance.y;
                 rad[(uint64_t)slot * 3 + 2] = conn.z * 1.0f + radiance.z;
-                W.flags[slot] = 2u;
             }
+            if (kLights || kNee) W.info[e] = staged << 2 | (cont ? 0u : 1u);
         }
         const uint32_t k = segAppend(outCount, emit, lost);
         if (k != OMV_SEG_NONE) {
             out.o[k] = f4of(nPos, nTnear);
             out.d[k] = f4of(nDir, __uint_as_float(slot));
+            out.t[k] = f4of(of, __uint_as_float(draws));
+            if (kNee) out.w[k] = escW;
         }
         if (kNee) {
             const uint32_t ke = segAppend(eqCount, envRay, lost);
@@ -1027,7 +1037,7 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
 // per-sample function does), and writes the sample of paths that ended
 // this round.
 __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_connect(WfState W, WfQueue in, WfSeg inCount, float* __restrict__ rad, int lights,
-                                                            int nee, int round, int gen) {
+                                                            int nee, int glow, int round, int gen) {
     const uint32_t gthreads = gridDim.x * blockDim.x;
     const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
     __shared__ SegTable cur;
@@ -1036,16 +1046,15 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_connect(WfState W, WfQueue i
     const uint64_t N = W.n;
     const bool slotIsEntry = gen && round == 1;   // round-1 rays computed from the slot: entry e is slot e
     for (uint32_t e = gtid; e < total; e += gthreads) {
-        const uint32_t slot = slotIsEntry ? e : __float_as_uint(in.d[cur.phys(e)].w);
-        const uint32_t fl = W.flags[slot];
+        const uint32_t info = W.info[e], fl = info & 3u;
         if (fl == 2u) continue;
+        const uint32_t slot = slotIsEntry ? e : __float_as_uint(in.d[cur.phys(e)].w);
         f3 conn = (lights && round > 1) ? xyz(W.conn[slot]) : mk3(0.0f, 0.0f, 0.0f);
         if (lights) {
-            const uint32_t nc = W.nconn[slot];
+            const uint32_t nc = info >> 2;
             for (uint32_t l = 0; l < nc; ++l) {
-                if (W.vis[(uint64_t)l * N + slot] != 2) continue;
-                f3 lc = mk3(W.cc[((uint64_t)l * 3 + 0) * N + slot], W.cc[((uint64_t)l * 3 + 1) * N + slot],
-                            W.cc[((uint64_t)l * 3 + 2) * N + slot]);
+                if (W.vis[(uint64_t)l * N + e] != 2) continue;
+                f3 lc = mk3(W.cc[((uint64_t)l * 3 + 0) * N + e], W.cc[((uint64_t)l * 3 + 1) * N + e], W.cc[((uint64_t)l * 3 + 2) * N + e]);
                 conn = mk3(lc.x + conn.x, lc.y + conn.y, lc.z + conn.z);
             }
             W.conn[slot] = f4of(conn, 0.0f);
@@ -1054,18 +1063,17 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_connect(WfState W, WfQueue i
         // by a path that ends this round
         const bool neeVis = nee && W.nvis[slot] == 2;
         if (!neeVis && fl != 1u) continue;
-        float4 rc = W.radc[slot];
+        float4 rc = glow ? W.rad[slot] : f4of(mk3(0.0f, 0.0f, 0.0f), 0.0f);
         if (neeVis) {
             const f3 c = xyz(W.neeC[slot]);
             rc.x = rc.x + c.x; rc.y = rc.y + c.y; rc.z = rc.z + c.z;
-            W.radc[slot] = rc;
+            W.rad[slot] = rc;
         }
         if (fl == 1u) {
             const f3 radiance = xyz(rc);
             rad[(uint64_t)slot * 3 + 0] = conn.x * 1.0f + radiance.x;
             rad[(uint64_t)slot * 3 + 1] = conn.y * 1.0f + radiance.y;
             rad[(uint64_t)slot * 3 + 2] = conn.z * 1.0f + radiance.z;
-            W.flags[slot] = 2u;
         }
     }
 }
@@ -1100,7 +1108,8 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TAIL_WAVES(kLights, kNee)) void omv_
         const uint32_t p = cur.phys(e);
         const float4 o = in.o[p], d = in.d[p];
         const uint32_t slot = __float_as_uint(d.w);
-        const float4 rc = W.radc[slot], th = W.thr[slot];
+        const float4 th = in.t[p];
+        const f3 radiance = kNee || S.any_emissive ? xyz(W.rad[slot]) : mk3(0.0f, 0.0f, 0.0f);
         LightSub ls;
         ls.idx = -1; ls.len = 0; ls.pos = mk3(0.0f, 0.0f, 0.0f); ls.intensity = ls.pos; ls.range = FLT_MAX;
         f3 conn = mk3(0.0f, 0.0f, 0.0f);
@@ -1114,9 +1123,9 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TAIL_WAVES(kLights, kNee)) void omv_
         WfLightVerts lv;
         lv.lv = W.lv; lv.N = N; lv.slot = slot;
         Rng cs;
-        rngRestore(cs, P.seed, STREAM_CAMERA, sample0 + slot, W.csn[slot]);
-        const f3 r = cameraRounds<kLights, kNee>(S, P, sample0 + slot, i0, xyz(o), xyz(d), o.w, xyz(th), th.w, xyz(rc), conn,
-                                                 __float_as_int(rc.w), cs, ls, lv, L);
+        rngRestore(cs, P.seed, STREAM_CAMERA, sample0 + slot, __float_as_uint(th.w));
+        const f3 r = cameraRounds<kLights, kNee>(S, P, sample0 + slot, i0, xyz(o), xyz(d), o.w, xyz(th), kNee ? in.w[p] : 1.0f, radiance,
+                                                 conn, i0, cs, ls, lv, L);
         rad[(uint64_t)slot * 3 + 0] = r.x;
         rad[(uint64_t)slot * 3 + 1] = r.y;
         rad[(uint64_t)slot * 3 + 2] = r.z;
@@ -1187,6 +1196,8 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_sort_scatter(WfQueue q, cons
         const uint32_t pos = atomicAdd(offs + keys[e], 1u);
         out.o[pos] = q.o[e];
         out.d[pos] = q.d[e];
+        out.t[pos] = q.t[e];
+        if (q.w) out.w[pos] = q.w[e];
     }
 }
 
@@ -1238,9 +1249,9 @@ uint32_t wavefrontSegCap(uint32_t nslots, int gridShade, int gridGen) {
 size_t wavefrontArenaBytes(uint32_t nslots, int lvCap, int lc, bool lights, bool nee, bool splat, bool sortRays, int gridShade, int gridGen) {
     const size_t N = nslots;
     const size_t Q = (size_t)OMV_QSEG * wavefrontSegCap(nslots, gridShade, gridGen);   // queue entries
-    size_t b = 6 * up(Q * 16)                        // three ray queues
-               + up(N * 16) + up(N * 8)              // hits
-               + 3 * up(N * 16) + 3 * up(N * 4);     // thr, radc, conn, csn, flags, nconn
+    size_t b = 9 * up(Q * 16) + (nee ? 3 * up(Q * 4) : 0)   // three ray queues
+               + up(N * 16) + up(N * 8)                      // hits
+               + 2 * up(N * 16) + up(N * 4);                 // rad, conn, info
     if (lights)
         b += up(N * 16) + 3 * up(N * 4) + up(N * (size_t)lvCap * 24) + up(N * (size_t)lc * 12) + up(N * (size_t)lc) +
              3 * up(Q * (size_t)lc * 16);
@@ -1288,20 +1299,24 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
     const size_t Q = (size_t)OMV_QSEG * segCap;
     uint8_t* cur = static_cast<uint8_t*>(L.arena);
     auto take = [&](size_t bytes) { uint8_t* p = cur; cur += up(bytes); return p; };
-    auto queue = [&]() { WfQueue q; q.o = reinterpret_cast<float4*>(take(Q * 16)); q.d = reinterpret_cast<float4*>(take(Q * 16)); return q; };
-    WfQueue qa = queue(), qb = queue(), qc = queue();
+    auto queue = [&](bool camera) {
+        WfQueue q;
+        q.o = reinterpret_cast<float4*>(take(Q * 16));
+        q.d = reinterpret_cast<float4*>(take(Q * 16));
+        q.t = camera ? reinterpret_cast<float4*>(take(Q * 16)) : nullptr;
+        q.w = camera && nee ? reinterpret_cast<float*>(take(Q * 4)) : nullptr;
+        return q;
+    };
+    WfQueue qa = queue(true), qb = queue(true), qc = queue(true);
     WfHits H;
     H.h = reinterpret_cast<float4*>(take(N * 16));
     H.id = reinterpret_cast<int2*>(take(N * 8));
     WfState W;
     std::memset(&W, 0, sizeof(W));
     W.n = n; W.lvCap = L.lvCap; W.lc = L.lc;
-    W.thr = reinterpret_cast<float4*>(take(N * 16));
-    W.radc = reinterpret_cast<float4*>(take(N * 16));
+    W.rad = reinterpret_cast<float4*>(take(N * 16));
     W.conn = reinterpret_cast<float4*>(take(N * 16));
-    W.csn = reinterpret_cast<uint32_t*>(take(N * 4));
-    W.flags = reinterpret_cast<uint32_t*>(take(N * 4));
-    W.nconn = reinterpret_cast<uint32_t*>(take(N * 4));
+    W.info = reinterpret_cast<uint32_t*>(take(N * 4));
     WfShadowQ sq;
     std::memset(&sq, 0, sizeof(sq));
     if (lights) {
@@ -1329,7 +1344,7 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
     if (nee) {
         W.neeC = reinterpret_cast<float4*>(take(N * 16));
         W.nvis = reinterpret_cast<uint8_t*>(take(N));
-        eq = queue();
+        eq = queue(false);
     }
     // queue counters: light round i reads lightCnt[i] (i = 1 .. lvCap-1) and
     // appends to lightCnt[i+1]; camera round i reads camCnt[i] (i = 1 .. B),
@@ -1492,8 +1507,8 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
             traced = nextInWavefront;
         }
         if (lights || nee)
-            hipLaunchKernelGGL(omv_wf_connect, dim3(L.blocksShade), blk, 0, stream, W, in, camCnt(i), L.rad, lights ? 1 : 0, nee ? 1 : 0, i,
-                               Gen1.gen);
+            hipLaunchKernelGGL(omv_wf_connect, dim3(L.blocksShade), blk, 0, stream, W, in, camCnt(i), L.rad, lights ? 1 : 0, nee ? 1 : 0,
+                               nee || S.any_emissive ? 1 : 0, i, Gen1.gen);
         if (sorted) {
             const WfQueue freed = in;
             in = spare;
