@@ -68,7 +68,7 @@ struct OmvInstance {
     float nrm[9];    // normal matrix: inverse of the transposed 3x3 (RenderMesh.h:36-43)
     int32_t mesh_id; // -1 = invalid instance
     int32_t blas_root;   // the mesh's BLAS root node (a copy of OmvMesh::blas_root: one dependent load less per instance entry)
-    int32_t pad;
+    int32_t mat_type;    // OMV_MAT_* of the mesh's material (a copy: the shading kernels sort hits by it)
 };
 
 struct OmvMaterial {
@@ -123,6 +123,7 @@ struct OmvSceneView {
     int32_t closest_only; // 1: visibility rays take the closest hit too (the occlusion early-out off)
     int32_t lights_leave; // 1: every light lies above each child box of the TLAS root on some axis, so every
                           // light ray (positive-octant directions) misses the scene and no light round has rays
+    int32_t hit_classes;  // material types (OMV_MAT_*) among the instances' meshes
     float   scene_lo[3], scene_inv[3];   // world box of the instances, 1 / its extent (0 if flat)
     int32_t bg_type, bg_w, bg_h;
     float   bg_const[3];

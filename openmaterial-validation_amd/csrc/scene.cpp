@@ -650,6 +650,7 @@ int RenderScene::commit(std::string& log) {
         d.blas_root = -1;
         if (in.meshId < 0) continue;
         d.blas_root = dmeshes[in.meshId].blas_root;
+        d.mat_type = mats_[dmeshes[in.meshId].mat_id].type;
         const OmvNode4& root = deviceBuild ? blasRoots[in.meshId] : nodes[dmeshes[in.meshId].blas_root];
         float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
         for (int k = 0; k < 4; ++k) {
@@ -788,6 +789,9 @@ int RenderScene::commit(std::string& log) {
     v.num_texs = (int)texs_.size(); v.num_lights = (int)lights_.size();
     v.tlas_root = tl.root;
     v.lights_leave = lightsLeave;
+    uint32_t types = 0;
+    for (const OmvInstance& in : dinsts) if (in.mesh_id >= 0) types |= 1u << in.mat_type;
+    for (; types; types &= types - 1) ++v.hit_classes;
     v.total_faces = faceBase;
     v.fc_subject = fcSubject_;
     v.any_emissive = anyEmissive;

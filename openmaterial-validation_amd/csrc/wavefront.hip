@@ -127,11 +127,9 @@ DEV unsigned long long* statSlot(unsigned long long* base) { return base + (bloc
 // over K counters instead of serialising on one (a wave-aggregated atomic on
 // one address costs ~11 ns of that address's time on MI355X; over 64
 // addresses ~0.35 ns).  Consumers walk the logical index 0 .. sum(cnt) - 1
-// region by region.  The host sizes cap so that no region can overflow (a
-// region is fed by ceil(grid/K) workgroups, each handling at most
-// OMV_BLOCK * ceil(N / threads) input entries, with at most `per` appends
-// each); a full region still drops the append and counts it in `lost`
-// rather than write out of bounds.  K = 1 is a plain compact queue.
+// region by region.  The host sizes cap so that no region can overflow
+// (wavefrontSegCap); a full region still drops the append and counts it in
+// `lost` rather than write out of bounds.  K = 1 is a plain compact queue.
 struct WfSeg {
     uint32_t* cnt;    // K counters (null: an empty queue)
     uint32_t K, cap;
@@ -755,27 +753,139 @@ __global__ __launch_bounds__(OMV_BLOCK, 6) void omv_wf_trace_cam1(OmvSceneView S
     flushCounters(statSlot(counters), rays, nCam, 0u, 0u, cnt);
 }
 
+// ------------------------------------------------------------- hit classes
+// The shading kernels are bound by VALU issue, and entry by entry a wave pays
+// for every branch any of its lanes takes: escape, mirror, PBR or diffuse
+// (lanes active 0.14 - 0.25 after the first bounce).  So a workgroup takes a
+// tile of entries at a time, sorts their indices by class in LDS -- escapes,
+// then the material types -- with every class starting at a multiple of 64,
+// and its waves take 64 indices of one class each.  Entries keep their order
+// within a class and wave, and what each path computes does not depend on it.
+// MI355X, unsorted -> sorted: masked scene with lights 640 x 479 x 16 6.21 ->
+// 5.82 ms, instanced 1080p x 16 8.90 -> 8.79 (instructions of its second round
+// 415 M -> 180 M; the round is then bound by memory).  With one type of
+// material sorting costs more than it saves (torus knot 4.59 -> 4.71 ms).
+constexpr uint32_t kShadeTile = 1024u, kShadeTileMin = 256u, kHitClasses = 4u, kNoEntry = 0xFFFFu;
+static_assert(OMV_BLOCK == 128, "two waves share a tile");
+static_assert(OMV_MAT_NONE == 0 && OMV_MAT_DIFFUSE == 3, "hit classes are the material types, class 0 the escapes");
+// Entries per tile: enough tiles for every workgroup to take several, and as
+// many entries as fit so that the padding of the classes stays small.  Not
+// sorted, OMV_BLOCK at a time: the entries of a scene whose materials are all
+// of one type (escapes are cheap beside the one kind of hit), and up to one
+// entry a thread, where the launch is bound by latency, not by issue.
+__host__ __device__ inline uint32_t shadeTile(uint32_t total, uint32_t grid, bool sorted) {
+    if (!sorted || total <= grid * OMV_BLOCK) return OMV_BLOCK;
+    const uint32_t want = total / (4u * grid);
+    return want >= kShadeTile ? kShadeTile : (want >= 2u * kShadeTileMin ? 2u * kShadeTileMin : kShadeTileMin);
+}
+// A workgroup's tiles: in row k the one of place (b + k * step) mod grid.  With
+// the same place in every row a workgroup would keep to the same columns of
+// the image whenever a row of tiles is a whole number of pixel rows (512
+// pixels x 64 samples: 4 pixel rows to 1024 workgroups), and some would shade
+// only sky (torus knot: 2.1 of 4 waves per SIMD resident on average; 4.76 ->
+// 4.59 ms with the step).  The
+// step, near 0.38 of the grid, is an odd multiple of OMV_QSEG, so a place keeps
+// its append region and its XCD.
+template <bool kSorted>
+struct TileWalk {
+    uint32_t row, place, step, tile, total, t0;
+    DEV explicit TileWalk(uint32_t tot) {
+        row = 0u; place = blockIdx.x; total = tot;
+        tile = kSorted ? shadeTile(tot, gridDim.x, true) : OMV_BLOCK;
+        step = gridDim.x > 2u * OMV_QSEG ? ((uint32_t)((uint64_t)gridDim.x * 391u >> 10) / OMV_QSEG | 1u) * OMV_QSEG : 0u;
+        t0 = place * tile;
+    }
+    DEV bool sorted() const { return kSorted && tile > OMV_BLOCK; }
+    DEV bool more() const { return row < total; }
+    DEV void next() {
+        row += gridDim.x * tile;
+        place += step;
+        if (place >= gridDim.x) place -= gridDim.x;
+        t0 = row + place * tile;
+    }
+};
+struct HitBins {
+    uint16_t list[kShadeTile + 64u * kHitClasses];   // tile-relative entries, kNoEntry in the padding
+    uint32_t wcnt[2][kHitClasses];
+    uint32_t begin, end;                             // chunks of 64: [0, begin) escapes, [begin, end) hits
+    // Sorts the entries [base, base + n) of id.  All threads of the workgroup
+    // call it; the waves may still be reading the tile before.
+    DEV void sort(const OmvSceneView& S, const int2* __restrict__ id, uint32_t base, uint32_t n) {
+        __syncthreads();
+        const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+        const uint64_t before = (1ull << lane) - 1ull;
+        uint32_t cls = 0u, cnt[kHitClasses] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (uint32_t k = 0; k < kShadeTile / 128u; ++k) {
+            const uint32_t i = (2u * k + wave) * 64u + lane;
+            if (2u * k * 64u >= n) break;
+            uint32_t c = 0u;
+            if (i < n) {
+                const int inst = id[base + i].x;
+                if (inst >= 0) c = (uint32_t)min(max(S.insts[inst].mat_type, 1), 3);
+            }
+            cls |= c << (2u * k);
+#pragma unroll
+            for (uint32_t j = 0; j < kHitClasses; ++j) cnt[j] += (uint32_t)__popcll(__ballot(i < n && c == j));
+        }
+        if (lane < kHitClasses) wcnt[wave][lane] = lane == 0u ? cnt[0] : (lane == 1u ? cnt[1] : (lane == 2u ? cnt[2] : cnt[3]));
+        for (uint32_t p = threadIdx.x; p < n + 64u * kHitClasses; p += OMV_BLOCK) list[p] = (uint16_t)kNoEntry;
+        __syncthreads();
+        uint32_t off[kHitClasses], at = 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < kHitClasses; ++j) {
+            if (j == 1u && threadIdx.x == 0u) begin = at >> 6;
+            off[j] = at + (wave ? wcnt[0][j] : 0u);
+            at += (wcnt[0][j] + wcnt[1][j] + 63u) & ~63u;
+        }
+        if (threadIdx.x == 0u) end = at >> 6;
+#pragma unroll
+        for (uint32_t k = 0; k < kShadeTile / 128u; ++k) {
+            const uint32_t i = (2u * k + wave) * 64u + lane;
+            if (2u * k * 64u >= n) break;
+            const uint32_t c = (cls >> (2u * k)) & 3u;
+            uint32_t pos = 0u;
+#pragma unroll
+            for (uint32_t j = 0; j < kHitClasses; ++j) {
+                const uint64_t m = __ballot(i < n && c == j);
+                if (c == j) pos = off[j] + (uint32_t)__popcll(m & before);
+                off[j] += (uint32_t)__popcll(m);
+            }
+            if (i < n) list[pos] = (uint16_t)i;
+        }
+        __syncthreads();
+    }
+};
+
 // ---------------------------------------------------------- shade light
 // Light-subpath vertex i (computePath with inv = false, BDPTRenderer.cpp:149-188)
 // and, with OMV_EXT_LIGHT_SPLAT (kSplat), its pinhole connection staged for
 // the visibility trace.
-template <bool kSplat>
+template <bool kSplat, bool kSorted>
 __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_shade_light(OmvSceneView S, omv_camera_desc cam, RP P, uint64_t sample0, int i, WfState W,
                                                                 WfQueue in, WfSeg inCount, WfHits H, WfQueue out, WfSeg outCount, WfShadowQ sq,
                                                                 WfSeg sqCount, unsigned long long* __restrict__ lost) {
-    const uint32_t gthreads = gridDim.x * blockDim.x;
-    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ HitBins bins;
     __shared__ SegTable cur;
     segLoad(cur, inCount);
     const uint32_t total = cur.total();
     const uint64_t N = W.n;
-    for (uint32_t e = gtid; e < total; e += gthreads) {
+    for (TileWalk<kSorted> w(total); w.more(); w.next()) {
+      if (w.t0 >= total) continue;
+      const uint32_t m = min(w.tile, total - w.t0);
+      if (w.sorted()) bins.sort(S, H.id, w.t0, m);
+      // a missed light ray ends its subpath: nothing to read or write
+      for (uint32_t ch = (w.sorted() ? bins.begin : 0u) + (threadIdx.x >> 6), end = w.sorted() ? bins.end : 2u; ch < end; ch += 2u) {
+        const uint32_t te = w.sorted() ? (uint32_t)bins.list[ch * 64u + (threadIdx.x & 63u)] : (threadIdx.x < m ? threadIdx.x : kNoEntry);
+        if (te == kNoEntry) continue;
+        const uint32_t e = w.t0 + te;
         const int2 id = H.id[e];
+        if (id.x < 0) continue;
         bool emit = false, spl = false;
         f3 nPos = mk3(0.0f, 0.0f, 0.0f), nDir = nPos, sPos = nPos, sDir = nPos, ctb = nPos;
         float nTnear = 0.0f, sTn = 0.0f, sD = 0.0f;
         uint32_t pix = 0, slot = 0;
-        if (id.x >= 0) {   // a missed light ray ends its subpath: nothing to read or write
+        {
             const float4 dd = in.d[cur.phys(e)];
             slot = __float_as_uint(dd.w);
             const f3 pDir = xyz(dd);
@@ -837,6 +947,7 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_shade_light(OmvSceneView S, 
                 sq.b[ks] = f4of(ctb, __uint_as_float(pix));
             }
         }
+      }
     }
 }
 
@@ -845,13 +956,12 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_shade_light(OmvSceneView S, 
 // the connections of that vertex staged for the visibility trace
 // (BDPTRenderer.cpp:266-297), the escape term (:251-258) and, with
 // OMV_EXT_HDRI_NEE, the next-event estimate staged for its visibility trace.
-template <bool kLights, bool kNee>
+template <bool kLights, bool kNee, bool kSorted>
 __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv_wf_shade_cam(OmvSceneView S, RP P, uint64_t sample0, int i, WfState W, WfQueue in,
                                                               WfSeg inCount, WfHits H, WfQueue out, WfSeg outCount, WfShadowQ sq,
                                                               WfSeg sqCount, WfQueue eq, WfSeg eqCount, float* __restrict__ rad, WfGen G,
                                                               unsigned long long* __restrict__ lost) {
-    const uint32_t gthreads = gridDim.x * blockDim.x;
-    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ HitBins bins;
     __shared__ SegTable cur;
     segLoad(cur, inCount);
     const uint32_t total = cur.total();
@@ -859,7 +969,14 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
     const int q = P.q;
     const bool gen = G.gen && i == 1;
     const bool glow = kNee || S.any_emissive;   // radiance is collected before the path's end
-    for (uint32_t e = gtid; e < total; e += gthreads) {
+    for (TileWalk<kSorted> w(total); w.more(); w.next()) {
+      if (w.t0 >= total) continue;
+      const uint32_t m = min(w.tile, total - w.t0);
+      if (w.sorted()) bins.sort(S, H.id, w.t0, m);
+      for (uint32_t ch = threadIdx.x >> 6, end = w.sorted() ? bins.end : 2u; ch < end; ch += 2u) {
+        const uint32_t te = w.sorted() ? (uint32_t)bins.list[ch * 64u + (threadIdx.x & 63u)] : (threadIdx.x < m ? threadIdx.x : kNoEntry);
+        if (te == kNoEntry) continue;
+        const uint32_t e = w.t0 + te;
         uint32_t slot;
         f3 pDir;
         f3 of = mk3(1.0f, 1.0f, 1.0f), radiance = mk3(0.0f, 0.0f, 0.0f);
@@ -1028,6 +1145,7 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
                 eq.d[ke] = f4of(eDir, __uint_as_float(slot));
             }
         }
+      }
     }
 }
 
@@ -1230,20 +1348,32 @@ constexpr size_t kAlign = 256;
 size_t up(size_t b) { return (b + kAlign - 1) & ~(kAlign - 1); }
 }  // namespace
 
-// Entries per append region of a queue fed by a launch of `grid`
-// workgroups over at most nslots input entries with one append each: the
-// workgroups of one region (ceil(grid / K)) handle at most OMV_BLOCK *
-// ceil(nslots / threads) entries each.  The producers are the shading
-// kernels (gridShade) and, for the round-1 light queue, generation
-// (gridGen); regions are sized for the larger of the two.  A queue holds
-// OMV_QSEG regions (>= nslots entries in all).
-static uint32_t segCapFor(uint32_t nslots, int grid) {
+// Entries per append region of a queue fed by at most nslots input entries
+// with one append each.  A region is fed by every OMV_QSEG-th workgroup.
+// Generation (gridGen workgroups) strides over its entries lane by lane; the
+// shading kernels (gridShade) take tiles of shadeTile entries, so with t of
+// them a workgroup handles at most ceil(t / grid) tiles and only
+// min(grid, t) workgroups have any.  A queue may hold fewer entries than
+// nslots and then has smaller tiles: each tile size counts at the largest
+// total that uses it.
+static uint32_t segCapGen(uint32_t nslots, int grid) {
     const uint64_t g = (uint64_t)std::max(grid, 1), threads = g * OMV_BLOCK;
     const uint64_t perBlock = (uint64_t)OMV_BLOCK * ((nslots + threads - 1) / threads);
     return (uint32_t)(((g + OMV_QSEG - 1) / OMV_QSEG) * perBlock);
 }
+static uint32_t segCapShade(uint32_t nslots, int grid) {
+    const uint64_t g = (uint64_t)std::max(grid, 1);
+    uint64_t cap = 0;
+    for (uint64_t tile = OMV_BLOCK; tile <= kShadeTile; tile *= 2) {
+        // (tiles of OMV_BLOCK entries serve any total when the scene is not sorted)
+        const uint64_t most = tile == kShadeTile || tile == OMV_BLOCK ? nslots : std::min<uint64_t>(nslots, 8 * tile * g - 1);
+        const uint64_t tiles = (most + tile - 1) / tile;
+        cap = std::max(cap, ((std::min(g, tiles) + OMV_QSEG - 1) / OMV_QSEG) * tile * ((tiles + g - 1) / g));
+    }
+    return (uint32_t)cap;
+}
 uint32_t wavefrontSegCap(uint32_t nslots, int gridShade, int gridGen) {
-    return std::max(segCapFor(nslots, gridShade), segCapFor(nslots, gridGen));
+    return std::max(segCapShade(nslots, gridShade), segCapGen(nslots, gridGen));
 }
 
 size_t wavefrontArenaBytes(uint32_t nslots, int lvCap, int lc, bool lights, bool nee, bool splat, bool sortRays, int gridShade, int gridGen) {
@@ -1274,11 +1404,11 @@ void wavefrontBlocksPerCU(int out[9]) {
         t = std::min(t, k);
     out[0] = t;
     out[4] = t;
-    out[1] = occ(omv_wf_shade_cam<true, true>, 0);
-    out[5] = occ(omv_wf_shade_cam<true, false>, 0);
-    out[6] = occ(omv_wf_shade_cam<false, true>, 0);
-    out[7] = occ(omv_wf_shade_cam<false, false>, 0);
-    out[2] = occ(omv_wf_shade_light<true>, 0);
+    out[1] = std::min(occ(omv_wf_shade_cam<true, true, true>, 0), occ(omv_wf_shade_cam<true, true, false>, 0));
+    out[5] = std::min(occ(omv_wf_shade_cam<true, false, true>, 0), occ(omv_wf_shade_cam<true, false, false>, 0));
+    out[6] = std::min(occ(omv_wf_shade_cam<false, true, true>, 0), occ(omv_wf_shade_cam<false, true, false>, 0));
+    out[7] = std::min(occ(omv_wf_shade_cam<false, false, true>, 0), occ(omv_wf_shade_cam<false, false, false>, 0));
+    out[2] = occ(omv_wf_shade_light<true, true>, 0);
     out[3] = occ(omv_wf_gen<true>, 0);
     out[8] = occ(omv_wf_trace_cam1, 0);
 }
@@ -1373,6 +1503,7 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
     unsigned long long* lost = L.counters + 6;   // the stats' overflow counter
     const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
     const dim3 blk(OMV_BLOCK);
+    const bool sorted = S.hit_classes > 1;   // shading sorts its entries by class
     const uint32_t xcds = L.xcdBands > 1 ? (uint32_t)L.xcdBands : 1u;
     auto mark = [&]() {
         if (L.traceEv && L.traceEvUsed && *L.traceEvUsed < L.traceEvCap) (void)hipEventRecord(L.traceEv[(*L.traceEvUsed)++], stream);
@@ -1416,13 +1547,13 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
             launchTrace(S.any_masked ? omv_wf_trace<1, true> : omv_wf_trace<1, false>, in, lightCnt(i), none, none, Gen0, kKeepSecondary);
             mark();
             if (splat) {
-                hipLaunchKernelGGL(omv_wf_shade_light<true>, dim3(L.blocksShade), blk, 0, stream, S, L.cam, P, L.sample0, i, W, in, lightCnt(i),
+                hipLaunchKernelGGL((sorted ? omv_wf_shade_light<true, true> : omv_wf_shade_light<true, false>), dim3(L.blocksShade), blk, 0, stream, S, L.cam, P, L.sample0, i, W, in, lightCnt(i),
                                    H, out, lightCnt(i + 1), sq, splCnt(i), lost);
                 mark();
                 launchTrace(S.any_masked ? omv_wf_trace<4, true> : omv_wf_trace<4, false>, in, none, splCnt(i), none, Gen0, kKeepSecondary);
                 mark();
             } else {
-                hipLaunchKernelGGL(omv_wf_shade_light<false>, dim3(L.blocksShade), blk, 0, stream, S, L.cam, P, L.sample0, i, W, in, lightCnt(i),
+                hipLaunchKernelGGL((sorted ? omv_wf_shade_light<false, true> : omv_wf_shade_light<false, false>), dim3(L.blocksShade), blk, 0, stream, S, L.cam, P, L.sample0, i, W, in, lightCnt(i),
                                    H, out, lightCnt(i + 1), sq, splCnt(i), lost);
             }
             std::swap(in, out);
@@ -1474,20 +1605,20 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
         traced = false;
         if (lights) {
             if (nee)
-                hipLaunchKernelGGL((omv_wf_shade_cam<true, true>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i), H,
+                hipLaunchKernelGGL((sorted ? omv_wf_shade_cam<true, true, true> : omv_wf_shade_cam<true, true, false>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i), H,
                                    out, camCnt(i + 1), sq, shCnt(i), eq, envCnt(i), L.rad, Gen1, lost);
             else
-                hipLaunchKernelGGL((omv_wf_shade_cam<true, false>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i),
+                hipLaunchKernelGGL((sorted ? omv_wf_shade_cam<true, false, true> : omv_wf_shade_cam<true, false, false>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i),
                                    H, out, camCnt(i + 1), sq, shCnt(i), eq, envCnt(i), L.rad, Gen1, lost);
         } else {
             if (nee)
-                hipLaunchKernelGGL((omv_wf_shade_cam<false, true>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i),
+                hipLaunchKernelGGL((sorted ? omv_wf_shade_cam<false, true, true> : omv_wf_shade_cam<false, true, false>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i),
                                    H, out, camCnt(i + 1), sq, shCnt(i), eq, envCnt(i), L.rad, Gen1, lost);
             else
-                hipLaunchKernelGGL((omv_wf_shade_cam<false, false>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i),
+                hipLaunchKernelGGL((sorted ? omv_wf_shade_cam<false, false, true> : omv_wf_shade_cam<false, false, false>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i),
                                    H, out, camCnt(i + 1), sq, shCnt(i), eq, envCnt(i), L.rad, Gen1, lost);
         }
-        bool sorted = false;
+        bool reordered = false;
         const bool nextInWavefront = i < B && i + 1 != i0;   // round i + 1 is traced by this schedule's round kernels
         if (L.sortRays && nextInWavefront) {
             // reorder the next round's rays (secondary rays) into the spare queue
@@ -1495,9 +1626,9 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
             hipLaunchKernelGGL(omv_wf_sort_keys, dim3(L.blocksShade), blk, 0, stream, S, out, camCnt(i + 1).cnt, sortKeys, sortHist);
             hipLaunchKernelGGL(omv_wf_sort_scan, dim3(1), dim3(1024), 0, stream, sortHist);
             hipLaunchKernelGGL(omv_wf_sort_scatter, dim3(L.blocksShade), blk, 0, stream, out, camCnt(i + 1).cnt, sortKeys, sortHist, spare);
-            sorted = true;
+            reordered = true;
         }
-        const WfQueue next = sorted ? spare : out;
+        const WfQueue next = reordered ? spare : out;
         // the next round's hits go to H, which this round's connect does not read
         if (fuse) {
             mark();
@@ -1509,7 +1640,7 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
         if (lights || nee)
             hipLaunchKernelGGL(omv_wf_connect, dim3(L.blocksShade), blk, 0, stream, W, in, camCnt(i), L.rad, lights ? 1 : 0, nee ? 1 : 0,
                                nee || S.any_emissive ? 1 : 0, i, Gen1.gen);
-        if (sorted) {
+        if (reordered) {
             const WfQueue freed = in;
             in = spare;
             spare = out;

@@ -359,3 +359,34 @@ def test_packet_traversal_keeps_the_film(pkg, wl, case):
     # nearest first), not its own, so its closest t culls a little less:
     # node and triangle counts are checked to 25 %
     _same([out[2], out[1]], visit_tol=0.25)
+
+
+@pytest.mark.parametrize("size", [(363, 362, 1), (700, 401, 2), (1449, 1451, 1), (2049, 2053, 1)])
+@pytest.mark.parametrize("kind", ["lights", "nee", "emissive", "one_type"])
+def test_sorted_shading_keeps_the_film(pkg, wl, kind, size):
+    """Shading sorts tiles of 256, 512 and 1024 entries by hit class in scenes
+    of several material types (a ragged last tile each), and takes unsorted
+    rows of entries in scenes of one; throughput and stream position travel in
+    the ray queue, the radiance so far beside it with emission or NEE.  Films
+    and ray counts equal the per-sample schedule's bit for bit."""
+    desc, view = wl.mixed_test_scene(hdr=True, lights=kind in ("lights", "emissive"))
+    if kind == "lights":   # low in the scene: light subpaths are shaded too
+        desc.lights.append(((-1.2, -0.6, -1.0), (30.0, 20.0, 10.0), -1.0))
+    if kind == "emissive":
+        desc.materials[2][1].update(emissive=(0.4, 0.2, 0.3), textures={2: 1, 3: 2})
+    if kind == "one_type":
+        for m in desc.meshes:
+            m["mat_id"] = 2 if m["mat_id"] != 0 else 0
+    view.width, view.height, spp = size
+    s = pkg.Scene()
+    desc.apply(s, pkg.pbr_desc)
+    cam = pkg.Camera(view.width, view.height, view.position, view.forward, view.up, view.yfov)
+    params = dict(samples_per_pixel=spp, camera_bounces=3, light_bounces=3, max_path_length=4, seed=17, extensions=2 if kind == "nee" else 0)
+    out = []
+    for sched in (pkg.SCHEDULE_WAVEFRONT, pkg.SCHEDULE_PER_SAMPLE):
+        r = pkg.Renderer(pkg.default_params(**params))
+        r.set_scene(s)
+        r.set_schedule(sched)
+        r.set_tuning(tail_round=3)
+        out.append((r.render(cam), r.stats()))
+    _same(out)
