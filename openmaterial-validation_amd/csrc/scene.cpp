@@ -169,6 +169,43 @@ void affineInverse(const float* M, float* out) {
     }
 }
 
+// Boxes that together hold the subtree of `root`: the root's children, the one
+// of largest area replaced by its own children while at most `most` remain
+// (most = 0: the children as they are; no node but the root is read).  An
+// instance's box is the box of these boxes turned by its matrix one by one,
+// which for a rotated mesh is far tighter than that of the turned root box, so
+// rays enter fewer instances that they miss: 60 rotated meshes of 33 K
+// triangles under lights, 1080p x 16 (MI355X), 6.59 -> 6.24 nodes per ray and
+// 8.78 -> 8.42 ms per render.
+constexpr int kCoverBoxes = 128;
+void coverBoxes(const OmvNode4* nodes, int root, int most, std::vector<BuildBox>& out) {
+    struct Item { float area; int node; BuildBox box; };   // node < 0: a leaf
+    auto smaller = [](const Item& a, const Item& b) { return a.area < b.area; };
+    std::vector<Item> heap;
+    auto addChildren = [&](int n) {
+        const OmvNode4& nd = nodes[n];
+        for (int k = 0; k < 4; ++k) {
+            if (nd.child[k] == OMV_EMPTY_CHILD) continue;
+            Item it;
+            it.node = nd.child[k] >= 0 ? nd.child[k] : -1;
+            const float lo[3] = {nd.lox[k], nd.loy[k], nd.loz[k]}, hi[3] = {nd.hix[k], nd.hiy[k], nd.hiz[k]};
+            float d[3];
+            for (int a = 0; a < 3; ++a) { it.box.lo[a] = lo[a]; it.box.hi[a] = hi[a]; d[a] = hi[a] - lo[a]; }
+            it.area = it.node < 0 ? -1.0f : d[0] * d[1] + d[1] * d[2] + d[2] * d[0];   // leaves are not replaced
+            heap.push_back(it);
+            std::push_heap(heap.begin(), heap.end(), smaller);
+        }
+    };
+    addChildren(root);
+    while (!heap.empty() && heap.front().node >= 0 && (int)heap.size() + 3 <= most) {
+        const int n = heap.front().node;
+        std::pop_heap(heap.begin(), heap.end(), smaller);
+        heap.pop_back();
+        addChildren(n);
+    }
+    for (const Item& it : heap) out.push_back(it.box);
+}
+
 int hipFail(hipError_t e, const char* what) {
     setError(std::string(what) + ": " + hipGetErrorString(e));
     return OMV_E_DEVICE;
@@ -635,10 +672,11 @@ int RenderScene::commit(std::string& log) {
         }
     }
     if (insts_.size() >= (1u << 29)) { setError("commit: too many instances"); return OMV_E_SCENE; }
-    // TLAS over world-space instance boxes (transformed BLAS root boxes, rounded outward)
+    // TLAS over world-space instance boxes (transformed boxes of the BLAS, see coverBoxes, rounded outward)
     std::vector<BuildBox> iboxes;
     std::vector<int> iids;
     std::vector<OmvInstance> dinsts(insts_.size());
+    std::vector<std::vector<BuildBox>> covers(meshes_.size());
     for (size_t i = 0; i < insts_.size(); ++i) {
         const HostInstance& in = insts_[i];
         OmvInstance& d = dinsts[i];
@@ -651,25 +689,30 @@ int RenderScene::commit(std::string& log) {
         if (in.meshId < 0) continue;
         d.blas_root = dmeshes[in.meshId].blas_root;
         d.mat_type = mats_[dmeshes[in.meshId].mat_id].type;
-        const OmvNode4& root = deviceBuild ? blasRoots[in.meshId] : nodes[dmeshes[in.meshId].blas_root];
-        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-        for (int k = 0; k < 4; ++k) {
-            if (root.child[k] == OMV_EMPTY_CHILD) continue;
-            lo[0] = std::min(lo[0], root.lox[k]); lo[1] = std::min(lo[1], root.loy[k]); lo[2] = std::min(lo[2], root.loz[k]);
-            hi[0] = std::max(hi[0], root.hix[k]); hi[1] = std::max(hi[1], root.hiy[k]); hi[2] = std::max(hi[2], root.hiz[k]);
+        std::vector<BuildBox>& cover = covers[in.meshId];
+        if (cover.empty()) {
+            if (deviceBuild) coverBoxes(&blasRoots[in.meshId], 0, 0, cover);   // the other nodes are in device memory
+            else coverBoxes(nodes.data(), dmeshes[in.meshId].blas_root, kCoverBoxes, cover);
         }
         double wl[3] = {INFINITY, INFINITY, INFINITY}, wh[3] = {-INFINITY, -INFINITY, -INFINITY};
-        for (int c = 0; c < 8; ++c) {
-            const double p[3] = {(c & 1) ? hi[0] : lo[0], (c & 2) ? hi[1] : lo[1], (c & 4) ? hi[2] : lo[2]};
-            for (int a = 0; a < 3; ++a) {
-                const double w = (double)in.tm[a * 4] * p[0] + (double)in.tm[a * 4 + 1] * p[1] + (double)in.tm[a * 4 + 2] * p[2] + (double)in.tm[a * 4 + 3];
-                wl[a] = std::min(wl[a], w);
-                wh[a] = std::max(wh[a], w);
+        double reach[3] = {0.0, 0.0, 0.0};   // the largest sum of terms behind a coordinate: rounding goes with it
+        for (const BuildBox& c : cover) {
+            for (int a = 0; a < 3; ++a) {   // the box M turns [lo, hi] into: centre +- sum |M| * half extent
+                double mid = (double)in.tm[a * 4 + 3], half = 0.0, terms = std::fabs((double)in.tm[a * 4 + 3]);
+                for (int k = 0; k < 3; ++k) {
+                    const double m = (double)in.tm[a * 4 + k], lo = c.lo[k], hi = c.hi[k];
+                    mid += m * 0.5 * (lo + hi);
+                    half += std::fabs(m) * 0.5 * (hi - lo);
+                    terms += std::fabs(m) * std::max(std::fabs(lo), std::fabs(hi));
+                }
+                wl[a] = std::min(wl[a], mid - half);
+                wh[a] = std::max(wh[a], mid + half);
+                reach[a] = std::max(reach[a], terms);
             }
         }
         BuildBox b;
         for (int a = 0; a < 3; ++a) {
-            const double pad = 1e-5 * (std::fabs(wl[a]) + std::fabs(wh[a])) + 1e-20;
+            const double pad = 1e-5 * std::max(std::fabs(wl[a]) + std::fabs(wh[a]), reach[a]) + 1e-20;
             b.lo[a] = std::nextafter((float)(wl[a] - pad), -INFINITY);
             b.hi[a] = std::nextafter((float)(wh[a] + pad), INFINITY);
         }

@@ -126,3 +126,53 @@ def test_refill_at_the_edges_of_a_list(pkg, wl, keep, size):
         assert np.array_equal(r.render(cam), want)
         for k in ("rays", "camera_rays", "light_rays", "shadow_rays"):
             assert r.stats()[k] == st[k], k
+
+
+@pytest.mark.parametrize("build", ["host", "device"])
+@pytest.mark.parametrize("place", [0, 1, 3])
+def test_turned_instances(pkg, wl, ref, place, build):
+    """Instance boxes come from several boxes of a mesh, each turned by the
+    instance's matrix: meshes of one leaf, of one triangle, far from their own
+    origin, plates that lie back in a plane of the world, turned, sheared and
+    mirrored.  Ids and tie flags are the oracle's, under both builders."""
+    scale, shift = PLACES[place]
+    d = wl.SceneDesc()
+    d.materials.append(("pbr", dict(base_color=(0.7, 0.6, 0.5, 1.0), metallic=0.3, roughness=0.4)))
+    tri = np.array([[-0.6, -0.4, 0.1], [0.7, -0.3, -0.2], [0.05, 0.65, 0.15]], np.float32)
+    d.meshes.append({"vertices": tri, "faces": np.array([[0, 1, 2]], np.uint32), "mat_id": 0})
+    v, f, _ = wl.plane(6, 6, 0.8, 0.0)
+    c, q = np.cos(0.6), np.sin(0.6)
+    turn = np.array([[c, -q, 0], [q, c, 0], [0, 0, 1]])   # the plate at 0.6 rad about z
+    d.meshes.append({"vertices": (v @ turn.T).astype(np.float32), "faces": f, "mat_id": 0})
+    v, f, _ = wl.grid_box(4, (0.9, 0.1, 0.05))
+    d.meshes.append({"vertices": v, "faces": f, "mat_id": 0})
+    v, f = wl.icosphere(3, 0.5)
+    d.meshes.append({"vertices": (v + np.array([30.0, 0.0, -20.0], np.float32)).astype(np.float32), "faces": f, "mat_id": 0})
+    rng = np.random.default_rng(5)
+    for i in range(40):
+        a = wl.trs((0, 0, 0), rng.normal(size=3), rng.uniform(0, 6.3), rng.uniform(0.3, 1.2, 3) * rng.choice([-1, 1], 3))
+        m = np.array(a, np.float64).reshape(-1, 4)
+        if i % 5 == 4:
+            m[:3, :3] = m[:3, :3] @ np.array([[1, 0.7, 0], [0, 1, -0.4], [0, 0, 1]])
+        if i % 4 == 1 and i < 20:   # the plates, turned back into y = const
+            m[:3, :3] = turn.T
+        at = rng.uniform(-1.8, 1.8, 3)
+        if i % 4 == 3:
+            at = at - m[:3, :3] @ np.array([30.0, 0.0, -20.0])
+        m[:3, :3] *= scale
+        m[:3, 3] = scale * at + np.array(shift)
+        d.instances.append((np.asarray(m, np.float32).reshape(np.shape(a)), i % 4))
+    d.fc_subject = "ipid"
+    cam = _camera(pkg, "free", scale, shift, 97, 83)
+    s = pkg.Scene()
+    s.set_build_mode(pkg.BUILD_DEVICE_LBVH if build == "device" else pkg.BUILD_HOST_SAH)
+    d.apply(s, pkg.pbr_desc)
+    r = pkg.Renderer(pkg.default_params(seed=3))
+    r.set_scene(s)
+    _, ids, tie = r.render_fc(cam)
+    rs = ref.Scene()
+    d.apply(rs, ref.pbr_desc)
+    _, rids, rtie = rs.render_fc(ref.default_params(seed=3), cam.desc())
+    assert np.array_equal(ids, rids)
+    assert np.array_equal(tie, rtie)
+    assert (ids[0] >= 0).mean() > 0.2
