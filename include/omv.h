@@ -396,8 +396,8 @@ typedef struct omv_render_tuning {
                                  one lane (same film): 0 = default, 1 = never
                                  (every round as its own trace, shade and
                                  connect launches), n >= 2 = from round n;
-                                 the default is 5 with point lights or NEE,
-                                 else 4                                      */
+                                 the default is 3 to 5: later with more
+                                 samples, and with point lights or NEE       */
 } omv_render_tuning;
 int omv_renderer_set_tuning(omv_renderer* r, const omv_render_tuning* t);
 int omv_renderer_get_tuning(const omv_renderer* r, omv_render_tuning* t);

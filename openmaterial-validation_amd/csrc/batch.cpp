@@ -88,6 +88,7 @@ int BatchRunner::prepare() {
         int dev = 0;
         (void)hipGetDevice(&dev);
         if ((e = hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return hipFail(e, "device attribute");
+        if (hipDeviceGetAttribute(&xcds_, hipDeviceAttributeNumberOfXccs, dev) != hipSuccess || xcds_ < 1) xcds_ = 1;
     }
     dropGraph();
     for (const Job& j : jobs_)
@@ -264,6 +265,13 @@ int BatchRunner::launchWavefrontJobs() {
         L.blocksShade = cus_ * shadeCamBlocksPerCU(wfPerCu_, J.scene->view().num_lights > 0,
                                                    (J.p.extensions & OMV_EXT_HDRI_NEE) && J.scene->view().env_tex_pdf);
         L.blocksGen = cus_ * wfPerCu_[3];
+        // The tail launch and the XCD bands, as a single render takes them: 48
+        // lightbox jobs of up to 384^2 x 48 on 8 streams 39.07 -> 38.13 ms, 20
+        // of up to 200^2 x 16 4.50 -> 4.19 ms, 5 of up to 128^2 x 8 1.24 ->
+        // 1.07 ms (MI355X).
+        L.tailRound = defaultTailRound(std::min(J.npix * (uint64_t)spp, wfMaxSlots_), J.scene->view().num_lights > 0,
+                                       (J.p.extensions & OMV_EXT_HDRI_NEE) && J.scene->view().env_tex_pdf);
+        L.xcdBands = J.scene->view().num_insts <= 4 ? 4 * xcds_ : 1;
         const uint64_t chunkPix = std::max<uint64_t>(1, wfMaxSlots_ / (uint64_t)spp);
         for (uint64_t pix0 = 0; rc == OMV_OK && pix0 < J.npix; pix0 += chunkPix) {
             const uint64_t np = std::min(chunkPix, J.npix - pix0);

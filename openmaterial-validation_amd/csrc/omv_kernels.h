@@ -89,6 +89,24 @@ int wavefrontCounterCount(int B, int lvCap);
 // lights, [6] with NEE, [7] with neither, [8] round-1 packet trace
 void wavefrontBlocksPerCU(int out[9]);
 inline int shadeCamBlocksPerCU(const int occ[9], bool lights, bool nee) { return lights ? (nee ? occ[1] : occ[5]) : (nee ? occ[6] : occ[7]); }
+// Camera round from which the wavefront hands the remaining paths of a chunk
+// to one tail launch (omv_wf_tail).  A round costs two or three launches that
+// each wait for their longest ray, whatever its size; the tail waits for its
+// longest path once but traces one path a lane.  So the fewer samples, the
+// earlier.  MI355X, ms per render from round 2 / 3 / 4 / 5:
+//   600 K samples: torus knot 0.63 0.76 0.89 1.00, with NEE 1.10 1.20 1.31
+//     1.43, asset with a light 0.83 0.96 1.04 1.11, 60 instances and lights
+//     0.76 0.84 0.94 1.04, mixed materials 0.97 0.80 0.90 0.92, masked with
+//     lights among them 2.07 1.93 1.95 2.00
+//   1.5 M: 0.98 0.99 1.11 1.21, 1.79 1.51 1.62 1.74, 1.15 1.21 1.30 1.38,
+//     0.95 1.01 1.10 1.21, 1.68 1.33 1.17 1.27, 3.62 2.95 2.92 2.93
+//   NEE 5.4 M: - 4.00 3.48 3.64; masked with lights 4.9 M: - - 5.94 5.80
+//   16.8 M torus knot: - 5.07 4.59 4.72; 33 M instanced: - - 9.39 8.78
+inline int defaultTailRound(uint64_t slots, bool lights, bool nee) {
+    if (!lights && !nee) return slots <= (1u << 21) ? 3 : 4;
+    if (slots <= (1u << 20)) return 3;
+    return slots <= (lights ? 1u << 22 : 1u << 23) ? 4 : 5;
+}
 hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream);
 // Path-replay adjoint over samples [sample0, sample0 + nsamples) (adjoint.hip).
 int adjointBlocksPerCU();

@@ -251,7 +251,7 @@ private:
     int wfPerCu_[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     uint64_t wfMaxSlots_ = 0;
     bool dirty_ = true;
-    int blocks_ = 0, cus_ = 0;
+    int blocks_ = 0, cus_ = 0, xcds_ = 1;
     uint64_t totalTiles_ = 0;
     omv_render_stats stats_{};
     hipStream_t stream_ = nullptr;

@@ -93,6 +93,35 @@ def test_batch_mixed_lights_and_zero_spp(pkg, wl):
         assert np.all(z[..., :3] == 0) and np.all(z[..., 3] == 1)
 
 
+@pytest.mark.parametrize("streams", [1, 3])
+@pytest.mark.parametrize("nee", [False, True])
+def test_batch_streams_deep_jobs(pkg, wl, nee, streams):
+    """Jobs on streams end in a tail launch and deal their queues to the XCDs:
+    paths that end before, in and after the tail's first round, scenes of few
+    and of many instances, each job's film that of a single render."""
+    desc, view = wl.mixed_test_scene(hdr=True, lights=True)
+    desc2, view2, _ = wl.large_instanced(width=48, height=27, spp=2, depth=6, count=24, tris_per=600, hdr_w=64, hdr_h=32)
+    scenes = [pkg.Scene(), pkg.Scene()]
+    desc.apply(scenes[0], pkg.pbr_desc)
+    desc2.apply(scenes[1], pkg.pbr_desc)
+    b = pkg.Batch()
+    plain = []
+    for j, depth in enumerate((1, 2, 3, 4, 8)):
+        for k, v in enumerate((view, view2)):
+            p = dict(samples_per_pixel=3, camera_bounces=depth, light_bounces=2, max_path_length=depth + 1, seed=j, extensions=pkg.EXT_HDRI_NEE if nee else 0)
+            cam = pkg.Camera(45, 31, v.position, v.forward, v.up, v.yfov)
+            r = pkg.Renderer(pkg.default_params(**p))
+            r.set_scene(scenes[k])
+            r.set_schedule(pkg.SCHEDULE_PER_SAMPLE)
+            plain.append(r.render(cam))
+            b.add_job(scenes[k], cam, pkg.default_params(**p))
+    b.set_tuning(streams=streams)
+    for _ in range(3):
+        b.run()
+        for j, want in enumerate(plain):
+            assert np.array_equal(b.film(j), want), j
+
+
 def test_batch_job_against_oracle(pkg, wl, ref):
     assets, jobs, scenes = _small_batch(pkg, wl, n_jobs=4)
     b = _batch(pkg, jobs, scenes)

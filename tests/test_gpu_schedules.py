@@ -390,3 +390,26 @@ def test_sorted_shading_keeps_the_film(pkg, wl, kind, size):
         r.set_tuning(tail_round=3)
         out.append((r.render(cam), r.stats()))
     _same(out)
+
+
+# samples at the edges of the default tail round: 2^20, 2^21, 2^22 and 2^23
+@pytest.mark.parametrize("size", [(1024, 1024, 1), (1025, 1024, 1), (1024, 1024, 2), (1025, 1024, 2),
+                                  (2048, 2048, 1), (2049, 2048, 1), (2048, 2048, 2), (2049, 2048, 2)])
+@pytest.mark.parametrize("kind", ["plain", "lights", "nee"])
+def test_default_tail_round_keeps_the_film(pkg, wl, kind, size):
+    w, h, spp = size
+    desc, view = wl.mixed_test_scene(hdr=True, lights=kind == "lights", masked=False)
+    s = pkg.Scene()
+    desc.apply(s, pkg.pbr_desc)
+    cam = pkg.Camera(w, h, view.position, view.forward, view.up, view.yfov)
+    out = []
+    for tail in (0, 1):
+        r = pkg.Renderer(pkg.default_params(samples_per_pixel=spp, camera_bounces=5, light_bounces=2, max_path_length=5, seed=4,
+                                            extensions=pkg.EXT_HDRI_NEE if kind == "nee" else 0))
+        r.set_scene(s)
+        if tail:
+            r.set_tuning(tail_round=tail)
+        out.append((r.render(cam), r.stats()))
+    assert np.array_equal(out[0][0], out[1][0])
+    for k in ("rays", "camera_rays", "light_rays", "shadow_rays", "samples"):
+        assert out[0][1][k] == out[1][1][k], k
