@@ -5,14 +5,14 @@
 //   1. one lane per triangle: box and centroid from the vertex pool;
 //      centroid bounds by a block reduction;
 //   2. 30-bit Morton code of each centroid in those bounds; stable LSD radix
-//      sort of (code, triangle) in four 8-bit passes -- each sort lane owns
-//      a contiguous chunk of 256 keys and walks it in order, so equal codes
-//      keep triangle order;
+//      sort of (code, triangle) in four 8-bit passes (device_sort.h), so
+//      equal codes keep triangle order;
 //   3. the binary radix tree over the sorted codes (Karras, "Maximizing
 //      parallelism in the construction of BVHs, octrees, and k-d trees",
 //      2012), codes made unique by appending the sorted position;
-//   4. boxes bottom-up: one lane per leaf climbs while it is the second
-//      child to arrive at a node (atomic counter per node);
+//   4. a node's box is the union of a run of sorted leaves: boxes of every
+//      aligned run of 2^k leaves first (lbRuns), of which a node takes at
+//      most two of each length;
 //   5. collapse into the 128-byte 4-wide nodes the traversal reads, one
 //      level per launch: a node takes its binary node's two children and
 //      keeps replacing the largest-area one by its children until it has
@@ -26,17 +26,22 @@
 // for bit; only node and triangle counts change.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
-#include <vector>
+#include <utility>
 
 #include "device_sort.h"
 #include "omv_kernels.h"
 
 namespace {
 
-constexpr int kChunk = 256;          // keys per sort lane
 constexpr int kBlock = 256;
 constexpr uint32_t kLeafBit = 0x80000000u;
+constexpr int kCollapseLevels = 16;  // collapse levels launched between two readbacks (even)
+
+// boxes of the aligned runs of 2^k sorted leaves, k = 0 .. count - 1: run j of
+// length 2^k is box off[k] + j, the last of a length possibly shorter
+struct LbRuns { uint32_t off[30]; int count; };
 
 __device__ inline float padDown(float v) { for (int k = 0; k < OMV_BOX_PAD_ULPS; ++k) v = nextafterf(v, -INFINITY); return v; }
 __device__ inline float padUp(float v) { for (int k = 0; k < OMV_BOX_PAD_ULPS; ++k) v = nextafterf(v, INFINITY); return v; }
@@ -122,6 +127,39 @@ __global__ void lbMorton(const float* __restrict__ cen, const float* __restrict_
     val[f] = f;
 }
 
+// 4a. Run boxes of lengths 2^(k0 + 1) .. 2^(k0 + 8) from those of 2^k0; at
+// k0 = 0 the leaves' boxes too, gathered into sorted order.  A leaf box is
+// read once and about two boxes a leaf are written, in up to four launches.
+__global__ __launch_bounds__(kBlock) void lbRuns(const uint32_t* __restrict__ val, const float* __restrict__ triBox, uint32_t n, int k0,
+                                                 LbRuns R, float* __restrict__ runs) {
+    __shared__ float red[6][kBlock];
+    const uint32_t t = threadIdx.x, i = blockIdx.x * kBlock + t;
+    const uint32_t m = (uint32_t)(((uint64_t)n + (1ull << k0) - 1) >> k0);
+    float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    if (i < m) {
+        const float* b = k0 == 0 ? triBox + (size_t)6 * val[i] : runs + (size_t)6 * (R.off[k0] + i);
+        for (int a = 0; a < 6; ++a) v[a] = b[a];
+        if (k0 == 0)
+            for (int a = 0; a < 6; ++a) runs[(size_t)6 * i + a] = v[a];
+    }
+    for (int a = 0; a < 6; ++a) red[a][t] = v[a];
+    for (int s = 1; s <= 8 && k0 + s < R.count; ++s) {
+        __syncthreads();
+        const uint32_t half = kBlock >> s, o = blockIdx.x * half + t;
+        if (t < half)
+            for (int a = 0; a < 3; ++a) {
+                v[a] = fminf(red[a][2 * t], red[a][2 * t + 1]);
+                v[3 + a] = fmaxf(red[3 + a][2 * t], red[3 + a][2 * t + 1]);
+            }
+        __syncthreads();
+        if (t < half) {
+            for (int a = 0; a < 6; ++a) red[a][t] = v[a];
+            if (o < (uint32_t)(((uint64_t)n + (1ull << (k0 + s)) - 1) >> (k0 + s)))
+                for (int a = 0; a < 6; ++a) runs[(size_t)6 * (R.off[k0 + s] + o) + a] = v[a];
+        }
+    }
+}
+
 // 3. radix tree; codes extended by the sorted position make them unique
 __device__ inline int prefixLen(const uint32_t* __restrict__ key, int n, int i, int j) {
     if (j < 0 || j >= n) return -1;
@@ -129,8 +167,11 @@ __device__ inline int prefixLen(const uint32_t* __restrict__ key, int n, int i, 
     return __clzll(a ^ b);
 }
 
-__global__ void lbTree(const uint32_t* __restrict__ key, int n, uint32_t* __restrict__ left, uint32_t* __restrict__ right,
-                       int* __restrict__ first, int* __restrict__ last, int* __restrict__ parentNode, int* __restrict__ parentLeaf) {
+// and 4b. each node's box from the run boxes.  200 K triangles: 38 us with the
+// run boxes made (MI355X); climbing from the leaves, a lane per leaf with a fence
+// for the device and a counter at every node, took 927 us.
+__global__ void lbTree(const uint32_t* __restrict__ key, int n, LbRuns R, const float* __restrict__ runs, uint32_t* __restrict__ left,
+                       uint32_t* __restrict__ right, int* __restrict__ first, int* __restrict__ last, float* __restrict__ nodeBox) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n - 1) return;
     const int d = prefixLen(key, n, i, i + 1) > prefixLen(key, n, i, i - 1) ? 1 : -1;
@@ -151,43 +192,19 @@ __global__ void lbTree(const uint32_t* __restrict__ key, int n, uint32_t* __rest
     const int lo = min(i, j), hi = max(i, j);
     first[i] = lo;
     last[i] = hi;
-    if (lo == gamma) { left[i] = kLeafBit | (uint32_t)gamma; parentLeaf[gamma] = i; }
-    else { left[i] = (uint32_t)gamma; parentNode[gamma] = i; }
-    if (hi == gamma + 1) { right[i] = kLeafBit | (uint32_t)(gamma + 1); parentLeaf[gamma + 1] = i; }
-    else { right[i] = (uint32_t)(gamma + 1); parentNode[gamma + 1] = i; }
-}
-
-__device__ inline void loadBox(const float* __restrict__ box, uint32_t idx, float lo[3], float hi[3]) {
-    for (int a = 0; a < 3; ++a) {
-        lo[a] = __hip_atomic_load(&box[(size_t)6 * idx + a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        hi[a] = __hip_atomic_load(&box[(size_t)6 * idx + 3 + a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    left[i] = lo == gamma ? kLeafBit | (uint32_t)gamma : (uint32_t)gamma;
+    right[i] = hi == gamma + 1 ? kLeafBit | (uint32_t)(gamma + 1) : (uint32_t)(gamma + 1);
+    float b[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    auto take = [&](uint32_t run) {
+        const float* q = runs + (size_t)6 * run;
+        for (int a = 0; a < 3; ++a) { b[a] = fminf(b[a], q[a]); b[3 + a] = fmaxf(b[3 + a], q[3 + a]); }
+    };
+    uint32_t from = (uint32_t)lo, to = (uint32_t)hi + 1u;   // whole runs of 2^k leaves in [lo, hi], k rising
+    for (int k = 0; from < to; ++k, from >>= 1, to >>= 1) {
+        if (from & 1u) take(R.off[k] + from++);
+        if (to & 1u) take(R.off[k] + --to);
     }
-}
-
-// 4. node boxes bottom-up (the second child to arrive builds the parent)
-__global__ void lbRefit(const uint32_t* __restrict__ val, const float* __restrict__ triBox, int n, const uint32_t* __restrict__ left,
-                        const uint32_t* __restrict__ right, const int* __restrict__ parentNode, const int* __restrict__ parentLeaf,
-                        float* __restrict__ leafBox, float* __restrict__ nodeBox, uint32_t* __restrict__ arrived) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t prim = val[i];
-    for (int a = 0; a < 6; ++a)
-        __hip_atomic_store(&leafBox[(size_t)6 * i + a], triBox[(size_t)6 * prim + a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    int p = n > 1 ? parentLeaf[i] : -1;
-    while (p >= 0) {
-        __threadfence();
-        if (atomicAdd(&arrived[p], 1u) == 0u) return;   // the sibling is not done yet
-        __threadfence();
-        float lo[3], hi[3], lo2[3], hi2[3];
-        const uint32_t l = left[p], r = right[p];
-        loadBox((l & kLeafBit) ? leafBox : nodeBox, l & ~kLeafBit, lo, hi);
-        loadBox((r & kLeafBit) ? leafBox : nodeBox, r & ~kLeafBit, lo2, hi2);
-        for (int a = 0; a < 3; ++a) {
-            __hip_atomic_store(&nodeBox[(size_t)6 * p + a], fminf(lo[a], lo2[a]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&nodeBox[(size_t)6 * p + 3 + a], fmaxf(hi[a], hi2[a]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        p = parentNode[p];
-    }
+    for (int a = 0; a < 6; ++a) nodeBox[(size_t)6 * i + a] = b[a];
 }
 
 struct BinRef {   // a binary tree node: internal index, or a leaf with kLeafBit
@@ -203,69 +220,81 @@ __device__ inline float halfArea(const float lo[3], const float hi[3]) {
     return d0 * d1 + d1 * d2 + d2 * d0;
 }
 
-// 5. one level of the collapse: jobs are (binary node, output node)
-__global__ void lbCollapse(const uint2* __restrict__ jobs, uint32_t njobs, const uint32_t* __restrict__ left, const uint32_t* __restrict__ right,
+// Counters of the collapse: [0] output nodes, [1] overflow, [2 + l] jobs of
+// level l of this batch of levels.  A later batch starts with the jobs left.
+__global__ void lbCollapseInit(uint32_t* __restrict__ c, uint2* __restrict__ jobs, bool start, uint32_t root) {
+    const uint32_t t = threadIdx.x;
+    const uint32_t left = start ? 1u : c[2 + kCollapseLevels];
+    __syncthreads();
+    if (t <= kCollapseLevels) c[2 + t] = t == 0 ? left : 0u;
+    if (t == 0 && start) { c[0] = 1u; c[1] = 0u; jobs[0] = make_uint2(root, 0u); }
+}
+
+// 5. one level of the collapse: jobs are (binary node, output node).  Their
+// number stays on the device, so a whole batch of levels is launched at once.
+__global__ void lbCollapse(const uint2* __restrict__ jobs, const uint32_t* __restrict__ jobCount, const uint32_t* __restrict__ left, const uint32_t* __restrict__ right,
                            const int* __restrict__ first, const int* __restrict__ last, const float* __restrict__ leafBox,
                            const float* __restrict__ nodeBox, int leafMax, int recBase, int nodeBase, uint32_t nodeCap,
                            OmvNode4* __restrict__ out, uint32_t* __restrict__ nodeCount, uint2* __restrict__ next, uint32_t* __restrict__ nextCount,
                            uint32_t* __restrict__ overflow) {
-    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-    if (t >= njobs) return;
-    const uint32_t b = jobs[t].x, o = jobs[t].y;
-    uint32_t kids[4];
-    int nk = 0;
-    if ((b & kLeafBit) || countOf(b, first, last) <= leafMax) {
-        kids[nk++] = b;   // a small root: one-child node holding a leaf
-    } else {
-        kids[nk++] = left[b];
-        kids[nk++] = right[b];
-        while (nk < 4) {
-            int best = -1;
-            float bestA = -1.0f;
-            for (int k = 0; k < nk; ++k) {
-                if ((kids[k] & kLeafBit) || countOf(kids[k], first, last) <= leafMax) continue;
-                float lo[3], hi[3];
-                for (int a = 0; a < 3; ++a) { lo[a] = nodeBox[(size_t)6 * kids[k] + a]; hi[a] = nodeBox[(size_t)6 * kids[k] + 3 + a]; }
-                const float ar = halfArea(lo, hi);
-                if (ar > bestA) { bestA = ar; best = k; }
-            }
-            if (best < 0) break;
-            const uint32_t inner = kids[best];
-            kids[best] = left[inner];
-            kids[nk++] = right[inner];
-        }
-    }
-    OmvNode4 nd;
-    for (int k = 0; k < 4; ++k) {
-        if (k >= nk) {
-            nd.child[k] = OMV_EMPTY_CHILD;
-            nd.entry[k] = OMV_ENT_NONE;
-            nd.lox[k] = nd.loy[k] = nd.loz[k] = nd.hix[k] = nd.hiy[k] = nd.hiz[k] = INFINITY;   // no ray hits it
-            continue;
-        }
-        const uint32_t c = kids[k];
-        const float* bx = (c & kLeafBit) ? leafBox + (size_t)6 * (c & ~kLeafBit) : nodeBox + (size_t)6 * c;
-        nd.lox[k] = padDown(bx[0]); nd.loy[k] = padDown(bx[1]); nd.loz[k] = padDown(bx[2]);
-        nd.hix[k] = padUp(bx[3]); nd.hiy[k] = padUp(bx[4]); nd.hiz[k] = padUp(bx[5]);
-        const int cnt = countOf(c, first, last);
-        if (cnt <= leafMax) {
-            nd.child[k] = -(recBase + firstOf(c, first) + 1);
-            nd.entry[k] = OMV_ENT(OMV_ENT_BLAS_LEAF, ((uint32_t)(recBase + firstOf(c, first)) << 3) | ((uint32_t)(cnt - 1) & 7u));
+    const uint32_t njobs = *jobCount;
+    for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t < njobs; t += gridDim.x * kBlock) {
+        const uint32_t b = jobs[t].x, o = jobs[t].y;
+        uint32_t kids[4];
+        int nk = 0;
+        if ((b & kLeafBit) || countOf(b, first, last) <= leafMax) {
+            kids[nk++] = b;   // a small root: one-child node holding a leaf
         } else {
-            const uint32_t idx = atomicAdd(nodeCount, 1u);
-            if (idx >= nodeCap) {   // cannot happen (one output node per binary node); keep the launch in bounds
-                atomicAdd(overflow, 1u);
+            kids[nk++] = left[b];
+            kids[nk++] = right[b];
+            while (nk < 4) {
+                int best = -1;
+                float bestA = -1.0f;
+                for (int k = 0; k < nk; ++k) {
+                    if ((kids[k] & kLeafBit) || countOf(kids[k], first, last) <= leafMax) continue;
+                    float lo[3], hi[3];
+                    for (int a = 0; a < 3; ++a) { lo[a] = nodeBox[(size_t)6 * kids[k] + a]; hi[a] = nodeBox[(size_t)6 * kids[k] + 3 + a]; }
+                    const float ar = halfArea(lo, hi);
+                    if (ar > bestA) { bestA = ar; best = k; }
+                }
+                if (best < 0) break;
+                const uint32_t inner = kids[best];
+                kids[best] = left[inner];
+                kids[nk++] = right[inner];
+            }
+        }
+        OmvNode4 nd;
+        for (int k = 0; k < 4; ++k) {
+            if (k >= nk) {
                 nd.child[k] = OMV_EMPTY_CHILD;
                 nd.entry[k] = OMV_ENT_NONE;
+                nd.lox[k] = nd.loy[k] = nd.loz[k] = nd.hix[k] = nd.hiy[k] = nd.hiz[k] = INFINITY;   // no ray hits it
                 continue;
             }
-            nd.child[k] = nodeBase + (int)idx;
-            nd.entry[k] = OMV_ENT(OMV_ENT_BLAS_NODE, nodeBase + (int)idx);
-            const uint32_t q = atomicAdd(nextCount, 1u);
-            next[q] = make_uint2(c, idx);
+            const uint32_t c = kids[k];
+            const float* bx = (c & kLeafBit) ? leafBox + (size_t)6 * (c & ~kLeafBit) : nodeBox + (size_t)6 * c;
+            nd.lox[k] = padDown(bx[0]); nd.loy[k] = padDown(bx[1]); nd.loz[k] = padDown(bx[2]);
+            nd.hix[k] = padUp(bx[3]); nd.hiy[k] = padUp(bx[4]); nd.hiz[k] = padUp(bx[5]);
+            const int cnt = countOf(c, first, last);
+            if (cnt <= leafMax) {
+                nd.child[k] = -(recBase + firstOf(c, first) + 1);
+                nd.entry[k] = OMV_ENT(OMV_ENT_BLAS_LEAF, ((uint32_t)(recBase + firstOf(c, first)) << 3) | ((uint32_t)(cnt - 1) & 7u));
+            } else {
+                const uint32_t idx = atomicAdd(nodeCount, 1u);
+                if (idx >= nodeCap) {   // cannot happen (one output node per binary node); keep the launch in bounds
+                    atomicAdd(overflow, 1u);
+                    nd.child[k] = OMV_EMPTY_CHILD;
+                    nd.entry[k] = OMV_ENT_NONE;
+                    continue;
+                }
+                nd.child[k] = nodeBase + (int)idx;
+                nd.entry[k] = OMV_ENT(OMV_ENT_BLAS_NODE, nodeBase + (int)idx);
+                const uint32_t q = atomicAdd(nextCount, 1u);
+                next[q] = make_uint2(c, idx);
+            }
         }
+        out[o] = nd;
     }
-    out[o] = nd;
 }
 
 // 6. triangle records in sorted order
@@ -290,10 +319,9 @@ namespace omv {
 
 // Scratch sizes for n triangles, in bytes (one allocation, carved below).
 size_t blasDeviceScratchBytes(uint32_t n) {
-    const uint64_t nc = (n + kChunk - 1) / kChunk;
-    // 22 arrays, each rounded up to an even number of words
-    return 4 * ((uint64_t)6 * n + 3 * n + 6 * blocks(n) + 8 + 4 * (uint64_t)n + 256 * nc + 4 * (uint64_t)n + 2 * (uint64_t)n +
-                6 * (uint64_t)n + 6 * (uint64_t)n + (uint64_t)n + 4 * (uint64_t)n + 8 + 2 * 22) + 256;
+    // 19 arrays, each rounded up to an even number of words
+    return 4 * ((uint64_t)6 * n + 3 * n + 6 * blocks(n) + 8 + 4 * (uint64_t)n + sortHistWords(n) + 4 * (uint64_t)n +
+                6 * (2 * (uint64_t)n + 32) + 6 * (uint64_t)n + 4 * (uint64_t)n + 2 + kCollapseLevels + 1 + 2 * 19) + 256;
 }
 
 hipError_t buildBlasDevice(const float* vtx, uint32_t vtxOff, uint32_t stride, const uint32_t* faces, uint32_t faceOff, uint32_t n,
@@ -302,7 +330,7 @@ hipError_t buildBlasDevice(const float* vtx, uint32_t vtxOff, uint32_t stride, c
     *root = -1; *nodeCount = 0; *depth = 0;
     if (n == 0 || nodeCap == 0) return hipSuccess;
     if (nodeCap > n) nodeCap = n;   // one output node per binary node at most: the job queues hold n entries
-    const uint32_t nb = blocks(n), nc = (n + kChunk - 1) / kChunk;
+    const uint32_t nb = blocks(n);
     uint32_t* p = static_cast<uint32_t*>(scratch);
     auto take = [&p](uint64_t words) { uint32_t* q = p; p += (words + 1) & ~(uint64_t)1; return q; };   // 8-byte aligned
     float* triBox = reinterpret_cast<float*>(take((uint64_t)6 * n));
@@ -313,53 +341,56 @@ hipError_t buildBlasDevice(const float* vtx, uint32_t vtxOff, uint32_t stride, c
     uint32_t* valA = take(n);
     uint32_t* keyB = take(n);
     uint32_t* valB = take(n);
-    uint32_t* hist = take((uint64_t)256 * nc);
+    uint32_t* hist = take(sortHistWords(n));
     uint32_t* left = take(n);
     uint32_t* right = take(n);
     int* first = reinterpret_cast<int*>(take(n));
     int* last = reinterpret_cast<int*>(take(n));
-    int* parentNode = reinterpret_cast<int*>(take(n));
-    int* parentLeaf = reinterpret_cast<int*>(take(n));
-    float* leafBox = reinterpret_cast<float*>(take((uint64_t)6 * n));
+    float* runs = reinterpret_cast<float*>(take(6 * (2 * (uint64_t)n + 32)));
     float* nodeBox = reinterpret_cast<float*>(take((uint64_t)6 * n));
-    uint32_t* arrived = take(n);
     uint2* jobsA = reinterpret_cast<uint2*>(take((uint64_t)2 * n));
     uint2* jobsB = reinterpret_cast<uint2*>(take((uint64_t)2 * n));
-    uint32_t* counters = take(8);   // [0] node count, [1] next jobs, [2] overflow
+    uint32_t* counters = take(2 + kCollapseLevels + 1);
 
+    LbRuns R;
+    R.count = 0;
+    for (uint64_t at = 0, m = n;; m = (m + 1) / 2) {   // n < 2^27: at most 28 lengths, fewer than 2 n + 32 boxes
+        R.off[R.count++] = (uint32_t)at;
+        at += m;
+        if (m == 1) break;
+    }
     hipError_t e;
     lbBoxes<<<nb, kBlock, 0, stream>>>(vtx, vtxOff, stride, faces, faceOff, n, triBox, cen, part);
     lbBounds<<<1, kBlock, 0, stream>>>(part, nb, bounds);
     lbMorton<<<nb, kBlock, 0, stream>>>(cen, bounds, n, keyA, valA);
-    if ((e = sortPairs32(keyA, valA, keyB, valB, hist, n, stream)) != hipSuccess) return e;
-    uint32_t* kIn = keyA; uint32_t* vIn = valA;
-    // the root has no parent
-    if ((e = hipMemsetAsync(parentNode, 0xFF, (size_t)n * 4, stream)) != hipSuccess) return e;
-    if (n > 1) lbTree<<<blocks(n - 1), kBlock, 0, stream>>>(kIn, (int)n, left, right, first, last, parentNode, parentLeaf);
-    if ((e = hipMemsetAsync(arrived, 0, (size_t)n * 4, stream)) != hipSuccess) return e;
-    lbRefit<<<nb, kBlock, 0, stream>>>(vIn, triBox, (int)n, left, right, parentNode, parentLeaf, leafBox, nodeBox, arrived);
-    lbRecords<<<nb, kBlock, 0, stream>>>(vtx, vtxOff, stride, faces, faceOff, vIn, n, records + (size_t)12 * recBase);
+    if ((e = sortPairs32(keyA, valA, keyB, valB, hist, n, 30, stream)) != hipSuccess) return e;
+    for (int k0 = 0; k0 == 0 || k0 + 1 < R.count; k0 += 8)
+        lbRuns<<<blocks(((uint64_t)n + (1ull << k0) - 1) >> k0), kBlock, 0, stream>>>(valA, triBox, n, k0, R, runs);
+    if (n > 1) lbTree<<<blocks(n - 1), kBlock, 0, stream>>>(keyA, (int)n, R, runs, left, right, first, last, nodeBox);
+    lbRecords<<<nb, kBlock, 0, stream>>>(vtx, vtxOff, stride, faces, faceOff, valA, n, records + (size_t)12 * recBase);
     if ((e = hipGetLastError()) != hipSuccess) return e;
 
-    // collapse, level by level from the root (binary node 0, or the single leaf)
-    const uint2 rootJob = make_uint2(n > 1 ? 0u : kLeafBit, 0u);
-    uint32_t init[3] = {1u, 0u, 0u};
-    if ((e = hipMemcpyAsync(jobsA, &rootJob, sizeof(rootJob), hipMemcpyHostToDevice, stream)) != hipSuccess) return e;
-    if ((e = hipMemcpyAsync(counters, init, sizeof(init), hipMemcpyHostToDevice, stream)) != hipSuccess) return e;
-    uint32_t njobs = 1;
+    // Collapse, level by level from the root (binary node 0, or the single
+    // leaf); the host reads the counts once per kCollapseLevels levels.  Level
+    // l holds at most 4^l jobs; a grid of more than 1024 workgroups strides.
+    const float* leafBox = runs;
     int levels = 0;
-    uint2* cur = jobsA; uint2* nxt = jobsB;
-    while (njobs > 0) {
-        ++levels;
-        if ((e = hipMemsetAsync(counters + 1, 0, 4, stream)) != hipSuccess) return e;
-        lbCollapse<<<blocks(njobs), kBlock, 0, stream>>>(cur, njobs, left, right, first, last, leafBox, nodeBox, leafMax, recBase, nodeBase,
-                                                        nodeCap, nodes + nodeBase, counters, nxt, counters + 1, counters + 2);
-        uint32_t c[3];
+    for (bool more = true, start = true; more; start = false) {
+        lbCollapseInit<<<1, 64, 0, stream>>>(counters, jobsA, start, n > 1 ? 0u : kLeafBit);
+        uint2* cur = jobsA; uint2* nxt = jobsB;
+        for (int l = 0; l < kCollapseLevels; ++l, std::swap(cur, nxt)) {
+            const uint64_t most = levels + l < 16 ? std::min<uint64_t>(n, 1ull << (2 * (levels + l))) : n;
+            lbCollapse<<<std::min(blocks(most), 1024u), kBlock, 0, stream>>>(cur, counters + 2 + l, left, right, first, last, leafBox, nodeBox,
+                                                                             leafMax, recBase, nodeBase, nodeCap, nodes + nodeBase, counters,
+                                                                             nxt, counters + 3 + l, counters + 1);
+        }
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        uint32_t c[2 + kCollapseLevels + 1];
         if ((e = hipMemcpyAsync(c, counters, sizeof(c), hipMemcpyDeviceToHost, stream)) != hipSuccess) return e;
         if ((e = hipStreamSynchronize(stream)) != hipSuccess) return e;
-        if (c[2]) return hipErrorInvalidValue;
-        njobs = c[1];
-        std::swap(cur, nxt);
+        if (c[1]) return hipErrorInvalidValue;
+        for (int l = 0; l < kCollapseLevels; ++l) levels += c[2 + l] != 0;
+        more = c[2 + kCollapseLevels] != 0;
         *nodeCount = (int)c[0];
     }
     *root = nodeBase;

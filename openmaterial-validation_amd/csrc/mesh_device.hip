@@ -164,7 +164,7 @@ namespace omv {
 
 size_t meshDeviceScratchBytes(uint32_t vn, uint32_t fn) {
     const uint64_t corners = 3ull * fn;
-    const uint64_t words = 4 * corners + 256ull * sortChunks((uint32_t)corners) + 2ull * vn + 7ull * fn + 8 + 2 * 9;
+    const uint64_t words = 4 * corners + sortHistWords((uint32_t)corners) + 2ull * vn + 7ull * fn + 8 + 2 * 9;
     return words * 4 + 256;
 }
 
@@ -182,7 +182,7 @@ hipError_t preprocessMeshDevice(float* vertices, uint32_t stride, uint32_t vn, c
     uint32_t* valA = take(corners);
     uint32_t* keyB = take(corners);
     uint32_t* valB = take(corners);
-    uint32_t* hist = take(256ull * sortChunks(corners));
+    uint32_t* hist = take(sortHistWords(corners));
     uint32_t* begin = take(vn);
     uint32_t* end = take(vn);
     float* faceData = reinterpret_cast<float*>(take(7ull * fn));
@@ -190,7 +190,7 @@ hipError_t preprocessMeshDevice(float* vertices, uint32_t stride, uint32_t vn, c
     hipError_t e;
     if ((e = hipMemsetAsync(bad, 0, 4, stream)) != hipSuccess) return e;
     mdCorners<<<grid(corners), kBlk, 0, stream>>>(faces, corners, vn, keyA, valA, bad);
-    if ((e = sortPairs32(keyA, valA, keyB, valB, hist, corners, stream)) != hipSuccess) return e;
+    if ((e = sortPairs32(keyA, valA, keyB, valB, hist, corners, 32 - __builtin_clz(vn), stream)) != hipSuccess) return e;
     if ((e = hipMemsetAsync(begin, 0, (size_t)vn * 4, stream)) != hipSuccess) return e;
     if ((e = hipMemsetAsync(end, 0, (size_t)vn * 4, stream)) != hipSuccess) return e;
     mdRanges<<<grid(corners), kBlk, 0, stream>>>(keyA, corners, vn, begin, end);

@@ -177,3 +177,47 @@ def test_device_mesh_preprocessing_bitexact(pkg, wl, kind):
     assert ma == mb
     assert np.array_equal(a, b), np.argwhere(a != b)[:5].tolist()
     assert np.all(np.isfinite(a))
+
+
+# triangles and vertices at the edges of a sort tile (1024 pairs; 3 corners a
+# triangle), of the sort's 8-bit passes (vertex ids below and from 2^8, 2^16),
+# of a digit's scan (256 tiles), of a workgroup's and a launch's run boxes
+# (256, 65536 triangles) and of the collapse's grid (1024 workgroups)
+SIZES = [(85, 255), (255, 256), (256, 257), (341, 100), (342, 100), (1023, 65535), (1024, 65536), (1025, 65537), (65535, 40000),
+         (65536, 30000), (65537, 30000), (87381, 1), (262145, 70000), (1200000, 300000)]
+
+
+@pytest.mark.parametrize("tris,verts", SIZES)
+def test_device_build_at_the_edges_of_its_tiles(pkg, wl, tris, verts):
+    """Triangle soups over few or many shared vertices (verts = 1: every
+    corner the same vertex): normals and tangents of the device build equal
+    the host's bit for bit, and its tree gives the same ids and ties."""
+    rng = np.random.default_rng(tris)
+    v = rng.uniform(-1, 1, (verts, 3)).astype(np.float32)
+    if verts > 300:   # small triangles: corners that are near each other along a curve
+        v = v[np.argsort(v[:, 0])]
+        f = (rng.integers(0, verts, (tris, 1)) + rng.integers(0, 40, (tris, 3))) % verts
+    else:
+        f = rng.integers(0, verts, (tris, 3))
+    d = wl.SceneDesc()
+    d.materials.append(("pbr", dict(base_color=(0.5, 0.5, 0.5, 1.0), metallic=0.2, roughness=0.4, textures={2: 0})))
+    d.textures.append(("rgba8", np.full((4, 4, 4), 128, np.uint8)))
+    d.meshes.append({"vertices": v, "faces": f.astype(np.uint32), "mat_id": 0, "uvs": [rng.uniform(0, 1, (verts, 2)).astype(np.float32)]})
+    d.instances.append((wl.trs((0.1, 0.0, -2.5), angle=0.3), 0))
+    d.fc_subject = "pid"
+    cam = pkg.Camera(61, 47, (0.0, 0.0, 0.0), (0.0, 0.0, -1.0), (0.0, 1.0, 0.0), 50.0)
+    out = []
+    for mode in (pkg.BUILD_HOST_SAH, pkg.BUILD_DEVICE_LBVH):
+        s = pkg.Scene()
+        s.set_build_mode(mode)
+        d.apply(s, pkg.pbr_desc)
+        r = pkg.Renderer(pkg.default_params(seed=4))
+        r.set_scene(s)
+        out.append((s.mesh_vertices(0)[0],) + tuple(r.render_fc(cam)) + (s.bvh_info(),))
+    a, b = out
+    for k in range(4):
+        assert np.array_equal(a[k], b[k]), k
+    assert a[4]["tri_records"] == b[4]["tri_records"] == tris
+    assert b[4]["nodes"] <= tris + 1
+    if verts > 1:
+        assert (a[2][0] >= 0).mean() > 0.02
