@@ -169,43 +169,6 @@ void affineInverse(const float* M, float* out) {
     }
 }
 
-// Boxes that together hold the subtree of `root`: the root's children, the one
-// of largest area replaced by its own children while at most `most` remain
-// (most = 0: the children as they are; no node but the root is read).  An
-// instance's box is the box of these boxes turned by its matrix one by one,
-// which for a rotated mesh is far tighter than that of the turned root box, so
-// rays enter fewer instances that they miss: 60 rotated meshes of 33 K
-// triangles under lights, 1080p x 16 (MI355X), 6.59 -> 6.24 nodes per ray and
-// 8.78 -> 8.42 ms per render.
-constexpr int kCoverBoxes = 128;
-void coverBoxes(const OmvNode4* nodes, int root, int most, std::vector<BuildBox>& out) {
-    struct Item { float area; int node; BuildBox box; };   // node < 0: a leaf
-    auto smaller = [](const Item& a, const Item& b) { return a.area < b.area; };
-    std::vector<Item> heap;
-    auto addChildren = [&](int n) {
-        const OmvNode4& nd = nodes[n];
-        for (int k = 0; k < 4; ++k) {
-            if (nd.child[k] == OMV_EMPTY_CHILD) continue;
-            Item it;
-            it.node = nd.child[k] >= 0 ? nd.child[k] : -1;
-            const float lo[3] = {nd.lox[k], nd.loy[k], nd.loz[k]}, hi[3] = {nd.hix[k], nd.hiy[k], nd.hiz[k]};
-            float d[3];
-            for (int a = 0; a < 3; ++a) { it.box.lo[a] = lo[a]; it.box.hi[a] = hi[a]; d[a] = hi[a] - lo[a]; }
-            it.area = it.node < 0 ? -1.0f : d[0] * d[1] + d[1] * d[2] + d[2] * d[0];   // leaves are not replaced
-            heap.push_back(it);
-            std::push_heap(heap.begin(), heap.end(), smaller);
-        }
-    };
-    addChildren(root);
-    while (!heap.empty() && heap.front().node >= 0 && (int)heap.size() + 3 <= most) {
-        const int n = heap.front().node;
-        std::pop_heap(heap.begin(), heap.end(), smaller);
-        heap.pop_back();
-        addChildren(n);
-    }
-    for (const Item& it : heap) out.push_back(it.box);
-}
-
 int hipFail(hipError_t e, const char* what) {
     setError(std::string(what) + ": " + hipGetErrorString(e));
     return OMV_E_DEVICE;
@@ -624,7 +587,6 @@ int RenderScene::commit(std::string& log) {
     }
     if ((deviceBuild ? (size_t)recTotal : tris.size() / 12) >= (1u << 27)) { setError("commit: more than 2^27 triangles"); return OMV_E_SCENE; }
     // device BLAS build: vertex and face pools first, then one build per mesh
-    std::vector<OmvNode4> blasRoots(meshes_.size());
     int deviceNodes = 0;
     if (deviceBuild) {
         hipError_t e;
@@ -636,8 +598,7 @@ int RenderScene::commit(std::string& log) {
                 nodeCap += (size_t)meshes_[i].fn;
                 scratch = std::max(scratch, blasDeviceScratchBytes((uint32_t)meshes_[i].fn));
             }
-        const size_t tlasCap = std::max<size_t>(1, insts_.size());
-        if ((e = dNodes_.reserve((nodeCap + tlasCap) * sizeof(OmvNode4))) != hipSuccess) return hipFail(e, "BVH nodes");
+        if ((e = dNodes_.reserve((nodeCap + std::max<size_t>(1, insts_.size())) * sizeof(OmvNode4))) != hipSuccess) return hipFail(e, "BVH nodes");
         if ((e = dTris_.reserve((size_t)recTotal * 12 * 4)) != hipSuccess) return hipFail(e, "triangle records");
         for (size_t i = 0; i < meshes_.size(); ++i)
             if (meshRec[i] >= 0 && (prepNormals[i] || prepTangents[i]))
@@ -667,16 +628,19 @@ int RenderScene::commit(std::string& log) {
             dmeshes[i].blas_root = root;
             deviceNodes += count;
             blasDepth = std::max(blasDepth, depth);
-            if ((e = hipMemcpy(&blasRoots[i], dNodes_.as<OmvNode4>() + root, sizeof(OmvNode4), hipMemcpyDeviceToHost)) != hipSuccess)
-                return hipFail(e, "BVH root readback");
         }
     }
     if (insts_.size() >= (1u << 29)) { setError("commit: too many instances"); return OMV_E_SCENE; }
-    // TLAS over world-space instance boxes (transformed boxes of the BLAS, see coverBoxes, rounded outward)
-    std::vector<BuildBox> iboxes;
-    std::vector<int> iids;
+    const size_t tlasCap = std::max<size_t>(1, insts_.size()), blasNodes = nodes.size();
+    if (!deviceBuild) {   // the TLAS nodes follow below
+        hipError_t e;
+        if ((e = dNodes_.reserve((blasNodes + tlasCap) * sizeof(OmvNode4))) != hipSuccess) return hipFail(e, "BVH nodes");
+        if (blasNodes && (e = hipMemcpy(dNodes_.ptr, nodes.data(), blasNodes * sizeof(OmvNode4), hipMemcpyHostToDevice)) != hipSuccess)
+            return hipFail(e, "upload nodes");
+    }
+    // TLAS over world-space instance boxes (made on the device from the nodes
+    // near each BLAS root, see instanceBoxesDevice), rounded outward
     std::vector<OmvInstance> dinsts(insts_.size());
-    std::vector<std::vector<BuildBox>> covers(meshes_.size());
     for (size_t i = 0; i < insts_.size(); ++i) {
         const HostInstance& in = insts_[i];
         OmvInstance& d = dinsts[i];
@@ -689,32 +653,29 @@ int RenderScene::commit(std::string& log) {
         if (in.meshId < 0) continue;
         d.blas_root = dmeshes[in.meshId].blas_root;
         d.mat_type = mats_[dmeshes[in.meshId].mat_id].type;
-        std::vector<BuildBox>& cover = covers[in.meshId];
-        if (cover.empty()) {
-            if (deviceBuild) coverBoxes(&blasRoots[in.meshId], 0, 0, cover);   // the other nodes are in device memory
-            else coverBoxes(nodes.data(), dmeshes[in.meshId].blas_root, kCoverBoxes, cover);
-        }
-        double wl[3] = {INFINITY, INFINITY, INFINITY}, wh[3] = {-INFINITY, -INFINITY, -INFINITY};
-        double reach[3] = {0.0, 0.0, 0.0};   // the largest sum of terms behind a coordinate: rounding goes with it
-        for (const BuildBox& c : cover) {
-            for (int a = 0; a < 3; ++a) {   // the box M turns [lo, hi] into: centre +- sum |M| * half extent
-                double mid = (double)in.tm[a * 4 + 3], half = 0.0, terms = std::fabs((double)in.tm[a * 4 + 3]);
-                for (int k = 0; k < 3; ++k) {
-                    const double m = (double)in.tm[a * 4 + k], lo = c.lo[k], hi = c.hi[k];
-                    mid += m * 0.5 * (lo + hi);
-                    half += std::fabs(m) * 0.5 * (hi - lo);
-                    terms += std::fabs(m) * std::max(std::fabs(lo), std::fabs(hi));
-                }
-                wl[a] = std::min(wl[a], mid - half);
-                wh[a] = std::max(wh[a], mid + half);
-                reach[a] = std::max(reach[a], terms);
-            }
-        }
+    }
+    std::vector<OmvInstanceBox> ibox(insts_.size());
+    if (!insts_.empty()) {
+        hipError_t e;
+        DeviceBuffer work;
+        const size_t bytes = ibox.size() * sizeof(OmvInstanceBox);
+        if ((e = dInsts_.upload(dinsts.data(), dinsts.size() * sizeof(OmvInstance))) != hipSuccess) return hipFail(e, "upload instances");
+        if ((e = work.reserve(bytes)) != hipSuccess) return hipFail(e, "instance boxes");
+        if ((e = instanceBoxesDevice(dNodes_.as<OmvNode4>(), dInsts_.as<OmvInstance>(), (uint32_t)insts_.size(), work.as<OmvInstanceBox>(),
+                                     nullptr)) != hipSuccess)
+            return hipFail(e, "instance box kernel launch");
+        if ((e = hipMemcpy(ibox.data(), work.ptr, bytes, hipMemcpyDeviceToHost)) != hipSuccess) return hipFail(e, "instance boxes");
+    }
+    std::vector<BuildBox> iboxes;
+    std::vector<int> iids;
+    for (size_t i = 0; i < insts_.size(); ++i) {
+        if (insts_[i].meshId < 0) continue;
+        const OmvInstanceBox& w = ibox[i];
         BuildBox b;
         for (int a = 0; a < 3; ++a) {
-            const double pad = 1e-5 * std::max(std::fabs(wl[a]) + std::fabs(wh[a]), reach[a]) + 1e-20;
-            b.lo[a] = std::nextafter((float)(wl[a] - pad), -INFINITY);
-            b.hi[a] = std::nextafter((float)(wh[a] + pad), INFINITY);
+            const double pad = 1e-5 * std::max(std::fabs(w.lo[a]) + std::fabs(w.hi[a]), w.reach[a]) + 1e-20;
+            b.lo[a] = std::nextafter((float)(w.lo[a] - pad), -INFINITY);
+            b.hi[a] = std::nextafter((float)(w.hi[a] + pad), INFINITY);
         }
         iboxes.push_back(b);
         iids.push_back((int)i);
@@ -810,12 +771,13 @@ int RenderScene::commit(std::string& log) {
         if ((e = dFaces_.upload(faces.data(), faces.size() * 4)) != hipSuccess) return hipFail(e, "upload faces");
     }
     if ((e = dMeshes_.upload(dmeshes.data(), dmeshes.size() * sizeof(OmvMesh))) != hipSuccess) return hipFail(e, "upload meshes");
-    if ((e = dInsts_.upload(dinsts.data(), dinsts.size() * sizeof(OmvInstance))) != hipSuccess) return hipFail(e, "upload instances");
     if ((e = dMats_.upload(mats_.data(), mats_.size() * sizeof(OmvMaterial))) != hipSuccess) return hipFail(e, "upload materials");
     if ((e = dTexs_.upload(dtex.data(), dtex.size() * sizeof(OmvTexture))) != hipSuccess) return hipFail(e, "upload textures");
     if ((e = dTexels_.upload(texels.data(), texels.size())) != hipSuccess) return hipFail(e, "upload texels");
     if (!deviceBuild) {
-        if ((e = dNodes_.upload(nodes.data(), nodes.size() * sizeof(OmvNode4))) != hipSuccess) return hipFail(e, "upload nodes");
+        if ((e = hipMemcpy(dNodes_.as<OmvNode4>() + blasNodes, nodes.data() + blasNodes, (nodes.size() - blasNodes) * sizeof(OmvNode4),
+                           hipMemcpyHostToDevice)) != hipSuccess)
+            return hipFail(e, "upload TLAS");
         if ((e = dTris_.upload(tris.data(), tris.size() * 4)) != hipSuccess) return hipFail(e, "upload triangles");
     }
     if ((e = dLights_.upload(lights_.data(), lights_.size() * sizeof(OmvLight))) != hipSuccess) return hipFail(e, "upload lights");

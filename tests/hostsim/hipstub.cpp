@@ -423,6 +423,10 @@ hipError_t buildBlasDevice(const float*, uint32_t, uint32_t, const uint32_t*, ui
     return hipSuccess;
 }
 size_t meshDeviceScratchBytes(uint32_t vn, uint32_t fn) { return 64 + (size_t)(vn + fn) * 64; }
+hipError_t instanceBoxesDevice(const OmvNode4*, const OmvInstance*, uint32_t n, OmvInstanceBox* out, hipStream_t) {
+    for (uint32_t i = 0; i < n; ++i) out[i] = {{-1.0, -1.0, -1.0}, {1.0, 1.0, 1.0}, {0.0, 0.0, 0.0}};
+    return hipSuccess;
+}
 hipError_t preprocessMeshDevice(float*, uint32_t, uint32_t, const uint32_t*, uint32_t, bool, bool, int, void*, hipStream_t, uint32_t* bad) {
     if (bad) *bad = 0;
     return hipSuccess;
