@@ -133,11 +133,15 @@ hipError_t buildBlasDevice(const float* vtx, uint32_t vtxOff, uint32_t stride, c
 size_t meshDeviceScratchBytes(uint32_t vn, uint32_t fn);
 hipError_t preprocessMeshDevice(float* vertices, uint32_t stride, uint32_t vn, const uint32_t* faces, uint32_t fn, bool normals,
                                 bool tangents, int uvOff, void* scratch, hipStream_t stream, uint32_t* badIndices);
-// World box of every instance and, per axis, the largest sum of the
-// magnitudes of the terms behind a coordinate (rounding goes with it); of an
-// instance without a BLAS (blas_root < 0) an empty box
+// bvh_device.hip: one pass over the instances at commit.  World box of every
+// instance and, per axis, the largest sum of the magnitudes of the terms
+// behind a coordinate (rounding goes with it); of an instance without a BLAS
+// (blas_root < 0) an empty box.  And the range of 1 / area over the world
+// triangles of an area above FLT_EPSILON, infinity and 0 if there are none.
 struct OmvInstanceBox { double lo[3], hi[3], reach[3]; };
-hipError_t instanceBoxesDevice(const OmvNode4* nodes, const OmvInstance* insts, uint32_t n, OmvInstanceBox* out, hipStream_t stream);
+struct OmvDensityRange { float lo, hi; };
+hipError_t instancePassDevice(const float* vtx, const uint32_t* faces, const OmvMesh* meshes, const OmvNode4* nodes, const OmvInstance* insts,
+                              uint32_t n, uint32_t maxFaces, OmvInstanceBox* boxes, OmvDensityRange* range, hipStream_t stream);
 hipError_t launchEnvBuild(const float* bg, int W, int H, float* rowProb, int* rowAlias, float* colProb, int* colAlias, float* texPdf,
                           void* scratch, hipStream_t stream);
 // 0: sample kernel (scene with lights), 1: FC kernel, 2: sample kernel (no lights), 3: batch kernel;

@@ -506,29 +506,6 @@ int RenderScene::commit(std::string& log) {
     for (size_t i = 0; i < lights_.size(); ++i)
         if (!lightSet_[i]) { setError("commit: light " + std::to_string(i) + " was never set"); return OMV_E_STATE; }
 
-    // FC density range (RenderScene.cpp:196-203, RenderMesh.cpp:277-297)
-    float minD = std::numeric_limits<float>::infinity(), maxD = 0.0f;
-    for (const auto& in : insts_) {
-        if (in.meshId < 0) continue;
-        const HostMesh& m = meshes_[in.meshId];
-        const float* T = in.tm;
-        for (int f = 0; f < m.fn; ++f) {
-            v3 P[3];
-            for (int k = 0; k < 3; ++k) {
-                const float* p = &m.V[(size_t)m.F[3 * f + k] * m.stride];
-                P[k] = mk(T[0] * p[0] + T[1] * p[1] + T[2] * p[2] + T[3], T[4] * p[0] + T[5] * p[1] + T[6] * p[2] + T[7],
-                          T[8] * p[0] + T[9] * p[1] + T[10] * p[2] + T[11]);
-            }
-            const float a = len(cross(mk(P[1].x - P[0].x, P[1].y - P[0].y, P[1].z - P[0].z),
-                                      mk(P[2].x - P[0].x, P[2].y - P[0].y, P[2].z - P[0].z))) / 2.0f;
-            if (a > std::numeric_limits<float>::epsilon()) {
-                const float d = 1.0f / (0.0f + a);
-                minD = std::min(minD, d);
-                maxD = std::max(maxD, d);
-            }
-        }
-    }
-
     // pools
     std::vector<float> vtx;
     std::vector<uint32_t> faces;
@@ -632,14 +609,18 @@ int RenderScene::commit(std::string& log) {
     }
     if (insts_.size() >= (1u << 29)) { setError("commit: too many instances"); return OMV_E_SCENE; }
     const size_t tlasCap = std::max<size_t>(1, insts_.size()), blasNodes = nodes.size();
+    hipError_t e;
     if (!deviceBuild) {   // the TLAS nodes follow below
-        hipError_t e;
+        if ((e = dVtx_.upload(vtx.data(), vtx.size() * 4)) != hipSuccess) return hipFail(e, "upload vertices");
+        if ((e = dFaces_.upload(faces.data(), faces.size() * 4)) != hipSuccess) return hipFail(e, "upload faces");
         if ((e = dNodes_.reserve((blasNodes + tlasCap) * sizeof(OmvNode4))) != hipSuccess) return hipFail(e, "BVH nodes");
         if (blasNodes && (e = hipMemcpy(dNodes_.ptr, nodes.data(), blasNodes * sizeof(OmvNode4), hipMemcpyHostToDevice)) != hipSuccess)
             return hipFail(e, "upload nodes");
     }
-    // TLAS over world-space instance boxes (made on the device from the nodes
-    // near each BLAS root, see instanceBoxesDevice), rounded outward
+    if ((e = dMeshes_.upload(dmeshes.data(), dmeshes.size() * sizeof(OmvMesh))) != hipSuccess) return hipFail(e, "upload meshes");
+    // The instances' pass on the device: world boxes for the TLAS, from the
+    // nodes near each BLAS root, and the FC density range (RenderScene.cpp:
+    // 196-203, RenderMesh.cpp:277-297)
     std::vector<OmvInstance> dinsts(insts_.size());
     for (size_t i = 0; i < insts_.size(); ++i) {
         const HostInstance& in = insts_[i];
@@ -655,16 +636,21 @@ int RenderScene::commit(std::string& log) {
         d.mat_type = mats_[dmeshes[in.meshId].mat_id].type;
     }
     std::vector<OmvInstanceBox> ibox(insts_.size());
+    OmvDensityRange density = {std::numeric_limits<float>::infinity(), 0.0f};
     if (!insts_.empty()) {
-        hipError_t e;
-        DeviceBuffer work;
+        DeviceBuffer work;   // the range, then the boxes
+        uint32_t maxFaces = 0;
+        for (const OmvMesh& m : dmeshes) if (m.valid) maxFaces = std::max(maxFaces, m.num_faces);
         const size_t bytes = ibox.size() * sizeof(OmvInstanceBox);
         if ((e = dInsts_.upload(dinsts.data(), dinsts.size() * sizeof(OmvInstance))) != hipSuccess) return hipFail(e, "upload instances");
-        if ((e = work.reserve(bytes)) != hipSuccess) return hipFail(e, "instance boxes");
-        if ((e = instanceBoxesDevice(dNodes_.as<OmvNode4>(), dInsts_.as<OmvInstance>(), (uint32_t)insts_.size(), work.as<OmvInstanceBox>(),
-                                     nullptr)) != hipSuccess)
-            return hipFail(e, "instance box kernel launch");
-        if ((e = hipMemcpy(ibox.data(), work.ptr, bytes, hipMemcpyDeviceToHost)) != hipSuccess) return hipFail(e, "instance boxes");
+        if ((e = work.reserve(16 + bytes)) != hipSuccess) return hipFail(e, "instance pass");
+        OmvInstanceBox* dBox = reinterpret_cast<OmvInstanceBox*>(work.as<uint8_t>() + 16);
+        if ((e = instancePassDevice(dVtx_.as<float>(), dFaces_.as<uint32_t>(), dMeshes_.as<OmvMesh>(), dNodes_.as<OmvNode4>(),
+                                    dInsts_.as<OmvInstance>(), (uint32_t)insts_.size(), maxFaces, dBox, work.as<OmvDensityRange>(),
+                                    nullptr)) != hipSuccess)
+            return hipFail(e, "instance pass launch");
+        if ((e = hipMemcpy(&density, work.ptr, sizeof(density), hipMemcpyDeviceToHost)) != hipSuccess) return hipFail(e, "density range");
+        if ((e = hipMemcpy(ibox.data(), dBox, bytes, hipMemcpyDeviceToHost)) != hipSuccess) return hipFail(e, "instance boxes");
     }
     std::vector<BuildBox> iboxes;
     std::vector<int> iids;
@@ -723,7 +709,7 @@ int RenderScene::commit(std::string& log) {
                     nd.entry[k] = OMV_ENT(OMV_ENT_TLAS_NODE, nd.child[k]);
                 }
         tl.root += deviceNodes;
-        hipError_t e = hipMemcpy(dNodes_.as<OmvNode4>() + deviceNodes, nodes.data(), nodes.size() * sizeof(OmvNode4), hipMemcpyHostToDevice);
+        e = hipMemcpy(dNodes_.as<OmvNode4>() + deviceNodes, nodes.data(), nodes.size() * sizeof(OmvNode4), hipMemcpyHostToDevice);
         if (e != hipSuccess) return hipFail(e, "upload TLAS");
     }
     // traversal stack bound: 3 siblings per BVH4 level plus the instance markers
@@ -765,12 +751,6 @@ int RenderScene::commit(std::string& log) {
     }
     texOffsets_.resize(dtex.size());
     for (size_t i = 0; i < dtex.size(); ++i) texOffsets_[i] = dtex[i].offset;
-    hipError_t e;
-    if (!deviceBuild) {
-        if ((e = dVtx_.upload(vtx.data(), vtx.size() * 4)) != hipSuccess) return hipFail(e, "upload vertices");
-        if ((e = dFaces_.upload(faces.data(), faces.size() * 4)) != hipSuccess) return hipFail(e, "upload faces");
-    }
-    if ((e = dMeshes_.upload(dmeshes.data(), dmeshes.size() * sizeof(OmvMesh))) != hipSuccess) return hipFail(e, "upload meshes");
     if ((e = dMats_.upload(mats_.data(), mats_.size() * sizeof(OmvMaterial))) != hipSuccess) return hipFail(e, "upload materials");
     if ((e = dTexs_.upload(dtex.data(), dtex.size() * sizeof(OmvTexture))) != hipSuccess) return hipFail(e, "upload textures");
     if ((e = dTexels_.upload(texels.data(), texels.size())) != hipSuccess) return hipFail(e, "upload texels");
@@ -811,7 +791,7 @@ int RenderScene::commit(std::string& log) {
     std::memcpy(v.bg_rot, bgRot_, sizeof(bgRot_));
     v.bg_scale = bgScale_;
     v.light_max = cdf.empty() ? 0.0f : cdf.back();
-    v.min_density = minD; v.max_density = maxD;
+    v.min_density = density.lo; v.max_density = density.hi;
 
     // environment importance sampling tables, built on the device
     if (bgType_ == OMV_BG_HDR && bgW_ > 0 && bgH_ > 0) {

@@ -423,8 +423,10 @@ hipError_t buildBlasDevice(const float*, uint32_t, uint32_t, const uint32_t*, ui
     return hipSuccess;
 }
 size_t meshDeviceScratchBytes(uint32_t vn, uint32_t fn) { return 64 + (size_t)(vn + fn) * 64; }
-hipError_t instanceBoxesDevice(const OmvNode4*, const OmvInstance*, uint32_t n, OmvInstanceBox* out, hipStream_t) {
-    for (uint32_t i = 0; i < n; ++i) out[i] = {{-1.0, -1.0, -1.0}, {1.0, 1.0, 1.0}, {0.0, 0.0, 0.0}};
+hipError_t instancePassDevice(const float*, const uint32_t*, const OmvMesh*, const OmvNode4*, const OmvInstance*, uint32_t n, uint32_t,
+                              OmvInstanceBox* boxes, OmvDensityRange* range, hipStream_t) {
+    for (uint32_t i = 0; i < n; ++i) boxes[i] = {{-1.0, -1.0, -1.0}, {1.0, 1.0, 1.0}, {0.0, 0.0, 0.0}};
+    *range = {1.0f, 1.0f};
     return hipSuccess;
 }
 hipError_t preprocessMeshDevice(float*, uint32_t, uint32_t, const uint32_t*, uint32_t, bool, bool, int, void*, hipStream_t, uint32_t* bad) {

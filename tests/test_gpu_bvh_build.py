@@ -221,3 +221,42 @@ def test_device_build_at_the_edges_of_its_tiles(pkg, wl, tris, verts):
     assert b[4]["nodes"] <= tris + 1
     if verts > 1:
         assert (a[2][0] >= 0).mean() > 0.02
+
+
+@pytest.mark.parametrize("mode", ["host", "device"])
+@pytest.mark.parametrize("counts", [(1, 1), (1024, 1), (1025, 3), (4, 4097), (300000, 5)])
+def test_density_range(pkg, wl, ref, counts, mode):
+    """The density subject's range over instances of two meshes, one of
+    single faces of a size that no other has (the range's two ends): at the
+    edges of the pass's grid, with scaled, mirrored and unused instances and
+    faces of no area, the oracle's colours."""
+    tris, insts = counts
+    rng = np.random.default_rng(tris)
+    x = np.linspace(-1, 1, tris + 1, dtype=np.float32)
+    v = np.concatenate([np.stack([x, 0 * x - 0.5, 0 * x], 1), np.stack([x, 0 * x + 0.5, 0 * x], 1)]).astype(np.float32)
+    i = np.arange(tris)
+    strip = np.stack([i, i + 1, tris + 1 + i], 1).astype(np.uint32)
+    big = np.array([[-1, -1, 0], [1, -1, 0], [0, 1, 0], [0, 1, 0]], np.float32)
+    d = wl.SceneDesc()
+    d.materials.append(("pbr", dict(base_color=(0.8, 0.6, 0.4, 1.0), metallic=0.0, roughness=0.5)))
+    d.meshes.append({"vertices": v, "faces": strip, "mat_id": 0})
+    d.meshes.append({"vertices": big, "faces": np.array([[0, 1, 2], [0, 2, 3]], np.uint32), "mat_id": 0})   # the second has no area
+    d.instances.append((wl.trs((0.0, 0.0, -4.0), scale=(-3.0, 2.5, 1.0)), 1))
+    for k in range(insts):
+        d.instances.append((wl.trs(rng.uniform(-1.0, 1.0, 3) + (0, 0, -2.5), angle=0.2 * k, scale=rng.uniform(0.2, 0.6, 3) * rng.choice([-1, 1], 3)), 0))
+    d.instances.append((wl.trs((0.0, 0.0, -3.0), scale=(0.05, 0.05, 1.0)), 1))
+    d.fc_subject = "md"
+    cam = pkg.Camera(64, 48, (0.0, 0.0, 0.0), (0.0, 0.0, -1.0), (0.0, 1.0, 0.0), 60.0)
+    s = pkg.Scene()
+    s.set_build_mode(pkg.BUILD_DEVICE_LBVH if mode == "device" else pkg.BUILD_HOST_SAH)
+    d.apply(s, pkg.pbr_desc)
+    r = pkg.Renderer(pkg.default_params(seed=4))
+    r.set_scene(s)
+    film, ids, tie = r.render_fc(cam)
+    rs = ref.Scene()
+    d.apply(rs, ref.pbr_desc)
+    rfilm, rids, _ = rs.render_fc(ref.default_params(seed=4), cam.desc())
+    same = (ids == rids).all(axis=0)
+    assert same.mean() > 0.999
+    np.testing.assert_allclose(film[same], rfilm[same], atol=1e-5, rtol=0)   # the paint's logarithms differ by a few ulp
+    assert np.unique(film[..., :3].reshape(-1, 3), axis=0).shape[0] >= (2 if tris == 1 else 3)
