@@ -495,12 +495,12 @@ int omv_renderer_render_detached(omv_renderer* r, omv_camera* c, const omv_scene
  * names them exists; cameras are copied at add time. */
 typedef struct omv_batch omv_batch;
 typedef struct omv_batch_tuning {
-    int blocks_per_cu;   /* per-pixel kernel: resident workgroups per CU
+    int blocks_per_cu;   /* one launch: resident workgroups per CU
                             (0 = occupancy limit)                          */
-    int tile_waves;      /* per-pixel kernel: samples per work item, about
+    int tile_waves;      /* one launch: samples per work item, about
                             256 * tile_waves (>= 1), in whole pixels       */
     int use_graph;       /* 1: replay a captured hipGraph, 0: plain launch */
-    int streams;         /* 0: one persistent per-pixel kernel over all
+    int streams;         /* 0: one persistent launch over all
                             jobs; N >= 1: each job's wavefront launch
                             sequence, jobs dealt over N streams so that one
                             job's last bounce rounds overlap other jobs    */
@@ -516,7 +516,7 @@ int omv_batch_get_tuning(const omv_batch* b, omv_batch_tuning* t);
 /* Times every candidate on the batch itself with plain launches (no graph
  * capture during the sweep), 'reps' runs each, keeps the fastest and reports
  * it in best (may be NULL): the jobs' wavefront sequences over 1, 2, 4 and 8
- * streams (no more streams than jobs) and the persistent per-pixel kernel at
+ * streams (no more streams than jobs) and the persistent launch at
  * each blocks_per_cu up to the occupancy limit x tile_waves 1, 2, 4.  The
  * starting use_graph is kept: the choice is captured once, at the next run. */
 int omv_batch_autotune(omv_batch* b, int reps, omv_batch_tuning* best);

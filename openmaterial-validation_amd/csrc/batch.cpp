@@ -335,7 +335,7 @@ int BatchRunner::run() {
 // sweep), reps runs each, and keeps the fastest; the chosen configuration is
 // captured once, at the next run, when the starting tuning asked for a graph.
 // Candidates: the jobs' wavefront sequences over 1, 2, 4 and 8 streams (no
-// more streams than jobs), and the persistent per-pixel kernel at every
+// more streams than jobs), and the persistent launch at every
 // resident-blocks-per-CU count up to the occupancy limit x 1, 2 or 4 waves
 // of pixels per work item.
 int BatchRunner::autotune(int reps, omv_batch_tuning* best) {

@@ -317,7 +317,7 @@ __global__ void lbRecords(const float* __restrict__ vtx, uint32_t vtxOff, uint32
 // four children it arrives at (or the box it ends in) by the instance's
 // matrix: centre +- sum |M| * half extent.  The union of up to 256 turned
 // boxes is far tighter on a rotated mesh than its turned root box, so rays
-// enter fewer instances that they miss: 60 rotated meshes of 33 K triangles
+// enter fewer instances that they miss: 200 rotated meshes of 10 K triangles
 // under lights, 1080p x 16 (MI355X), 6.59 -> 6.21 nodes per ray and 8.78 ->
 // 8.39 ms per render.
 __global__ __launch_bounds__(kBlock) void lbInstanceBoxes(const OmvNode4* __restrict__ nodes, const OmvInstance* __restrict__ insts, uint32_t n,

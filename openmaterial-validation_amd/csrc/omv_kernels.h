@@ -33,7 +33,7 @@ void packBatchJob(void* dst, const OmvSceneView& S, const omv_camera_desc& cam, 
                   uint64_t npix);
 hipError_t launchBatch(const void* jobs, int njobs, const uint64_t* tileEnd, uint64_t totalTiles, int tileWaves,
                        unsigned long long* counters, float* lv, uint32_t* gstack, int blocks, bool nee, hipStream_t stream);
-// Allocation-free render (noalloc.hip): one persistent per-pixel kernel over
+// Allocation-free render (noalloc.hip): one persistent launch over tiles with
 // the file-scope scratch array; statsOut (may be null: no wait) receives the
 // 8 counters after the stream has finished.  On failure err / what say why.
 int renderNoalloc(const OmvSceneView& S, const omv_camera_desc& cam, const omv_renderer_params& p, float* film, hipStream_t stream,
@@ -85,7 +85,7 @@ uint32_t wavefrontSegCap(uint32_t nslots, int gridShade, int gridGen);
 size_t wavefrontArenaBytes(uint32_t nslots, int lvCap, int lc, bool lights, bool nee, bool splat, bool sortRays, int gridShade, int gridGen);
 int wavefrontCounterCount(int B, int lvCap);
 // resident blocks per CU: [0] trace, [1] camera shading with lights + NEE,
-// [2] light shading, [3] gen, [4] persistent trace, [5] camera shading with
+// [2] light shading, [3] gen, [4] as [0], [5] camera shading with
 // lights, [6] with NEE, [7] with neither, [8] round-1 packet trace
 void wavefrontBlocksPerCU(int out[9]);
 inline int shadeCamBlocksPerCU(const int occ[9], bool lights, bool nee) { return lights ? (nee ? occ[1] : occ[5]) : (nee ? occ[6] : occ[7]); }

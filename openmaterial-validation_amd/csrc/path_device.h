@@ -975,7 +975,7 @@ DEV bool offer(Hit& h, float t, float u, float v, int inst, int prim) {
 // 4-wide slab test, conservative (Ize 2013: tmax scaled by 1 + 2*gamma(3)).
 // An empty slot (planes at +inf, entry E_NONE) tests as a miss or, when
 // tfar * kUp overflows to +inf, as a hit at +inf; either way its E_NONE
-// entry is never pushed (pushSorted), so no entry check is needed here.
+// entry is never pushed, so no entry check is needed here.
 DEV void boxTest4(const OmvNode4& nd, const f3& o, const f3& idir, float tnear, float tfar, float tent[4], bool hit[4]) {
     const float kUp = 1.0000004f;
 #pragma unroll

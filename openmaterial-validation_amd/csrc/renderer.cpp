@@ -294,7 +294,7 @@ int BDPTRenderer::renderDetached(PinholeCamera& cam, const RenderScene& eval, do
 }
 
 // Allocation-free render: validates on the host, then one persistent
-// per-pixel launch over the fixed scratch array (noalloc.hip).  Touches none
+// launch over the fixed scratch array (noalloc.hip).  Touches none
 // of this renderer's buffers, streams or events.
 int BDPTRenderer::renderNoalloc(const PinholeCamera& cam, float* film, hipStream_t stream, omv_render_stats* st) {
     if (!scene_ || !scene_->committed()) { setError("render_noalloc: no committed scene"); return OMV_E_STATE; }
