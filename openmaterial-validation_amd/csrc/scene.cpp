@@ -638,19 +638,23 @@ int RenderScene::commit(std::string& log) {
     std::vector<OmvInstanceBox> ibox(insts_.size());
     OmvDensityRange density = {std::numeric_limits<float>::infinity(), 0.0f};
     if (!insts_.empty()) {
-        DeviceBuffer work;   // the range, then the boxes
         uint32_t maxFaces = 0;
         for (const OmvMesh& m : dmeshes) if (m.valid) maxFaces = std::max(maxFaces, m.num_faces);
-        const size_t bytes = ibox.size() * sizeof(OmvInstanceBox);
-        if ((e = dInsts_.upload(dinsts.data(), dinsts.size() * sizeof(OmvInstance))) != hipSuccess) return hipFail(e, "upload instances");
-        if ((e = work.reserve(16 + bytes)) != hipSuccess) return hipFail(e, "instance pass");
-        OmvInstanceBox* dBox = reinterpret_cast<OmvInstanceBox*>(work.as<uint8_t>() + 16);
+        // the range and the boxes lie behind the instances: an allocation and
+        // its release would take longer than the pass
+        const size_t bytes = (dinsts.size() * sizeof(OmvInstance) + 15) & ~(size_t)15, boxBytes = ibox.size() * sizeof(OmvInstanceBox);
+        if ((e = dInsts_.reserve(bytes + 16 + boxBytes)) != hipSuccess) return hipFail(e, "instances");
+        if ((e = hipMemcpy(dInsts_.ptr, dinsts.data(), dinsts.size() * sizeof(OmvInstance), hipMemcpyHostToDevice)) != hipSuccess)
+            return hipFail(e, "upload instances");
+        uint8_t* out = dInsts_.as<uint8_t>() + bytes;
         if ((e = instancePassDevice(dVtx_.as<float>(), dFaces_.as<uint32_t>(), dMeshes_.as<OmvMesh>(), dNodes_.as<OmvNode4>(),
-                                    dInsts_.as<OmvInstance>(), (uint32_t)insts_.size(), maxFaces, dBox, work.as<OmvDensityRange>(),
-                                    nullptr)) != hipSuccess)
+                                    dInsts_.as<OmvInstance>(), (uint32_t)insts_.size(), maxFaces, reinterpret_cast<OmvInstanceBox*>(out + 16),
+                                    reinterpret_cast<OmvDensityRange*>(out), nullptr)) != hipSuccess)
             return hipFail(e, "instance pass launch");
-        if ((e = hipMemcpy(&density, work.ptr, sizeof(density), hipMemcpyDeviceToHost)) != hipSuccess) return hipFail(e, "density range");
-        if ((e = hipMemcpy(ibox.data(), dBox, bytes, hipMemcpyDeviceToHost)) != hipSuccess) return hipFail(e, "instance boxes");
+        std::vector<uint8_t> got(16 + boxBytes);
+        if ((e = hipMemcpy(got.data(), out, got.size(), hipMemcpyDeviceToHost)) != hipSuccess) return hipFail(e, "instance pass");
+        std::memcpy(&density, got.data(), sizeof(density));
+        std::memcpy(ibox.data(), got.data() + 16, boxBytes);
     }
     std::vector<BuildBox> iboxes;
     std::vector<int> iids;
