@@ -39,7 +39,7 @@ enum { OMV_BG_NONE = 0, OMV_BG_CONSTANT = 1, OMV_BG_HDR = 2 };
 #define OMV_ENT_INST 3u
 #define OMV_ENT(kind, payload) (((uint32_t)(kind) << OMV_ENT_SHIFT) | (uint32_t)(payload))
 #define OMV_ENT_END 0xFFFFFFFFu    // end of an instance's BLAS (stack only)
-#define OMV_ENT_NONE 0xFFFFFFFEu   // empty child slot (never pushed)
+#define OMV_ENT_NONE 0xFFFFFFFEu   // empty child slot (dropped where it is taken up)
 #define OMV_ENT_DONE 0xFFFFFFFDu   // bottom of the stack: the traversal is over
 static_assert(OMV_BVH_LEAF_MAX >= 1 && OMV_BVH_LEAF_MAX <= 8, "leaf size must fit the entry's 3-bit count");
 

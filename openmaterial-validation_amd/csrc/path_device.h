@@ -1127,11 +1127,13 @@ struct Trav {
         // is at least as near, so the traversal ends here
         if (h.inst >= 0 && h.t <= tstop) cur = E_DONE;
     }
-    // entry into an instance, or the end of one
+    // entry into an instance, the end of one, or an empty slot that node() took
     DEV void inst(const OmvSceneView& S, Stack& st, Counters& c) {
-        if (cur == (uint32_t)E_END) {
-            curInst = -1;
-            boxRay(wo, wd, box);
+        if (cur >= (uint32_t)E_NONE) {
+            if (cur == (uint32_t)E_END) {
+                curInst = -1;
+                boxRay(wo, wd, box);
+            }
             cur = st.pop();
             return;
         }
@@ -1153,7 +1155,10 @@ struct Trav {
     // fetched by the direction's signs (nearRows).  A child that is missed
     // gets the key +inf; the 5-comparator network sorts (distance, entry)
     // pairs as doubles, two instructions a comparator.  An empty slot (planes
-    // at +inf) is always missed, since tcull is finite.
+    // at +inf) is missed on every axis that culls, since tcull is finite; a ray
+    // that culls on none (a non-finite or tiny one, as instances of a singular
+    // matrix make) takes it for hit, and inst() drops its E_NONE.  Comparing
+    // the entries here instead would cost four instructions on every visit.
     DEV void node(const OmvSceneView& S, Stack& st, Counters& c) {
         ++c.nodes;
         const char* base = reinterpret_cast<const char*>(S.nodes);

@@ -176,3 +176,72 @@ def test_turned_instances(pkg, wl, ref, place, build):
     assert np.array_equal(ids, rids)
     assert np.array_equal(tie, rtie)
     assert (ids[0] >= 0).mean() > 0.2
+
+
+def _inside(value):
+    """What a program can pass for a place: none of it is refused."""
+    return {"inf_x": (np.inf, 0.0, 0.0), "nan": (np.nan,) * 3, "inf": (np.inf, -np.inf, np.inf), "minus_inf": (-np.inf,) * 3}[value]
+
+
+ODD = ["flat", "flatter", "point", "far"] + [f"{k}_{v}" for k in ("instance", "light", "camera") for v in ("inf_x", "nan", "inf", "minus_inf")]
+
+
+@pytest.mark.parametrize("build", ["host", "device"])
+@pytest.mark.parametrize("odd", ODD)
+def test_rays_that_cull_on_no_axis(pkg, wl, ref, odd, build):
+    """Instances of a singular matrix (their inverse is inf and NaN), of a
+    scale beyond the slab test's range, and instances, lights and cameras at
+    places that are not finite: the box test may cull on no axis, so empty
+    child slots are taken for hit.  Ids are the oracle's; rounds, film tiles,
+    wave packets and the allocation-free render give the per-sample schedule's
+    film."""
+    import torch
+    d = _scene(wl, 1.0, (0, 0, 0))
+    cam = _camera(pkg, "free", 1.0, (0, 0, 0))
+    kind, _, value = odd.partition("_")
+    rng = np.random.default_rng(6)
+    for k in range(6):   # turned plates, boxes and spheres, each under the odd matrix
+        at = rng.uniform(-1.0, 1.0, 3) + (0.0, 0.6, 0.0)
+        scale = {"flat": (1, 1, 0), "flatter": (0, 1, 0), "point": (0, 0, 0), "far": (1e32, 1e32, 1e32)}.get(kind, (0.3, 0.3, 0.3))
+        m = np.array(wl.trs(tuple(at), rng.normal(size=3), 0.7 + k, scale), np.float32)
+        if kind == "instance":
+            m.reshape(-1, 4)[:3, 3] = _inside(value)
+        d.instances.append((m, k % 3))
+    if kind == "light":
+        d.lights.append((_inside(value), (40.0,) * 3, -1.0))
+    if kind == "camera":
+        cam.set_viewpoint(_inside(value), (1, 0, 0), (0, 1, 0), (0, 0, -1))
+    d.fc_subject = "ipid"
+    s = pkg.Scene()
+    s.set_build_mode(pkg.BUILD_DEVICE_LBVH if build == "device" else pkg.BUILD_HOST_SAH)
+    d.apply(s, pkg.pbr_desc)
+    params = dict(samples_per_pixel=2, camera_bounces=4, light_bounces=3, max_path_length=5, seed=9)
+    print(f"odd case {odd} {build}", flush=True)
+    r = pkg.Renderer(pkg.default_params(seed=3))
+    r.set_scene(s)
+    _, ids, tie = r.render_fc(cam)
+    rs = ref.Scene()
+    d.apply(rs, ref.pbr_desc)
+    _, rids, rtie = rs.render_fc(ref.default_params(seed=3), cam.desc())
+    assert np.array_equal(ids, rids) and np.array_equal(tie, rtie)
+    if kind == "far":   # the camera is inside: every ray hits, at distances whose squares overflow
+        assert (ids[0] >= 0).all()
+        return
+    if kind != "camera":
+        assert (ids[0] >= 0).mean() > 0.2
+    one = pkg.Renderer(pkg.default_params(**params))
+    one.set_scene(s)
+    one.set_schedule(pkg.SCHEDULE_PER_SAMPLE)
+    want = one.render(cam)
+    assert one.stats()["stack_overflows"] == 0
+    for tuning in (dict(), dict(tail_round=1), dict(tail_round=2), dict(traversal=2), dict(sort_rays=2)):
+        r = pkg.Renderer(pkg.default_params(**params))
+        r.set_scene(s)
+        if tuning:
+            r.set_tuning(**tuning)
+        assert np.array_equal(r.render(cam), want, equal_nan=True), tuning
+    film = torch.empty(cam.desc().height, cam.desc().width, 4, device="cuda")
+    torch.cuda.synchronize()   # the film's allocation, before a stream that does not wait for torch's
+    one.render_noalloc(cam, film.data_ptr())
+    torch.cuda.synchronize()
+    assert np.array_equal(film.cpu().numpy().reshape(want.shape), want, equal_nan=True)
