@@ -71,10 +71,10 @@ struct WfHits {
 };
 struct WfState {
     uint32_t n;        // slots
-    float4* rad;       // camera radiance so far xyz (written and read with emission or OMV_EXT_HDRI_NEE only)
+    float4* rad;       // camera radiance so far xyz (written and read with emission or OMV_EXT_HDRI_NEE, and for info state 3)
     float4* conn;      // connection sum xyz
-    uint32_t* info;    // [entry of the round] connections staged << 2 | 0 running, 1 ends after this round's
-                       // connections, 2 written (lights or OMV_EXT_HDRI_NEE only)
+    uint32_t* info;    // [entry of the round] connections staged << 2 | 0 running, 1 ends after this round's connections,
+                       // 2 written, 3 ends with a radiance that is not finite in rad (lights or OMV_EXT_HDRI_NEE only)
     float4* lthr;      // light throughput xyz, first-hit attenuation rD
     uint32_t* lsn;     // light stream draws consumed
     int* lidx;         // sampled light
@@ -204,6 +204,11 @@ DEV uint32_t segAppendKeyed(const WfSeg& g, bool want, uint32_t key, uint32_t nk
 }
 
 DEV f3 xyz(const float4& v) { return mk3(v.x, v.y, v.z); }
+// The radiance of a path that has met no emission: the per-sample function
+// adds throughput * 0 at every vertex, which is 0 while the throughput is
+// finite and NaN from the vertex on where a component overflowed (it does not
+// become finite again), so the throughput of the last vertex tells it.
+DEV f3 darkRadiance(const f3& of) { return mk3(0.0f + of.x * 0.0f, 0.0f + of.y * 0.0f, 0.0f + of.z * 0.0f); }
 DEV float4 f4of(const f3& v, float w) { float4 r; r.x = v.x; r.y = v.y; r.z = v.z; r.w = w; return r; }
 
 // Round-1 rays of sample s: the camera ray (PinholeCamera::getRay, 2 draws
@@ -998,7 +1003,7 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
                 of = xyz(th);
                 draws = __float_as_uint(th.w);
                 if (kNee) escIn = in.w[p];
-                if (glow) radiance = xyz(W.rad[slot]);
+                radiance = glow ? xyz(W.rad[slot]) : darkRadiance(of);
             }
         }
         int n = i;   // vertices so far: every round before this one added one
@@ -1128,7 +1133,11 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_SHADE_WAVES(kLights, kNee)) void omv
                 rad[(uint64_t)slot * 3 + 1] = conn.y * 1.0f + radiance.y;
                 rad[(uint64_t)slot * 3 + 2] = conn.z * 1.0f + radiance.z;
             }
-            if (kLights || kNee) W.info[e] = staged << 2 | (cont ? 0u : 1u);
+            if (kLights || kNee) {
+                const bool dark = glow || (radiance.x == 0.0f && radiance.y == 0.0f && radiance.z == 0.0f);
+                if (!cont && !dark) W.rad[slot] = f4of(radiance, 0.0f);
+                W.info[e] = staged << 2 | (cont ? 0u : (dark ? 1u : 3u));
+            }
         }
         const uint32_t k = segAppend(outCount, emit, lost);
         if (k != OMV_SEG_NONE) {
@@ -1180,14 +1189,14 @@ __global__ __launch_bounds__(OMV_BLOCK) void omv_wf_connect(WfState W, WfQueue i
         // the radiance so far is needed by a visible next-event estimate and
         // by a path that ends this round
         const bool neeVis = nee && W.nvis[slot] == 2;
-        if (!neeVis && fl != 1u) continue;
-        float4 rc = glow ? W.rad[slot] : f4of(mk3(0.0f, 0.0f, 0.0f), 0.0f);
+        if (!neeVis && fl == 0u) continue;
+        float4 rc = glow || fl == 3u ? W.rad[slot] : f4of(mk3(0.0f, 0.0f, 0.0f), 0.0f);
         if (neeVis) {
             const f3 c = xyz(W.neeC[slot]);
             rc.x = rc.x + c.x; rc.y = rc.y + c.y; rc.z = rc.z + c.z;
             W.rad[slot] = rc;
         }
-        if (fl == 1u) {
+        if (fl != 0u) {
             const f3 radiance = xyz(rc);
             rad[(uint64_t)slot * 3 + 0] = conn.x * 1.0f + radiance.x;
             rad[(uint64_t)slot * 3 + 1] = conn.y * 1.0f + radiance.y;
@@ -1227,7 +1236,7 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TAIL_WAVES(kLights, kNee)) void omv_
         const float4 o = in.o[p], d = in.d[p];
         const uint32_t slot = __float_as_uint(d.w);
         const float4 th = in.t[p];
-        const f3 radiance = kNee || S.any_emissive ? xyz(W.rad[slot]) : mk3(0.0f, 0.0f, 0.0f);
+        const f3 radiance = kNee || S.any_emissive ? xyz(W.rad[slot]) : darkRadiance(xyz(th));
         LightSub ls;
         ls.idx = -1; ls.len = 0; ls.pos = mk3(0.0f, 0.0f, 0.0f); ls.intensity = ls.pos; ls.range = FLT_MAX;
         f3 conn = mk3(0.0f, 0.0f, 0.0f);

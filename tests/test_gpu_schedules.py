@@ -413,3 +413,32 @@ def test_default_tail_round_keeps_the_film(pkg, wl, kind, size):
     assert np.array_equal(out[0][0], out[1][0])
     for k in ("rays", "camera_rays", "light_rays", "shadow_rays", "samples"):
         assert out[0][1][k] == out[1][1][k], k
+
+
+@pytest.mark.parametrize("lights", [False, True])
+@pytest.mark.parametrize("bounces", [2, 3, 7])
+@pytest.mark.parametrize("factor", [1e12, 1e25, np.inf])
+def test_throughput_that_overflows(pkg, wl, lights, bounces, factor):
+    """Base colours so bright that the throughput overflows after a vertex or
+    two: the per-sample function's radiance is NaN from there on (throughput *
+    0 emission), and every schedule gives its film: paths that end by the
+    round, by an escape, in the tail, with and without connections."""
+    desc, view = wl.mixed_test_scene(hdr=True, lights=lights)
+    view.width, view.height = 61, 43
+    desc.materials = [("pbr", dict(m[1], base_color=(factor, 0.5, 0.7 * factor, 1.0))) if m[0] == "pbr" else m for m in desc.materials]
+    s = pkg.Scene()
+    desc.apply(s, pkg.pbr_desc)
+    cam = pkg.Camera(view.width, view.height, view.position, view.forward, view.up, view.yfov)
+    params = dict(samples_per_pixel=2, camera_bounces=bounces, light_bounces=2, max_path_length=6, seed=3)
+    one = pkg.Renderer(pkg.default_params(**params))
+    one.set_scene(s)
+    one.set_schedule(pkg.SCHEDULE_PER_SAMPLE)
+    want = one.render(cam)
+    bad = ~np.isfinite(want[..., :3])
+    assert bad.any() and not bad.all()
+    for tuning in (dict(), dict(tail_round=1), dict(tail_round=2), dict(tail_round=3), dict(tail_round=1, sort_rays=2)):
+        r = pkg.Renderer(pkg.default_params(**params))
+        r.set_scene(s)
+        if tuning:
+            r.set_tuning(**tuning)
+        assert np.array_equal(r.render(cam), want, equal_nan=True), tuning

@@ -224,9 +224,6 @@ def test_rays_that_cull_on_no_axis(pkg, wl, ref, odd, build):
     d.apply(rs, ref.pbr_desc)
     _, rids, rtie = rs.render_fc(ref.default_params(seed=3), cam.desc())
     assert np.array_equal(ids, rids) and np.array_equal(tie, rtie)
-    if kind == "far":   # the camera is inside: every ray hits, at distances whose squares overflow
-        assert (ids[0] >= 0).all()
-        return
     if kind != "camera":
         assert (ids[0] >= 0).mean() > 0.2
     one = pkg.Renderer(pkg.default_params(**params))
