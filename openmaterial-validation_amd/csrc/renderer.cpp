@@ -414,12 +414,12 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
     const uint64_t npix = (uint64_t)cam.desc.width * cam.desc.height;
     const int spp = p.samples_per_pixel;
     const int lvCap = std::max(std::min(p.light_bounces + 1, std::max(p.max_path_length, 1)), 1);
-    if (!splat_ && npix * (uint64_t)spp <= kTileSamples && defaultTuning(tuning_)) return renderTiles(cam, lvCap);
     const int lc = std::max(1, std::min(lvCap, std::max(p.max_path_length, 1)));
     const uint64_t maxSlots = tuning_.chunk_samples > 0 ? (uint64_t)tuning_.chunk_samples : (lights ? kWfSlotsLights : kWfSlots);
     const uint64_t chunkPix = std::max<uint64_t>(1, maxSlots / (uint64_t)spp);
     const uint64_t slots = std::min(npix, chunkPix) * (uint64_t)spp;
     if (slots * (uint64_t)lc >= (1ull << 32)) { setError("render: too many samples per pixel for one chunk"); return OMV_E_RANGE; }
+    if (!splat_ && npix * (uint64_t)spp <= kTileSamples && defaultTuning(tuning_)) return renderTiles(cam, lvCap);
     if (!wfPerCu_[0]) wavefrontBlocksPerCU(wfPerCu_);
     // resident traversal workgroups per CU: the occupancy limit of the traversal kernels
     const int traceOcc = wfPerCu_[0];

@@ -89,3 +89,19 @@ def test_default_schedule_at_the_tile_limit(pkg, wl, lights, ext):
         for k in ("samples", "rays", "camera_rays", "light_rays", "shadow_rays", "stack_overflows"):
             assert a[k] == b[k], k
         assert (a["trace_launches"] == 1) == (w * h * 4 <= 1 << 18)
+
+
+@pytest.mark.parametrize("chunk", [0, 1 << 18])
+def test_refused_however_few_samples(pkg, wl, chunk):
+    """Samples x connections per vertex past 32 bits are refused, on the tile launch of small renders as in rounds."""
+    _, s, cam = _scene(pkg, wl, 512, 512)
+    for vertices, refused in ((1 << 14, True), (64, False)):
+        r = pkg.Renderer(pkg.default_params(samples_per_pixel=1, camera_bounces=2, light_bounces=vertices - 1, max_path_length=vertices))
+        r.set_scene(s)
+        if chunk:
+            r.set_tuning(chunk_samples=chunk)
+        if refused:
+            with pytest.raises(RuntimeError, match="too many samples per pixel"):
+                r.render(cam)
+        else:
+            r.render(cam)
