@@ -1040,16 +1040,25 @@ DEV void boxTest4Rows(const OmvNode4* nodes, uint32_t idx, uint32_t rows, const 
 // 2^-24 each.  The builders widen every child plane by 4 ulps (>= 4 * 2^-24
 // |p|) and the bias carries 6 * 2^-24 |o r|, so a box the exact ray meets is
 // never missed; the widening also covers the rounding of a hit's t, as
-// kBoxUp does on the far side.  A component below 1e-30 (0, NaN) does not
-// cull on its axis: idir 0, nb -inf, fb +inf.
+// kBoxUp does on the far side.  Where 1 / d or o / d is not finite nb, fb or
+// both are infinite or NaN, which the minima and maxima drop: the axis does
+// not cull.  A component of exactly 0 keeps the ray in a slab for good or out
+// of it: with idir the power of two that takes |o| (at least 1) just below
+// 2^127, the same products have the sign of p - o, a slab that starts behind
+// o gets a near distance of 0 or less, one that ends before o a negative far
+// one, and the bound of 6 * 2^-24 * 2^127 keeps slabs that end within 6 ulps
+// of o, for boxes up to a distance of 6e31.  (Without culling on such an axis
+// a ray visits every box along it: torus knot of 100 K triangles 512^2 x 16,
+// rays with x = 0, 18.6 -> 1.7 ms on MI355X.)
 struct BoxRay { f3 idir, nb, fb; uint32_t rows; };
 DEV void boxAxis(float o, float d, float& idir, float& nb, float& fb) {
-    const float r = __builtin_amdgcn_rcpf(d);
-    const float od = o * r;
-    const bool ok = fabsf(d) >= 1e-30f;
-    idir = ok ? r : 0.0f;
-    nb = ok ? __builtin_fmaf(fabsf(od), -3.57627869e-7f, -od) : -INFINITY;   // 6 * 2^-24
-    fb = ok ? __builtin_fmaf(fabsf(od), 3.57627869e-7f, -od) : INFINITY;
+    const uint32_t e = max(__float_as_uint(o) & 0x7F800000u, 126u << 23);   // |o| < 2^(e' - 126), e' = e >> 23
+    const bool zero = d == 0.0f;
+    idir = zero ? __uint_as_float((380u << 23) - e) : __builtin_amdgcn_rcpf(d);   // 2^(253 - e')
+    const float od = o * idir;
+    const float m = zero ? 1.70141183e38f : fabsf(od);   // 2^127
+    nb = __builtin_fmaf(m, -3.57627869e-7f, -od);        // 6 * 2^-24
+    fb = __builtin_fmaf(m, 3.57627869e-7f, -od);
 }
 DEV void boxRay(const f3& o, const f3& d, BoxRay& b) {
     boxAxis(o.x, d.x, b.idir.x, b.nb.x, b.fb.x);

@@ -134,3 +134,39 @@ def test_tiny_and_huge_directions(trav, wl, size):
     meshes, insts = scene(wl, rng)
     extra = [(turned(rng, (size,) * 3, np.zeros(3)), k % 2) for k in range(3)]
     check(trav(meshes, insts + extra, rays(rng)), (0.1, 1.0))
+
+
+@pytest.mark.parametrize("zero", [(0,), (1,), (2,), (0, 1), (0, 2), (1, 2)])
+@pytest.mark.parametrize("place", ["free", "edge", "flat", "far"])
+def test_zero_components_cull(trav, wl, zero, place):
+    """A ray with components of exactly 0 (either sign) hits what it has to,
+    on the very edge of boxes too, and visits no more than a ray that is
+    turned away from the axis by 1e-4."""
+    rng = np.random.default_rng(5)
+    v, f = wl.icosphere(4, 0.7)
+    n, q = 400, 24
+    g = np.linspace(-1, 1, q, dtype=np.float32)
+    plate = np.stack(np.meshgrid(g, np.zeros(1, np.float32), g, indexing="ij"), -1).reshape(-1, 3)
+    i = (np.arange(q - 1)[:, None] * q + np.arange(q - 1)).ravel()
+    pf = np.concatenate([np.stack([i, i + 1, i + q], 1), np.stack([i + 1, i + q + 1, i + q], 1)])
+    meshes, m = [(v, f), (plate, pf)], np.eye(4)
+    m[:3, 3] = {"far": (7e4, -2e4, 3e3)}.get(place, (0, 0, 0))
+    target = rng.uniform(-0.6, 0.6, (n, 3))
+    if place == "edge":
+        target = np.where(rng.random((n, 3)) < 0.5, 0.7 * rng.choice([-1, 0, 1], (n, 3)), target)
+    d = rng.normal(size=(n, 3))
+    d[:, list(zero)] = 0.0
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    d[: n // 2, list(zero)] = -0.0
+    o = np.float32(m[:3, 3]) + (target - 3.0 * d)
+    if place == "flat":   # along and beside a plate on y = 0, among its vertices' planes
+        o[:, 1] = np.float32(m[1, 3]) + rng.choice([0.0, 1e-7, -1e-7, 1e-30, -1e-40], n)
+    r = np.concatenate([o, d, np.zeros((n, 1)), np.full((n, 1), FAR)], 1).astype(np.float32)
+    insts = [(m, 1 if place == "flat" else 0)]
+    got = trav(meshes, insts, r)
+    check(got)
+    if place in ("free", "far"):
+        assert (got[:, 0] >= 0).mean() > 0.3
+        turn = r.copy()
+        turn[:, 3:6] += np.where(turn[:, 3:6] == 0, np.float32(1e-4), 0)
+        assert got[:, 3].mean() <= 1.2 * trav(meshes, insts, turn)[:, 3].mean() + 2
