@@ -219,6 +219,26 @@ struct Collapser {
 
 }  // namespace
 
+bool meshPivot(const float* vertices, size_t stride, const uint32_t* faces, int fn, float pivot[3]) {
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    const size_t corners = (size_t)3 * std::max(fn, 0), step = std::max<size_t>(1, corners / 64);
+    for (size_t i = 0; i < corners; i += step) {
+        const float* p = vertices + (size_t)faces[i] * stride;
+        growBox(lo, hi, p, p);
+    }
+    float size = 0.0f, away = 0.0f;
+    for (int a = 0; a < 3; ++a) {
+        pivot[a] = 0.5f * lo[a] + 0.5f * hi[a];
+        size = std::max(size, hi[a] - lo[a]);
+        away = std::max(away, std::fabs(pivot[a]));
+        if (!std::isfinite(pivot[a])) away = -1.0f;
+        if (away < 0.0f) break;
+    }
+    if (away > 256.0f * size) return true;
+    pivot[0] = pivot[1] = pivot[2] = 0.0f;
+    return false;
+}
+
 Bvh4Result buildBvh4(const std::vector<BuildBox>& boxes, int leafMax, int leafBase, std::vector<OmvNode4>& pool, bool tlas) {
     Bvh4Result r;
     if (boxes.empty()) return r;

@@ -2,8 +2,8 @@
 // the host binned-SAH builder (bvh.cpp) when commit time matters more than
 // the last node visit (batched validation jobs).
 //
-//   1. one lane per triangle: box and centroid from the vertex pool;
-//      centroid bounds by a block reduction;
+//   1. one lane per triangle: box (relative to the mesh's pivot) and centroid
+//      from the vertex pool; centroid bounds by a block reduction;
 //   2. 30-bit Morton code of each centroid in those bounds; stable LSD radix
 //      sort of (code, triangle) in four 8-bit passes (device_sort.h), so
 //      equal codes keep triangle order;
@@ -49,7 +49,7 @@ __device__ inline float padUp(float v) { for (int k = 0; k < OMV_BOX_PAD_ULPS; +
 
 // 1. triangle boxes and centroids; block partials of the centroid bounds
 __global__ void lbBoxes(const float* __restrict__ vtx, uint32_t vtxOff, uint32_t stride, const uint32_t* __restrict__ faces,
-                        uint32_t faceOff, uint32_t n, float* __restrict__ box, float* __restrict__ cen, float* __restrict__ part) {
+                        uint32_t faceOff, uint32_t n, float3 pivot, float* __restrict__ box, float* __restrict__ cen, float* __restrict__ part) {
     __shared__ float red[6][kBlock];
     const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -60,8 +60,9 @@ __global__ void lbBoxes(const float* __restrict__ vtx, uint32_t vtxOff, uint32_t
             for (int a = 0; a < 3; ++a) { lo[a] = fminf(lo[a], p[a]); hi[a] = fmaxf(hi[a], p[a]); }
         }
         for (int a = 0; a < 3; ++a) {
-            box[(size_t)6 * f + a] = lo[a];
-            box[(size_t)6 * f + 3 + a] = hi[a];
+            const float at = a == 0 ? pivot.x : (a == 1 ? pivot.y : pivot.z);
+            box[(size_t)6 * f + a] = omv::planeFrom(lo[a], at, false);
+            box[(size_t)6 * f + 3 + a] = omv::planeFrom(hi[a], at, true);
             c[a] = cm[a] = 0.5f * lo[a] + 0.5f * hi[a];
             cen[(size_t)3 * f + a] = c[a];
         }
@@ -320,8 +321,8 @@ __global__ void lbRecords(const float* __restrict__ vtx, uint32_t vtxOff, uint32
 // enter fewer instances that they miss: 200 rotated meshes of 10 K triangles
 // under lights, 1080p x 16 (MI355X), 6.59 -> 6.21 nodes per ray and 8.78 ->
 // 8.39 ms per render.
-__global__ __launch_bounds__(kBlock) void lbInstanceBoxes(const OmvNode4* __restrict__ nodes, const OmvInstance* __restrict__ insts, uint32_t n,
-                                                          omv::OmvInstanceBox* __restrict__ out, omv::OmvDensityRange* __restrict__ range) {
+__global__ __launch_bounds__(kBlock) void lbInstanceBoxes(const OmvNode4* __restrict__ nodes, const OmvInstance* __restrict__ insts,
+                                                          const float* __restrict__ pivots, uint32_t n, omv::OmvInstanceBox* __restrict__ out, omv::OmvDensityRange* __restrict__ range) {
     if (blockIdx.x == 0 && threadIdx.x == 0) { range->lo = INFINITY; range->hi = 0.0f; }   // for lbDensity after this launch
     const uint32_t i = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
     if (i >= n) return;
@@ -334,7 +335,7 @@ __global__ __launch_bounds__(kBlock) void lbInstanceBoxes(const OmvNode4* __rest
             const double t = (double)in.xfm[4 * a + 3];
             double mid = t, half = 0.0, terms = fabs(t);
             for (int c = 0; c < 3; ++c) {
-                const double m = (double)in.xfm[4 * a + c], l = bl[c], h = bh[c];
+                const double m = (double)in.xfm[4 * a + c], at = pivots ? pivots[4 * i + c] : 0.0f, l = at + bl[c], h = at + bh[c];
                 mid += m * 0.5 * (l + h);
                 half += fabs(m) * 0.5 * (h - l);
                 terms += fabs(m) * fmax(fabs(l), fabs(h));
@@ -417,7 +418,7 @@ size_t blasDeviceScratchBytes(uint32_t n) {
 }
 
 hipError_t buildBlasDevice(const float* vtx, uint32_t vtxOff, uint32_t stride, const uint32_t* faces, uint32_t faceOff, uint32_t n,
-                           int leafMax, int recBase, int nodeBase, uint32_t nodeCap, OmvNode4* nodes, float* records, void* scratch,
+                           const float pivot[3], int leafMax, int recBase, int nodeBase, uint32_t nodeCap, OmvNode4* nodes, float* records, void* scratch,
                            hipStream_t stream, int* root, int* nodeCount, int* depth) {
     *root = -1; *nodeCount = 0; *depth = 0;
     if (n == 0 || nodeCap == 0) return hipSuccess;
@@ -452,7 +453,7 @@ hipError_t buildBlasDevice(const float* vtx, uint32_t vtxOff, uint32_t stride, c
         if (m == 1) break;
     }
     hipError_t e;
-    lbBoxes<<<nb, kBlock, 0, stream>>>(vtx, vtxOff, stride, faces, faceOff, n, triBox, cen, part);
+    lbBoxes<<<nb, kBlock, 0, stream>>>(vtx, vtxOff, stride, faces, faceOff, n, make_float3(pivot[0], pivot[1], pivot[2]), triBox, cen, part);
     lbBounds<<<1, kBlock, 0, stream>>>(part, nb, bounds);
     lbMorton<<<nb, kBlock, 0, stream>>>(cen, bounds, n, keyA, valA);
     if ((e = sortPairs32(keyA, valA, keyB, valB, hist, n, 30, stream)) != hipSuccess) return e;
@@ -491,9 +492,9 @@ hipError_t buildBlasDevice(const float* vtx, uint32_t vtxOff, uint32_t stride, c
 }
 
 hipError_t instancePassDevice(const float* vtx, const uint32_t* faces, const OmvMesh* meshes, const OmvNode4* nodes, const OmvInstance* insts,
-                              uint32_t n, uint32_t maxFaces, OmvInstanceBox* boxes, OmvDensityRange* range, hipStream_t stream) {
+                              const float* pivots, uint32_t n, uint32_t maxFaces, OmvInstanceBox* boxes, OmvDensityRange* range, hipStream_t stream) {
     if (n == 0) return hipSuccess;
-    lbInstanceBoxes<<<(n + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, stream>>>(nodes, insts, n, boxes, range);
+    lbInstanceBoxes<<<(n + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, stream>>>(nodes, insts, pivots, n, boxes, range);
     // about four triangles a lane of the largest mesh, 4096 workgroups in all
     const uint32_t gx = std::min(std::max(blocks((uint64_t)maxFaces) / 4, 1u), 1024u), gy = std::min(n, std::max(4096u / gx, 1u));
     lbDensity<<<dim3(gx, gy), kBlock, 0, stream>>>(vtx, faces, meshes, insts, n, reinterpret_cast<uint32_t*>(range));

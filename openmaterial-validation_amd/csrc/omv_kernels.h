@@ -123,11 +123,19 @@ hipError_t launchDetached(const OmvSceneView& S0, const OmvSceneView& S1, const 
 hipError_t launchPost(const float* film, float* tmp, float* outF, uint8_t* outU8, int w, int h, float A, float gamma, bool denoise,
                       hipStream_t stream);
 // Environment alias tables (env.hip); scratch holds 4*W*H + 2*H + 2 words.
+// A box plane p relative to a pivot, rounded outward.
+__host__ __device__ inline float planeFrom(float p, float pivot, bool upper) {
+    const float d = p - pivot;
+    const double exact = (double)p - (double)pivot;
+    if (upper ? (double)d < exact : (double)d > exact) return nextafterf(d, upper ? INFINITY : -INFINITY);
+    return d;
+}
 // bvh_device.hip: one mesh's BLAS built on the device (linear BVH collapsed
-// into OmvNode4) into nodes[nodeBase ...] and records[12 * recBase ...]
+// into OmvNode4) into nodes[nodeBase ...] and records[12 * recBase ...], its
+// boxes relative to pivot (on the host)
 size_t blasDeviceScratchBytes(uint32_t n);
 hipError_t buildBlasDevice(const float* vtx, uint32_t vtxOff, uint32_t stride, const uint32_t* faces, uint32_t faceOff, uint32_t n,
-                           int leafMax, int recBase, int nodeBase, uint32_t nodeCap, OmvNode4* nodes, float* records, void* scratch,
+                           const float pivot[3], int leafMax, int recBase, int nodeBase, uint32_t nodeCap, OmvNode4* nodes, float* records, void* scratch,
                            hipStream_t stream, int* root, int* nodeCount, int* depth);
 // mesh_device.hip: commitMesh's normals / tangents of one mesh on the device
 size_t meshDeviceScratchBytes(uint32_t vn, uint32_t fn);
@@ -138,10 +146,11 @@ hipError_t preprocessMeshDevice(float* vertices, uint32_t stride, uint32_t vn, c
 // behind a coordinate (rounding goes with it); of an instance without a BLAS
 // (blas_root < 0) an empty box.  And the range of 1 / area over the world
 // triangles of an area above FLT_EPSILON, infinity and 0 if there are none.
+// (pivots: OmvSceneView::pivots)
 struct OmvInstanceBox { double lo[3], hi[3], reach[3]; };
 struct OmvDensityRange { float lo, hi; };
 hipError_t instancePassDevice(const float* vtx, const uint32_t* faces, const OmvMesh* meshes, const OmvNode4* nodes, const OmvInstance* insts,
-                              uint32_t n, uint32_t maxFaces, OmvInstanceBox* boxes, OmvDensityRange* range, hipStream_t stream);
+                              const float* pivots, uint32_t n, uint32_t maxFaces, OmvInstanceBox* boxes, OmvDensityRange* range, hipStream_t stream);
 hipError_t launchEnvBuild(const float* bg, int W, int H, float* rowProb, int* rowAlias, float* colProb, int* colAlias, float* texPdf,
                           void* scratch, hipStream_t stream);
 // 0: sample kernel (scene with lights), 1: FC kernel, 2: sample kernel (no lights), 3: batch kernel;

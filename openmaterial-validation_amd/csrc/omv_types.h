@@ -44,7 +44,7 @@ enum { OMV_BG_NONE = 0, OMV_BG_CONSTANT = 1, OMV_BG_HDR = 2 };
 static_assert(OMV_BVH_LEAF_MAX >= 1 && OMV_BVH_LEAF_MAX <= 8, "leaf size must fit the entry's 3-bit count");
 
 struct alignas(64) OmvNode4 {
-    float lox[4], hix[4], loy[4], hiy[4], loz[4], hiz[4];   // child boxes; an empty slot's planes are all +inf
+    float lox[4], hix[4], loy[4], hiy[4], loz[4], hiz[4];   // child boxes (a BLAS's: less the mesh's pivot); an empty slot's planes are all +inf
     int32_t child[4];    // >= 0 internal node; < 0 leaf: -(first+1) (tri record / instance id); empty: OMV_EMPTY_CHILD
     uint32_t entry[4];   // the child's stack entry (OMV_ENT), OMV_ENT_NONE for an empty slot
 };
@@ -111,6 +111,7 @@ struct OmvSceneView {
     const uint8_t*     texels;
     const OmvNode4*    nodes;
     const float*       tris;      // 12 floats per record
+    const float*       pivots;    // 4 floats per instance: its mesh's pivot; null: 0 for all (meshPivot)
     const OmvLight*    lights;
     const float*       light_cdf;
     const float*       bg;        // 4 floats per texel (rgb + pad)

@@ -1036,38 +1036,43 @@ DEV void boxTest4Rows(const OmvNode4* nodes, uint32_t idx, uint32_t rows, const 
 // and instance: nb for a near plane (error bound taken off) and fb for a far
 // one (added).  Conservative: with r = v_rcp_f32(d) (1 ulp) the computed
 // distance is off the exact (p - o) / d by at most 3 roundings of |p r| (r,
-// the multiply-add) and 5 of |o r| (r, o * r, the bias, the multiply-add),
-// 2^-24 each.  The builders widen every child plane by 4 ulps (>= 4 * 2^-24
-// |p|) and the bias carries 6 * 2^-24 |o r|, so a box the exact ray meets is
-// never missed; the widening also covers the rounding of a hit's t, as
-// kBoxUp does on the far side.  Where 1 / d or o / d is not finite nb, fb or
-// both are infinite or NaN, which the minima and maxima drop: the axis does
-// not cull.  A component of exactly 0 keeps the ray in a slab for good or out
-// of it: with idir the power of two that takes |o| (at least 1) just below
-// 2^127, the same products have the sign of p - o, a slab that starts behind
-// o gets a near distance of 0 or less, one that ends before o a negative far
-// one, and the bound of 6 * 2^-24 * 2^127 keeps slabs that end within 6 ulps
-// of o, for boxes up to a distance of 6e31.  (Without culling on such an axis
-// a ray visits every box along it: torus knot of 100 K triangles 512^2 x 16,
-// rays with x = 0, 18.6 -> 1.7 ms on MI355X.)
+// the multiply-add) and 6 of |o r| (r, o * r, the bias, the multiply-add, o
+// itself: in a BLAS o and p are relative to the mesh's pivot), 2^-24 each.
+// The builders widen every child plane by 4 ulps (>= 4 * 2^-24 |p|) and the
+// bias carries 6 * 2^-24 |o r|, so a box the exact ray meets is never missed;
+// the widening also covers the rounding of a hit's t, as kBoxUp does on the
+// far side.  Where 1 / d or o / d is not finite nb, fb or both are infinite or
+// NaN, which the minima and maxima drop: the axis does not cull.
 struct BoxRay { f3 idir, nb, fb; uint32_t rows; };
-DEV void boxAxis(float o, float d, float& idir, float& nb, float& fb) {
-    const uint32_t e = max(__float_as_uint(o) & 0x7F800000u, 126u << 23);   // |o| < 2^(e' - 126), e' = e >> 23
-    const bool zero = d == 0.0f;
-    idir = zero ? __uint_as_float((380u << 23) - e) : __builtin_amdgcn_rcpf(d);   // 2^(253 - e')
-    const float od = o * idir;
-    const float m = zero ? 1.70141183e38f : fabsf(od);   // 2^127
-    nb = __builtin_fmaf(m, -3.57627869e-7f, -od);        // 6 * 2^-24
-    fb = __builtin_fmaf(m, 3.57627869e-7f, -od);
+DEV void boxAxis(float o, float r, float& idir, float& nb, float& fb) {
+    const float od = o * r;
+    idir = r;
+    nb = __builtin_fmaf(fabsf(od), -3.57627869e-7f, -od);   // 6 * 2^-24
+    fb = __builtin_fmaf(fabsf(od), 3.57627869e-7f, -od);
 }
 DEV void boxRay(const f3& o, const f3& d, BoxRay& b) {
-    boxAxis(o.x, d.x, b.idir.x, b.nb.x, b.fb.x);
-    boxAxis(o.y, d.y, b.idir.y, b.nb.y, b.fb.y);
-    boxAxis(o.z, d.z, b.idir.z, b.nb.z, b.fb.z);
+    boxAxis(o.x, __builtin_amdgcn_rcpf(d.x), b.idir.x, b.nb.x, b.fb.x);
+    boxAxis(o.y, __builtin_amdgcn_rcpf(d.y), b.idir.y, b.nb.y, b.fb.y);
+    boxAxis(o.z, __builtin_amdgcn_rcpf(d.z), b.idir.z, b.nb.z, b.fb.z);
     b.rows = nearRows(b.idir);
     // computed where it is asked for: hoisted out of the mask loop it would be
     // kept in scratch memory across the traversal
     asm volatile("" : "+v"(b.idir.x), "+v"(b.idir.y), "+v"(b.idir.z));
+}
+// A component of exactly 0 keeps the ray in a slab for good or out of it: with
+// idir the power of two that takes |o| (at least 1) just below 2^127, the same
+// products have the sign of p - o, a slab that starts behind o gets a near
+// distance of 0 or less, one that ends before o a negative far one, and 6 *
+// 2^-24 * 2^127 on either side keeps slabs that end within 6 ulps of o, for
+// boxes up to a distance of 6e31.  (Without culling on such an axis a ray
+// visits every box along it: torus knot of 100 K triangles 512^2 x 16, rays
+// with x = 0, 18.6 -> 1.7 ms on MI355X.)
+DEV void boxAxisZero(float o, float d, float& idir, float& nb, float& fb) {
+    if (d != 0.0f) return;
+    const uint32_t e = max(__float_as_uint(o) & 0x7F800000u, 126u << 23);   // |o| < 2^(e' - 126), e' = e >> 23
+    idir = __uint_as_float((380u << 23) - e);                               // 2^(253 - e')
+    nb = __builtin_fmaf(-o, idir, -6.08472288e31f);
+    fb = __builtin_fmaf(-o, idir, 6.08472288e31f);
 }
 constexpr float kBoxUp = 1.0000004f;
 
@@ -1115,6 +1120,7 @@ struct Trav {
         wo = o; wd = d;
         boxRay(o, d, box);
         curInst = -1;
+        if (__builtin_expect(__ballot(zeroAxis()) != 0ull, 0)) reBox(S);
         st.push(E_DONE, c);
         cur = (E_TLAS_NODE << E_KIND_SHIFT) | (uint32_t)S.tlas_root;
         return true;
@@ -1135,6 +1141,32 @@ struct Trav {
         // a hit at or before tstop decides an occlusion query: the closest hit
         // is at least as near, so the traversal ends here
         if (h.inst >= 0 && h.t <= tstop) cur = E_DONE;
+    }
+    // some direction component of `box` is 0 (or denormal)
+    DEV bool zeroAxis() const { return fmaxf(fmaxf(fabsf(box.idir.x), fabsf(box.idir.y)), fabsf(box.idir.z)) == INFINITY; }
+    // `box` made again for the level the traversal is at, with what boxRay
+    // leaves out: zero components and the pivots of meshes far from their
+    // origin.  Rare, and from the world ray anew so that nothing is held in
+    // registers for it: looking whether it is needed takes 0.8 % of the
+    // traversal time of 200 instances (selects in boxRay and a branch for the
+    // pivots in inst() took 2 %).
+    DEV void reBox(const OmvSceneView& S) {
+        f3 o = wo, d = wd;
+        if (curInst >= 0) {
+            const float* I = S.insts[curInst].inv;
+            o = mk3(I[0] * wo.x + I[1] * wo.y + I[2] * wo.z + I[3], I[4] * wo.x + I[5] * wo.y + I[6] * wo.z + I[7],
+                    I[8] * wo.x + I[9] * wo.y + I[10] * wo.z + I[11]);
+            d = mk3(I[0] * wd.x + I[1] * wd.y + I[2] * wd.z, I[4] * wd.x + I[5] * wd.y + I[6] * wd.z, I[8] * wd.x + I[9] * wd.y + I[10] * wd.z);
+            if (S.pivots) {
+                const float4 p = reinterpret_cast<const float4*>(S.pivots)[curInst];
+                o = mk3(o.x - p.x, o.y - p.y, o.z - p.z);
+            }
+        }
+        boxRay(o, d, box);
+        boxAxisZero(o.x, d.x, box.idir.x, box.nb.x, box.fb.x);
+        boxAxisZero(o.y, d.y, box.idir.y, box.nb.y, box.fb.y);
+        boxAxisZero(o.z, d.z, box.idir.z, box.nb.z, box.fb.z);
+        box.rows = nearRows(box.idir);
     }
     // entry into an instance, the end of one, or an empty slot that node() took
     DEV void inst(const OmvSceneView& S, Stack& st, Counters& c) {
@@ -1224,7 +1256,10 @@ DEV void Trav::iterate(const OmvSceneView& S, Stack& st, Counters& c) {
     for (int k = 0; k < kNodeSteps; ++k)
         if (isNode()) node(S, st, c);
     if (isLeaf()) leaf(S, st, c);
-    if (!isNode() && !isLeaf() && more()) inst(S, st, c);
+    if (!isNode() && !isLeaf() && more()) {
+        inst(S, st, c);
+        if (__builtin_expect(S.pivots != nullptr || __ballot(zeroAxis()) != 0ull, 0)) reBox(S);
+    }
 }
 DEV bool traceClosest(const OmvSceneView& S, const f3& o, const f3& d, float tnear, float tfar, Hit& h, Stack& st, Counters& c,
                       float tstop = -1.0f) {

@@ -112,7 +112,7 @@ private:
     size_t deviceBytes_ = 0;
     std::vector<uint64_t> texOffsets_;   // byte offsets in the device texel pool
     OmvSceneView view_{};
-    DeviceBuffer dVtx_, dFaces_, dMeshes_, dInsts_, dMats_, dTexs_, dTexels_, dNodes_, dTris_, dLights_, dCdf_, dBg_, dEnv_, dEnvScratch_;
+    DeviceBuffer dVtx_, dFaces_, dMeshes_, dInsts_, dPivots_, dMats_, dTexs_, dTexels_, dNodes_, dTris_, dLights_, dCdf_, dBg_, dEnv_, dEnvScratch_;
 };
 
 // Page-locked host memory (hipHostMalloc) for films, so a film is read back

@@ -510,6 +510,9 @@ int RenderScene::commit(std::string& log) {
     std::vector<float> vtx;
     std::vector<uint32_t> faces;
     std::vector<OmvMesh> dmeshes(meshes_.size());
+    struct Pivot { float at[3]; };
+    std::vector<Pivot> pivots(meshes_.size(), Pivot{{0.0f, 0.0f, 0.0f}});   // what a mesh's boxes are relative to
+    bool anyPivot = false;
     std::vector<OmvNode4> nodes;
     std::vector<float> tris;
     int faceBase = 0, blasDepth = 0;
@@ -533,6 +536,7 @@ int RenderScene::commit(std::string& log) {
         if (!m.valid) continue;
         vtx.insert(vtx.end(), m.V.begin(), m.V.end());
         faces.insert(faces.end(), m.F.begin(), m.F.end());
+        anyPivot = meshPivot(m.V.data(), (size_t)m.stride, m.F.data(), m.fn, pivots[i].at) || anyPivot;
         if (deviceBuild) {   // built on the GPU below, records in mesh order
             meshRec[i] = recTotal;
             recTotal += m.fn;
@@ -545,6 +549,10 @@ int RenderScene::commit(std::string& log) {
             for (int k = 0; k < 3; ++k) {
                 const float* p = &m.V[(size_t)m.F[3 * f + k] * m.stride];
                 for (int a = 0; a < 3; ++a) { b.lo[a] = std::min(b.lo[a], p[a]); b.hi[a] = std::max(b.hi[a], p[a]); }
+            }
+            for (int a = 0; a < 3; ++a) {
+                b.lo[a] = planeFrom(b.lo[a], pivots[i].at[a], false);
+                b.hi[a] = planeFrom(b.hi[a], pivots[i].at[a], true);
             }
         }
         const int recBase = (int)(tris.size() / 12);
@@ -599,7 +607,7 @@ int RenderScene::commit(std::string& log) {
             const HostMesh& m = meshes_[i];
             int root = -1, count = 0, depth = 0;
             e = buildBlasDevice(dVtx_.as<float>(), dmeshes[i].vtx_offset, dmeshes[i].stride, dFaces_.as<uint32_t>(), dmeshes[i].face_offset,
-                                (uint32_t)m.fn, OMV_BVH_LEAF_MAX, meshRec[i], deviceNodes, (uint32_t)m.fn, dNodes_.as<OmvNode4>(),
+                                (uint32_t)m.fn, pivots[i].at, OMV_BVH_LEAF_MAX, meshRec[i], deviceNodes, (uint32_t)m.fn, dNodes_.as<OmvNode4>(),
                                 dTris_.as<float>(), work.ptr, nullptr, &root, &count, &depth);
             if (e != hipSuccess) return hipFail(e, "device BVH build");
             dmeshes[i].blas_root = root;
@@ -635,6 +643,12 @@ int RenderScene::commit(std::string& log) {
         d.blas_root = dmeshes[in.meshId].blas_root;
         d.mat_type = mats_[dmeshes[in.meshId].mat_id].type;
     }
+    std::vector<float> ipivots(anyPivot ? 4 * insts_.size() : 0, 0.0f);
+    if (anyPivot) {
+        for (size_t i = 0; i < insts_.size(); ++i)
+            if (insts_[i].meshId >= 0) std::memcpy(&ipivots[4 * i], pivots[insts_[i].meshId].at, sizeof(Pivot));
+        if ((e = dPivots_.upload(ipivots.data(), ipivots.size() * 4)) != hipSuccess) return hipFail(e, "upload pivots");
+    }
     std::vector<OmvInstanceBox> ibox(insts_.size());
     OmvDensityRange density = {std::numeric_limits<float>::infinity(), 0.0f};
     if (!insts_.empty()) {
@@ -648,7 +662,7 @@ int RenderScene::commit(std::string& log) {
             return hipFail(e, "upload instances");
         uint8_t* out = dInsts_.as<uint8_t>() + bytes;
         if ((e = instancePassDevice(dVtx_.as<float>(), dFaces_.as<uint32_t>(), dMeshes_.as<OmvMesh>(), dNodes_.as<OmvNode4>(),
-                                    dInsts_.as<OmvInstance>(), (uint32_t)insts_.size(), maxFaces, reinterpret_cast<OmvInstanceBox*>(out + 16),
+                                    dInsts_.as<OmvInstance>(), anyPivot ? dPivots_.as<float>() : nullptr, (uint32_t)insts_.size(), maxFaces, reinterpret_cast<OmvInstanceBox*>(out + 16),
                                     reinterpret_cast<OmvDensityRange*>(out), nullptr)) != hipSuccess)
             return hipFail(e, "instance pass launch");
         std::vector<uint8_t> got(16 + boxBytes);
@@ -773,6 +787,7 @@ int RenderScene::commit(std::string& log) {
     v.vtx = dVtx_.as<float>(); v.faces = dFaces_.as<uint32_t>(); v.meshes = dMeshes_.as<OmvMesh>();
     v.insts = dInsts_.as<OmvInstance>(); v.mats = dMats_.as<OmvMaterial>(); v.texs = dTexs_.as<OmvTexture>();
     v.texels = dTexels_.as<uint8_t>(); v.nodes = dNodes_.as<OmvNode4>(); v.tris = dTris_.as<float>();
+    v.pivots = anyPivot ? dPivots_.as<float>() : nullptr;
     v.lights = dLights_.as<OmvLight>(); v.light_cdf = dCdf_.as<float>(); v.bg = dBg_.as<float>();
     v.num_meshes = (int)meshes_.size(); v.num_insts = (int)insts_.size(); v.num_mats = (int)mats_.size();
     v.num_texs = (int)texs_.size(); v.num_lights = (int)lights_.size();
@@ -817,7 +832,7 @@ int RenderScene::commit(std::string& log) {
     nodeCount_ = (int)nodes.size() + deviceNodes;
     bvhDepth_ = tl.depth + blasDepth;
     recordCount_ = deviceBuild ? recTotal : (int)(tris.size() / 12);
-    deviceBytes_ = dVtx_.bytes + dFaces_.bytes + dMeshes_.bytes + dInsts_.bytes + dMats_.bytes + dTexs_.bytes + dTexels_.bytes +
+    deviceBytes_ = dVtx_.bytes + dFaces_.bytes + dMeshes_.bytes + dInsts_.bytes + dPivots_.bytes + dMats_.bytes + dTexs_.bytes + dTexels_.bytes +
                    dNodes_.bytes + dTris_.bytes + dLights_.bytes + dCdf_.bytes + dBg_.bytes + dEnv_.bytes;
     committed_ = true;
     return OMV_OK;

@@ -579,7 +579,7 @@ DEV uint64_t wuni64(uint64_t v) { return ((uint64_t)wuni((uint32_t)(v >> 32)) <<
 struct PacketRay {   // one lane's ray and closest hit
     f3 wo, wd, widir;   // world ray
     TriRay op;          // object ray of the packet's current instance
-    f3 oidir;
+    f3 oo, oidir;       // ... for its boxes: origin less the mesh's pivot
     Hit h;
     float tnear, tfar;
     DEV bool found() const { return h.inst >= 0; }
@@ -630,6 +630,11 @@ DEV void packetTrace(const OmvSceneView& S, PacketRay& R, uint64_t M0, uint32_t*
                             I[8] * o.x + I[9] * o.y + I[10] * o.z + I[11]);
                 f3 od = mk3(I[0] * d.x + I[1] * d.y + I[2] * d.z, I[4] * d.x + I[5] * d.y + I[6] * d.z, I[8] * d.x + I[9] * d.y + I[10] * d.z);
                 ok = rayPrep(oo, od, R.op);
+                R.oo = oo;
+                if (S.pivots) {
+                    const float4 p = reinterpret_cast<const float4*>(S.pivots)[inst];
+                    R.oo = mk3(oo.x - p.x, oo.y - p.y, oo.z - p.z);
+                }
                 R.oidir = mk3(1.0f / od.x, 1.0f / od.y, 1.0f / od.z);
             }
             const uint64_t M2 = __ballot(ok);
@@ -650,7 +655,7 @@ DEV void packetTrace(const OmvSceneView& S, PacketRay& R, uint64_t M0, uint32_t*
         const float tb = R.h.t;
         float tent[4]; bool hit[4];
         if (kind == E_TLAS_NODE) boxTest4(nd, R.wo, R.widir, R.tnear, tb, tent, hit);
-        else boxTest4(nd, R.op.o, R.oidir, R.tnear, tb, tent, hit);
+        else boxTest4(nd, R.oo, R.oidir, R.tnear, tb, tent, hit);
         if (act) ++c.nodes;
         uint64_t m[4];
 #pragma unroll

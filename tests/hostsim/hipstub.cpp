@@ -417,13 +417,13 @@ hipError_t launchPost(const float*, float*, float*, uint8_t*, int, int, float, f
     return hipSuccess;
 }
 size_t blasDeviceScratchBytes(uint32_t n) { return 64 + (size_t)n * 64; }
-hipError_t buildBlasDevice(const float*, uint32_t, uint32_t, const uint32_t*, uint32_t, uint32_t, int, int, int, uint32_t, OmvNode4*, float*, void*,
-                           hipStream_t, int* root, int* nodeCount, int* depth) {
+hipError_t buildBlasDevice(const float*, uint32_t, uint32_t, const uint32_t*, uint32_t, uint32_t, const float*, int, int, int, uint32_t, OmvNode4*,
+                           float*, void*, hipStream_t, int* root, int* nodeCount, int* depth) {
     *root = 0; *nodeCount = 1; *depth = 1;
     return hipSuccess;
 }
 size_t meshDeviceScratchBytes(uint32_t vn, uint32_t fn) { return 64 + (size_t)(vn + fn) * 64; }
-hipError_t instancePassDevice(const float*, const uint32_t*, const OmvMesh*, const OmvNode4*, const OmvInstance*, uint32_t n, uint32_t,
+hipError_t instancePassDevice(const float*, const uint32_t*, const OmvMesh*, const OmvNode4*, const OmvInstance*, const float*, uint32_t n, uint32_t,
                               OmvInstanceBox* boxes, OmvDensityRange* range, hipStream_t) {
     for (uint32_t i = 0; i < n; ++i) boxes[i] = {{-1.0, -1.0, -1.0}, {1.0, 1.0, 1.0}, {0.0, 0.0, 0.0}};
     *range = {1.0f, 1.0f};

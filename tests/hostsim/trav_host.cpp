@@ -71,13 +71,14 @@ template <class T> T rd() {
 int main() {
     std::vector<OmvNode4> nodes;
     std::vector<float> tris;
-    struct Mesh { int root, first, count; float lo[3], hi[3]; };
+    struct Mesh { int root, first, count; float lo[3], hi[3], pivot[3]; bool far; };
     std::vector<Mesh> meshes(rd<int32_t>());
     for (Mesh& m : meshes) {
         std::vector<float> v((size_t)3 * rd<int32_t>());
-        std::vector<int32_t> f((size_t)3 * rd<int32_t>());
+        std::vector<uint32_t> f((size_t)3 * rd<int32_t>());
         for (float& x : v) x = rd<float>();
-        for (int32_t& i : f) i = rd<int32_t>();
+        for (uint32_t& i : f) i = rd<uint32_t>();
+        m.far = omv::meshPivot(v.data(), 3, f.data(), (int)(f.size() / 3), m.pivot);
         std::vector<omv::BuildBox> boxes(f.size() / 3);
         for (int a = 0; a < 3; ++a) { m.lo[a] = INFINITY; m.hi[a] = -INFINITY; }
         for (size_t t = 0; t < boxes.size(); ++t)
@@ -87,6 +88,8 @@ int main() {
                 boxes[t].hi[a] = std::fmax(p, std::fmax(q, r));
                 m.lo[a] = std::fmin(m.lo[a], boxes[t].lo[a]);
                 m.hi[a] = std::fmax(m.hi[a], boxes[t].hi[a]);
+                boxes[t].lo[a] = omv::planeFrom(boxes[t].lo[a], m.pivot[a], false);
+                boxes[t].hi[a] = omv::planeFrom(boxes[t].hi[a], m.pivot[a], true);
             }
         m.first = (int)(tris.size() / 12);
         m.count = (int)boxes.size();
@@ -100,6 +103,9 @@ int main() {
     }
     std::vector<OmvInstance> insts(rd<int32_t>());
     std::vector<omv::BuildBox> iboxes;
+    std::vector<float> pivots;
+    bool anyPivot = false;
+    for (const Mesh& m : meshes) anyPivot = anyPivot || m.far;
     for (OmvInstance& in : insts) {
         std::memset(&in, 0, sizeof(in));
         in.mesh_id = rd<int32_t>();
@@ -107,6 +113,7 @@ int main() {
         for (float& x : in.inv) x = rd<float>();
         const Mesh& m = meshes[in.mesh_id];
         in.blas_root = m.root;
+        pivots.insert(pivots.end(), {m.pivot[0], m.pivot[1], m.pivot[2], 0.0f});
         omv::BuildBox b;
         for (int a = 0; a < 3; ++a) {
             double mid = in.xfm[4 * a + 3], half = 0.0, reach = std::fabs(mid);
@@ -131,6 +138,7 @@ int main() {
     OmvSceneView S;
     std::memset(&S, 0, sizeof(S));
     S.nodes = nodes.data(); S.insts = insts.data(); S.tris = tris.data();
+    S.pivots = anyPivot ? pivots.data() : nullptr;
     S.num_insts = (int)insts.size(); S.tlas_root = tl.root;
 
     std::vector<uint32_t> spill((size_t)(OMV_STACK_TOTAL - OMV_STACK_LDS) * OMV_BLOCK);

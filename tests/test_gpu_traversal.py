@@ -242,3 +242,62 @@ def test_rays_that_cull_on_no_axis(pkg, wl, ref, odd, build):
     one.render_noalloc(cam, film.data_ptr())
     torch.cuda.synchronize()
     assert np.array_equal(film.cpu().numpy().reshape(want.shape), want, equal_nan=True)
+
+
+@pytest.mark.parametrize("build", ["host", "device"])
+@pytest.mark.parametrize("away", [250.0, 262.0, 4e3, 3e5, 2e6])
+def test_meshes_far_from_their_origin(pkg, wl, ref, away, build):
+    """Meshes on either side of the distance (256 times their size) from which
+    their boxes are relative to a pivot, turned and scaled, among meshes about
+    their origin: the oracle's ids, one film in every schedule, and about as
+    many node visits as for the same mesh about its origin."""
+    v, f = wl.icosphere(3, 0.5)
+    at = np.float32([away, -0.25 * away, 0.5 * away])
+    far = (v + at).astype(np.float32)
+    rng = np.random.default_rng(8)
+    places = [(rng.normal(size=3), rng.uniform(0, 6.3), rng.uniform(0.4, 1.0, 3), rng.uniform(-1.5, 1.5, 3)) for _ in range(16)]
+
+    def scene(moved):
+        d = wl.SceneDesc()
+        d.materials.append(("pbr", dict(base_color=(0.7, 0.6, 0.5, 1.0), metallic=0.3, roughness=0.4)))
+        d.meshes.append({"vertices": far if moved else (far - at).astype(np.float32), "faces": f, "mat_id": 0})
+        d.meshes.append({"vertices": v, "faces": f, "mat_id": 0})
+        for k, (axis, angle, size, place) in enumerate(places):
+            m = np.array(wl.trs((0, 0, 0), axis, angle, size), np.float64).reshape(4, 4)
+            m[:3, 3] = place - (m[:3, :3] @ at.astype(np.float64) if moved and k % 2 == 0 else 0.0)
+            d.instances.append((m.astype(np.float32), k % 2))
+        d.lights.append(((2.0, 3.0, 2.0), (40.0,) * 3, -1.0))
+        d.background = ("const", (0.2, 0.3, 0.4))
+        d.fc_subject = "ipid"
+        s = pkg.Scene()
+        s.set_build_mode(pkg.BUILD_DEVICE_LBVH if build == "device" else pkg.BUILD_HOST_SAH)
+        d.apply(s, pkg.pbr_desc)
+        return d, s
+
+    cam = _camera(pkg, "free", 1.0, (0, 0, 0), 97, 83)
+    d, s = scene(True)
+    r = pkg.Renderer(pkg.default_params(seed=3))
+    r.set_scene(s)
+    _, ids, tie = r.render_fc(cam)
+    visits = r.stats()["nodes_visited"]
+    rs = ref.Scene()
+    d.apply(rs, ref.pbr_desc)
+    _, rids, rtie = rs.render_fc(ref.default_params(seed=3), cam.desc())
+    assert np.array_equal(ids, rids) and np.array_equal(tie, rtie)
+    assert (ids[0] >= 0).mean() > 0.2
+    _, near = scene(False)
+    r.set_scene(near)
+    r.render_fc(cam)
+    if away < 1e5:   # farther off, the instances' boxes carry the rounding of their own transforms
+        assert visits <= 1.2 * r.stats()["nodes_visited"]
+    params = dict(samples_per_pixel=2, camera_bounces=4, light_bounces=3, max_path_length=5, seed=9)
+    one = pkg.Renderer(pkg.default_params(**params))
+    one.set_scene(s)
+    one.set_schedule(pkg.SCHEDULE_PER_SAMPLE)
+    want = one.render(cam)
+    for tuning in (dict(), dict(tail_round=1), dict(traversal=2)):
+        r = pkg.Renderer(pkg.default_params(**params))
+        r.set_scene(s)
+        if tuning:
+            r.set_tuning(**tuning)
+        assert np.array_equal(r.render(cam), want), tuning

@@ -170,3 +170,25 @@ def test_zero_components_cull(trav, wl, zero, place):
         turn = r.copy()
         turn[:, 3:6] += np.where(turn[:, 3:6] == 0, np.float32(1e-4), 0)
         assert got[:, 3].mean() <= 1.2 * trav(meshes, insts, turn)[:, 3].mean() + 2
+
+
+@pytest.mark.parametrize("away", [0.0, 1e3, 1e5, 1e6])
+def test_meshes_far_from_their_origin(trav, wl, away):
+    """A mesh moved away in its own coordinates and back by its instance: the
+    slab test's slack goes with the size of the mesh, not with the distance,
+    so a ray visits hardly more nodes than for the mesh in place."""
+    rng = np.random.default_rng(6)
+    v, f = wl.icosphere(4, 0.7)
+    at = np.float32([away, -0.5 * away, 0.25 * away])
+    far = v + at
+    m, back = np.eye(4), np.eye(4)
+    back[:3, 3] = -at.astype(np.float64)
+    r = rays(rng, 300)
+    r[:, :3] *= 0.5
+    d = -r[:, :3] + rng.uniform(-0.6, 0.6, (len(r), 3))
+    r[:, 3:6] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    got = trav([(far, f)], [(back, 0)], r)
+    check(got, (0.3, 1.0))
+    # the mesh that rounding has made of it, in place
+    near = trav([(far - at, f)], [(m, 0)], r)
+    assert got[:, 3].mean() <= 1.2 * near[:, 3].mean() + 1
