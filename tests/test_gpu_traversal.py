@@ -50,10 +50,9 @@ def _scene(wl, scale, shift):
 def _camera(pkg, frame, scale, shift, w=37, h=29):
     cam = pkg.Camera(w, h, yfov=50.0)
     x, y, z = FRAMES[frame]
-    # Off the meshes' planes of symmetry, where a whole frame of rays with x = 0
-    # runs along shared edges: there both triangles are hit, at t's that differ
-    # in the last bits, more than the slab test's slack on grazing rays, so
-    # that either may be culled by the other's t (the oracle pads by 1e-6).
+    # Off the meshes' planes of symmetry: there a whole frame of rays with x = 0
+    # runs along shared edges, where the oracle's own boxes (padded by 1e-6) may
+    # leave out one of two faces hit at the same t (test_rays_along_shared_edges).
     x0, y0 = 0.0137, 0.0 if frame == "y0" else 0.5071
     at = {"along_x": (-4.0, y0, -1.0 + x0), "minus_y": (x0, 4.0, -1.0)}.get(frame, (x0, y0, 4.0))
     cam.set_viewpoint(tuple(scale * a + b for a, b in zip(at, shift)), x, y, z)
@@ -83,6 +82,48 @@ def test_ids_match_the_oracle(pkg, wl, ref, frame, place):
     assert np.array_equal(tie, rtie)
     if frame == "free" and scale > 1e-10:
         assert (ids[0] >= 0).mean() > 0.2   # the view does hit geometry
+
+
+@pytest.mark.parametrize("build", ["host", "device"])
+@pytest.mark.parametrize("place", [0, 1, 2, 3])
+@pytest.mark.parametrize("frame", ["x0", "y0", "along_z", "along_x", "minus_y"])
+def test_rays_along_shared_edges(pkg, wl, ref, frame, place, build):
+    """A camera on the meshes' planes of symmetry: rays run along edges that
+    two faces share, and along flat boxes' planes.  Both faces have to be
+    seen: ids and tie flags are those of a loop over all triangles."""
+    import ctypes as C
+    scale, shift = PLACES[place]
+    d = _scene(wl, scale, shift)
+    d.lights.clear()
+    d.fc_subject = "ipid"
+    w, h, seed = 23, 17, 3
+    cam = pkg.Camera(w, h, yfov=50.0)
+    at = {"along_x": (-4.0, 0.5, -1.0), "minus_y": (0.0, 4.0, -1.0)}.get(frame, (0.0, 0.0 if frame == "y0" else 0.5, 4.0))
+    cam.set_viewpoint(tuple(scale * a + b for a, b in zip(at, shift)), *FRAMES[frame])
+    s = pkg.Scene()
+    s.set_build_mode(pkg.BUILD_DEVICE_LBVH if build == "device" else pkg.BUILD_HOST_SAH)
+    d.apply(s, pkg.pbr_desc)
+    r = pkg.Renderer(pkg.default_params(seed=seed))
+    r.set_scene(s)
+    _, ids, tie = r.render_fc(cam)
+    rs = ref.Scene()
+    d.apply(rs, ref.pbr_desc)
+    lib, desc = ref.lib(), ref.CameraDesc.from_buffer_copy(cam.desc())
+    want, wtie = np.full((2, h, w), -1), np.zeros((h, w), int)
+    for p in range(w * h):   # the pass's ray of every pixel: jitter from the camera stream, origin off the position by its ulps
+        bits, o, dv = (C.c_uint32 * 4)(), np.zeros(3, np.float32), np.zeros(3, np.float32)
+        lib.ref_philox4x32_10((C.c_uint32 * 4)(0, 0, p, 0), (C.c_uint32 * 2)(seed, 0), bits)
+        lib.ref_camera_ray(C.byref(desc), p % w, p // w, lib.ref_u01(bits[0]), lib.ref_u01(bits[1]), ref.ptr(o), ref.ptr(dv))
+        o = o + np.float32(3 * 2.0**-23) * max(np.float32(1), np.abs(o).max()) * dv
+        hit = rs.closest_hit(o, dv, bvh=False)[0]
+        if hit:
+            want[:, p // w, p % w], wtie[p // w, p % w] = (hit[4], hit[3]), hit[5]
+    base = np.cumsum([0] + [len(m["faces"]) for m in d.meshes])
+    ids = ids.reshape(4, h, w)
+    got = np.where(ids[0] >= 0, ids[0] - base[np.maximum(ids[1], 0)], -1)
+    assert np.array_equal(got, want[0]) and np.array_equal(ids[3], want[1])
+    assert np.array_equal(np.asarray(tie).reshape(h, w), wtie)
+    assert (got >= 0).mean() > 0.2
 
 
 @pytest.mark.parametrize("place", [0, 1, 3])
