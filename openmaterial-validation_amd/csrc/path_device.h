@@ -1036,8 +1036,8 @@ DEV void boxTest4Rows(const OmvNode4* nodes, uint32_t idx, uint32_t rows, const 
 // and instance: nb for a near plane (error bound taken off) and fb for a far
 // one (added).  Conservative: with r = v_rcp_f32(d) (1 ulp) the computed
 // distance is off the exact (p - o) / d by at most 3 roundings of |p r| (r,
-// the multiply-add) and 6 of |o r| (r, o * r, the bias, the multiply-add, o
-// itself: in a BLAS o and p are relative to the mesh's pivot), 2^-24 each.
+// the multiply-add) and 5 of |o r| (r, o * r, the bias, the multiply-add),
+// 2^-24 each.
 // The builders widen every child plane by 4 ulps (>= 4 * 2^-24 |p|) and the
 // bias carries 6 * 2^-24 |o r|, so a box the exact ray meets is never missed;
 // the widening also covers the rounding of a hit's t, as kBoxUp does on the
@@ -1144,6 +1144,7 @@ struct Trav {
     }
     // some direction component of `box` is 0 (or denormal)
     DEV bool zeroAxis() const { return fmaxf(fmaxf(fabsf(box.idir.x), fabsf(box.idir.y)), fabsf(box.idir.z)) == INFINITY; }
+    DEV static void widen(float& nb, float& fb) { const float e = 0.5f * (fb - nb); nb -= e; fb += e; }
     // `box` made again for the level the traversal is at, with what boxRay
     // leaves out: zero components and the pivots of meshes far from their
     // origin.  Rare, and from the world ray anew so that nothing is held in
@@ -1163,6 +1164,11 @@ struct Trav {
             }
         }
         boxRay(o, d, box);
+        if (S.pivots) {   // o is rounded once more: twice the bias
+            widen(box.nb.x, box.fb.x);
+            widen(box.nb.y, box.fb.y);
+            widen(box.nb.z, box.fb.z);
+        }
         boxAxisZero(o.x, d.x, box.idir.x, box.nb.x, box.fb.x);
         boxAxisZero(o.y, d.y, box.idir.y, box.nb.y, box.fb.y);
         boxAxisZero(o.z, d.z, box.idir.z, box.nb.z, box.fb.z);
