@@ -187,9 +187,9 @@ int BatchRunner::prepareWavefront(const std::vector<int>& order) {
         }
     }
     if (!fork_ && (e = hipEventCreateWithFlags(&fork_, hipEventDisableTiming)) != hipSuccess) return hipFail(e, "hipEventCreate");
-    if (!wfPerCu_[0]) wavefrontBlocksPerCU(wfPerCu_);
+    if (!wfPerCu_.trace) wfPerCu_ = wavefrontBlocksPerCU();
     wfMaxSlots_ = 1ull << 22;
-    const int blocksTrace = cus_ * wfPerCu_[0];
+    const int blocksTrace = cus_ * wfPerCu_.trace;
     size_t arena = 0, rad = 0;
     int ncnt = 0;
     for (int j : order) {
@@ -204,7 +204,7 @@ int BatchRunner::prepareWavefront(const std::vector<int>& order) {
         if (slots * (uint64_t)lc >= (1ull << 32)) { setError("batch: too many samples per pixel for one chunk"); return OMV_E_RANGE; }
         const bool nee = (J.p.extensions & OMV_EXT_HDRI_NEE) && J.scene->view().env_tex_pdf;
         arena = std::max(arena, wavefrontArenaBytes((uint32_t)slots, lvCap, lc, lights, nee, false, false,
-                                                    cus_ * shadeCamBlocksPerCU(wfPerCu_, lights, nee), cus_ * wfPerCu_[3]));
+                                                    cus_ * wfPerCu_.shade[lights][nee], cus_ * wfPerCu_.gen));
         rad = std::max(rad, (size_t)slots * 3 * sizeof(float));
         ncnt = std::max(ncnt, wavefrontCounterCount(J.p.camera_bounces, lvCap));
     }
@@ -261,16 +261,15 @@ int BatchRunner::launchWavefrontJobs() {
         L.lc = std::max(1, std::min(lvCap, std::max(J.p.max_path_length, 1)));
         L.arena = r.arena.ptr; L.qcount = r.qcount.as<uint32_t>(); L.rad = r.rad.as<float>(); L.gstack = r.gstack.as<uint32_t>();
         L.counters = dCounters_.as<unsigned long long>();
-        L.blocksTrace = cus_ * wfPerCu_[0];
-        L.blocksShade = cus_ * shadeCamBlocksPerCU(wfPerCu_, J.scene->view().num_lights > 0,
-                                                   (J.p.extensions & OMV_EXT_HDRI_NEE) && J.scene->view().env_tex_pdf);
-        L.blocksGen = cus_ * wfPerCu_[3];
+        L.blocksTrace = cus_ * wfPerCu_.trace;
+        const bool lights = J.scene->view().num_lights > 0, nee = (J.p.extensions & OMV_EXT_HDRI_NEE) && J.scene->view().env_tex_pdf;
+        L.blocksShade = cus_ * wfPerCu_.shade[lights][nee];
+        L.blocksGen = cus_ * wfPerCu_.gen;
         // The tail launch and the XCD bands, as a single render takes them: 48
         // lightbox jobs of up to 384^2 x 48 on 8 streams 39.07 -> 38.13 ms, 20
         // of up to 200^2 x 16 4.50 -> 4.19 ms, 5 of up to 128^2 x 8 1.24 ->
         // 1.07 ms (MI355X).
-        L.tailRound = defaultTailRound(std::min(J.npix * (uint64_t)spp, wfMaxSlots_), J.scene->view().num_lights > 0,
-                                       (J.p.extensions & OMV_EXT_HDRI_NEE) && J.scene->view().env_tex_pdf);
+        L.tailRound = defaultTailRound(std::min(J.npix * (uint64_t)spp, wfMaxSlots_), lights, nee);
         L.xcdBands = J.scene->view().num_insts <= 4 ? 4 * xcds_ : 1;
         const uint64_t chunkPix = std::max<uint64_t>(1, wfMaxSlots_ / (uint64_t)spp);
         for (uint64_t pix0 = 0; rc == OMV_OK && pix0 < J.npix; pix0 += chunkPix) {

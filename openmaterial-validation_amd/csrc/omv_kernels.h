@@ -84,11 +84,10 @@ hipError_t launchTiles(const OmvSceneView& S, const omv_camera_desc& cam, const 
 uint32_t wavefrontSegCap(uint32_t nslots, int gridShade, int gridGen);
 size_t wavefrontArenaBytes(uint32_t nslots, int lvCap, int lc, bool lights, bool nee, bool splat, bool sortRays, int gridShade, int gridGen);
 int wavefrontCounterCount(int B, int lvCap);
-// resident blocks per CU: [0] trace, [1] camera shading with lights + NEE,
-// [2] light shading, [3] gen, [4] as [0], [5] camera shading with
-// lights, [6] with NEE, [7] with neither, [8] round-1 packet trace
-void wavefrontBlocksPerCU(int out[9]);
-inline int shadeCamBlocksPerCU(const int occ[9], bool lights, bool nee) { return lights ? (nee ? occ[1] : occ[5]) : (nee ? occ[6] : occ[7]); }
+// Resident workgroups per CU of the traversal, the generation, the round-1
+// packet trace and the camera shading [lights][nee] kernels.
+struct WfOccupancy { int trace, gen, packet, shade[2][2]; };
+WfOccupancy wavefrontBlocksPerCU();
 // Camera round from which the wavefront hands the remaining paths of a chunk
 // to one tail launch (omv_wf_tail).  A round costs two or three launches that
 // each wait for their longest ray, whatever its size; the tail waits for its

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/omv.h"
+#include "omv_kernels.h"
 #include "omv_types.h"
 
 namespace omv {
@@ -178,7 +179,7 @@ private:
     int schedule_ = OMV_SCHEDULE_WAVEFRONT;
     omv_render_tuning tuning_{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     OmvSceneView viewForLaunch() const;   // the scene view with the tuning's traversal order
-    int wfPerCu_[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    WfOccupancy wfPerCu_{};   // trace 0: not asked yet
     int tilePerCu_[4] = {0, 0, 0, 0};   // [lights][nee]
     RenderScene* scene_ = nullptr;
     omv_render_stats stats_{};
@@ -248,7 +249,7 @@ private:
     };
     std::deque<StreamRes> sres_;
     hipEvent_t fork_ = nullptr;
-    int wfPerCu_[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    WfOccupancy wfPerCu_{};   // trace 0: not asked yet
     uint64_t wfMaxSlots_ = 0;
     bool dirty_ = true;
     int blocks_ = 0, cus_ = 0, xcds_ = 1;

@@ -420,17 +420,17 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
     const uint64_t slots = std::min(npix, chunkPix) * (uint64_t)spp;
     if (slots * (uint64_t)lc >= (1ull << 32)) { setError("render: too many samples per pixel for one chunk"); return OMV_E_RANGE; }
     if (!splat_ && npix * (uint64_t)spp <= kTileSamples && defaultTuning(tuning_)) return renderTiles(cam, lvCap);
-    if (!wfPerCu_[0]) wavefrontBlocksPerCU(wfPerCu_);
+    if (!wfPerCu_.trace) wfPerCu_ = wavefrontBlocksPerCU();
     // resident traversal workgroups per CU: the occupancy limit of the traversal kernels
-    const int traceOcc = wfPerCu_[0];
+    const int traceOcc = wfPerCu_.trace;
     const int blocksTrace = cus_ * (tuning_.trace_blocks_per_cu > 0 ? std::min(tuning_.trace_blocks_per_cu, traceOcc) : traceOcc);
     hipError_t e;
     if ((e = dStack_.reserve((uint64_t)blocksTrace * OMV_BLOCK * (OMV_STACK_TOTAL - OMV_STACK_LDS) * sizeof(uint32_t))) != hipSuccess)
         return hipFail(e, "stack spill");
     const bool nee = (p.extensions & OMV_EXT_HDRI_NEE) && S.env_tex_pdf;
-    const int blocksShade = cus_ * shadeCamBlocksPerCU(wfPerCu_, lights, nee);
+    const int blocksShade = cus_ * wfPerCu_.shade[lights][nee];
     if ((e = dArena_.reserve(wavefrontArenaBytes((uint32_t)slots, lvCap, lc, lights, nee, splat_ != nullptr, tuning_.sort_rays == 2,
-                                                 blocksShade, cus_ * wfPerCu_[3]))) != hipSuccess)
+                                                 blocksShade, cus_ * wfPerCu_.gen))) != hipSuccess)
         return hipFail(e, "wavefront state");
     if ((e = dQcount_.reserve(wavefrontCounterCount(p.camera_bounces, lvCap) * sizeof(uint32_t))) != hipSuccess) return hipFail(e, "queue counters");
     if ((e = dRad_.reserve(slots * 3 * sizeof(float))) != hipSuccess) return hipFail(e, "sample buffer");
@@ -441,7 +441,7 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
     L.counters = dCounters_.as<unsigned long long>();
     L.blocksTrace = blocksTrace;
     L.blocksShade = blocksShade;
-    L.blocksGen = cus_ * wfPerCu_[3];
+    L.blocksGen = cus_ * wfPerCu_.gen;
     L.traceKeep = tuning_.trace_keep;
     L.splat = splat_;
     L.sortRays = tuning_.sort_rays == 2;
@@ -457,7 +457,7 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
     L.tailRound = tuning_.tail_round == 1 ? 0
                  : (tuning_.tail_round >= 2 ? tuning_.tail_round : defaultTailRound(slots, lights, nee));
     const bool packets = tuning_.traversal == 2;
-    L.blocksPacket = packets ? cus_ * wfPerCu_[8] : 0;
+    L.blocksPacket = packets ? cus_ * wfPerCu_.packet : 0;
     // an event pair around every traversal launch: (2 light + 3 camera rounds) per chunk
     const uint64_t chunks = (npix + chunkPix - 1) / chunkPix;
     const size_t evNeed = (size_t)std::min<uint64_t>(1u << 14, chunks * 2 * (uint64_t)(2 * lvCap + 3 * p.camera_bounces));

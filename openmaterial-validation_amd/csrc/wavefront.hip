@@ -1409,22 +1409,22 @@ size_t wavefrontArenaBytes(uint32_t nslots, int lvCap, int lc, bool lights, bool
 // lightCnt, camCnt, shCnt, envCnt, splCnt, OMV_QSEG counters each (see launchWavefront)
 int wavefrontCounterCount(int B, int lvCap) { return OMV_QSEG * (2 * (lvCap + 2) + 3 * (B + 2)); }
 
-void wavefrontBlocksPerCU(int out[9]) {
+WfOccupancy wavefrontBlocksPerCU() {
     const size_t lds = (size_t)OMV_STACK_LDS * OMV_BLOCK * sizeof(uint32_t);
     int t = occ(omv_wf_trace<0, true>, lds);
     for (int k : {occ(omv_wf_trace<0, false>, lds), occ(omv_wf_trace<1, true>, lds), occ(omv_wf_trace<1, false>, lds),
                   occ(omv_wf_trace<4, true>, lds), occ(omv_wf_trace<4, false>, lds), occ(omv_wf_trace<5, true>, lds),
                   occ(omv_wf_trace<5, false>, lds)})
         t = std::min(t, k);
-    out[0] = t;
-    out[4] = t;
-    out[1] = std::min(occ(omv_wf_shade_cam<true, true, true>, 0), occ(omv_wf_shade_cam<true, true, false>, 0));
-    out[5] = std::min(occ(omv_wf_shade_cam<true, false, true>, 0), occ(omv_wf_shade_cam<true, false, false>, 0));
-    out[6] = std::min(occ(omv_wf_shade_cam<false, true, true>, 0), occ(omv_wf_shade_cam<false, true, false>, 0));
-    out[7] = std::min(occ(omv_wf_shade_cam<false, false, true>, 0), occ(omv_wf_shade_cam<false, false, false>, 0));
-    out[2] = occ(omv_wf_shade_light<true, true>, 0);
-    out[3] = occ(omv_wf_gen<true>, 0);
-    out[8] = occ(omv_wf_trace_cam1, 0);
+    WfOccupancy o;
+    o.trace = t;
+    o.gen = occ(omv_wf_gen<true>, 0);
+    o.packet = occ(omv_wf_trace_cam1, 0);
+    o.shade[1][1] = std::min(occ(omv_wf_shade_cam<true, true, true>, 0), occ(omv_wf_shade_cam<true, true, false>, 0));
+    o.shade[1][0] = std::min(occ(omv_wf_shade_cam<true, false, true>, 0), occ(omv_wf_shade_cam<true, false, false>, 0));
+    o.shade[0][1] = std::min(occ(omv_wf_shade_cam<false, true, true>, 0), occ(omv_wf_shade_cam<false, true, false>, 0));
+    o.shade[0][0] = std::min(occ(omv_wf_shade_cam<false, false, true>, 0), occ(omv_wf_shade_cam<false, false, false>, 0));
+    return o;
 }
 
 // One chunk of whole pixels: samples [sample0, sample0 + nslots).
