@@ -24,9 +24,11 @@
 
 // ============================================================== kernels
 // Plain render: one sample per lane at a time over [sample0, sample0 + nsamples),
-// persistent grid; radiance per sample for the ordered film reduction.
+// persistent grid; radiance per sample for the ordered film reduction.  Bound
+// to the waves per SIMD its registers about give (166 - 256 VGPRs): with
+// lights and NEE it would otherwise run at one, for 5 registers.
 template <bool kLights, bool kNee, bool kSplat>
-__global__ __launch_bounds__(OMV_BLOCK) void omv_bdpt_kernel(OmvSceneView S, omv_camera_desc cam, RP P, int spp,
+__global__ __launch_bounds__(OMV_BLOCK, kLights || kNee ? 2 : 3) void omv_bdpt_kernel(OmvSceneView S, omv_camera_desc cam, RP P, int spp,
                                                              uint64_t sample0, uint64_t nsamples, float* __restrict__ rad,
                                                              float* __restrict__ lv, uint32_t* __restrict__ gstack,
                                                              unsigned long long* __restrict__ counters, float* __restrict__ splat) {
@@ -59,8 +61,9 @@ struct OmvJobDev {
     float* film;
 };
 
+// (two waves per SIMD: see omv_tile_kernel, which renders the same tiles)
 template <bool kNee>
-__global__ __launch_bounds__(OMV_BLOCK) void omv_batch_kernel(const OmvJobDev* __restrict__ jobs, int njobs,
+__global__ __launch_bounds__(OMV_BLOCK, 2) void omv_batch_kernel(const OmvJobDev* __restrict__ jobs, int njobs,
                                                               const uint64_t* __restrict__ tileEnd, uint64_t totalTiles,
                                                               int tileWaves, unsigned long long* __restrict__ work,
                                                               float* __restrict__ lv, uint32_t* __restrict__ gstack,

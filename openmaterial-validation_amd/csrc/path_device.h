@@ -973,9 +973,9 @@ DEV bool offer(Hit& h, float t, float u, float v, int inst, int prim) {
 }
 
 // 4-wide slab test, conservative (Ize 2013: tmax scaled by 1 + 2*gamma(3)).
-// An empty slot (planes at +inf, entry E_NONE) tests as a miss or, when
-// tfar * kUp overflows to +inf, as a hit at +inf; either way its E_NONE
-// entry is never pushed, so no entry check is needed here.
+// An empty slot (planes at +inf, entry E_NONE) may test as a hit (tfar * kUp
+// overflowing to +inf, or a ray whose distances are all NaN): the callers go
+// by the entry.
 DEV void boxTest4(const OmvNode4& nd, const f3& o, const f3& idir, float tnear, float tfar, float tent[4], bool hit[4]) {
     const float kUp = 1.0000004f;
 #pragma unroll
@@ -1044,16 +1044,17 @@ DEV void boxTest4Rows(const OmvNode4* nodes, uint32_t idx, uint32_t rows, const 
 // far side.  Where 1 / d or o / d is not finite nb, fb or both are infinite or
 // NaN, which the minima and maxima drop: the axis does not cull.
 struct BoxRay { f3 idir, nb, fb; uint32_t rows; };
-DEV void boxAxis(float o, float r, float& idir, float& nb, float& fb) {
+constexpr float kBoxBias = 3.57627869e-7f;   // 6 * 2^-24
+DEV void boxAxis(float o, float r, float bias, float& idir, float& nb, float& fb) {
     const float od = o * r;
     idir = r;
-    nb = __builtin_fmaf(fabsf(od), -3.57627869e-7f, -od);   // 6 * 2^-24
-    fb = __builtin_fmaf(fabsf(od), 3.57627869e-7f, -od);
+    nb = __builtin_fmaf(fabsf(od), -bias, -od);
+    fb = __builtin_fmaf(fabsf(od), bias, -od);
 }
 DEV void boxRay(const f3& o, const f3& d, BoxRay& b) {
-    boxAxis(o.x, __builtin_amdgcn_rcpf(d.x), b.idir.x, b.nb.x, b.fb.x);
-    boxAxis(o.y, __builtin_amdgcn_rcpf(d.y), b.idir.y, b.nb.y, b.fb.y);
-    boxAxis(o.z, __builtin_amdgcn_rcpf(d.z), b.idir.z, b.nb.z, b.fb.z);
+    boxAxis(o.x, __builtin_amdgcn_rcpf(d.x), kBoxBias, b.idir.x, b.nb.x, b.fb.x);
+    boxAxis(o.y, __builtin_amdgcn_rcpf(d.y), kBoxBias, b.idir.y, b.nb.y, b.fb.y);
+    boxAxis(o.z, __builtin_amdgcn_rcpf(d.z), kBoxBias, b.idir.z, b.nb.z, b.fb.z);
     b.rows = nearRows(b.idir);
     // computed where it is asked for: hoisted out of the mask loop it would be
     // kept in scratch memory across the traversal
@@ -1093,7 +1094,11 @@ DEV bool keyHit(Key a) { return __uint_as_float(a.y) < INFINITY; }
 // traversal is at, set when an instance is entered and left.  The result
 // does not depend on the visiting order: boxes are tested conservatively
 // against the current closest t, triangles accept t in (tnear, t_closest],
-// and offer() keeps the (t, instance, primitive) minimum.
+// and offer() keeps the (t, instance, primitive) minimum.  (The rounding of a
+// triangle's t has no bound at grazing angles, so a face that an almost
+// parallel ray hits a hair before the closest one so far can be culled by it:
+// with boxes tightened by an ulp one pixel in 2 M changed; the trees of both
+// builders gave the same films over 1.2e8 rays.)
 struct Trav {
     f3 wo, wd;       // world ray
     BoxRay box;      // the ray in the space of cur's node
@@ -1144,7 +1149,6 @@ struct Trav {
     }
     // some direction component of `box` is 0 (or denormal)
     DEV bool zeroAxis() const { return fmaxf(fmaxf(fabsf(box.idir.x), fabsf(box.idir.y)), fabsf(box.idir.z)) == INFINITY; }
-    DEV static void widen(float& nb, float& fb) { const float e = 0.5f * (fb - nb); nb -= e; fb += e; }
     // `box` made again for the level the traversal is at, with what boxRay
     // leaves out: zero components and the pivots of meshes far from their
     // origin.  Rare, and from the world ray anew so that nothing is held in
@@ -1152,27 +1156,21 @@ struct Trav {
     // traversal time of 200 instances (selects in boxRay and a branch for the
     // pivots in inst() took 2 %).
     DEV void reBox(const OmvSceneView& S) {
-        f3 o = wo, d = wd;
-        if (curInst >= 0) {
-            const float* I = S.insts[curInst].inv;
-            o = mk3(I[0] * wo.x + I[1] * wo.y + I[2] * wo.z + I[3], I[4] * wo.x + I[5] * wo.y + I[6] * wo.z + I[7],
-                    I[8] * wo.x + I[9] * wo.y + I[10] * wo.z + I[11]);
-            d = mk3(I[0] * wd.x + I[1] * wd.y + I[2] * wd.z, I[4] * wd.x + I[5] * wd.y + I[6] * wd.z, I[8] * wd.x + I[9] * wd.y + I[10] * wd.z);
-            if (S.pivots) {
-                const float4 p = reinterpret_cast<const float4*>(S.pivots)[curInst];
-                o = mk3(o.x - p.x, o.y - p.y, o.z - p.z);
-            }
-        }
-        boxRay(o, d, box);
-        if (S.pivots) {   // o is rounded once more: twice the bias
-            widen(box.nb.x, box.fb.x);
-            widen(box.nb.y, box.fb.y);
-            widen(box.nb.z, box.fb.z);
-        }
-        boxAxisZero(o.x, d.x, box.idir.x, box.nb.x, box.fb.x);
-        boxAxisZero(o.y, d.y, box.idir.y, box.nb.y, box.fb.y);
-        boxAxisZero(o.z, d.z, box.idir.z, box.nb.z, box.fb.z);
+        reAxis(S, 0, wo.x, wd.x, box.idir.x, box.nb.x, box.fb.x);
+        reAxis(S, 1, wo.y, wd.y, box.idir.y, box.nb.y, box.fb.y);
+        reAxis(S, 2, wo.z, wd.z, box.idir.z, box.nb.z, box.fb.z);
         box.rows = nearRows(box.idir);
+    }
+    DEV void reAxis(const OmvSceneView& S, int a, float o, float d, float& idir, float& nb, float& fb) {
+        if (curInst >= 0) {
+            const float* I = S.insts[curInst].inv + 4 * a;
+            o = I[0] * wo.x + I[1] * wo.y + I[2] * wo.z + I[3];
+            d = I[0] * wd.x + I[1] * wd.y + I[2] * wd.z;
+            if (S.pivots) o = o - S.pivots[4 * curInst + a];
+        }
+        boxAxis(o, __builtin_amdgcn_rcpf(d), S.pivots ? 2.0f * kBoxBias : kBoxBias, idir, nb, fb);   // o is rounded once more
+        boxAxisZero(o, d, idir, nb, fb);
+        asm volatile("" ::: "memory");   // an axis at a time: no loads ahead
     }
     // entry into an instance, the end of one, or an empty slot that node() took
     DEV void inst(const OmvSceneView& S, Stack& st, Counters& c) {
@@ -1242,8 +1240,9 @@ struct Trav {
     DEV void iterate(const OmvSceneView& S, Stack& st, Counters& c);
 };
 
-// Traversal launches are bound by VALU issue (0.8 - 0.99 of the issue cycles
-// on MI355X, a quarter of the lanes active on secondary rays), so what counts
+// Traversal launches are bound by VALU issue (MI355X: 0.75 - 0.84 of the issue
+// cycles in the first two rounds, 0.4 of the lanes active on secondary rays;
+// later rounds are short and wait for fetches), so what counts
 // is instructions per entry and how many entry kinds an iteration mixes.  The
 // blocks of the loop are taken by the lanes whose entry is of that kind, and
 // a wave pays each block that any of its lanes needs; a ray visits four to
