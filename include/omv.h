@@ -336,7 +336,8 @@ int omv_renderer_get_stats(const omv_renderer* r, omv_render_stats* out);
  *                            traversal kernel and a shading kernel
  *                            (+ connection visibility and sum with lights);
  *                            with the default tuning a render of at most
- *                            2^18 samples is one launch over film tiles
+ *                            2^18 samples, 64 a pixel, is one launch over
+ *                            film tiles
  *                            (counted as one traversal launch);
  *   OMV_SCHEDULE_PER_SAMPLE  one persistent kernel, one lane per sample. */
 #define OMV_SCHEDULE_WAVEFRONT   0
@@ -498,7 +499,9 @@ typedef struct omv_batch_tuning {
     int blocks_per_cu;   /* one launch: resident workgroups per CU
                             (0 = occupancy limit)                          */
     int tile_waves;      /* one launch: samples per work item, about
-                            256 * tile_waves (>= 1), in whole pixels       */
+                            256 * tile_waves in whole pixels, at least one
+                            pixel, at most 64 pixels and (but for one pixel
+                            of more) 1024 samples, so >= 4 are alike       */
     int use_graph;       /* 1: replay a captured hipGraph, 0: plain launch */
     int streams;         /* 0: one persistent launch over all
                             jobs; N >= 1: each job's wavefront launch

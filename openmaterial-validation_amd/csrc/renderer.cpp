@@ -21,14 +21,6 @@ constexpr uint64_t kChunkSamples = 1ull << 24;   // per-sample radiance buffer: 
 // of one MI355X's 288 GB; chunk_samples lowers it.
 constexpr uint64_t kWfSlots = 1ull << 25;
 constexpr uint64_t kWfSlotsLights = 1ull << 25;
-// Round-1 camera rays are traced as wave packets (omv_wf_trace_cam1) only on
-// request (tuning traversal = 2).  Measured on MI355X (kernel ms per render,
-// per-ray -> packets), first with the branchy triangle setup: at 64 samples
-// per pixel torus knot 512^2 8.55 -> 8.38, instanced 960x540 15.06 ->
-// 14.89; at 16: instanced 1080p 15.06 -> 15.13.  Once the per-ray traversal
-// got the branch-free triangle setup and stack fast paths: torus knot 512^2
-// x 64 6.36 -> 6.41, 1024^2 x 16 6.23 -> 6.26, instanced 1080p x 16 12.48
-// -> 12.61, x 4 4.74 -> 5.12.
 // Samples up to which a render with the default tuning runs as one launch
 // over film tiles instead of ray-queue rounds: its 20 and more launches each
 // wait for their longest ray, which is most of a small render.  MI355X,
@@ -36,7 +28,13 @@ constexpr uint64_t kWfSlotsLights = 1ull << 25;
 // without point lights, NEE, masked, 60 instances): 12 K samples 0.29 - 1.36
 // -> 0.17 - 0.81, 192 K 0.30 - 1.62 -> 0.29 - 0.97; at 600 K 0.37 - 2.05 ->
 // 0.50 - 2.04, tiles 1.3 x faster to 1.3 x slower.
+// And at most one batch of a wave per pixel: a pixel's samples are one wave's,
+// 64 at a time, so more of them are a serial chain.  Tiles against rounds, films
+// of 8^2 to 64^2 on three kinds of scene: 64 samples a pixel 1.07 - 1.5 times as
+// fast, 96 0.76 - 1.05, 128 0.72 - 1.07, 256 0.47 - 0.66; 8^2 x 1024 6.1 ms
+// against 0.75, 1 pixel x 2^18 824 ms against 16.
 constexpr uint64_t kTileSamples = 1ull << 18;
+constexpr int kTileSpp = 64;
 bool defaultTuning(const omv_render_tuning& t) {
     const omv_render_tuning none{};
     return std::memcmp(&t, &none, sizeof(t)) == 0;
@@ -419,7 +417,7 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
     const uint64_t chunkPix = std::max<uint64_t>(1, maxSlots / (uint64_t)spp);
     const uint64_t slots = std::min(npix, chunkPix) * (uint64_t)spp;
     if (slots * (uint64_t)lc >= (1ull << 32)) { setError("render: too many samples per pixel for one chunk"); return OMV_E_RANGE; }
-    if (!splat_ && npix * (uint64_t)spp <= kTileSamples && defaultTuning(tuning_)) return renderTiles(cam, lvCap);
+    if (!splat_ && spp <= kTileSpp && npix * (uint64_t)spp <= kTileSamples && defaultTuning(tuning_)) return renderTiles(cam, lvCap);
     if (!wfPerCu_.trace) wfPerCu_ = wavefrontBlocksPerCU();
     // resident traversal workgroups per CU: the occupancy limit of the traversal kernels
     const int traceOcc = wfPerCu_.trace;
@@ -456,6 +454,14 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
     L.xcdBands = tuning_.xcd_bands > 0 ? tuning_.xcd_bands : (S.num_insts <= 4 ? 4 * xcds_ : 1);
     L.tailRound = tuning_.tail_round == 1 ? 0
                  : (tuning_.tail_round >= 2 ? tuning_.tail_round : defaultTailRound(slots, lights, nee));
+    // Round-1 camera rays are traced as wave packets (omv_wf_trace_cam1) only on
+    // request (tuning traversal = 2).  Measured on MI355X (kernel ms per render,
+    // per-ray -> packets), first with the branchy triangle setup: at 64 samples
+    // per pixel torus knot 512^2 8.55 -> 8.38, instanced 960x540 15.06 ->
+    // 14.89; at 16: instanced 1080p 15.06 -> 15.13.  Once the per-ray traversal
+    // got the branch-free triangle setup and stack fast paths: torus knot 512^2
+    // x 64 6.36 -> 6.41, 1024^2 x 16 6.23 -> 6.26, instanced 1080p x 16 12.48
+    // -> 12.61, x 4 4.74 -> 5.12.
     const bool packets = tuning_.traversal == 2;
     L.blocksPacket = packets ? cus_ * wfPerCu_.packet : 0;
     // an event pair around every traversal launch: (2 light + 3 camera rounds) per chunk

@@ -105,3 +105,19 @@ def test_refused_however_few_samples(pkg, wl, chunk):
                 r.render(cam)
         else:
             r.render(cam)
+
+
+@pytest.mark.parametrize("size,spp,tiles", [((8, 8), 64, True), ((8, 8), 65, False), ((1, 1), 64, True), ((1, 1), 4096, False),
+                                            ((64, 64), 64, True), ((4, 4), 3000, False), ((512, 512), 1, True), ((513, 512), 1, False)])
+def test_many_samples_on_few_pixels(pkg, wl, size, spp, tiles):
+    """The tile launch takes a pixel's samples 64 at a time in one wave, so it
+    is for up to 64 samples a pixel (and 2^18 in all); either way the film is
+    the per-sample schedule's."""
+    desc, s, cam = _scene(pkg, wl, *size)
+    params = dict(samples_per_pixel=spp, camera_bounces=4, light_bounces=2, max_path_length=5, seed=5)
+    r, q = pkg.Renderer(pkg.default_params(**params)), pkg.Renderer(pkg.default_params(**params))
+    q.set_schedule(pkg.SCHEDULE_PER_SAMPLE)
+    for x in (r, q):
+        x.set_scene(s)
+    assert np.array_equal(r.render(cam), q.render(cam))
+    assert (r.stats()["trace_launches"] == 1) == tiles
