@@ -398,7 +398,8 @@ typedef struct omv_render_tuning {
                                  (every round as its own trace, shade and
                                  connect launches), n >= 2 = from round n;
                                  the default is 3 to 5: later with more
-                                 samples, and with point lights or NEE       */
+                                 samples, with point lights or NEE, and where
+                                 few paths escape                            */
 } omv_render_tuning;
 int omv_renderer_set_tuning(omv_renderer* r, const omv_render_tuning* t);
 int omv_renderer_get_tuning(const omv_renderer* r, omv_render_tuning* t);

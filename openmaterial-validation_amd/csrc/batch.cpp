@@ -269,7 +269,10 @@ int BatchRunner::launchWavefrontJobs() {
         // lightbox jobs of up to 384^2 x 48 on 8 streams 39.07 -> 38.13 ms, 20
         // of up to 200^2 x 16 4.50 -> 4.19 ms, 5 of up to 128^2 x 8 1.24 ->
         // 1.07 ms (MI355X).
-        L.tailRound = defaultTailRound(std::min(J.npix * (uint64_t)spp, wfMaxSlots_), lights, nee);
+        // The earlier tail of open scenes: 8 jobs of 256^2 x 12 in a closed room
+        // 37.7 -> 31.5 ms without it (MI355X).
+        L.tailRound = J.scene->encloses(J.cam.position) ? lateTailRound(lights, nee)
+                                                        : earlyTailRound(std::min(J.npix * (uint64_t)spp, wfMaxSlots_), lights, nee);
         L.xcdBands = J.scene->view().num_insts <= 4 ? 4 * xcds_ : 1;
         const uint64_t chunkPix = std::max<uint64_t>(1, wfMaxSlots_ / (uint64_t)spp);
         for (uint64_t pix0 = 0; rc == OMV_OK && pix0 < J.npix; pix0 += chunkPix) {

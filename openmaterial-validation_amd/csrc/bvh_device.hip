@@ -22,8 +22,8 @@
 //   6. triangle records (v0 + id, v1, v2) in sorted order.
 //
 // The closest hit does not depend on the tree (watertight test, ties broken
-// by (t, instance, primitive)), so films equal the host-built scene's bit
-// for bit; only node and triangle counts change.
+// by (t, instance, primitive); see Trav for grazing hits), so films equal the
+// host-built scene's bit for bit; only node and triangle counts change.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

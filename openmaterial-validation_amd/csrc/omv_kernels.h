@@ -62,6 +62,11 @@ struct WfLaunch {
     int roundEvAt;             // done (or at the end when there are fewer rounds)
     int xcdBands;              // > 1: traversal queues dealt to this many XCDs in chunks (L2 locality); else plain stride
     int tailRound;             // >= 2: camera rounds tailRound .. B run as one launch (omv_wf_tail); else round by round
+    // tailEarly >= 3: already from round tailEarly on if at most 3/4 of the paths start round 2.  Their number goes
+    // to `alive` (pinned memory, with an event), and the host waits for it while the device runs that round
+    int tailEarly;
+    uint32_t* alive;
+    hipEvent_t aliveEv;
     int blocksPacket;          // > 0: round-1 camera rays traced as wave packets (omv_wf_trace_cam1) on this many workgroups
 };
 // Pixels of a tile that one wave renders sample by sample (renderTile): about
@@ -101,7 +106,17 @@ WfOccupancy wavefrontBlocksPerCU();
 //     0.95 1.01 1.10 1.21, 1.68 1.33 1.17 1.27, 3.62 2.95 2.92 2.93
 //   NEE 5.4 M: - 4.00 3.48 3.64; masked with lights 4.9 M: - - 5.94 5.80
 //   16.8 M torus knot: - 5.07 4.59 4.72; 33 M instanced: - - 9.39 8.78
-inline int defaultTailRound(uint64_t slots, bool lights, bool nee) {
+// (At 1.5 M scenes of one material type would gain from an earlier round still:
+// with lights from 2, NEE from 3; mixed and masked ones from 4.)
+// That holds while most paths escape: 0.12 - 0.65 of them start round 2 in those
+// scenes, 0.01 - 0.18 round 3.  In a closed room 0.86 - 0.95 start round 2 and
+// the tail is full of long paths: from round 3 / 4 / 5, 1 M samples, depth 20,
+// 5.16 4.28 3.84 without lights, 30.5 26.5 23.6 with; 2 M, depth 8, 5.46 4.84
+// 4.57, 29.6 25.8 23.3.  There the tail starts at lateTailRound.  A render
+// counts the paths that start round 2; batches, which are captured, go by
+// where the camera is (RenderScene::encloses).
+inline int lateTailRound(bool lights, bool nee) { return lights || nee ? 5 : 4; }
+inline int earlyTailRound(uint64_t slots, bool lights, bool nee) {
     if (!lights && !nee) return slots <= (1u << 21) ? 3 : 4;
     if (slots <= (1u << 20)) return 3;
     return slots <= (lights ? 1u << 22 : 1u << 23) ? 4 : 5;

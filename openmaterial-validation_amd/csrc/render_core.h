@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/omv.h"
+#include "bvh.h"
 #include "omv_kernels.h"
 #include "omv_types.h"
 
@@ -78,6 +79,8 @@ public:
     int commit(std::string& log);
 
     bool committed() const { return committed_; }
+    // true when the rays from p along all six axis directions meet the world box of an instance: a camera in a room
+    bool encloses(const float p[3]) const;
     const OmvSceneView& view() const { return view_; }
     int meshInfo(int id, int* vn, int* fn, int* stride, int* mat) const;
     int vertices(int id, float* out, size_t cap) const;
@@ -111,6 +114,7 @@ private:
     bool committed_ = false;
     int nodeCount_ = 0, bvhDepth_ = 0, recordCount_ = 0, stackBound_ = 0;
     size_t deviceBytes_ = 0;
+    std::vector<BuildBox> instBoxes_;    // world boxes of the instances
     std::vector<uint64_t> texOffsets_;   // byte offsets in the device texel pool
     OmvSceneView view_{};
     DeviceBuffer dVtx_, dFaces_, dMeshes_, dInsts_, dPivots_, dMats_, dTexs_, dTexels_, dNodes_, dTris_, dLights_, dCdf_, dBg_, dEnv_, dEnvScratch_;
@@ -203,6 +207,7 @@ private:
     // stream marking where the next chunk may start
     hipStream_t stream2_ = nullptr;
     hipEvent_t chunkEv_[3] = {nullptr, nullptr, nullptr};
+    hipEvent_t aliveEv_[2] = {nullptr, nullptr};   // the count of round 2's paths is on the host (per chunk stream)
     DeviceBuffer dArena2_, dQcount2_, dRad2_, dStack2_;
 };
 

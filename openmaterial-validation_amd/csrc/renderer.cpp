@@ -103,6 +103,7 @@ BDPTRenderer::~BDPTRenderer() {
     for (auto& e : ev_) if (e) (void)hipEventDestroy(e);
     for (auto& e : traceEv_) (void)hipEventDestroy(e);
     for (auto& e : chunkEv_) if (e) (void)hipEventDestroy(e);
+    for (auto& e : aliveEv_) if (e) (void)hipEventDestroy(e);
     if (hostStage_) (void)hipHostFree(hostStage_);
     if (stream2_) (void)hipStreamDestroy(stream2_);
     if (stream_) (void)hipStreamDestroy(stream_);
@@ -182,7 +183,7 @@ int BDPTRenderer::render(PinholeCamera& cam, float* filmDev) {
     // the film the kernels write: the renderer's (read back into the camera)
     // or the caller's device buffer (left in device memory)
     film_ = filmDev ? filmDev : dFilm_.as<float>();
-    if (!hostStage_ && (e = hipHostMalloc(&hostStage_, 8 * sizeof(unsigned long long), hipHostMallocDefault)) != hipSuccess) {
+    if (!hostStage_ && (e = hipHostMalloc(&hostStage_, 9 * sizeof(unsigned long long), hipHostMallocDefault)) != hipSuccess) {
         hostStage_ = nullptr;
         return hipFail(e, "counter staging");
     }
@@ -453,7 +454,15 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
     // 11.00 with one band per XCD)
     L.xcdBands = tuning_.xcd_bands > 0 ? tuning_.xcd_bands : (S.num_insts <= 4 ? 4 * xcds_ : 1);
     L.tailRound = tuning_.tail_round == 1 ? 0
-                 : (tuning_.tail_round >= 2 ? tuning_.tail_round : defaultTailRound(slots, lights, nee));
+                 : (tuning_.tail_round >= 2 ? tuning_.tail_round : lateTailRound(lights, nee));
+    L.tailEarly = tuning_.tail_round == 0 ? earlyTailRound(slots, lights, nee) : 0;
+    if (L.tailEarly >= L.tailRound) L.tailEarly = 0;
+    if (L.tailEarly) {
+        for (auto& ev : aliveEv_)
+            if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return hipFail(e, "hipEventCreate");
+        L.alive = reinterpret_cast<uint32_t*>(static_cast<unsigned long long*>(hostStage_) + 8);
+        L.aliveEv = aliveEv_[0];
+    }
     // Round-1 camera rays are traced as wave packets (omv_wf_trace_cam1) only on
     // request (tuning traversal = 2).  Measured on MI355X (kernel ms per render,
     // per-ray -> packets), first with the branchy triangle setup: at 64 samples
@@ -494,6 +503,7 @@ int BDPTRenderer::renderWavefront(PinholeCamera& cam, double& kernelMs) {
         st[1] = stream2_;
         Ls[1].arena = dArena2_.ptr; Ls[1].qcount = dQcount2_.as<uint32_t>(); Ls[1].rad = rad[1] = dRad2_.as<float>();
         Ls[1].gstack = dStack2_.as<uint32_t>();
+        if (L.tailEarly) { Ls[1].alive = L.alive + 1; Ls[1].aliveEv = aliveEv_[1]; }
         const int stagger = tuning_.chunk_stagger > 0 ? tuning_.chunk_stagger : 1;
         for (int k = 0; k < 2; ++k) { Ls[k].roundEv = chunkEv_[k]; Ls[k].roundEvAt = stagger; }
     }

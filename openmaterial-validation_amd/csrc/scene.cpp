@@ -685,6 +685,8 @@ int RenderScene::commit(std::string& log) {
         iids.push_back((int)i);
     }
     Bvh4Result tl = buildBvh4(iboxes, 1, 0, nodes, true);
+    instBoxes_.clear();
+    if (iboxes.size() <= 4096) instBoxes_ = iboxes;   // encloses() is not worth a longer look
     float sceneLo[3] = {INFINITY, INFINITY, INFINITY}, sceneHi[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (const BuildBox& b : iboxes)
         for (int a = 0; a < 3; ++a) { sceneLo[a] = std::min(sceneLo[a], b.lo[a]); sceneHi[a] = std::max(sceneHi[a], b.hi[a]); }
@@ -836,6 +838,18 @@ int RenderScene::commit(std::string& log) {
                    dNodes_.bytes + dTris_.bytes + dLights_.bytes + dCdf_.bytes + dBg_.bytes + dEnv_.bytes;
     committed_ = true;
     return OMV_OK;
+}
+
+bool RenderScene::encloses(const float p[3]) const {
+    int met = 0;
+    for (const BuildBox& b : instBoxes_)
+        for (int a = 0; a < 3; ++a) {
+            const int u = (a + 1) % 3, v = (a + 2) % 3;
+            if (!(b.lo[u] <= p[u] && p[u] <= b.hi[u] && b.lo[v] <= p[v] && p[v] <= b.hi[v])) continue;
+            if (b.hi[a] >= p[a]) met |= 1 << (2 * a);
+            if (b.lo[a] <= p[a]) met |= 2 << (2 * a);
+        }
+    return met == 63;
 }
 
 int RenderScene::updateTexture(int texId, const void* src) {

@@ -324,10 +324,10 @@ struct XcdList {
 // direction comes from a rejection loop, cheaper to keep than to redo) by
 // appending to the segmented round-1 light queue (lightSeg, whose regions
 // are sized for this launch's grid) -- except a ray that
-// misses all four child boxes of the TLAS root: the traversal's first step
-// is that same test (boxTest4Rows, tnear 0, tfar FLT_MAX), after which it
-// ends without a hit, so such a ray is not traced.  Its trace is still
-// counted (one ray, one light ray, the root's node visit), and light round
+// misses all four child boxes of the TLAS root (boxTest4Rows, conservative,
+// tnear 0, tfar FLT_MAX): it hits nothing and is not traced.  Its trace is
+// still counted (one ray, one light ray, the root's node visit; the traversal's
+// own test of the root is a little wider and may visit more), and light round
 // 1 leaves its subpath at the light vertex, as for a traced miss.  A light
 // that lies above every root child on some axis has all its rays culled
 // (lightBelowRoot); their directions are not drawn.
@@ -1265,6 +1265,16 @@ __global__ __launch_bounds__(OMV_BLOCK, OMV_TAIL_WAVES(kLights, kNee)) void omv_
     flushCounters(statSlot(counters), L.rays, L.camRays, 0u, L.shadowRays, L.cnt);
 }
 
+// The entries of a queue, into host memory.
+__global__ void omv_wf_alive(WfSeg q, uint32_t* __restrict__ out) {
+    __shared__ SegTable cur;
+    segLoad(cur, q);
+    if (threadIdx.x == 0) {
+        *out = cur.total();
+        __threadfence_system();
+    }
+}
+
 // ----------------------------------------------------------- ray sorting
 // A round's secondary camera rays reordered by (direction octant, cell of a
 // 16^3 grid over the scene box, Morton order) with a counting sort, so that
@@ -1583,27 +1593,20 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
     const bool fuse = lights || nee;
     // rounds i0 .. B in one launch (0: none); the round before i0 leaves
     // its camera rays untraced for it
-    const int i0 = L.tailRound >= 2 && L.tailRound <= B ? L.tailRound : 0;
+    int i0 = L.tailRound >= 2 && L.tailRound <= B ? L.tailRound : 0;
+    const bool ask = L.tailEarly >= 3 && L.tailEarly <= B;
     bool traced = false;   // the camera rays of round i were traced by the previous fused launch
     bool roundEvDone = false;
     for (int i = 1; i <= B; ++i) {
+        if (ask && i == L.tailEarly - 1) {   // before this round's fused launch, which traces the next round's rays
+            if ((e = hipEventSynchronize(L.aliveEv)) != hipSuccess) return e;
+            if (*L.alive <= n - n / 4) i0 = L.tailEarly;
+        }
         if (i == i0) {
+            auto tail = lights ? (nee ? omv_wf_tail<true, true> : omv_wf_tail<true, false>)
+                               : (nee ? omv_wf_tail<false, true> : omv_wf_tail<false, false>);
             mark();
-            if (lights) {
-                if (nee)
-                    hipLaunchKernelGGL((omv_wf_tail<true, true>), dim3(L.blocksTrace), blk, lds, stream, S, P, L.sample0, i, W, in, camCnt(i),
-                                       L.rad, L.gstack, stats);
-                else
-                    hipLaunchKernelGGL((omv_wf_tail<true, false>), dim3(L.blocksTrace), blk, lds, stream, S, P, L.sample0, i, W, in, camCnt(i),
-                                       L.rad, L.gstack, stats);
-            } else {
-                if (nee)
-                    hipLaunchKernelGGL((omv_wf_tail<false, true>), dim3(L.blocksTrace), blk, lds, stream, S, P, L.sample0, i, W, in, camCnt(i),
-                                       L.rad, L.gstack, stats);
-                else
-                    hipLaunchKernelGGL((omv_wf_tail<false, false>), dim3(L.blocksTrace), blk, lds, stream, S, P, L.sample0, i, W, in, camCnt(i),
-                                       L.rad, L.gstack, stats);
-            }
+            hipLaunchKernelGGL(tail, dim3(L.blocksTrace), blk, lds, stream, S, P, L.sample0, i, W, in, camCnt(i), L.rad, L.gstack, stats);
             mark();
             break;
         }
@@ -1631,6 +1634,10 @@ hipError_t launchWavefront(const WfLaunch& L, hipStream_t stream) {
             else
                 hipLaunchKernelGGL((sorted ? omv_wf_shade_cam<false, false, true> : omv_wf_shade_cam<false, false, false>), dim3(L.blocksShade), blk, 0, stream, S, P, L.sample0, i, W, in, camCnt(i),
                                    H, out, camCnt(i + 1), sq, shCnt(i), eq, envCnt(i), L.rad, Gen1, lost);
+        }
+        if (ask && i == 1) {
+            hipLaunchKernelGGL(omv_wf_alive, dim3(1), dim3(64), 0, stream, camCnt(2), L.alive);
+            if ((e = hipEventRecord(L.aliveEv, stream)) != hipSuccess) return e;
         }
         bool reordered = false;
         const bool nextInWavefront = i < B && i + 1 != i0;   // round i + 1 is traced by this schedule's round kernels

@@ -442,3 +442,66 @@ def test_throughput_that_overflows(pkg, wl, lights, bounces, factor):
         if tuning:
             r.set_tuning(**tuning)
         assert np.array_equal(r.render(cam), want, equal_nan=True), tuning
+
+
+def _room(wl, lights):
+    """A closed room (a sphere seen from inside) with a box in it."""
+    d = wl.SceneDesc()
+    d.materials.append(("pbr", dict(base_color=(0.8, 0.8, 0.7, 1.0), metallic=0.0, roughness=0.8)))
+    v, f = wl.icosphere(4, 6.0)
+    d.meshes.append({"vertices": v, "faces": f[:, ::-1].copy(), "mat_id": 0})
+    v, f, uv = wl.grid_box(3, (0.7, 0.7, 0.7))
+    d.meshes.append({"vertices": v, "faces": f, "mat_id": 0, "uvs": [uv]})
+    d.instances += [(wl.trs((0, 0, 0)), 0), (wl.trs((0.2, -0.3, -3.0), angle=0.4), 1)]
+    if lights:
+        d.lights.append(((1.0, 2.0, 0.0), (60.0,) * 3, -1.0))
+    d.background = ("const", (0.2, 0.3, 0.4))
+    return d, wl.View(200, 140, (0.3, 0.2, 1.0), (0.0, 0.0, -1.0), yfov=70.0)
+
+
+@pytest.mark.parametrize("bounces", [2, 3, 4, 7])
+@pytest.mark.parametrize("lights", [False, True])
+@pytest.mark.parametrize("closed", [False, True])
+def test_tail_starts_later_in_closed_rooms(pkg, wl, closed, lights, bounces):
+    """By default the tail launch of a render of 400 K samples starts at round 3
+    while most paths escape, and at the round for the largest renders when
+    more than 3/4 of them go on after the first vertex; the film is that of
+    every round on its own."""
+    desc, view = _room(wl, lights) if closed else wl.mixed_test_scene(hdr=True, lights=lights)
+    view.width, view.height = 200, 140
+    s = pkg.Scene()
+    desc.apply(s, pkg.pbr_desc)
+    cam = pkg.Camera(view.width, view.height, view.position, view.forward, view.up, view.yfov)
+    films, launches = [], []
+    for tail in (0, 1, (5 if lights else 4) if closed else 3):
+        r = pkg.Renderer(pkg.default_params(samples_per_pixel=15, camera_bounces=bounces, light_bounces=2, max_path_length=6, seed=8))
+        r.set_scene(s)
+        if tail:
+            r.set_tuning(tail_round=tail)
+        films.append(r.render(cam).copy())
+        launches.append(r.stats()["trace_launches"])
+    assert np.array_equal(films[0], films[1]) and np.array_equal(films[0], films[2])
+    assert launches[0] == launches[2]
+
+
+def test_batch_in_a_closed_room(pkg, wl):
+    """Stream jobs, captured, whose cameras are in a room or outside: the plain renders' films."""
+    b = pkg.Batch()
+    want, scenes = [], []
+    for closed in (True, False):
+        for lights in (False, True):
+            desc, view = _room(wl, lights) if closed else wl.mixed_test_scene(hdr=True, lights=lights)
+            s = pkg.Scene()
+            desc.apply(s, pkg.pbr_desc)
+            scenes.append(s)
+            cam = pkg.Camera(83, 61, view.position, view.forward, view.up, view.yfov)
+            p = pkg.default_params(samples_per_pixel=5, camera_bounces=6, light_bounces=2, max_path_length=6, seed=4)
+            b.add_job(s, cam, p)
+            r = pkg.Renderer(p)
+            r.set_scene(s)
+            want.append(r.render(cam).copy())
+    b.set_tuning(streams=3, use_graph=True)
+    for _ in range(3):
+        b.run()
+        for j, film in enumerate(want):
+            assert np.array_equal(b.film(j), film), j
