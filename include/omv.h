@@ -336,8 +336,9 @@ int omv_renderer_get_stats(const omv_renderer* r, omv_render_stats* out);
  *                            traversal kernel and a shading kernel
  *                            (+ connection visibility and sum with lights);
  *                            with the default tuning a render of at most
- *                            2^18 samples, 64 a pixel, is one launch over
- *                            film tiles
+ *                            2^18 samples (2^16 with instances on all six
+ *                            sides of the camera), 64 a pixel, is one launch
+ *                            over film tiles
  *                            (counted as one traversal launch);
  *   OMV_SCHEDULE_PER_SAMPLE  one persistent kernel, one lane per sample. */
 #define OMV_SCHEDULE_WAVEFRONT   0

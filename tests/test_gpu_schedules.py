@@ -484,6 +484,16 @@ def test_tail_starts_later_in_closed_rooms(pkg, wl, closed, lights, bounces):
     assert launches[0] == launches[2]
 
 
+@pytest.mark.parametrize("spp,closed,tiles", [(2, True, True), (3, True, False), (3, False, True), (9, False, True), (10, False, False)])
+def test_small_renders_in_closed_rooms(pkg, wl, spp, closed, tiles):
+    """The tile launch is for at most 2^18 samples, 2^16 in a closed room; the film is the per-sample schedule's."""
+    desc, view = _room(wl, True) if closed else wl.mixed_test_scene(hdr=True, lights=True)
+    view.width, view.height = 200, 140
+    (a, sa), (b, _) = _both(pkg, desc, view, samples_per_pixel=spp, camera_bounces=5, light_bounces=2, max_path_length=6, seed=8)
+    assert np.array_equal(a, b)
+    assert (sa["trace_launches"] == 1) == tiles
+
+
 def test_batch_in_a_closed_room(pkg, wl):
     """Stream jobs, captured, whose cameras are in a room or outside: the plain renders' films."""
     b = pkg.Batch()
