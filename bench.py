@@ -564,7 +564,8 @@ def main():
             roofline["traffic_source"] = traffic_src
             roofline["measured_hbm_gbs"] = round(traffic / (dom_ms * 1e-3) / 1e9, 1)
             roofline["measured_hbm_frac"] = round(traffic / (dom_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)
-            roofline["limiter"] = "dependent node-fetch latency and lane divergence (measured HBM rate well below peak)"
+            roofline["limiter"] = ("VALU issue at half the lanes (about 0.7 of the issue cycles over a render's traversal), dependent "
+                                   "node-fetch latency in the late rounds (measured HBM rate well below peak)")
     line = {
         "metric": "BDPT paths/s (Mrays/s beside it) on 1 GPU", "value": round(paths_per_s, 1), "unit": "paths/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(elapsed / args.steps * 1e3, 3),
